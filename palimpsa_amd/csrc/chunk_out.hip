@@ -1,0 +1,400 @@
+// Chunked Palimpsa forward, outputs: chunk_out_kernel.
+//
+// From the state at the start of every tile (chunk_states.hip, or the two kernels of chunk_fwd.hip) all tiles of 64
+// tokens are worked in parallel.  Inside a tile the recurrence is run token by token on the vector units in fp32,
+//   M <- f_t M + v_t k_t^T,   I <- f_t I + b_t (k_t*k_t)^T + (1 - f_t) Ip,   o_t = scale (M / I) q_t
+// (the naive recurrence, chunk_palimpsa_forgetting_scalar.py:712-717 of the reference; its associative scan over a
+// register tile, :190-207, is what the chunked kernel of the reference does instead).
+//
+// Why not on the matrix cores: a state entry costs four plain fp32 instructions to advance (two per branch).  As prefix
+// products it costs 12 matrix instructions of 16 cycles per 16 entries of a lane plus the operands, more issue time than
+// the four, and rounds the operands.  What bounds the kernel is vector issue: per entry and token six fp32
+// instructions and one reciprocal.
+//
+// How a SIMD of gfx950 issues these (measured with one kind of instruction per wave): a wave issues one instruction per 4.3
+// cycles; two waves can issue an fp32 add / mul / fma each in the same 4 cycles, as can one of these beside an integer,
+// conversion or DPP instruction, but a reciprocal (8.3 cycles) runs with no other vector instruction, and the oldest
+// wave goes first.  So (1) a wave that reaches its reciprocals is starved by the older ones' fp32 instructions, and those
+// then run alone at half rate: the reciprocals of a token are issued as one burst at raised wave priority
+// (s_setprio; B=8 T=2048 H=12 64x64: 185 -> 161 us); (2) fp32 instructions with a scalar-register operand do not pair
+// (every operand comes from LDS into vector registers, wave-uniform ones too); (3) an odd number of waves on a
+// SIMD leaves one without a partner (two or four waves, not three: __launch registers <= 128).
+// Ideal by these rates: 6 x 2.15 + 8.3 = 21.2 cycles per entry and wave; measured 25.6 (slope over the batch size).
+// Against the earlier kernels on the matrix cores: 64x64 B=8 T=2048 H=12 250 -> 155 us, 128x128 B=2 T=4096 H=16
+// 568 -> 388, 96x96 B=8 T=2048 H=16 0.287 -> 0.202 ps per entry, fp32 rows at 64x64 570 -> 160 us (they ran split operands).
+//
+// Layout: a wave holds a block of the state, NG lanes along the key columns x 64 / NG lanes along the value rows, DN
+// columns x DD rows per lane in registers.  Blocking the registers both ways keeps the LDS traffic low (3 DN + 2 DD words
+// per DN x DD entries), and the sum over the key columns is mostly in-lane.
+#include <type_traits>
+
+#include "chunk_common.h"
+#include "pal_host.h"
+#include "pal_profile.h"
+
+namespace pal {
+
+constexpr int kOT = 8;   // tokens per staging step: two buffers of them let four workgroups of four waves share a unit's LDS
+
+// lane -> (column group, row group) of a wave; the bits of the column group are the ones the sum over the columns
+// moves along (see OutLanes::reduce)
+template <int NG>
+struct OutLanes {
+  static constexpr int DG = 64 / NG;
+  static __device__ __forceinline__ int col(int lane) {
+    if constexpr (NG == 4) return (lane >> 2) & 3;
+    else if constexpr (NG == 8) return ((lane >> 2) & 3) | ((lane & 1) << 2);
+    else return lane & (NG - 1);
+  }
+  static __device__ __forceinline__ int row(int lane) {
+    if constexpr (NG == 4) return (lane & 3) | ((lane >> 4) << 2);
+    else if constexpr (NG == 8) return ((lane >> 1) & 1) | ((lane >> 4) << 1);
+    else return lane / NG;
+  }
+  // the lanes that hold a copy of a total after the reduction
+  static __device__ __forceinline__ bool first(int lane) {
+    if constexpr (NG == 4) return true;
+    else if constexpr (NG == 8) return (lane & 1) == 0;
+    else if constexpr (NG == 16) return (lane & 3) == 0;
+    else return (lane & 19) == 0;
+  }
+  // sum over lane bits 0, 1 and 4, as far as they belong to the column group; every lane gets the total
+  static __device__ __forceinline__ float sum_other(float x) {
+    if constexpr (NG >= 8) x += dpp<0xB1>(x);    // quad_perm [1,0,3,2]
+    if constexpr (NG >= 16) x += dpp<0x4E>(x);   // quad_perm [2,3,0,1]
+    if constexpr (NG == 32) {
+      float y = x;
+      swap_rows(x, y);
+      x += y;
+    }
+    return x;
+  }
+  template <int CTRL>
+  static __device__ __forceinline__ float dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+  }
+};
+// lanes with bit 3 clear: x summed over bit 3; set: y.  (DPP with a bank mask: two instructions; the s_nop covers the
+// wait states a DPP read needs after a VALU write, which the compiler cannot see inside the assembly)
+__device__ __forceinline__ float pair_bit3(float x, float y) {
+  float r;
+  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc" : "=&v"(r) : "v"(x), "v"(y));
+  return r;
+}
+// the same for bit 2
+__device__ __forceinline__ float pair_bit2(float x, float y) {
+  float r;
+  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %2, %2 row_shr:4 row_mask:0xf bank_mask:0xa" : "=&v"(r) : "v"(x), "v"(y));
+  return r;
+}
+
+// x <- x f + c in one instruction (the compiler would copy c first and accumulate into the copy)
+__device__ __forceinline__ void fma3(float& x, float f, float c) {
+  asm("v_fma_f32 %0, %0, %1, %2" : "+v"(x) : "v"(f), "v"(c));
+}
+
+template <typename TIn>
+struct Raw4;
+template <>
+struct Raw4<bf16_t> { typedef bf16x4 type; };
+template <>
+struct Raw4<float> { typedef f32x4 type; };
+
+// pieces of a lane's DN columns: DN / 4 pieces of four, then two, then one; every piece is contiguous over the lanes
+template <int NG, int DN>
+__device__ __forceinline__ void lds_cols(const float* row, int ng, float* out) {
+  constexpr int N4 = DN / 4;
+#pragma unroll
+  for (int p = 0; p < N4; ++p) *(f32x4*)&out[4 * p] = *(const f32x4*)&row[p * NG * 4 + ng * 4];
+  if constexpr ((DN & 3) >= 2) {
+    const f32x2 x = *(const f32x2*)&row[N4 * 4 * NG + ng * 2];
+    out[4 * N4] = x[0]; out[4 * N4 + 1] = x[1];
+  }
+  if constexpr (DN & 1) out[DN - 1] = row[(DN - 1) * NG + ng];
+}
+template <int NG, int DN>
+__device__ __forceinline__ constexpr int col_of(int i, int ng) {
+  constexpr int N4 = DN / 4;
+  if (i < 4 * N4) return (i / 4) * NG * 4 + ng * 4 + i % 4;
+  if ((DN & 3) >= 2 && i < 4 * N4 + 2) return 4 * N4 * NG + ng * 2 + (i - 4 * N4);
+  return (DN - 1) * NG + ng;
+}
+template <int DD>
+__device__ __forceinline__ void lds_rows(const float* p, float* out) {
+  if constexpr (DD % 4 == 0) {
+#pragma unroll
+    for (int x = 0; x < DD / 4; ++x) *(f32x4*)&out[4 * x] = *(const f32x4*)&p[4 * x];
+  } else if constexpr (DD % 2 == 0) {
+#pragma unroll
+    for (int x = 0; x < DD / 2; ++x) {
+      const f32x2 y = *(const f32x2*)&p[2 * x];
+      out[2 * x] = y[0]; out[2 * x + 1] = y[1];
+    }
+  } else {
+#pragma unroll
+    for (int x = 0; x < DD; ++x) out[x] = p[x];
+  }
+}
+
+// a lane's operands of one token
+template <int NG, int DN, int DD>
+struct OutRow {
+  float k[DN], kk[DN], q[DN], vb[2 * DD];
+  f32x2 fc;
+  __device__ __forceinline__ void load(const float* row, int ng, int d0) {
+    constexpr int DKP = NG * DN;
+    fc = *(const f32x2*)row;
+    lds_cols<NG, DN>(row + 4, ng, k);
+    lds_cols<NG, DN>(row + 4 + DKP, ng, kk);
+    lds_rows<2 * DD>(row + 4 + 3 * DKP + 2 * d0, vb);
+    lds_cols<NG, DN>(row + 4 + 2 * DKP, ng, q);
+  }
+};
+
+template <typename TIn, int NG, int DN, int DD, bool HAS_VAR>
+__global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(HAS_VAR ? 2 : 4)))
+void chunk_out_kernel(ChunkArgs a, int W) {
+  extern __shared__ float smem[];
+  typedef typename Raw4<TIn>::type raw4;
+  constexpr int DKP = NG * DN;              // key columns of the lanes (dk, or up to 16 more that stay zero)
+  constexpr int ROWS = (64 / NG) * DD;      // value rows of a wave
+  constexpr int TU = 4 / DD;                // tokens per iteration
+  const int NT = W * 64, VR = W * ROWS;     // threads and value rows of the workgroup
+  constexpr int oK = 4, oKK = oK + DKP, oQ = oKK + DKP, oVB = oQ + DKP;
+  const int STRIDE = oVB + 2 * VR;          // floats per staged token: f, c, -, -, k, k*k, q, (v, b) of every row
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int H = a.H, dk = a.dk, dv = a.dv;
+  const int cidx = (int)(blockIdx.x / H), h = (int)(blockIdx.x % H);
+  const int r0 = (int)blockIdx.y * VR;
+  int seq, t0, clen, cis;
+  chunk_lookup(a, cidx, seq, t0, clen, cis);
+  float* sFC = smem;                        // [64][2] f_t, (1 - f_t) Ip
+  float* sRow = sFC + 2 * kC;               // [2][kOT][STRIDE]
+  const float Ip = a.Ip[h];
+  // every fetch of the set-up is issued before the first is used
+  const float gt = (w == 0 && lane < clen) ? load_gate(a.gt, (int64_t)(t0 + lane) * H + h, a.gate_bf16) : 0.f;
+  const float gh = a.g[h] * kLog2e;
+  const TIn* kp = (const TIn*)a.k + qk_row(a, t0, h);
+  const TIn* qp = (const TIn*)a.q + qk_row(a, t0, h);
+  const TIn* vp = (const TIn*)a.v + ((int64_t)t0 * H + h) * dv + r0;
+  const TIn* bp = (const TIn*)a.b + ((int64_t)t0 * H + h) * dv + r0;
+  const int qs = (int)qk_stride(a), vs = H * dv;
+  // staging items: (token, four columns) of k and q, (token, four rows) of v and b
+  const int nk4 = dk >> 2, nv4 = min(VR, dv - r0) >> 2;
+  raw4 rk, rq, rv, rb;
+  const int s_kq = tid / nk4, c_kq = tid - s_kq * nk4, s_vb = tid / nv4, c_vb = tid - s_vb * nv4;
+  auto fetch = [&](int s0) {
+    if (s_kq < kOT && s0 + s_kq < clen) {
+      rk = *(const raw4*)(kp + (int64_t)(s0 + s_kq) * qs + 4 * c_kq);
+      rq = *(const raw4*)(qp + (int64_t)(s0 + s_kq) * qs + 4 * c_kq);
+    }
+    if (s_vb < kOT && s0 + s_vb < clen) {
+      rv = *(const raw4*)(vp + (int64_t)(s0 + s_vb) * vs + 4 * c_vb);
+      rb = *(const raw4*)(bp + (int64_t)(s0 + s_vb) * vs + 4 * c_vb);
+    }
+  };
+  auto put_kq = [&](float* row, int c, raw4 k4, raw4 q4) {
+    f32x4 x, xx, y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { x[e] = (float)k4[e]; xx[e] = x[e] * x[e]; y[e] = (float)q4[e]; }
+    *(f32x4*)&row[oK + 4 * c] = x;
+    *(f32x4*)&row[oKK + 4 * c] = xx;
+    *(f32x4*)&row[oQ + 4 * c] = y;
+  };
+  auto deposit = [&](int s0, int buf) {
+    float* base = sRow + buf * kOT * STRIDE;
+    if (tid < kOT) *(f32x2*)&base[tid * STRIDE] = *(const f32x2*)&sFC[2 * (s0 + tid)];   // s0 + tid < 64
+    if (s_kq < kOT && s0 + s_kq < clen) put_kq(base + s_kq * STRIDE, c_kq, rk, rq);
+    if (s_vb < kOT && s0 + s_vb < clen) {
+      float* p = &base[s_vb * STRIDE + oVB + 8 * c_vb];
+      *(f32x4*)p = f32x4{(float)rv[0], (float)rb[0], (float)rv[1], (float)rb[1]};
+      *(f32x4*)(p + 4) = f32x4{(float)rv[2], (float)rb[2], (float)rv[3], (float)rb[3]};
+    }
+    // wide keys on few waves: the items of k, q beyond the fetched ones
+    for (int idx = tid + NT; idx < kOT * nk4; idx += NT) {
+      const int s = idx / nk4, c = idx - s * nk4;
+      if (s0 + s < clen)
+        put_kq(base + s * STRIDE, c, *(const raw4*)(kp + (int64_t)(s0 + s) * qs + 4 * c),
+               *(const raw4*)(qp + (int64_t)(s0 + s) * qs + 4 * c));
+    }
+  };
+  fetch(0);
+  const int ng = OutLanes<NG>::col(lane), dg = OutLanes<NG>::row(lane);
+  const int d0 = w * ROWS + dg * DD;        // first value row of the lane inside the workgroup
+  float M[DD][DN], I[DD][DN];
+  {
+    const float* mu = a.chunk_mu + (((int64_t)cidx * H + h) * dv + r0) * dk;
+    const float* Is = a.chunk_I + (((int64_t)cidx * H + h) * dv + r0) * dk;
+#pragma unroll
+    for (int j = 0; j < DD; ++j) {
+      const bool on = r0 + d0 + j < dv;
+      const int64_t ro = (int64_t)(on ? d0 + j : 0) * dk;
+      auto piece = [&](auto width, int i) {
+        constexpr int VW = decltype(width)::value;
+        const int c = col_of<NG, DN>(i, ng);
+        float x[VW], y[VW];
+        const bool in = DKP == 0 || c < dk;
+        load_vec<VW>(mu + ro + (in ? c : 0), x);
+        load_vec<VW>(Is + ro + (in ? c : 0), y);
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+          M[j][i + e] = on && in ? x[e] * y[e] : 0.f;
+          I[j][i + e] = on && in ? y[e] : 1.f;
+        }
+      };
+#pragma unroll
+      for (int p = 0; p < DN / 4; ++p) piece(std::integral_constant<int, 4>{}, 4 * p);
+      if constexpr ((DN & 3) >= 2) piece(std::integral_constant<int, 2>{}, 4 * (DN / 4));
+      if constexpr (DN & 1) piece(std::integral_constant<int, 1>{}, DN - 1);
+    }
+  }
+  if (w == 0) {
+    const float f = fast_exp2(-gt * gh);
+    *(f32x2*)&sFC[2 * lane] = f32x2{f, (1.f - f) * Ip};
+  }
+  // rows and columns beyond the head dims stay zero in both buffers
+  if (DKP != dk || VR > dv - r0) {
+    for (int idx = tid; idx < 2 * kOT * STRIDE; idx += NT) sRow[idx] = 0.f;
+  }
+  __syncthreads();
+  deposit(0, 0);
+  __syncthreads();
+
+  // The totals of DD rows x TU tokens are reduced together: four values, of which lane bits 3 and 2 select one
+  const int sel = 2 * ((lane >> 3) & 1) + ((lane >> 2) & 1);
+  const int dsel = sel % DD, tsel = sel / DD;
+  const bool writer = OutLanes<NG>::first(lane) && r0 + d0 + dsel < dv;
+  auto reduce = [&](const float* x) {
+    return OutLanes<NG>::sum_other(pair_bit2(pair_bit3(x[0], x[2]), pair_bit3(x[1], x[3])));
+  };
+  const int64_t orow = ((int64_t)t0 * H + h) * dv + r0 + d0 + dsel;
+
+  OutRow<NG, DN, DD> x;
+  for (int s0 = 0; s0 < clen; s0 += kOT) {
+    const int buf = (s0 / kOT) & 1;
+    const bool more = s0 + kOT < clen;
+    if (more) fetch(s0 + kOT);
+    const int nt = min(kOT, clen - s0);
+    const float* row = sRow + buf * kOT * STRIDE;
+    x.load(row, ng, d0);
+#pragma unroll 1
+    for (int tt = 0; tt < nt; tt += TU, row += TU * STRIDE) {
+      float acc[4], accv[4];
+#pragma unroll
+      for (int u = 0; u < TU; ++u) {
+        float r[DD][DN], qc[DN];
+#pragma unroll
+        for (int i = 0; i < DN; ++i) {
+#pragma unroll
+          for (int j = 0; j < DD; ++j) {
+            M[j][i] = fmaf(x.vb[2 * j], x.k[i], M[j][i] * x.fc[0]);
+            fma3(I[j][i], x.fc[0], x.fc[1]);
+            I[j][i] = fmaf(x.vb[2 * j + 1], x.kk[i], I[j][i]);
+          }
+          qc[i] = x.q[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the next token's operands are requested here: the burst of reciprocals hides their latency (after the last
+        // token of a step: rows of the other buffer or, at its end, not yet written; they are read again below)
+        x.load(row + (u + 1) * STRIDE, ng, d0);
+        __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+        for (int i = 0; i < DN; ++i)
+#pragma unroll
+          for (int j = 0; j < DD; ++j) r[j][i] = fast_rcp(I[j][i]);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < DD; ++j) { acc[u * DD + j] = 0.f; accv[u * DD + j] = 0.f; }
+#pragma unroll
+        for (int i = 0; i < DN; ++i)
+#pragma unroll
+          for (int j = 0; j < DD; ++j) {
+            float& y = acc[u * DD + j];
+            y = fmaf(M[j][i] * r[j][i], qc[i], y);
+            if constexpr (HAS_VAR) accv[u * DD + j] = fmaf(qc[i] * qc[i], r[j][i], accv[u * DD + j]);
+          }
+      }
+      const int t = s0 + tt + tsel;
+      const bool wr = writer && t < clen;
+      const int64_t oo = orow + (int64_t)t * vs;
+      const float out = reduce(acc);
+      if (wr) ((TIn*)a.o)[oo] = from_f32<TIn>(out * a.scale);
+      if constexpr (HAS_VAR) {
+        const float outv = reduce(accv);
+        if (wr) store_rt(a.o_var, oo, outv * a.scale, a.var_bf16);
+      }
+    }
+    if (more) deposit(s0 + kOT, buf ^ 1);
+    __syncthreads();
+  }
+}
+
+// Waves per workgroup for nw waves of value rows: the hardware deals the waves of a workgroup out to the four SIMDs in
+// order, so four (or two) to a workgroup load them evenly and five or six do not (96x96, twelve waves: 0.202 ps per
+// entry in workgroups of four, 0.225 in threes, 0.26 in sixes; 48x96, six waves: 0.207 in twos, 0.224 in threes, 0.26 in one
+// six; 80x80, ten waves: 0.257 in twos, 0.35 in fives).
+static int out_waves(int nw) {
+  if (nw <= 4) return nw;
+  if (nw % 4 == 0) return 4;
+  if (nw % 2 == 0) return 2;
+  return nw % 4 == 3 ? 4 : 3;
+}
+
+template <typename TIn, int NG, int DN, int DD>
+static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
+  constexpr int ROWS = (64 / NG) * DD;
+  static_assert(ROWS <= 32, "one staging item of v, b per thread");
+  const int nw = (a.dv + ROWS - 1) / ROWS;            // waves over the value rows
+  const int W = out_waves(nw), slices = (nw + W - 1) / W;
+  const int64_t blocks = (int64_t)a.total_chunks * a.H;
+  if (blocks > 0x7fffffff) return PAL_E_DIM;
+  const size_t lds = sizeof(float) * (2 * kC + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
+  if (lds > kMaxLds) return PAL_E_HEADDIM;
+  auto go = [&](auto kern) -> int {
+    if (int rc = allow_lds((const void*)kern, lds)) return rc;
+    PAL_TIMED_LAUNCH(kKernChunkOut, s, kern, dim3((unsigned)blocks, (unsigned)slices), dim3(64 * W), lds, s, a, W);
+    return 0;
+  };
+  const int rc = (a.flags & PAL_FLAG_HAS_VAR) ? go(&chunk_out_kernel<TIn, NG, DN, DD, true>) : go(&chunk_out_kernel<TIn, NG, DN, DD, false>);
+  if (rc) return rc;
+  PAL_HIP_LAUNCH_CHECK();
+  return PAL_OK;
+}
+
+template <typename TIn, int NG, int DN>
+static int launch_out_dn(const ChunkArgs& a, hipStream_t s) {
+  // Two value rows per lane where that still gives every SIMD two waves; below, one row: half the work per wave and
+  // twice the waves (one sequence of 777 tokens, 16 heads of 64x64: 28 us with two rows, 23 with one; B=2 T=2048 H=12 64x64,
+  // three waves per SIMD: 49.6 against 51.0).
+  const int64_t waves = (int64_t)a.total_chunks * a.H * ((a.dv * NG + 127) / 128);
+  if (waves <= 2048) return launch_out_dd<TIn, NG, DN, 1>(a, s);
+  return launch_out_dd<TIn, NG, DN, 2>(a, s);
+}
+
+template <typename TIn>
+static int launch_out_t(const ChunkArgs& a, hipStream_t s) {
+  switch ((a.dk + 15) / 16) {
+    case 1: return launch_out_dn<TIn, 4, 4>(a, s);
+    case 2: return launch_out_dn<TIn, 4, 8>(a, s);
+    case 3: return launch_out_dn<TIn, 8, 6>(a, s);
+    case 4: return launch_out_dn<TIn, 8, 8>(a, s);
+    case 5: return launch_out_dn<TIn, 16, 5>(a, s);
+    case 6: return launch_out_dn<TIn, 16, 6>(a, s);
+    case 7: return launch_out_dn<TIn, 16, 7>(a, s);
+    case 8: return launch_out_dn<TIn, 16, 8>(a, s);
+    case 9: case 10: return launch_out_dn<TIn, 32, 5>(a, s);
+    case 11: case 12: return launch_out_dn<TIn, 32, 6>(a, s);
+    case 13: case 14: return launch_out_dn<TIn, 32, 7>(a, s);
+    case 15: case 16: return launch_out_dn<TIn, 32, 8>(a, s);
+    default: return PAL_E_HEADDIM;
+  }
+}
+
+int launch_out(const ChunkArgs& a, int dtype, hipStream_t s) {
+  return dtype == PAL_DTYPE_BF16 ? launch_out_t<bf16_t>(a, s) : launch_out_t<float>(a, s);
+}
+
+}  // namespace pal
