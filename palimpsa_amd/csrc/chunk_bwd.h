@@ -1,0 +1,80 @@
+// Pieces shared by the kernels of the chunked backward (chunk_bwd.hip, chunk_bwd_tile.hip).
+#pragma once
+#include "chunk_common.h"
+
+namespace pal {
+
+struct BwdArgs {
+  ChunkArgs c;
+  const void *d_o, *d_o_var;
+  void *dq, *dk, *dv, *db;
+  float *dgt, *dg, *dIp, *d_init_mu, *d_init_I;
+  void *wDM, *wDJ;        // [total_chunks,H,dv,dk] local carries, then incoming carries, in the dtype of the rows
+  float* wFtot;           // [total_chunks,H] log2 of the total decay of a tile
+  float* wSig;            // [total_chunks,H] sum over the tile of dJloc
+  float* wE;              // [H, tokens]  local part of d log f
+  float* wInitPart;       // [n_seqs,H,dv*dk/256] partial sums of dJ_0
+  float* wDgTile;         // [total_chunks,H] the tiles' shares of dg
+  float* wQK;             // [tokens,H,2,dk] dq, dk summed so far, where a tile takes several slices of value rows (bf16 rows)
+  int32_t tokens;
+  int32_t apply_alias;     // carry apply: db^carry shares LDS with the bf16 carries (large head dims)
+};
+
+// A launch of the tile kernel covers a rectangle of the state: `cols` key columns from n0 on, and value rows from r0 on.
+// Larger heads take several: groups of 64, 48 or 32 key columns (16 for a head of 16), in each of them slices of 64, 48,
+// 32 or 16 value rows.  (96 columns as 64 + 32, 80 as 48 + 32: workgroups of four or two waves, two or four of them to a
+// compute unit.  One workgroup of eight waves has nothing to fill its barriers and its set-up with: 96x96, 32768 packed
+// tokens, 16 heads: 5.5 ms, as rectangles 4.2.  A rectangle costs, in ps per state entry and token at B=8 T=2048 H=16, 0.77
+// (64x64: columns x rows), 0.86 (64x48), 0.87 (64x32), 0.98 (48x64), 1.00 (48x48), 1.12 (48x32), 1.06 (32x64), 0.99 (32x48,
+// 32x32), 1.8 (16x16): hence 96 rows as 48 + 48, where neither piece pays for a small one.)
+struct TileRect {
+  int n0, cols, r0, flags;
+};
+constexpr int kRectColsBefore = 1, kRectRowsBefore = 2, kRectRowsAfter = 4;   // launches that came before, come after
+inline int tile_piece(int n) { return n == 80 ? 48 : n >= 64 ? 64 : n; }
+inline int tile_rows(int cols, int n) { return cols == 16 ? (n >= 48 ? 48 : 16) : n == 96 ? 48 : tile_piece(n); }   // (16 columns: one wave's staging)
+
+constexpr int kHalf = 32;          // tokens of a half tile: the contraction length of one matrix instruction
+constexpr int kHS = kHalf + 8;     // row stride (bf16) of the transposed half tiles: 16-byte reads stay aligned
+
+// tokens per step for DT x DN state entries per lane: mu and 1 / I of a step stay in registers
+__host__ __device__ constexpr int tile_g(int DT, int DN) { return DT * DN <= 9 ? 8 : 4; }
+__host__ __device__ constexpr int rows_pad(int DT) { return DT == 3 ? 4 : DT; }
+__host__ __device__ constexpr int vb_stride(int DT, bool var) { return (var ? 4 : 3) * 16 * rows_pad(DT) + 4; }
+
+// LDS (floats): running decay, (f, (1 - f) Ip) per token, decay weights of every step's state, their factors of the
+// base state, X_t, partial (S, X); base states; transposed v, b of both halves (of one, and the first half's in the
+// partial sums' memory at the start, where that lets two workgroups share a compute unit); two buffers of staged rows
+// and of partial dv, db
+struct TileLds {
+  int oFC, oW, oFB, oX, oXS, oBase, oT, oKQ, oVB, oPart, both, total;
+};
+__host__ __device__ constexpr TileLds tile_lds(int DT, int DN, int nbw, bool var, bool f32) {
+  TileLds L = {};
+  const int G = tile_g(DT, DN), half = (f32 ? 2 : 1) * 16 * DT * kHS;   // (two tensors of bf16)
+  for (int both = 1; both >= 0; --both) {
+    int o = kC;
+    L.oFC = o; o += 2 * (kC + 2);
+    L.oW = o; o += (kC / G + 1) * kHalf;
+    L.oFB = o; o += kC / G + 4;
+    L.oX = o; o += kC;
+    L.oXS = o; o += 2 * nbw * 2 * G;
+    o = (o + 3) & ~3;
+    L.oBase = o; o += nbw * 2 * DT * 64 * 4;
+    L.oT = o; o += (both ? 2 : 1) * half;
+    L.oKQ = o; o += 2 * nbw * G * 32;
+    L.oVB = o; o += 2 * G * vb_stride(DT, var);
+    const int part = 2 * nbw * G * 32 * DT;
+    L.oPart = o; o += both || part > half ? part : half;
+    L.both = both;
+    L.total = o;
+    const int fit = 160 * 1024 / 4 / (nbw > 2 ? 2 : 4);
+    if (o <= fit) break;
+  }
+  return L;
+}
+
+template <typename TIn, bool VAR>
+int launch_tile_t(const BwdArgs& A, hipStream_t s);   // chunk_bwd_tile_*.hip
+
+}  // namespace pal

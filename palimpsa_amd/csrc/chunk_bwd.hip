@@ -9,21 +9,15 @@
 // (:360-384).  All tiles of 64 tokens are processed in parallel; what crosses a
 // tile boundary is handled by two small extra passes (scan, apply); the gate gradient is finished in the second:
 //
-//  local   per (tile, head): recompute M_t, I_t from the tile-start state (as the
-//          forward does), form dMloc/dJloc, dq; feed them straight from the MFMA
-//          accumulators into the reverse contraction dM^loc = L^T dMloc (k index =
-//          token, so accumulator registers are already in operand layout); from it
-//          the tile-local parts of dv, db, dk and the carry the tile hands to its
-//          predecessor, R_loc = f_first * dM^loc_first.
+//  local   per (tile, head): chunk_bwd_tile.hip -- dq, the tile's own parts of dv, db, dk and of the gate gradient, and
+//          the carry the tile hands to its predecessor, R_loc = f_first * dM^loc_first.
 //  scan    per state entry: R_{c-1} = R_loc,c + F_C,c R_c backwards over the tiles
 //          of a sequence (the role of curr_dM/curr_dI, :429-430); also yields the
 //          gradients of the initial state.
 //  apply   per (tile, head): adds the carry terms a_s R k_s etc. to dv, db, dk
 //          with four small MFMA products.
-//  gate    d log f_s = <dM_s, f_s M_{s-1}> + <dJ_s, f_s J_{s-1}>, evaluated without any
-//          cancellation (the reference un-shifts the state by dividing by f, :409-412):
-//            local part   gamma_s = <dM^loc_s, S_s> + <dJ^loc_s, S^J_s>, S_s = f_s M_{s-1} from a
-//                         strictly-lower-triangular MFMA product in the layout of dM^loc;
+//  gate    d log f_s = <dM_s, f_s M_{s-1}> + <dJ_s, f_s J_{s-1}>:
+//            local part   gamma_s of the tile kernel;
 //            carry part   sum_{r<s, r in tile} beta_r + F_C (<R_M, M_0> + <R_J, J_0>), with
 //                         beta_r = <v_r, dv^carry_r> + <b_r, db^carry_r> from the apply pass and
 //                         (M_0, J_0) the state at the start of the tile.
@@ -32,627 +26,13 @@
 //          a last small kernel sums the shares per head.
 #include <type_traits>
 
-#include "chunk_common.h"
+#include "chunk_bwd.h"
 #include "pal_host.h"
 #include "pal_profile.h"
 
 namespace pal {
 
 void fill_chunk_args(ChunkArgs& a, const PalDims* d, const PalFwdTensors* t);
-
-struct BwdArgs {
-  ChunkArgs c;
-  const void *d_o, *d_o_var;
-  void *dq, *dk, *dv, *db;
-  float *dgt, *dg, *dIp, *d_init_mu, *d_init_I;
-  void *wDM, *wDJ;        // [total_chunks,H,dv,dk] local carries, then incoming carries, in the dtype of the rows
-  float* wFtot;           // [total_chunks,H] log2 of the total decay of a tile
-  float* wSig;            // [total_chunks,H] sum over the tile of dJloc
-  float* wE;              // [H, tokens]  local part of d log f
-  float* wInitPart;       // [n_seqs,H,dv*dk/256] partial sums of dJ_0
-  float* wDgTile;         // [total_chunks,H] the tiles' shares of dg
-  int32_t tokens;
-  int32_t apply_alias;     // carry apply: db^carry shares LDS with the bf16 carries (large head dims)
-};
-
-constexpr int kVS2 = 68;
-// local pass: rows the consumers run behind the first producer (the second producer runs one row behind it)
-constexpr int kLagC = 2;
-// value rows staged at a time: 8 with two column blocks per workgroup, so that two such workgroups fit a compute unit's LDS
-__host__ __device__ constexpr int local_dg(int NB, bool prec) { return (!prec && NB == 2) ? 8 : 16; }
-
-
-// ------------------------------------------------- local pass, four wave roles
-// One workgroup per (tile, head).  For every value row d the tile recomputes M_t, I_t for its 64 tokens
-// (orientation [t, n]), forms dMloc/dJloc and dq, contracts them backwards in time (dM^loc[n, s]) and
-// runs the dv/db/dk/gate epilogue on the result.
-// Organised for four waves per SIMD: one wave issues a VALU instruction every 5-9 cycles at best while
-// the SIMD can start one every 2-3, so the work on a block of 16 key columns is cut into four roles
-// small enough for 128 registers each.  A workgroup has 4*NB waves; wave = role*NB + (column block).
-//   roles 0/1 ("producers", tokens 0..31 / 32..63): recompute the states of one value row for 16 key
-//     columns, form dMloc/dJloc and dq, and leave packed bf16 operands P^M, P^J (local gradients) and X^M, X^J
-//     (rank-one updates) of their half of the tile in an LDS slot;
-//   roles 2/3 ("consumers", column tokens s in 0..31 / 32..63): pick their half's slot up two iterations after the
-//     first producer wrote its own and do the reverse contraction, the strictly-lower product and the
-//     dv/db/dk/gate epilogue.
-// Every role has its own loop (its own register allocation) with the same sequence of barriers.
-// The tile is worked as two halves of 32 tokens coupled through LDS (see the producers).
-// NB <= 4 column blocks are in flight at a time (16 waves); a wider head dim takes several passes over
-// the tile, the later ones adding their dv/db/gate contributions to those of the earlier ones.
-// PREC (fp32 rows): every operand is carried as two bf16 halves and every product takes three matrix instructions
-// (split_bf16 / mfma16_split); the LDS slots hold twice the operands and a wave may use 256 registers
-// (two waves per SIMD), so at most 2 column blocks are in flight.
-// Three column blocks (dk = 48) are 12 waves, three per SIMD and one workgroup per compute unit (its LDS): that
-// instance may use 168 registers.
-template <typename TIn, int NB, bool HAS_VAR, bool MULTI, bool PREC>
-__global__ __launch_bounds__(4 * NB * 64) __attribute__((amdgpu_waves_per_eu(PREC ? 2 : (NB == 3 ? 3 : 4))))
-void chunk_bwd_local_roles_kernel(BwdArgs A) {
-  const ChunkArgs& a = A.c;
-  extern __shared__ float smem[];
-  constexpr int NST = HAS_VAR ? 4 : 3;  // staged tensors: v, b, do, (dovar)
-  constexpr int DG = local_dg(NB, PREC);   // value rows per staging group
-  constexpr int STG = DG * kVS2;
-  float* sC = smem;                      // [64] running log2 decay
-  float* sF = sC + kC;                   // [64] decay from before the half of the tile: 2^c_t (t < 32), 2^(c_t - c_31)
-  float* sSt = sF + kC;                  // [2][NST][DG][kVS2]
-  float* sPv = sSt + 2 * NST * STG;      // [NB][DG][64] per-wave partial dv
-  float* sPb = sPv + NB * DG * kC;       // [NB][DG][64] per-wave partial db
-  // The second producer runs one value row behind the first (it takes the state after token 31 from it), the
-  // consumers follow two rows behind.  The first producer's half of a slot is then alive for three rows, the second
-  // one's for two:
-  //   sX  [NB][3 x {P^M_0, P^J_0, X^M_0, X^J_0} | 2 x {P^M_1, P^J_1, X^M_1, X^J_1}][64 lanes]
-  //       (PREC: each group of four is followed by its four lo halves),
-  //   sMJ [NB][3 slots][M_0, J_0, M_31, J_31, what flows back over token 31 (M, J)][16]   (see the producers).
-  float* sMJ = sPb + NB * DG * kC;
-  constexpr int XS = PREC ? 2 : 1;
-  bf16x8* sX = (bf16x8*)(sMJ + NB * 288);
-  // [NB][DG rows][4][M 0..3, J 0..3] first column of dM^loc, dJ^loc of a group of value rows (the carry to the previous tile)
-  float* sCar = (float*)(sX + NB * 20 * XS * 64);
-  // [NB][64] d log f partials of the consumer waves, then [2 NB] sums of dJloc: written after the last row of a pass,
-  // when the operand slots are dead, so they share their memory
-  float* sRed = (float*)sX;
-  const int tid = threadIdx.x;
-  int lane = tid & 63, i = lane & 15, g = lane >> 4;   // re-derived per pass from an opaque copy, see below
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: role branches are scalar
-  const int role = wave / NB, nbl = wave - role * NB;   // nbl: column block inside the current group
-  const int H = a.H, dk = a.dk, dv = a.dv;
-  // NB blocks of 16 key columns are handled at a time; wider heads take several passes over the tile
-  const int nb_total = dk >> 4, n_pass = MULTI ? (nb_total + NB - 1) / NB : 1;   // MULTI = false: dk == 16*NB
-  const int cidx = blockIdx.x / H, h = blockIdx.x % H;
-  int seq, t0, clen, cis;
-  chunk_lookup(a, cidx, seq, t0, clen, cis);
-  const float Ip = a.Ip[h];
-  const float gh = a.g[h] * kLog2e;
-  const float scale = a.scale;
-  const bool fold = !PREC && a.init_mu == nullptr;
-
-  if (wave == 0) {
-    const float gt = (lane < clen) ? load_gate(a.gt, (int64_t)(t0 + lane) * H + h, a.gate_bf16) : 0.f;
-    const float c = wave_inclusive_scan(-gt * gh, lane);
-    sC[lane] = c;
-    const float c31 = __shfl(c, 31);   // every lane takes part: not inside the conditional
-    sF[lane] = fast_exp2(lane >= 32 ? c - c31 : c);
-    if (lane == 63) A.wFtot[(int64_t)cidx * H + h] = c;
-  }
-  // Global addresses are kept as a wave-uniform base plus a 32-bit lane offset, so that the
-  // loop-invariant parts live in scalar registers.
-  // Staging of DG value rows x 64 tokens (v, b, do, dovar) and the dv/db flush: threads 0..16 DG - 1,
-  // thread = (token s, quad of rows q4).
-  const int64_t row0 = ((int64_t)t0 * H + h) * dv;
-  const TIn* vp = (const TIn*)a.v + row0;
-  const TIn* bp = (const TIn*)a.b + row0;
-  const TIn* dop = (const TIn*)A.d_o + row0;
-  const int st_s = tid / (DG / 4), st_q = tid % (DG / 4);
-  const bool st_on = tid < kC * DG / 4;
-  const unsigned st_off = (unsigned)(st_s * H * dv + 4 * st_q);
-  auto stage = [&](int dg) {
-    if (!st_on) return;
-    float st[NST][4];
-    // the lane offset is made opaque here so that no per-lane 64-bit address is kept across the loop
-    unsigned off = st_off;
-    asm volatile("" : "+v"(off));
-    if (st_s < clen) {
-      load_vec<4>(vp + dg * DG + off, st[0]);
-      load_vec<4>(bp + dg * DG + off, st[1]);
-      load_vec<4>(dop + dg * DG + off, st[2]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[2][e] *= scale;
-      if (HAS_VAR) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st[NST - 1][e] = scale * load_rt(A.d_o_var, row0 + dg * DG + off + e, a.var_bf16);
-      }
-    } else {
-#pragma unroll
-      for (int x = 0; x < NST; ++x)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st[x][e] = 0.f;
-    }
-    const int buf = dg & 1;
-#pragma unroll
-    for (int x = 0; x < NST; ++x)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sSt[((buf * NST + x) * DG + 4 * st_q + e) * kVS2 + st_s] = st[x][e];
-  };
-  const int64_t rs = qk_stride(a);      // token stride of q, k
-  const int64_t rso = (int64_t)H * dk;  // token stride of dq, dk (one row per value head)
-  const int64_t tile_off = (((int64_t)cidx * H + h) * dv) * dk;
-  const int n_groups = dv / DG;
-  int pass = 0, nb = nbl, n_act = NB;   // set per pass: global column block of this wave, active blocks
-
-  // end of one iteration, identical for every role: stage the next group of DG value rows mid-group
-  // into the other buffer, synchronise, and flush dv/db once the consumers have finished a group
-  auto iter_tail = [&](int it) {
-    if ((it & (DG - 1)) == DG / 2 && it / DG + 1 < n_groups) stage(it / DG + 1);
-    __syncthreads();
-    if (it >= kLagC && ((it - kLagC) & (DG - 1)) == DG - 1) {
-      const int dg = (it - kLagC) / DG;
-      if (st_on && st_s < clen) {
-        unsigned off = st_off;
-        asm volatile("" : "+v"(off));
-        TIn* dvo = (TIn*)A.dv + row0 + dg * DG + off;
-        TIn* dbo = (TIn*)A.db + row0 + dg * DG + off;
-        float sv[4] = {0.f, 0.f, 0.f, 0.f}, sb_[4] = {0.f, 0.f, 0.f, 0.f};
-        if (MULTI && pass > 0) {   // later passes add to what the earlier column groups left
-          load_vec<4>(dvo, sv);
-          load_vec<4>(dbo, sb_);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-#pragma unroll
-          for (int w = 0; w < NB; ++w) {
-            if (!MULTI || w < n_act) {
-              sv[e] += sPv[(w * DG + 4 * st_q + e) * kC + st_s];
-              sb_[e] += sPb[(w * DG + 4 * st_q + e) * kC + st_s];
-            }
-          }
-        }
-        store_vec<4>(dvo, sv);
-        store_vec<4>(dbo, sb_);
-      }
-      // carry handed to the previous tile, f_first * dM^loc at the first token: thread = (column block, row, quad of columns)
-      if (tid < n_act * DG * 4) {
-        const int w = tid / (DG * 4), row = (tid >> 2) & (DG - 1), q4 = tid & 3;
-        const float f_first = fast_exp2(sC[0]);
-        const f32x4 cm = *(const f32x4*)&sCar[tid * 8], cj = *(const f32x4*)&sCar[tid * 8 + 4];
-        const float rm[4] = {f_first * cm[0], f_first * cm[1], f_first * cm[2], f_first * cm[3]};
-        const float rj[4] = {f_first * cj[0], f_first * cj[1], f_first * cj[2], f_first * cj[3]};
-        const int64_t co = tile_off + (int64_t)(dg * DG + row) * dk + 16 * (pass * NB + w) + 4 * q4;
-        store_vec<4>((TIn*)A.wDM + co, rm);
-        store_vec<4>((TIn*)A.wDJ + co, rj);
-      }
-      __syncthreads();
-    }
-  };
-
-  // ------------------------------------------------------------------ the tile as two halves of 32 tokens
-  // A causal product over 64 tokens costs 6 matrix instructions per 16 columns (token blocks of 16 against
-  // K = 16, 32, 48, 64, padded to multiples of 32), over two halves of 32 tokens 4: the second half starts from the
-  // state after token 31, which the first producer has in its accumulators and leaves in sMJ for the second one, a
-  // row behind.  The reverse contraction of the first half needs what flows back over the border,
-  // f_32 dM^loc_32 = sum_{t >= 32} 2^(c_t - c_31) dMloc_t: the second producer sums it from its local gradients and
-  // the first consumer adds it to the local gradient of token 31 in its operand.  The two producers are then the
-  // same code on tokens 0..31 and 32..63 and each consumer reads only its own half's operands: 24 matrix
-  // instructions (PREC: 72) and 16 KB of LDS traffic per value row and column block.
-  //   sMJ slot of a row (d mod 3): [M_0, J_0, M_31, J_31, f_32 dM^loc_32, f_32 dJ^loc_32][16 key columns]
-  // How the state before a half (M_p, J_p) enters its products:
-  //   FOLD (bf16 operands, no initial state): it rides in the operand of the half's first token,
-  //     X'_first = X_first + f_first (M_p, J_p), since the decay from before the half to token t is L[t,first] f_first;
-  //     the strictly-lower product gets it for the first token itself as a virtual token in its last contraction slot
-  //     (token 31 / 63, which is never below a column token of the half).  The state is rounded to bf16 there like
-  //     every other operand; a J_0 below zero (an initial state with I_0 < Ip) would cancel against Ip, so launches
-  //     with an initial state take the next form;
-  //   else in fp32: M_t = Fh_t M_p + (product), with Fh_t = sF[t] the decay from before the half; the strictly-lower
-  //     product of bf16 operands takes Fh_s M_p through the virtual token (on every column), that of split
-  //     operands (PREC) adds it in fp32.
-  auto producer = [&](auto hfc, auto foldc) {
-    constexpr int HF = decltype(hfc)::value;   // tokens 32HF .. 32HF+31
-    constexpr bool FOLD = decltype(foldc)::value;
-    bf16x8 Lop[2];            // L[t,s] inside the half: t = 32HF+16tl+i, s = 32HF+8g+j <= t
-    bf16x8 Lol[PREC ? 2 : 1]; // PREC: its lo halves
-    float kk[8], kk2[8];      // k and its square in operand layout (n = i, s = 32HF+8g+j)
-    float qq[8];              // q in result layout (t = 32HF+16tl+4g+r, n = i)
-    float dq[8];
-    // second half: 2^(c_t - c_31), the weight of token t in what flows back to token 31 (bf16 pairs / PREC: fp32)
-    bf16x2 wD[(HF && !PREC) ? 4 : 1];
-    float wDf[(HF && PREC) ? 8 : 1];
-    float sigacc = 0.f;
-    {
-      const TIn* kp = (const TIn*)a.k + qk_row(a, t0, h) + 16 * nb;
-      const TIn* qp = (const TIn*)a.q + qk_row(a, t0, h) + 16 * nb;
-      float ct[2], cs[8];
-#pragma unroll
-      for (int tl = 0; tl < 2; ++tl) ct[tl] = sC[32 * HF + 16 * tl + i];
-      *(f32x4*)&cs[0] = *(const f32x4*)&sC[32 * HF + 8 * g];
-      *(f32x4*)&cs[4] = *(const f32x4*)&sC[32 * HF + 8 * g + 4];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int s = 32 * HF + 8 * g + j;
-        const bool ok = s < clen;
-        const float kv = to_f32((kp + (int64_t)(ok ? s : 0) * rs)[i]);
-        kk[j] = ok ? kv : 0.f;
-        kk2[j] = kk[j] * kk[j];
-#pragma unroll
-        for (int tl = 0; tl < 2; ++tl) {
-          const int t = 32 * HF + 16 * tl + i;
-          const float lv = (s <= t) ? fast_exp2(ct[tl] - cs[j]) : 0.f;
-          const bf16_t lh = (bf16_t)lv;
-          Lop[tl][j] = lh;
-          if constexpr (PREC) Lol[tl][j] = (bf16_t)(lv - (float)lh);
-        }
-      }
-#pragma unroll
-      for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int t = 32 * HF + 16 * tl + 4 * g + r;
-          const bool ok = t < clen;
-          const float qv = to_f32((qp + (int64_t)(ok ? t : 0) * rs)[i]);
-          qq[tl * 4 + r] = ok ? qv : 0.f;
-          dq[tl * 4 + r] = 0.f;
-        }
-      if (HF) {
-#pragma unroll
-        for (int tl = 0; tl < 2; ++tl) {
-          const f32x4 w4 = *(const f32x4*)&sF[32 + 16 * tl + 4 * g];
-          if constexpr (PREC) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) wDf[tl * 4 + r] = w4[r];
-          } else {
-            wD[tl * 2] = pack2(w4[0], w4[1]);
-            wD[tl * 2 + 1] = pack2(w4[2], w4[3]);
-          }
-        }
-      }
-    }
-    // first half: tile-start state of the next value row (entry of the own key column n = i), fetched one row ahead
-    const float* cmu = a.chunk_mu + tile_off + 16 * nb;
-    const float* cI = a.chunk_I + tile_off + 16 * nb;
-    float mu_n = 0.f, I_n = 0.f;
-    if (!HF) { mu_n = cmu[i]; I_n = cI[i]; }
-    // FOLD: decay of the incoming state into the first token of the half, on the lanes that hold that token's operand
-    const float f0m = (FOLD && g == 0) ? sF[32 * HF] : 0.f;
-    int b3 = 0;                                 // d mod 3: the row's slot of sMJ and of the first producer's operands
-    for (int it = 0; it < dv + kLagC; ++it) {
-      if (it >= HF && it - HF < dv) {
-        const int d = it - HF, dd = d & (DG - 1), buf = (d / DG) & 1;
-        const float* sV = sSt + (buf * NST + 0) * STG + dd * kVS2;
-        const float* sB = sSt + (buf * NST + 1) * STG + dd * kVS2;
-        const float* sDo = sSt + (buf * NST + 2) * STG + dd * kVS2;
-        const float* sDov = sSt + (buf * NST + NST - 1) * STG + dd * kVS2;
-        float* mj = sMJ + (nbl * 3 + b3) * 96;
-        float Mp, Jp;   // state before the first token of the half
-        if (!HF) {
-          const float mu0 = mu_n, I0 = I_n;
-          const int64_t dn = (int64_t)min(d + 1, dv - 1) * dk;
-          mu_n = (cmu + dn)[i];
-          I_n = (cI + dn)[i];
-          Mp = mu0 * I0;
-          Jp = I0 - Ip;
-          if (g == 0) { mj[i] = Mp; mj[16 + i] = Jp; }
-        } else {
-          Mp = mj[32 + i];
-          Jp = mj[48 + i];
-        }
-        bf16x8 XM, XJ;
-        bf16x8 XMl, XJl;   // PREC: the lo halves
-        {
-          const f32x4 v0 = *(const f32x4*)&sV[32 * HF + 8 * g], v1 = *(const f32x4*)&sV[32 * HF + 8 * g + 4];
-          const f32x4 b0 = *(const f32x4*)&sB[32 * HF + 8 * g], b1 = *(const f32x4*)&sB[32 * HF + 8 * g + 4];
-          if constexpr (PREC) {
-            float xm[8], xj[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              xm[j] = kk[j] * (j < 4 ? v0[j & 3] : v1[j & 3]);
-              xj[j] = kk2[j] * (j < 4 ? b0[j & 3] : b1[j & 3]);
-            }
-            split_bf16(xm, XM, XMl);
-            split_bf16(xj, XJ, XJl);
-          } else {
-            const float fM = f0m * Mp, fJ = f0m * Jp;
-#pragma unroll
-            for (int j = 0; j < 8; j += 2) {
-              const float va = j < 4 ? v0[j & 3] : v1[j & 3], vb = j < 4 ? v0[(j & 3) + 1] : v1[(j & 3) + 1];
-              const float ba = j < 4 ? b0[j & 3] : b1[j & 3], bb = j < 4 ? b0[(j & 3) + 1] : b1[(j & 3) + 1];
-              const bool tok0 = FOLD && j == 0;
-              const bf16x2 pm = pack2(tok0 ? fmaf(kk[j], va, fM) : kk[j] * va, kk[j + 1] * vb);
-              const bf16x2 pj = pack2(tok0 ? fmaf(kk2[j], ba, fJ) : kk2[j] * ba, kk2[j + 1] * bb);
-              XM[j] = pm[0]; XM[j + 1] = pm[1];
-              XJ[j] = pj[0]; XJ[j + 1] = pj[1];
-            }
-          }
-        }
-        bf16x8 PM, PJ;
-        float pmf[PREC ? 8 : 1], pjf[PREC ? 8 : 1];   // PREC: the local gradients in fp32 until they are split
-        float backM = 0.f, backJ = 0.f;
-#pragma unroll
-        for (int tl = 0; tl < 2; ++tl) {
-          const int tb = 2 * HF + tl;
-          f32x4 accM = {0.f, 0.f, 0.f, 0.f};
-          f32x4 accI = {Ip, Ip, Ip, Ip};
-          if constexpr (PREC) {
-            accM = mfma16_split(Lop[tl], Lol[tl], XM, XMl, accM);
-            accI = mfma16_split(Lop[tl], Lol[tl], XJ, XJl, accI);
-          } else {
-            accM = mfma16(Lop[tl], XM, accM);
-            accI = mfma16(Lop[tl], XJ, accI);
-          }
-          f32x4 Fv = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (!FOLD) Fv = *(const f32x4*)&sF[16 * tb + 4 * g];
-          const f32x4 dov = *(const f32x4*)&sDo[16 * tb + 4 * g];
-          f32x4 dvv = {0.f, 0.f, 0.f, 0.f};
-          if (HAS_VAR) dvv = *(const f32x4*)&sDov[16 * tb + 4 * g];
-          float dMl[4], dJl[4];
-          float M3 = 0.f, I3 = 0.f;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float Mf = FOLD ? accM[r] : fmaf(Fv[r], Mp, accM[r]);
-            const float If = FOLD ? accI[r] : fmaf(Fv[r], Jp, accI[r]);
-            if (r == 3) { M3 = Mf; I3 = If; }
-            const float rI = fast_rcp(If);
-            const float mu = Mf * rI;
-            const float q = qq[tl * 4 + r];
-            dMl[r] = (dov[r] * q) * rI;
-            dJl[r] = -(dMl[r] * mu);
-            dq[tl * 4 + r] = fmaf(mu, dov[r], dq[tl * 4 + r]);
-            if (HAS_VAR) {
-              const float wq = dvv[r] * q;          // scale*dovar*q
-              const float w = wq * q * rI;          // scale*dovar*q^2/I
-              dJl[r] = fmaf(-w, rI, dJl[r]);
-              dq[tl * 4 + r] = fmaf(2.f * wq, rI, dq[tl * 4 + r]);
-            }
-            if constexpr (PREC) sigacc += dJl[r];
-          }
-          if (!HF && tl == 1 && g == 3) {   // state after token 31 for the second half of the row
-            mj[32 + i] = M3;
-            mj[48 + i] = I3 - Ip;
-          }
-          const int o4 = tl * 4;
-          if constexpr (PREC) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              pmf[o4 + r] = dMl[r];
-              pjf[o4 + r] = dJl[r];
-              if (HF) {   // what flows back over the border
-                backM = fmaf(wDf[o4 + r], dMl[r], backM);
-                backJ = fmaf(wDf[o4 + r], dJl[r], backJ);
-              }
-            }
-          } else {
-            const bf16x2 m0 = pack2(dMl[0], dMl[1]), m1 = pack2(dMl[2], dMl[3]);
-            const bf16x2 j0 = pack2(dJl[0], dJl[1]), j1 = pack2(dJl[2], dJl[3]);
-            // the sum of dJloc (for dIp) from the packed pairs: one instruction per two entries
-            const bf16x2 one2 = {(bf16_t)1.f, (bf16_t)1.f};
-            sigacc = __builtin_amdgcn_fdot2_f32_bf16(j0, one2, sigacc, false);
-            sigacc = __builtin_amdgcn_fdot2_f32_bf16(j1, one2, sigacc, false);
-            if (HF) {   // what flows back over the border, from the packed pairs
-              backM = __builtin_amdgcn_fdot2_f32_bf16(m0, wD[tl * 2], backM, false);
-              backM = __builtin_amdgcn_fdot2_f32_bf16(m1, wD[tl * 2 + 1], backM, false);
-              backJ = __builtin_amdgcn_fdot2_f32_bf16(j0, wD[tl * 2], backJ, false);
-              backJ = __builtin_amdgcn_fdot2_f32_bf16(j1, wD[tl * 2 + 1], backJ, false);
-            }
-            PM[o4 + 0] = m0[0]; PM[o4 + 1] = m0[1]; PM[o4 + 2] = m1[0]; PM[o4 + 3] = m1[1];
-            PJ[o4 + 0] = j0[0]; PJ[o4 + 1] = j0[1]; PJ[o4 + 2] = j1[0]; PJ[o4 + 3] = j1[1];
-          }
-        }
-        if (HF) {   // sums over the four lane rows: row 0 gets the mean branch's total, row 1 the precision branch's
-          const float tot = rows4_sum_x4(backM, backJ, 0.f, 0.f);
-          if (g < 2) mj[64 + 16 * g + i] = tot;
-        }
-        bf16x8* mine = sX + ((nbl * 20 + (HF ? 12 + 4 * (d & 1) : 4 * b3)) * XS) * 64 + lane;
-        if constexpr (PREC) {
-          bf16x8 PMl, PJl;
-          split_bf16(pmf, PM, PMl);
-          split_bf16(pjf, PJ, PJl);
-          mine[4 * 64] = PMl; mine[5 * 64] = PJl; mine[6 * 64] = XMl; mine[7 * 64] = XJl;
-        }
-        mine[0] = PM; mine[64] = PJ; mine[2 * 64] = XM; mine[3 * 64] = XJ;
-        b3 = (b3 == 2) ? 0 : b3 + 1;
-      }
-      iter_tail(it);
-    }
-    TIn* dqp = (TIn*)A.dq + ((int64_t)t0 * H + h) * dk + 16 * nb;
-#pragma unroll
-    for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 32 * HF + 16 * tl + 4 * g + r;
-        if (t < clen) (dqp + (int64_t)t * rso)[i] = from_f32<TIn>(dq[tl * 4 + r]);
-      }
-    const float x = wave_sum(sigacc);
-    if (lane == 0) sRed[NB * kC + HF * NB + nbl] = x;
-  };
-
-  // ------------------------------------------------------------------ consumers
-  auto consumer = [&](auto hfc, auto foldc) {
-    constexpr int HF = decltype(hfc)::value;   // column tokens 32HF .. 32HF+31 (blocks sb = 2HF+sl)
-    constexpr bool FOLD = decltype(foldc)::value;
-    bf16x8 Lr[2];     // reverse operand inside the half: contraction (g,j) <-> token t = 32HF + 16(j/4) + 4g + j%4 >= s
-    bf16x8 Ls[2];     // strictly-lower operand: contraction token s' = 32HF + 8g + j < column token s = 16sb+i
-    bf16x8 Lrl[PREC ? 2 : 1], Lsl[PREC ? 2 : 1];   // PREC: their lo halves
-    float kr[8], kr2[8];   // k and its square in result layout (s = 16sb+i, n = 4g+r)
-    float dkM[8], dkJ[8];
-    float gate[2], Fs[2];
-    {
-      const TIn* kp4 = (const TIn*)a.k + qk_row(a, t0, h) + 16 * nb;
-      float ct[2], cs[8], ctt[8];
-#pragma unroll
-      for (int sl = 0; sl < 2; ++sl) ct[sl] = sC[16 * (2 * HF + sl) + i];
-      *(f32x4*)&cs[0] = *(const f32x4*)&sC[32 * HF + 8 * g];
-      *(f32x4*)&cs[4] = *(const f32x4*)&sC[32 * HF + 8 * g + 4];
-      *(f32x4*)&ctt[0] = *(const f32x4*)&sC[32 * HF + 4 * g];
-      *(f32x4*)&ctt[4] = *(const f32x4*)&sC[32 * HF + 16 + 4 * g];
-#pragma unroll
-      for (int sl = 0; sl < 2; ++sl) {
-        const int s = 16 * (2 * HF + sl) + i;
-        Fs[sl] = sF[s];   // decay from before the half to the column token
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int sp = 32 * HF + 8 * g + j;
-          float lv = (sp < s) ? fast_exp2(ct[sl] - cs[j]) : 0.f;
-          // the virtual token (bf16 operands): the state before the half, for the half's first token only when the
-          // operands carry it already (FOLD), else for every column token
-          if (!PREC && g == 3 && j == 7) lv = (FOLD && s != 32 * HF) ? 0.f : Fs[sl];
-          const bf16_t lh = (bf16_t)lv;
-          Ls[sl][j] = lh;
-          if constexpr (PREC) Lsl[sl][j] = (bf16_t)(lv - (float)lh);
-          const int t = 32 * HF + 16 * (j >> 2) + 4 * g + (j & 3);
-          const float rv = (t >= s) ? fast_exp2(ctt[j] - ct[sl]) : 0.f;
-          const bf16_t rh = (bf16_t)rv;
-          Lr[sl][j] = rh;
-          if constexpr (PREC) Lrl[sl][j] = (bf16_t)(rv - (float)rh);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) { kr[sl * 4 + r] = 0.f; dkM[sl * 4 + r] = 0.f; dkJ[sl * 4 + r] = 0.f; }
-        if (s < clen) load_vec<4>(kp4 + (int64_t)s * rs + 4 * g, &kr[sl * 4]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) kr2[sl * 4 + r] = kr[sl * 4 + r] * kr[sl * 4 + r];
-        gate[sl] = 0.f;
-      }
-    }
-    // the carries between tiles are kept in the dtype of the rows: bf16 rows feed them to the matrix cores in bf16
-    // anyway (carry apply), and the scan that sums them over the tiles runs in fp32 registers.  The consumer of the
-    // first column token parks them per group of value rows; the flush of the group scales and stores them.
-    float* car = sCar + ((nbl * DG) * 4 + g) * 8;
-    // after the 4-way transposing reduction, row g of the wave holds dv (g<2) or db (g>=2) of token block g&1
-    float* pw = ((g < 2) ? sPv : sPb) + nbl * DG * kC + 16 * (2 * HF + (g & 1)) + i;
-    int b3 = 0;   // d mod 3
-    for (int it = 0; it < dv + kLagC; ++it) {
-      if (it >= kLagC) {
-        const int d = it - kLagC, dd = d & (DG - 1), buf = (d / DG) & 1;
-        const float* sV = sSt + (buf * NST + 0) * STG + dd * kVS2;
-        const float* sB = sSt + (buf * NST + 1) * STG + dd * kVS2;
-        // the own half's operands
-        const bf16x8* ph = sX + ((nbl * 20 + (HF ? 12 + 4 * (d & 1) : 4 * b3)) * XS) * 64 + lane;
-        const float* mj = sMJ + (nbl * 3 + b3) * 96;
-        b3 = (b3 == 2) ? 0 : b3 + 1;
-        bf16x8 PM = ph[0], PJ = ph[64], XM = ph[2 * 64], XJ = ph[3 * 64];
-        bf16x8 PMl, PJl, XMl, XJl;   // PREC: the lo halves
-        f32x4 MpT = {0.f, 0.f, 0.f, 0.f}, JpT = {0.f, 0.f, 0.f, 0.f};   // PREC: state before the half, key columns n = 4g+r
-        if constexpr (PREC) {
-          PMl = ph[4 * 64]; PJl = ph[5 * 64]; XMl = ph[6 * 64]; XJl = ph[7 * 64];
-          MpT = *(const f32x4*)&mj[32 * HF + 4 * g];
-          JpT = *(const f32x4*)&mj[32 * HF + 16 + 4 * g];
-        } else {
-          // virtual token of the strictly-lower products: the state before the half's first token (key column n = i)
-          const bf16x2 st2 = pack2(mj[32 * HF + i], mj[32 * HF + 16 + i]);
-          if (g == 3) { XM[7] = st2[0]; XJ[7] = st2[1]; }
-        }
-        if (!HF) {
-          // what flows back over the border joins the local gradient of token 31 (element 7 of the lanes g = 3)
-          const float bm = mj[64 + i], bj = mj[80 + i];
-          if (g == 3) {
-            if constexpr (PREC) {
-              const float xm = ((float)PM[7] + (float)PMl[7]) + bm, xj = ((float)PJ[7] + (float)PJl[7]) + bj;
-              const bf16_t mh = (bf16_t)xm, jh = (bf16_t)xj;
-              PM[7] = mh; PMl[7] = (bf16_t)(xm - (float)mh);
-              PJ[7] = jh; PJl[7] = (bf16_t)(xj - (float)jh);
-            } else {
-              PM[7] = (bf16_t)((float)PM[7] + bm);
-              PJ[7] = (bf16_t)((float)PJ[7] + bj);
-            }
-          }
-        }
-        float dvp[2], dbp[2];
-        const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int sl = 0; sl < 2; ++sl) {
-          const int sb = 2 * HF + sl;
-          f32x4 aM, aJ, sM, sJ;
-          if constexpr (PREC) {
-            aM = mfma16_split(PM, PMl, Lr[sl], Lrl[sl], z4);
-            aJ = mfma16_split(PJ, PJl, Lr[sl], Lrl[sl], z4);
-            sM = mfma16_split(XM, XMl, Ls[sl], Lsl[sl], z4);
-            sJ = mfma16_split(XJ, XJl, Ls[sl], Lsl[sl], z4);
-          } else {
-            aM = mfma16(PM, Lr[sl], z4);
-            aJ = mfma16(PJ, Lr[sl], z4);
-            // S[n, s] = f_s M_{s-1}: strictly-lower product in the same [n, s] layout
-            sM = mfma16(XM, Ls[sl], z4);
-            sJ = mfma16(XJ, Ls[sl], z4);
-          }
-          const float vS = sV[16 * sb + i];
-          const float bS = sB[16 * sb + i];
-          float dvs = 0.f, dbs = 0.f, gm = gate[sl];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            dvs = fmaf(aM[r], kr[sl * 4 + r], dvs);
-            dbs = fmaf(aJ[r], kr2[sl * 4 + r], dbs);
-            dkM[sl * 4 + r] = fmaf(aM[r], vS, dkM[sl * 4 + r]);
-            dkJ[sl * 4 + r] = fmaf(aJ[r], bS, dkJ[sl * 4 + r]);
-            const float Ss = PREC ? fmaf(Fs[sl], MpT[r], sM[r]) : sM[r];
-            const float SJ = PREC ? fmaf(Fs[sl], JpT[r], sJ[r]) : sJ[r];
-            gm = fmaf(aM[r], Ss, gm);
-            gm = fmaf(aJ[r], SJ, gm);
-          }
-          gate[sl] = gm;
-          dvp[sl] = dvs;
-          dbp[sl] = dbs;
-          if (!HF && sl == 0 && i == 0) {
-            *(f32x4*)&car[dd * 32] = aM;
-            *(f32x4*)&car[dd * 32 + 4] = aJ;
-          }
-        }
-        pw[dd * kC] = rows4_sum_x4(dvp[0], dvp[1], dbp[0], dbp[1]);
-      }
-      iter_tail(it);
-    }
-    TIn* dkp = (TIn*)A.dk + ((int64_t)t0 * H + h) * dk + 16 * nb;
-#pragma unroll
-    for (int sl = 0; sl < 2; ++sl) {
-      const int s = 16 * (2 * HF + sl) + i;
-      if (s < clen) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          (dkp + (int64_t)s * rso)[4 * g + r] = from_f32<TIn>(fmaf(2.f * kr[sl * 4 + r], dkJ[sl * 4 + r], dkM[sl * 4 + r]));
-      }
-      const float x = rows4_sum(gate[sl]);
-      if (g == 0) sRed[nbl * kC + 16 * (2 * HF + sl) + i] = x;
-    }
-  };
-
-  // every role runs dv+1 iterations with the same barriers; a wave whose column block lies beyond dk
-  // (last pass of a head dim that is not a multiple of 16*NB) only keeps the barriers
-  float gm_tot = 0.f, sg_tot = 0.f;   // threads 0..63: gate term of token tid; thread 0: sum of dJloc
-  for (pass = 0; pass < n_pass; ++pass) {
-    nb = pass * NB + nbl;
-    n_act = MULTI ? min(NB, nb_total - pass * NB) : NB;
-    // the per-role constants that do not depend on the column block (decay operands) must be computed
-    // inside the role that uses them: hoisted above the role branches or out of this loop they would be
-    // live for all four roles at once
-    asm volatile("" : "+v"(lane));
-    i = lane & 15;
-    g = lane >> 4;
-    stage(0);
-    __syncthreads();
-    if (MULTI && nbl >= n_act) {
-      for (int it = 0; it < dv + kLagC; ++it) iter_tail(it);
-    } else if (fold) {
-      if constexpr (!PREC) {
-        if (role == 0) producer(std::integral_constant<int, 0>{}, std::true_type{});
-        else if (role == 1) producer(std::integral_constant<int, 1>{}, std::true_type{});
-        else if (role == 2) consumer(std::integral_constant<int, 0>{}, std::true_type{});
-        else consumer(std::integral_constant<int, 1>{}, std::true_type{});
-      }
-    } else if (role == 0) producer(std::integral_constant<int, 0>{}, std::false_type{});
-    else if (role == 1) producer(std::integral_constant<int, 1>{}, std::false_type{});
-    else if (role == 2) consumer(std::integral_constant<int, 0>{}, std::false_type{});
-    else consumer(std::integral_constant<int, 1>{}, std::false_type{});
-    __syncthreads();
-    if (tid < kC) {
-#pragma unroll
-      for (int w = 0; w < NB; ++w)
-        if (!MULTI || w < n_act) gm_tot += sRed[w * kC + tid];
-      if (tid == 0) {
-#pragma unroll
-        for (int w = 0; w < NB; ++w)
-          if (!MULTI || w < n_act) sg_tot += sRed[NB * kC + w] + sRed[NB * kC + NB + w];
-      }
-    }
-    __syncthreads();
-  }
-  if (tid < clen) A.wE[(int64_t)h * A.tokens + t0 + tid] = gm_tot;
-  if (tid == 0) A.wSig[(int64_t)cidx * H + h] = sg_tot;
-}
 
 // ----------------------------------------------------------------- carry scan
 // R_{c-1} = R_loc,c + F_c R_c backwards over the tiles of a sequence: one thread per four consecutive state
@@ -1189,7 +569,7 @@ __global__ __launch_bounds__(64) void chunk_bwd_head_reduce_kernel(BwdArgs A) {
 }
 
 struct BwdLayout {
-  size_t oDM, oDJ, oFtot, oSig, oE, oInit, oDgTile, oDqFull, oDkFull, total;
+  size_t oDM, oDJ, oFtot, oSig, oE, oInit, oDgTile, oDqFull, oDkFull, oQK, total;
 };
 
 // dq, dk of a q/k head shared by `rep` value heads: the kernels leave one row per value head ([tokens, H, dk]) in the
@@ -1254,6 +634,8 @@ static BwdLayout bwd_layout(const PalDims* d) {
     L.oDqFull = o; o = align256(o + full);
     L.oDkFull = o; o = align256(o + full);
   }
+  L.oQK = o;
+  if (tile_rows(tile_piece(d->dk), d->dv) < d->dv && d->dtype == PAL_DTYPE_BF16) o = align256(o + tokens * d->n_heads * d->dk * 2 * 4);
   L.total = o;
   return L;
 }
@@ -1261,30 +643,12 @@ static BwdLayout bwd_layout(const PalDims* d) {
 // Launch shapes that depend on the head dims only; worked out before the first launch so that a head-dim pair the
 // backward cannot serve is refused while nothing has been enqueued.
 struct BwdPlan {
-  int nb_local;        // column blocks per pass of the tile kernel
-  size_t lds_local;
   size_t lds_apply;
   int apply_alias, apply_seq, apply_ksmax;
 };
 
-static size_t local_lds_bytes(int NB, bool var, bool prec) {
-  const int DG = local_dg(NB, prec);
-  return sizeof(float) * (2 * kC + 2 * (var ? 4 : 3) * DG * kVS2 + 2 * NB * DG * kC + NB * 288 + NB * DG * 32) +
-         (size_t)NB * 20 * (prec ? 2 : 1) * 64 * 16;
-}
-
 // prec: the fp32-accurate variants (fp32 rows without PAL_FLAG_FP32_FAST)
-static int bwd_plan(int dk, int dv, bool var, bool prec, BwdPlan& P) {
-  const int nb_total = dk / 16;
-  if (nb_total < 1 || nb_total > 16) return PAL_E_HEADDIM;
-  // At most 4 column blocks (16 waves, 128 registers each: one workgroup per compute unit) in flight; wider heads
-  // take several passes.  Passes of 4 blocks when they divide the head dim, else passes of 2: two workgroups of
-  // 8 waves then share a compute unit and fill each other's barrier waits, which measured 14-17 % faster than
-  // passes of 3 (12 waves, one workgroup per unit) at dk = 80 and 96 and the same as 4 + 3 at dk = 112.
-  P.nb_local = nb_total <= 4 ? nb_total : (nb_total % 4 == 0 ? 4 : 2);
-  if (prec && P.nb_local > 2) P.nb_local = 2;   // 16-operand slots: at most two column blocks fit the LDS
-  P.lds_local = local_lds_bytes(P.nb_local, var, prec);
-  if (P.lds_local > kMaxLds) return PAL_E_HEADDIM;
+static int bwd_plan(int dk, int dv, bool prec, BwdPlan& P) {
   const int dmax = dk > dv ? dk : dv;
   const size_t rt_bytes = (prec ? 2 : 1) * 2 * (size_t)2 * dk * (dv + 8), o_bytes = sizeof(float) * kC * (dmax + 4);
   if (prec && dmax > 128) return PAL_E_HEADDIM;
@@ -1303,44 +667,6 @@ static int bwd_plan(int dk, int dv, bool var, bool prec, BwdPlan& P) {
   P.lds_apply = lds;
   P.apply_ksmax = dmax <= 64 ? 2 : dmax <= 128 ? 4 : 8;
   return PAL_OK;
-}
-
-template <typename TIn, int NB, bool PREC>
-static int launch_local_nb(const BwdArgs& A, hipStream_t s) {
-  const bool var = A.c.flags & PAL_FLAG_HAS_VAR;
-  const int64_t blocks = (int64_t)A.c.total_chunks * A.c.H;
-  if (blocks > 0x7fffffff) return PAL_E_DIM;
-  // four wave roles per block of 16 key columns, NB such blocks at a time (see chunk_bwd_local_roles_kernel)
-  const int NT = 4 * NB * 64;
-  const size_t lds = local_lds_bytes(NB, var, PREC);
-  if (lds > kMaxLds) return PAL_E_HEADDIM;
-  const bool multi = A.c.dk != 16 * NB;
-  auto go = [&](auto kern) -> int {
-    if (int rc = allow_lds((const void*)kern, lds)) return rc;
-    PAL_TIMED_LAUNCH(kKernBwdLocal, s, kern, dim3((unsigned)blocks), dim3(NT), lds, s, A);
-    return 0;
-  };
-  int rc;
-  if constexpr (NB == 2 || NB == 4) {   // the only block counts that run several passes (see bwd_plan)
-    if (multi) rc = var ? go(&chunk_bwd_local_roles_kernel<TIn, NB, true, true, PREC>) : go(&chunk_bwd_local_roles_kernel<TIn, NB, false, true, PREC>);
-    else rc = var ? go(&chunk_bwd_local_roles_kernel<TIn, NB, true, false, PREC>) : go(&chunk_bwd_local_roles_kernel<TIn, NB, false, false, PREC>);
-  } else {
-    rc = var ? go(&chunk_bwd_local_roles_kernel<TIn, NB, true, false, PREC>) : go(&chunk_bwd_local_roles_kernel<TIn, NB, false, false, PREC>);
-  }
-  if (rc) return rc;
-  PAL_HIP_LAUNCH_CHECK();
-  return PAL_OK;
-}
-
-template <typename TIn, bool PREC>
-static int launch_local(const BwdArgs& A, const BwdPlan& P, hipStream_t s) {
-  switch (P.nb_local) {
-    case 1: return launch_local_nb<TIn, 1, PREC>(A, s);
-    case 2: return launch_local_nb<TIn, 2, PREC>(A, s);
-    case 3: if constexpr (!PREC) return launch_local_nb<TIn, 3, false>(A, s); else return PAL_E_HEADDIM;
-    case 4: if constexpr (!PREC) return launch_local_nb<TIn, 4, false>(A, s); else return PAL_E_HEADDIM;
-    default: return PAL_E_HEADDIM;
-  }
 }
 
 template <typename TIn, int KSMAX, bool SEQ, bool PREC>
@@ -1364,7 +690,7 @@ extern "C" size_t pal_chunk_bwd_workspace_bytes(const PalDims* d) {
   if (pal_validate_dims(d) != PAL_OK || d->total_chunks <= 0) return 0;
   pal::BwdPlan P;
   const bool prec = d->dtype == PAL_DTYPE_F32 && !(d->flags & PAL_FLAG_FP32_FAST);
-  if (pal::bwd_plan(d->dk, d->dv, (d->flags & PAL_FLAG_HAS_VAR) != 0, prec, P) != PAL_OK) return 0;
+  if (pal::bwd_plan(d->dk, d->dv, prec, P) != PAL_OK) return 0;
   return pal::bwd_layout(d).total;
 }
 
@@ -1372,7 +698,7 @@ extern "C" int pal_chunk_bwd_supported(int32_t dk, int32_t dv, int32_t dtype, ui
   if (dk < 16 || dk > 256 || (dk & 15) || dv < 16 || dv > 256 || (dv & 15)) return PAL_E_HEADDIM;
   if (dtype != PAL_DTYPE_F32 && dtype != PAL_DTYPE_BF16) return PAL_E_DTYPE;
   pal::BwdPlan P;
-  return pal::bwd_plan(dk, dv, true, dtype == PAL_DTYPE_F32 && !(flags & PAL_FLAG_FP32_FAST), P);
+  return pal::bwd_plan(dk, dv, dtype == PAL_DTYPE_F32 && !(flags & PAL_FLAG_FP32_FAST), P);
 }
 
 extern "C" int pal_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const PalBwdTensors* gr, void* workspace,
@@ -1392,7 +718,7 @@ extern "C" int pal_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const Pal
   if (rc) return rc;
   BwdPlan P;
   const bool prec = dd.dtype == PAL_DTYPE_F32 && !(dd.flags & PAL_FLAG_FP32_FAST);
-  rc = bwd_plan(dd.dk, dd.dv, (dd.flags & PAL_FLAG_HAS_VAR) != 0, prec, P);
+  rc = bwd_plan(dd.dk, dd.dv, prec, P);
   if (rc) return rc;
   if ((int64_t)dd.total_chunks * dd.n_heads > 0x7fffffff ||
       (int64_t)dd.n_seqs * dd.n_heads * carry_scan_blocks((int64_t)dd.dv * dd.dk) > 0x7fffffff)
@@ -1416,10 +742,13 @@ extern "C" int pal_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const Pal
   A.wFtot = (float*)(ws + L.oFtot); A.wSig = (float*)(ws + L.oSig);
   A.wE = (float*)(ws + L.oE); A.wInitPart = (float*)(ws + L.oInit);
   A.wDgTile = (float*)(ws + L.oDgTile);
+  A.wQK = (float*)(ws + L.oQK);
   A.tokens = dd.batch * dd.seq_len;
   hipStream_t s = (hipStream_t)stream;
   const bool bf = dd.dtype == PAL_DTYPE_BF16;
-  rc = bf ? launch_local<bf16_t, false>(A, P, s) : prec ? launch_local<float, true>(A, P, s) : launch_local<float, false>(A, P, s);
+  const bool var = dd.flags & PAL_FLAG_HAS_VAR;
+  rc = bf ? (var ? launch_tile_t<bf16_t, true>(A, s) : launch_tile_t<bf16_t, false>(A, s))
+          : (var ? launch_tile_t<float, true>(A, s) : launch_tile_t<float, false>(A, s));
   if (rc) return rc;
   {
     const int64_t blocks = (int64_t)dd.n_seqs * dd.n_heads * carry_scan_blocks((int64_t)dd.dv * dd.dk);

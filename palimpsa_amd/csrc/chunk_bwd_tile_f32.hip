@@ -1,0 +1,6 @@
+// Instances of the tile kernel of the chunked backward: fp32 rows, without the gradient of the uncertainty output.
+#include "chunk_bwd_tile.h"
+
+namespace pal {
+template int launch_tile_t<float, false>(const BwdArgs&, hipStream_t);
+}

@@ -1,0 +1,44 @@
+"""The chunked backward's tile kernel at the edges of its launches: one and several groups of key columns and slices of
+value rows (64, 48, 32, 16 of each), tiles that end inside a step, at a step, in the first or the second half; with and
+without the uncertainty output and an initial state; fp32 rows at the fp32 bar, bf16 rows at the bf16 one."""
+import pytest
+import torch
+
+from oracle import palimpsa_oracle as po
+from tests import helpers as hp
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("q", "k", "v", "b", "gt", "g", "Ip")
+
+
+@pytest.mark.parametrize("dk,dv", [(16, 64), (16, 48), (32, 16), (32, 80), (48, 96), (64, 112), (80, 32), (96, 48), (128, 64)])
+@pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_tile_kernel_launches(gpu_device, dk, dv, rows):
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    H = 2
+    for T, var, init in ((3, False, False), (33, True, False), (64, False, True), (103, True, True)):
+        inp = hp.rounded(po.make_inputs(1, T, H, dk, dv, seed=dk + dv + T), rows)
+        inp["g"] = torch.tensor([0.3, 5.0])
+        gen = torch.Generator().manual_seed(T)
+        mu0 = I0 = None
+        if init:
+            mu0 = 0.1 * torch.randn(1, H, dv, dk, generator=gen)
+            I0 = inp["Ip"].view(1, H, 1, 1) + torch.rand(1, H, dv, dk, generator=gen)
+        o_ref, _, _, _ = hp.oracle_forward(inp, mu0=mu0, I0=I0, dtype=torch.float64)
+        # squared-error loss: dO correlated with the state, dg and dIp well conditioned
+        do = (o_ref - 0.3 * torch.randn(1, T, H, dv, generator=gen)).float()
+        dov = 0.3 * torch.randn(1, T, H, dv, generator=gen) if var else None
+        ref = hp.oracle_grads(inp, do, dov, mu0=mu0, I0=I0)
+        leaves = {n: inp[n].to(gpu_device).clone().requires_grad_(True) for n in NAMES}
+        if init:
+            leaves["mu0"], leaves["I0"] = (x.to(gpu_device).requires_grad_(True) for x in (mu0, I0))
+        out = chunk_palimpsa(*[leaves[n] for n in NAMES], initial_mu_state=leaves.get("mu0"), initial_I_state=leaves.get("I0"),
+                             output_uncertainty=var)
+        loss = ((out[0] if var else out).float() * do.to(gpu_device)).sum()
+        if var:
+            loss = loss + (out[1].float() * dov.to(gpu_device)).sum()
+        got = torch.autograd.grad(loss, list(leaves.values()))
+        for n, x in zip(leaves, got):
+            err = hp.max_rel(x, ref[n])
+            assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (T, var, init, n, err)
