@@ -146,6 +146,26 @@ def load() -> C.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native host path of the eager calls (csrc/host_ext.cpp), bound to the loaded library; its functions return
+    None for a call that is not a plain one, which then takes the Python route."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as ext
+        except ImportError as e:
+            raise ImportError(f"palimpsa_amd/_host.so: {e}; build it with `python -m palimpsa_amd.build`") from e
+        ext.bind([C.cast(getattr(lib, name), C.c_void_p).value for name in (
+            "pal_recurrent_fwd", "pal_gla_recurrent_fwd", "pal_chunk_fwd", "pal_chunk_bwd", "pal_chunk_bwd_workspace_bytes",
+            "pal_chunk_bwd_supported", "pal_strerror")])
+        _host = ext
+    return _host
+
+
 # How the chunked entry points build the tile-start states (PAL_FLAG_STATES_* of the C ABI): 0 = chosen by shape,
 # 1 = two kernels, 2 = one pass wherever it applies.  A knob of this Python layer for tests and measurements (the
 # library itself keeps no such state); initial value from the environment variable PALIMPSA_STATE_PASS_MODE.

@@ -1,4 +1,4 @@
-"""Build libpalimpsa_hip.so (gfx950) from palimpsa_amd/csrc with hipcc.
+"""Build libpalimpsa_hip.so (gfx950) from palimpsa_amd/csrc with hipcc, and the host extension module _host.so.
 
 Usage: ``python -m palimpsa_amd.build [--force]``.  The library is written
 in-tree (palimpsa_amd/lib/) and carries no torch dependency: it is plain HIP
@@ -16,6 +16,8 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
+HOST_SRC = os.path.join(CSRC, "host_ext.cpp")
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 LIB_PATH = os.path.join(LIB_DIR, "libpalimpsa_hip.so")
 
 ARCH = "gfx950"
@@ -79,6 +81,28 @@ def build(force: bool = False, jobs: int = 8) -> str:
     return LIB_PATH
 
 
+def build_host(force: bool = False) -> str:
+    """Compile the extension module of the native host path (host code only, against the installed torch)."""
+    import sysconfig
+
+    import torch
+
+    deps = [HOST_SRC, os.path.join(os.path.dirname(PKG_DIR), "include", "palimpsa_hip.h")]
+    if not force and os.path.exists(HOST_PATH) and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(p) for p in deps):
+        return HOST_PATH
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"] +
+           [f"-I{p}" for p in inc] + [HOST_SRC, "-o", HOST_PATH, f"-L{os.path.join(root, 'lib')}"] +
+           ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SRC}:\n{r.stdout}\n{r.stderr}")
+    return HOST_PATH
+
+
 if __name__ == "__main__":
-    p = build(force="--force" in sys.argv)
-    print(p)
+    print(build(force="--force" in sys.argv))
+    print(build_host(force="--force" in sys.argv))

@@ -246,7 +246,15 @@ def chunk_palimpsa(q, k, v, b, gt, g, Ip, initial_mu_state=None, initial_I_state
         scale = q.shape[-1] ** -0.5
     if not isinstance(chunk_size, int) or chunk_size <= 0:
         raise ValueError(f"chunk_size must be a positive int, got {chunk_size!r}")
-    if _ops.available() and torch.compiler.is_compiling():
+    compiling = torch.compiler.is_compiling()
+    if not compiling and q.is_cuda and (cu_seqlens is None or (q.dim() == 4 and q.shape[0] == 1)):
+        meta = None if cu_seqlens is None else cm.chunk_meta(cu_seqlens, q.shape[1], q.device)[0]
+        r = L.host().chunk_fwd(q, k, v, b, gt, g, Ip, initial_mu_state, initial_I_state, scale, output_uncertainty,
+                               L.state_pass_flags(), meta, cu_seqlens, _WINDOW_STATE_BYTES)
+        if r is not None:
+            out = (r[0], r[1]) if output_uncertainty else r[0]
+            return (out, r[2], r[3]) if output_final_state else out
+    if _ops.available() and compiling:
         # under a tracer the work is handed over as opaque library ops (see _custom_ops.py)
         if cu_seqlens is not None and q.shape[0] != 1:
             raise ValueError(f"Batch size must be 1 for Varlen, got {q.shape[0]}")

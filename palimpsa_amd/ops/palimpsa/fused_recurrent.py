@@ -210,7 +210,14 @@ def fused_recurrent_palimpsa(
             raise ValueError("Initial states mismatch sequence length.")
     if scale is None:
         scale = k.shape[-1] ** -0.5
-    if _ops.available() and torch.compiler.is_compiling():
+    compiling = torch.compiler.is_compiling()
+    if not compiling and cu_seqlens is None and q.is_cuda:
+        r = L.host().recurrent_fwd(q, k, v, b, gt, g, Ip, scale, initial_mu_state, initial_I_state, output_final_state,
+                                   output_uncertainty, L.state_pass_flags())
+        if r is not None:
+            out = (r[0], r[1]) if output_uncertainty else r[0]
+            return (out, r[2], r[3]) if output_final_state else out
+    if _ops.available() and compiling:
         # under a tracer the work is handed over as opaque library ops (see _custom_ops.py)
         o, o_var, final_mu_state, final_I_state = _ops.recurrent_fwd(
             q, k, v, b, gt, g, Ip, initial_mu_state, initial_I_state, float(scale), bool(output_final_state),

@@ -192,13 +192,23 @@ def chunk_simple_gla(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: Optio
     return ChunkSimpleGLA.apply(q, k, v, g, scale, initial_state, output_final_state, cu_seqlens)
 
 
-@cm.no_compile
 def fused_recurrent_simple_gla(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: Optional[torch.Tensor] = None,
                                scale: Optional[float] = None, initial_state: Optional[torch.Tensor] = None,
                                output_final_state: bool = False, cu_seqlens: Optional[torch.Tensor] = None):
     """Token-serial (decode) form; returns ``(o, final_state | None)``.  Without autograd it runs a kernel that keeps
     the state in the ``[N, H, dk, dv]`` layout of the caller (one read and one write of the state per call; the
     result may be written over ``initial_state`` by passing it again as the next call's initial state)."""
+    if not torch.compiler.is_compiling() and cu_seqlens is None and g is not None and q.is_cuda and v.dim() == 4:
+        r = L.host().gla_recurrent_fwd(q, k, v, g, _minus_one_rate(v.shape[2], q.device),
+                                       q.shape[-1] ** -0.5 if scale is None else scale, initial_state, output_final_state,
+                                       L.state_pass_flags())
+        if r is not None:
+            return r
+    return _fused_recurrent_simple_gla(q, k, v, g, scale, initial_state, output_final_state, cu_seqlens)
+
+
+@cm.no_compile
+def _fused_recurrent_simple_gla(q, k, v, g, scale, initial_state, output_final_state, cu_seqlens):
     needs_grad = torch.is_grad_enabled() and any(
         isinstance(x, torch.Tensor) and x.requires_grad for x in (q, k, v, g, initial_state))
     if needs_grad:

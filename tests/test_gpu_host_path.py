@@ -1,0 +1,63 @@
+"""The native host path of the eager calls against the Python route, which a call with a strided row tensor takes: the same
+kernels on the same values, so results, states and gradients are equal bit for bit."""
+import pytest
+import torch
+
+from oracle import palimpsa_oracle as po
+from tests import helpers as hp
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("q", "k", "v", "b", "gt", "g", "Ip")
+
+
+def _strided(x):
+    return torch.cat([x, x], -1)[..., : x.shape[-1]]
+
+
+@pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("T,init,var,cu,bf16_gates", [(1, True, False, None, False), (70, False, True, None, True),
+                                                      (150, True, True, [0, 17, 17, 150], False)])
+def test_native_and_python_routes_agree(gpu_device, rows, T, init, var, cu, bf16_gates):
+    from palimpsa_amd import _lib as L
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa, fused_recurrent_palimpsa
+    from palimpsa_amd.ops.simple_gla import fused_recurrent_simple_gla
+    B, H, dk, dv = 1 if cu else 2, 4, 32, 48
+    inp = hp.rounded(po.make_inputs(B, T, H, dk, dv, seed=T), rows)
+    x = {n: inp[n].to(gpu_device) for n in NAMES}
+    x["q"], x["k"] = x["q"][:, :, :2].contiguous(), x["k"][:, :, :2].contiguous()   # two heads share a q/k row
+    if bf16_gates:
+        x["gt"] = x["gt"].bfloat16()
+    N = len(cu) - 1 if cu else B
+    cu_t = None if cu is None else torch.tensor(cu, dtype=torch.int32, device=gpu_device)
+    s = dict(initial_mu_state=torch.randn(N, H, dv, dk, device=gpu_device),
+             initial_I_state=2 + torch.rand(N, H, dv, dk, device=gpu_device)) if init else {}
+    host = L.host()
+
+    def run(f, native, grad):
+        y = {n: (t.clone().requires_grad_(grad)) for n, t in list(x.items()) + list(s.items())}
+        args = [y[n] for n in NAMES]
+        assert args[0].is_contiguous()
+        if not native:
+            args[0] = _strided(args[0])
+            assert not args[0].is_contiguous()
+        with torch.set_grad_enabled(grad):
+            out = f(*args, **{n: y[n] for n in s}, output_final_state=True, output_uncertainty=var, cu_seqlens=cu_t)
+        o = list(out[0]) if var else [out[0]]
+        res = o + list(out[1:])
+        if grad:
+            res += torch.autograd.grad([z.float().square().sum() for z in o], list(y.values()))
+        return res
+
+    for f, grad in ((chunk_palimpsa, False), (chunk_palimpsa, True), (fused_recurrent_palimpsa, False)):
+        for a, b in zip(run(f, True, grad), run(f, False, grad)):
+            assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), (f.__name__, grad)
+    if cu is None:
+        g = -x["gt"].float()
+        S = torch.randn(N, H, dk, dv, device=gpu_device) if init else None
+        a = fused_recurrent_simple_gla(x["q"], x["k"], x["v"], g, initial_state=S, output_final_state=True)
+        b = fused_recurrent_simple_gla(_strided(x["q"]), x["k"], x["v"], g, initial_state=S, output_final_state=True)
+        assert all(torch.equal(y, z) for y, z in zip(a, b))
+        ipad = (x["q"], x["k"], x["v"], x["b"], x["gt"], x["g"], x["Ip"], 1.0, None, None, False, False, 0)
+        assert host.recurrent_fwd(*ipad) is not None
+        assert host.recurrent_fwd(_strided(x["q"]), *ipad[1:]) is None
