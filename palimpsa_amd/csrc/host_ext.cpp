@@ -104,6 +104,14 @@ bool wants_grad(std::initializer_list<const Tensor*> ts, const OptT& a, const Op
   return (a && a->requires_grad()) || (b && b->requires_grad());
 }
 
+// A tensor with a forward-mode tangent (a dual number, whether or not it requires grad): the autograd Functions of the
+// Python route refuse it, a plain kernel call would hand back results without a tangent, a derivative of zero.
+bool has_tangent(std::initializer_list<const Tensor*> ts, const OptT& a, const OptT& b) {
+  for (const Tensor* t : ts)
+    if (t->defined() && t->_fw_grad(/*level=*/0).defined()) return true;
+  return (a && a->_fw_grad(0).defined()) || (b && b->_fw_grad(0).defined());
+}
+
 void* stream_of(const c10::Device& dev) { return (void*)c10::hip::getCurrentHIPStream(dev.index()).stream(); }
 
 // ---------------------------------------------------------------------------------------------- token-serial forward
@@ -112,6 +120,7 @@ py::object recurrent_fwd(const Tensor& q, const Tensor& k, const Tensor& v, cons
                          const Tensor& Ip, double scale, const OptT& mu, const OptT& I, bool final_state, bool var,
                          int64_t mode_flags) {
   if (wants_grad({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I) || mu.has_value() != I.has_value()) return py::none();
+  if (has_tangent({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I)) return py::none();
   Call c(q, k, v, &b, gt, g, &Ip, scale, 0);
   if (!c.ok) return py::none();
   switch (c.dk) {   // the head dims that the token-serial kernels are compiled for
@@ -143,7 +152,7 @@ py::object recurrent_fwd(const Tensor& q, const Tensor& k, const Tensor& v, cons
 // the same without the precision state: (o, final | None), or None; states [N, H, dk, dv]
 py::object gla_recurrent_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& rate, double scale,
                              const OptT& S, bool final_state, int64_t mode_flags) {
-  if (wants_grad({&q, &k, &v, &g}, S, std::nullopt)) return py::none();
+  if (wants_grad({&q, &k, &v, &g}, S, std::nullopt) || has_tangent({&q, &k, &v, &g}, S, std::nullopt)) return py::none();
   Call c(q, k, v, nullptr, g, rate, nullptr, scale, 0);
   if (!c.ok) return py::none();
   const c10::Device dev = q.device();
@@ -266,6 +275,7 @@ py::object chunk_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Te
                      const OptT& cu, int64_t window_bytes) {
   if (mu.has_value() != I.has_value() || meta.has_value() != cu.has_value()) return py::none();
   if (cu && (cu->dim() != 1 || cu->numel() < 2)) return py::none();
+  if (has_tangent({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I)) return py::none();
   Call c(q, k, v, &b, gt, g, &Ip, scale, cu ? cu->numel() - 1 : 0);
   if (!c.ok) return py::none();
   const c10::Device dev = q.device();

@@ -61,3 +61,28 @@ def test_native_and_python_routes_agree(gpu_device, rows, T, init, var, cu, bf16
         ipad = (x["q"], x["k"], x["v"], x["b"], x["gt"], x["g"], x["Ip"], 1.0, None, None, False, False, 0)
         assert host.recurrent_fwd(*ipad) is not None
         assert host.recurrent_fwd(_strided(x["q"]), *ipad[1:]) is None
+
+
+def _plain_call(dev, T=3, H=2, dk=16, dv=16, grad=()):
+    inp = po.make_inputs(1, T, H, dk, dv, seed=5)
+    x = [inp[n].to(dev) for n in NAMES]
+    for i in grad:
+        x[i].requires_grad_(True)
+    return x
+
+
+@pytest.mark.parametrize("which", range(9), ids=list(NAMES) + ["mu0", "I0"])
+@pytest.mark.parametrize("grad_mode", [False, True])
+def test_forward_mode_stays_refused(gpu_device, which, grad_mode):
+    """No operator has a forward-mode formula: a dual number is refused, with gradients on or off, and never comes back
+    without its tangent."""
+    import torch.autograd.forward_ad as fw
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa, fused_recurrent_palimpsa
+    x = _plain_call(gpu_device)
+    s = [torch.zeros(1, 2, 16, 16, device=gpu_device), torch.ones(1, 2, 16, 16, device=gpu_device)]
+    for f in (chunk_palimpsa, fused_recurrent_palimpsa):
+        with fw.dual_level(), torch.set_grad_enabled(grad_mode):
+            y = x + s
+            y[which] = fw.make_dual(y[which], torch.ones_like(y[which]))
+            with pytest.raises(NotImplementedError):
+                f(*y[:7], initial_mu_state=y[7], initial_I_state=y[8])
