@@ -13,6 +13,7 @@
 #include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 
@@ -104,6 +105,13 @@ bool wants_grad(std::initializer_list<const Tensor*> ts, const OptT& a, const Op
   return (a && a->requires_grad()) || (b && b->requires_grad());
 }
 
+// No tracer (torch.jit.trace), functorch transform (vmap, grad, jvp) and no dispatch mode is listening on this thread: each
+// would see the output allocations of a call but not the kernel that fills them.  (torch switches each of them on by a
+// dispatch key that it includes for the thread.)
+bool unobserved() {
+  return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+}
+
 // A tensor with a forward-mode tangent (a dual number, whether or not it requires grad): the autograd Functions of the
 // Python route refuse it, a plain kernel call would hand back results without a tangent, a derivative of zero.
 bool has_tangent(std::initializer_list<const Tensor*> ts, const OptT& a, const OptT& b) {
@@ -119,7 +127,8 @@ void* stream_of(const c10::Device& dev) { return (void*)c10::hip::getCurrentHIPS
 py::object recurrent_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, const Tensor& gt, const Tensor& g,
                          const Tensor& Ip, double scale, const OptT& mu, const OptT& I, bool final_state, bool var,
                          int64_t mode_flags) {
-  if (wants_grad({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I) || mu.has_value() != I.has_value()) return py::none();
+  if (!unobserved() || mu.has_value() != I.has_value()) return py::none();
+  if (wants_grad({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I)) return py::none();
   if (has_tangent({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I)) return py::none();
   Call c(q, k, v, &b, gt, g, &Ip, scale, 0);
   if (!c.ok) return py::none();
@@ -152,7 +161,7 @@ py::object recurrent_fwd(const Tensor& q, const Tensor& k, const Tensor& v, cons
 // the same without the precision state: (o, final | None), or None; states [N, H, dk, dv]
 py::object gla_recurrent_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& rate, double scale,
                              const OptT& S, bool final_state, int64_t mode_flags) {
-  if (wants_grad({&q, &k, &v, &g}, S, std::nullopt) || has_tangent({&q, &k, &v, &g}, S, std::nullopt)) return py::none();
+  if (!unobserved() || wants_grad({&q, &k, &v, &g}, S, std::nullopt) || has_tangent({&q, &k, &v, &g}, S, std::nullopt)) return py::none();
   Call c(q, k, v, nullptr, g, rate, nullptr, scale, 0);
   if (!c.ok) return py::none();
   const c10::Device dev = q.device();
@@ -273,7 +282,7 @@ struct ChunkNode : torch::autograd::Function<ChunkNode> {
 py::object chunk_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, const Tensor& gt, const Tensor& g,
                      const Tensor& Ip, const OptT& mu, const OptT& I, double scale, bool var, int64_t mode_flags, const OptT& meta,
                      const OptT& cu, int64_t window_bytes) {
-  if (mu.has_value() != I.has_value() || meta.has_value() != cu.has_value()) return py::none();
+  if (!unobserved() || mu.has_value() != I.has_value() || meta.has_value() != cu.has_value()) return py::none();
   if (cu && (cu->dim() != 1 || cu->numel() < 2)) return py::none();
   if (has_tangent({&q, &k, &v, &b, &gt, &g, &Ip}, mu, I)) return py::none();
   Call c(q, k, v, &b, gt, g, &Ip, scale, cu ? cu->numel() - 1 : 0);

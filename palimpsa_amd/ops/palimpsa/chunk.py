@@ -254,8 +254,9 @@ def chunk_palimpsa(q, k, v, b, gt, g, Ip, initial_mu_state=None, initial_I_state
         if r is not None:
             out = (r[0], r[1]) if output_uncertainty else r[0]
             return (out, r[2], r[3]) if output_final_state else out
-    if _ops.available() and compiling:
-        # under a tracer the work is handed over as opaque library ops (see _custom_ops.py)
+    if _ops.available() and (compiling or torch.jit.is_tracing()):
+        # under a tracer the work is handed over as opaque library ops (see _custom_ops.py); torch.jit.trace too: what
+        # it records of the Function below gives other values when the trace runs
         if cu_seqlens is not None and q.shape[0] != 1:
             raise ValueError(f"Batch size must be 1 for Varlen, got {q.shape[0]}")
         mode_flags = L.state_pass_flags()

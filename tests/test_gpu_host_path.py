@@ -86,3 +86,40 @@ def test_forward_mode_stays_refused(gpu_device, which, grad_mode):
             y[which] = fw.make_dual(y[which], torch.ones_like(y[which]))
             with pytest.raises(NotImplementedError):
                 f(*y[:7], initial_mu_state=y[7], initial_I_state=y[8])
+
+
+@pytest.mark.filterwarnings("ignore")
+def test_traced_call_runs_the_kernels_again(gpu_device):
+    """torch.jit.trace records the call as an operation that the trace repeats on its inputs, not the allocation of its
+    outputs alone."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa, fused_recurrent_palimpsa
+    x = _plain_call(gpu_device)
+    with torch.no_grad():
+        for f in (chunk_palimpsa, fused_recurrent_palimpsa):
+            traced = torch.jit.trace(lambda q: f(q, *x[1:]), (x[0],), check_trace=False)
+            for q in (x[0], 2.0 * x[0], x[0].flip(1).contiguous()):
+                junk = torch.full_like(x[2], 1e6)   # what an unfilled output would be likely to hold
+                del junk
+                assert torch.equal(traced(q), f(q, *x[1:])), f.__name__
+
+
+def test_transforms_and_dispatch_modes_take_the_python_route(gpu_device):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from palimpsa_amd import _lib as L
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    x = _plain_call(gpu_device)
+    native = (*x, None, None, 1.0, False, 0, None, None, 1 << 30)
+    assert L.host().chunk_fwd(*native) is not None
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert L.host().chunk_fwd(*native) is None
+        assert chunk_palimpsa(*x).shape == x[2].shape
+    with pytest.raises(RuntimeError):   # the Function has no vmap rule
+        torch.vmap(lambda q: chunk_palimpsa(q, *x[1:]))(torch.stack([x[0]] * 2))
+    with pytest.raises(RuntimeError):   # nor one for functorch's gradients
+        torch.func.grad(lambda q: chunk_palimpsa(q, *x[1:]).sum())(x[0])
