@@ -149,6 +149,20 @@ def load() -> C.CDLL:
 _host = None
 
 
+def _check_host(ext) -> None:
+    """The extension module passes C structs to the library by itself: both have to be built from the same header, and it
+    uses torch's C++ interface, which has to be that of the torch that is loaded."""
+    import torch
+
+    want = (PAL_ABI_VERSION, C.sizeof(PalDims), C.sizeof(PalFwdTensors), C.sizeof(PalBwdTensors))
+    have = tuple(getattr(ext, "abi", ()))
+    built = getattr(ext, "torch_version", None)
+    if have != want or built != torch.__version__:
+        raise ImportError(
+            f"{getattr(ext, '__file__', 'palimpsa_amd._host')}: ABI version and struct sizes {have} != expected {want}, or "
+            f"built for torch {built}, not {torch.__version__}; rebuild with `python -m palimpsa_amd.build`")
+
+
 def host():
     """The native host path of the eager calls (csrc/host_ext.cpp), bound to the loaded library; its functions return
     None for a call that is not a plain one, which then takes the Python route."""
@@ -158,12 +172,17 @@ def host():
         try:
             from . import _host as ext
         except ImportError as e:
-            raise ImportError(f"palimpsa_amd/_host.so: {e}; build it with `python -m palimpsa_amd.build`") from e
-        ext.bind([C.cast(getattr(lib, name), C.c_void_p).value for name in (
-            "pal_recurrent_fwd", "pal_gla_recurrent_fwd", "pal_chunk_fwd", "pal_chunk_bwd", "pal_chunk_bwd_workspace_bytes",
-            "pal_chunk_bwd_supported", "pal_strerror")])
+            raise ImportError(f"palimpsa_amd._host: {e}; build it with `python -m palimpsa_amd.build` (needs g++ and the "
+                              "headers of the installed torch)") from e
+        _check_host(ext)
+        ext.bind([C.cast(getattr(lib, name), C.c_void_p).value for name in _HOST_FUNCTIONS])
         _host = ext
     return _host
+
+
+# the library's functions that the extension module calls, in the order of its table
+_HOST_FUNCTIONS = ("pal_recurrent_fwd", "pal_gla_recurrent_fwd", "pal_chunk_fwd", "pal_chunk_bwd",
+                   "pal_chunk_bwd_workspace_bytes", "pal_chunk_bwd_supported", "pal_strerror")
 
 
 # How the chunked entry points build the tile-start states (PAL_FLAG_STATES_* of the C ABI): 0 = chosen by shape,

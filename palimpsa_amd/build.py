@@ -2,7 +2,9 @@
 
 Usage: ``python -m palimpsa_amd.build [--force]``.  The library is written
 in-tree (palimpsa_amd/lib/) and carries no torch dependency: it is plain HIP
-behind the C ABI of include/palimpsa_hip.h.
+behind the C ABI of include/palimpsa_hip.h.  The extension module is host code
+against the headers of the installed torch and of Python (g++, or $CXX); it is
+built again when the torch version or the interpreter changes.
 """
 from __future__ import annotations
 
@@ -11,13 +13,16 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 HOST_SRC = os.path.join(CSRC, "host_ext.cpp")
-HOST_PATH = os.path.join(PKG_DIR, "_host.so")
+# the extension module is tied to the interpreter it was built for: its name says so, and another one does not load it
+HOST_PATH = os.path.join(PKG_DIR, "_host" + sysconfig.get_config_var("EXT_SUFFIX"))
+HOST_STAMP = os.path.join(OBJ_DIR, "host_ext.stamp")
 LIB_PATH = os.path.join(LIB_DIR, "libpalimpsa_hip.so")
 
 ARCH = "gfx950"
@@ -66,6 +71,13 @@ def _compile_one(src: str, force: bool) -> str:
 
 
 def build(force: bool = False, jobs: int = 8) -> str:
+    """Build the shared library and the extension module (which hold the same C structs).  Returns the library's path."""
+    path = build_library(force, jobs)
+    build_host(force)
+    return path
+
+
+def build_library(force: bool = False, jobs: int = 8) -> str:
     """Compile every .hip under csrc/ and link the shared library.  Returns its path."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
@@ -81,28 +93,42 @@ def build(force: bool = False, jobs: int = 8) -> str:
     return LIB_PATH
 
 
+def _host_stamp() -> str:
+    """What the extension module was built against."""
+    import torch
+
+    return f"torch {torch.__version__}, python {sys.version.split()[0]} {sysconfig.get_config_var('SOABI')}"
+
+
 def build_host(force: bool = False) -> str:
     """Compile the extension module of the native host path (host code only, against the installed torch)."""
-    import sysconfig
-
     import torch
 
     deps = [HOST_SRC, os.path.join(os.path.dirname(PKG_DIR), "include", "palimpsa_hip.h")]
-    if not force and os.path.exists(HOST_PATH) and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(p) for p in deps):
+    stamp = _host_stamp()
+    if (not force and os.path.exists(HOST_PATH) and os.path.exists(HOST_STAMP) and open(HOST_STAMP).read() == stamp
+            and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(p) for p in deps)):
         return HOST_PATH
     root = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
     inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
            os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
-    cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"] +
+    cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+            f'-DPAL_TORCH_VERSION="{torch.__version__}"'] +
            [f"-I{p}" for p in inc] + [HOST_SRC, "-o", HOST_PATH, f"-L{os.path.join(root, 'lib')}"] +
            ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed on {HOST_SRC}:\n{r.stdout}\n{r.stderr}")
+    untagged = os.path.join(PKG_DIR, "_host.so")   # would load in place of a tagged one, whatever interpreter it is for
+    if os.path.exists(untagged):
+        os.remove(untagged)
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    with open(HOST_STAMP, "w") as f:
+        f.write(stamp)
     return HOST_PATH
 
 
 if __name__ == "__main__":
     print(build(force="--force" in sys.argv))
-    print(build_host(force="--force" in sys.argv))
+    print(HOST_PATH)

@@ -311,6 +311,9 @@ py::object chunk_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Te
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
+  // what this module was built from; the loader compares it before it binds the library
+  m.attr("abi") = py::make_tuple(PAL_ABI_VERSION, sizeof(PalDims), sizeof(PalFwdTensors), sizeof(PalBwdTensors));
+  m.attr("torch_version") = PAL_TORCH_VERSION;
   m.def("bind", &bind);
   m.def("recurrent_fwd", &recurrent_fwd);
   m.def("gla_recurrent_fwd", &gla_recurrent_fwd);

@@ -4,6 +4,8 @@ No kernel is launched here."""
 import ctypes as C
 import os
 import re
+import sys
+import sysconfig
 
 import numpy as np
 import pytest
@@ -298,3 +300,50 @@ def test_missing_library_fails_loudly(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libpalimpsa_hip.so"))
     with pytest.raises(ImportError, match="palimpsa_amd.build"):
         _lib.load()
+
+
+def test_host_module_is_checked_before_it_is_bound(L, monkeypatch):
+    """The extension module hands C structs to the library by itself: one of another header or another torch is refused."""
+    import types
+
+    import torch
+    good = L.host()
+    assert tuple(good.abi) == (L.PAL_ABI_VERSION, C.sizeof(L.PalDims), C.sizeof(L.PalFwdTensors),
+                               C.sizeof(L.PalBwdTensors))
+    L._check_host(good)
+    for abi, version in (((L.PAL_ABI_VERSION - 1, *good.abi[1:]), torch.__version__),
+                         ((good.abi[0], good.abi[1] - 4, *good.abi[2:]), torch.__version__),
+                         (good.abi, "2.0.0"), ((), None)):
+        bound = []
+        stub = types.SimpleNamespace(abi=abi, torch_version=version, bind=bound.append)
+        monkeypatch.setattr(L, "_host", None)
+        monkeypatch.setitem(sys.modules, "palimpsa_amd._host", stub)
+        monkeypatch.setattr("palimpsa_amd._host", stub, raising=False)
+        with pytest.raises(ImportError, match="rebuild"):
+            L.host()
+        assert not bound
+
+
+def test_build_covers_the_host_module(monkeypatch):
+    """One build makes the library and the module from the same header; the module is rebuilt for another torch."""
+    from palimpsa_amd import build
+    assert build.HOST_PATH.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+    calls = []
+    monkeypatch.setattr(build, "build_library", lambda force, jobs: calls.append("library"))
+    monkeypatch.setattr(build, "build_host", lambda force=False: calls.append("host"))
+    build.build()
+    assert calls == ["library", "host"]
+    monkeypatch.undo()
+    build.build_host()
+
+    class Ran(Exception):
+        pass
+
+    def run(*a, **k):
+        raise Ran
+
+    monkeypatch.setattr(build.subprocess, "run", run)
+    assert build.build_host() == build.HOST_PATH       # up to date
+    monkeypatch.setattr(build, "_host_stamp", lambda: "torch 0")
+    with pytest.raises(Ran):
+        build.build_host()
