@@ -175,14 +175,14 @@ def host():
             raise ImportError(f"palimpsa_amd._host: {e}; build it with `python -m palimpsa_amd.build` (needs g++ and the "
                               "headers of the installed torch)") from e
         _check_host(ext)
-        ext.bind([C.cast(getattr(lib, name), C.c_void_p).value for name in _HOST_FUNCTIONS])
+        ext.bind([C.cast(getattr(lib, name), C.c_void_p).value for name in _HOST_FUNCTIONS], check)
         _host = ext
     return _host
 
 
 # the library's functions that the extension module calls, in the order of its table
 _HOST_FUNCTIONS = ("pal_recurrent_fwd", "pal_gla_recurrent_fwd", "pal_chunk_fwd", "pal_chunk_bwd",
-                   "pal_chunk_bwd_workspace_bytes", "pal_chunk_bwd_supported", "pal_strerror")
+                   "pal_chunk_bwd_workspace_bytes", "pal_chunk_bwd_supported")
 
 
 # How the chunked entry points build the tile-start states (PAL_FLAG_STATES_* of the C ABI): 0 = chosen by shape,

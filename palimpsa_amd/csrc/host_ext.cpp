@@ -9,6 +9,7 @@
 //
 // The kernels are reached through the C ABI of palimpsa_hip.h, whose addresses the Python loader hands over once (bind).
 #include <Python.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
@@ -32,12 +33,27 @@ struct Abi {
   int (*chunk_bwd)(const PalDims*, const PalFwdTensors*, const PalBwdTensors*, void*, size_t, void*);
   size_t (*chunk_bwd_workspace_bytes)(const PalDims*);
   int (*chunk_bwd_supported)(int32_t, int32_t, int32_t, uint32_t);
-  const char* (*strerror)(int);
 } abi;
+py::handle raise_code;   // (code, where): raises what the Python routes raise for a code of the library
 
-void bind(const std::vector<uintptr_t>& p) {
-  TORCH_CHECK(p.size() == 7, "bind: seven addresses");
+void bind(const std::vector<uintptr_t>& p, py::object check) {
+  TORCH_CHECK(p.size() * sizeof(p[0]) == sizeof(abi), "bind: number of addresses");
   memcpy(&abi, p.data(), sizeof(abi));
+  raise_code = check.release();   // held for the life of the process
+}
+
+// For the autograd node, whose backward runs on a thread of the engine: a Python exception that the engine carries over.
+[[noreturn]] void fail(int rc, const char* where) {
+  py::gil_scoped_acquire gil;
+  try {
+    raise_code(rc, where);
+    PyErr_SetString(PyExc_RuntimeError, where);   // (not reached: the codes are errors)
+  } catch (py::error_already_set& e) {
+    e.restore();
+  }
+  python_error err;
+  err.persist();
+  throw err;
 }
 
 // kernel calls without the interpreter lock where the thread holds it (a launch may wait for room in the queue)
@@ -223,7 +239,7 @@ struct ChunkNode : torch::autograd::Function<ChunkNode> {
     Call c(q, k, v, &b, gt, g, &Ip, scale, cu.defined() ? cu.numel() - 1 : 0);
     ChunkOut out;
     const int rc = chunk_forward(c, q, k, v, b, gt, g, Ip, mu, I, var, (uint32_t)flags, meta, cu, tiles, out);
-    TORCH_CHECK_VALUE(rc == 0, "pal_chunk_fwd: ", abi.strerror(rc), " (code ", rc, ")");
+    if (rc) fail(rc, "pal_chunk_fwd");
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({q, k, v, b, gt, g, Ip, mu, I, meta, cu, out.tile_mu, out.tile_I});
     ctx->saved_data["scale"] = scale;
@@ -270,7 +286,7 @@ struct ChunkNode : torch::autograd::Function<ChunkNode> {
     Tensor ws = at::empty({(int64_t)std::max<size_t>(bytes, 16)}, q.options().dtype(at::kByte).requires_grad(false));
     int rc;
     { NoGil off; rc = abi.chunk_bwd(&c.dims, &t, &w, ws.mutable_data_ptr(), bytes, stream_of(q.device())); }
-    TORCH_CHECK(rc == 0, "pal_chunk_bwd: ", abi.strerror(rc), " (code ", rc, ")");
+    if (rc) fail(rc, "pal_chunk_bwd");
     if (gt.scalar_type() != at::kFloat) dgt = dgt.to(gt.scalar_type());
     const Tensor none;
     return {dq, dk, dv, db, dgt, dg, dIp, dmu, dI, none, none, none, none, none, none};
@@ -297,8 +313,13 @@ py::object chunk_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Te
   const uint32_t flags = (uint32_t)mode_flags | (cu ? PAL_FLAG_VARLEN : 0) | (mu ? PAL_FLAG_HAS_INIT : 0) | (var ? PAL_FLAG_HAS_VAR : 0);
   if (grad) {
     if (abi.chunk_bwd_supported((int32_t)c.dk, (int32_t)c.dv, c.dims.dtype, (uint32_t)mode_flags)) return py::none();
-    auto r = ChunkNode::apply(q, k, v, b, gt, g, Ip, mu, I, meta, cu, scale, var, (int64_t)flags, tiles);
-    return py::make_tuple(r[0], var ? py::cast(r[3]) : py::none(), r[1], r[2]);
+    try {
+      auto r = ChunkNode::apply(q, k, v, b, gt, g, Ip, mu, I, meta, cu, scale, var, (int64_t)flags, tiles);
+      return py::make_tuple(r[0], var ? py::cast(r[3]) : py::none(), r[1], r[2]);
+    } catch (python_error& e) {
+      e.restore();
+      throw py::error_already_set();
+    }
   }
   ChunkOut out;
   const Tensor none;

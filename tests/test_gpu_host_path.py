@@ -123,3 +123,34 @@ def test_transforms_and_dispatch_modes_take_the_python_route(gpu_device):
         torch.vmap(lambda q: chunk_palimpsa(q, *x[1:]))(torch.stack([x[0]] * 2))
     with pytest.raises(RuntimeError):   # nor one for functorch's gradients
         torch.func.grad(lambda q: chunk_palimpsa(q, *x[1:]).sum())(x[0])
+
+
+def test_library_codes_raise_what_the_python_route_raises(gpu_device):
+    """A code of the library, forward or backward (there on a thread of the autograd engine): the same exception from both
+    routes.  The library's functions are replaced by ones that return the code and launch nothing."""
+    import ctypes as C
+
+    from palimpsa_amd import _lib as L
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    host, lib = L.host(), L.load()
+    addresses = {n: C.cast(getattr(lib, n), C.c_void_p).value for n in L._HOST_FUNCTIONS}
+    fwd_t = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_void_p)
+    bwd_t = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p)
+    try:
+        for code in (L.PAL_E_WORKSPACE, L.PAL_E_ALIGN, L.PAL_E_DIM, 700):
+            with pytest.raises(Exception) as want:
+                L.check(code, "pal_chunk_bwd")
+            x = _plain_call(gpu_device, grad=range(7))
+            host.bind([*(dict(addresses, pal_chunk_bwd=C.cast(f := bwd_t(lambda *a: code), C.c_void_p).value)).values()], L.check)
+            out = chunk_palimpsa(*x)
+            assert "ChunkNode" in out.grad_fn.name()
+            with pytest.raises(Exception) as got:
+                out.sum().backward()
+            assert type(got.value) is type(want.value) and str(got.value) == str(want.value)
+            assert getattr(got.value, "code", None) == getattr(want.value, "code", None)
+            host.bind([*(dict(addresses, pal_chunk_fwd=C.cast(f := fwd_t(lambda *a: code), C.c_void_p).value)).values()], L.check)  # noqa: F841
+            with pytest.raises(type(want.value)):
+                chunk_palimpsa(*x)
+    finally:
+        host.bind([*addresses.values()], L.check)
+    chunk_palimpsa(*x).sum().backward()
