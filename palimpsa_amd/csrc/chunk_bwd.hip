@@ -159,7 +159,10 @@ __global__ __launch_bounds__(256, 2) void chunk_bwd_carry_apply_kernel(BwdArgs A
   //   d log f_t = (local part, from the tile kernel) + (carry terms of the earlier tokens of the tile) + (boundary term),
   //   dgt_t = -g d log f_t, and the tile's share of dg = -sum_t gt_t d log f_t.
   auto gate_grad = [&](float bc, float bnd) {
-    const float pre = wave_inclusive_scan(bc, lane) - bc;
+    // sum over the earlier tokens alone (the sum with this token's own term, less that term, would lose what an earlier
+    // strong decay has left of the others)
+    const float before = __shfl_up(bc, 1);
+    const float pre = wave_inclusive_scan(lane ? before : 0.f, lane);
     const float dlogf = tok_ok ? e_l + pre + bnd : 0.f;
     if (tok_ok) A.dgt[tokL * H + h] = -a.g[h] * dlogf;
     const float share = wave_sum(-gt_l * dlogf);

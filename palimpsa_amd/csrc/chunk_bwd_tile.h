@@ -4,7 +4,7 @@
 // the gate's gradient, and the carry R_loc = f_first dM_first that the tile hands to its predecessor (chunk_bwd.hip).
 // With G_t = scale do_t q_t^T, r = 1 / I_t and mu = M_t r, per state entry and token (the reference's reverse
 // recurrence, chunk_palimpsa_forgetting_scalar.py:360-434):
-//   forward  M <- f_t M + v_t k_t        I <- f_t I + b_t k_t^2 + (1 - f_t) Ip
+//   forward  M <- f_t M + v_t k_t        J <- f_t J + b_t k_t^2   (J = I - Ip)
 //   reverse  dM <- f_{t+1} dM + G r      dJ <- f_{t+1} dJ - G r mu
 //   dq = sum_d scale do mu    dv = sum_n dM k    db = sum_n dJ k^2    dk = sum_d dM v + 2 k sum_d dJ b
 // all of it token by token in fp32 on the vector units.
@@ -12,9 +12,9 @@
 // The reverse sweep needs mu and r of every token in reverse order.  A tile is worked in steps of kG tokens from its
 // end: the state before a step is recomputed from the state before its half of the tile by two matrix products over at
 // most 32 tokens (k weighted by the decay against v, and k^2 against b; bf16 operands, two halves of each for fp32
-// rows), the step's tokens are advanced forward leaving mu, r of its tokens in registers, then worked in reverse.
+// rows), the step's tokens are advanced forward leaving their states in registers, then worked in reverse.
 //
-// What bounds it: vector issue.  Per entry and token 16 fp32 instructions and a reciprocal, and about 8 more for the sums
+// What bounds it: vector issue.  Per entry and token 19 fp32 instructions and a reciprocal, and about 8 more for the sums
 // over lanes, the recomputed states, staging and the sums over waves; two waves per SIMD (the registers), each of
 // which issues an instruction per 5.4 cycles.  As products on the matrix cores (12 prefix and 12 suffix instructions of
 // 16 cycles per 16 entries of a lane, operands exchanged through LDS between waves of different roles) the same pass took
@@ -25,14 +25,16 @@
 // 48 columns loads all four SIMDs.  As many tokens per step as the registers hold: the fixed cost of a step (about
 // 3000 cycles of a SIMD per wave beside 48 per entry and token) is what small pieces pay.
 //
-// Gate: gamma_t = <dM_t, f_t M_{t-1}> + <dJ_t, f_t J_{t-1}>.  <dMloc, M> + <dJloc, J> = Ip sum(G r mu) (=: Ip S_t), so
-//   gamma_t = gamma_{t+1} + Ip S_t - <dv_t, v_t> - <db_t, b_t>
-// inside a step, from fp32 row sums (with the uncertainty's gradient Go = scale dovar q^2, one more term - sum(Go r)): per
-// state entry and token it costs the one addition of S.  gamma of the first token of the next step is formed from its
-// definition, so that what the recomputed states are off by does not add up over the steps.
+// Gate: gamma_t = f_t (<dM_t, M_{t-1}> + <dJ_t, J_{t-1}>), formed as it stands: where a token decays strongly, what is left of
+// the state is of the order of f_t, and so is gamma.  (The states of the step are in registers, so that it takes two
+// instructions per entry and token and the one that makes I out of J.  gamma_{t+1} + Ip sum(G r mu) - <dv_t, v_t> - <db_t, b_t>
+// is the same number for one addition, but as a difference of terms of order 1: with every fifth token at f = e^-18 the
+// gradients of these tokens were off by 200 times their size in fp32.  The definition costs 531 -> 555 us at B=8 T=2048 H=12
+// 64x64; fp32 rows B=8 T=2048 H=8 64x64 went from 636 to 612, since the reciprocals of a token are now taken beside its
+// products instead of with the forward sweep.)  The first token of a step sees the state after the step before it in time:
+// its gamma is formed there, that of the tile's first token from the state at the start of the tile.
 #pragma once
 #include <type_traits>
-
 
 #include "chunk_bwd.h"
 #include "pal_host.h"
@@ -64,8 +66,8 @@ __device__ __forceinline__ float pair_bit2(float x, float y) {
 //     lanes of row g get p_g and q_g.
 template <int DT, int DN>
 struct TokSums {
-  float o[2 * DN], p[4], q[4], S, X;
-  float y0, y1, y2, y3, z0, z1, sx;
+  float o[2 * DN], p[4], q[4], X;
+  float y0, y1, y2, y3, z0, z1;
   __device__ __forceinline__ void stage_a() {
     if constexpr (DN == 4) {
       asm("s_nop 1\n\t"
@@ -119,7 +121,6 @@ struct TokSums {
     } else {
       asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(p[0]), "+v"(p[1]));
     }
-    sx = pair_bit3(S, X);
   }
   __device__ __forceinline__ void stage_c() {
     asm("s_nop 1\n\t"
@@ -140,10 +141,6 @@ __device__ __forceinline__ float dpp_quad(float x) {
 __device__ __forceinline__ float quad_sum(float x) {
   x += dpp_quad<0xB1>(x);    // quad_perm [1,0,3,2]
   return x + dpp_quad<0x4E>(x);   // quad_perm [2,3,0,1]
-}
-// x <- x f + c in one instruction (the compiler would copy c first and accumulate into the copy)
-__device__ __forceinline__ void fma3(float& x, float f, float c) {
-  asm("v_fma_f32 %0, %0, %1, %2" : "+v"(x) : "v"(f), "v"(c));
 }
 
 template <typename TIn>
@@ -167,14 +164,13 @@ __device__ __forceinline__ void lds_vals(const float* p, float* out) {
   }
 }
 
-// what both sweeps read of a token: its k, v, b, and (f, (1 - f) Ip)
+// what both sweeps read of a token: its k, v, b and f
 template <int DT>
 struct TokFwd {
   f32x4 k;
-  float v[DT], b[DT];
-  f32x2 fc;
-  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* pfc, int plane) {
-    fc = *(const f32x2*)pfc;
+  float v[DT], b[DT], f;
+  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* pf, int plane) {
+    f = *pf;
     k = *(const f32x4*)kq;
     lds_vals<DT>(vb, v);
     lds_vals<DT>(vb + plane, b);
@@ -185,11 +181,11 @@ template <int DT, bool VAR>
 struct TokRev {
   f32x4 q;
   float d_o[DT], d_ov[VAR ? DT : 1], fn;
-  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* pfc, int plane) {
+  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* pf, int plane) {
     q = *(const f32x4*)(kq + 16);
     lds_vals<DT>(vb + 2 * plane, d_o);
     if constexpr (VAR) lds_vals<DT>(vb + 3 * plane, d_ov);
-    fn = pfc[2];
+    fn = pf[1];
   }
 };
 
@@ -211,7 +207,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   constexpr int kG = tile_g(DT, DN), kSub = kC / kG;   // tokens per step, steps per tile
   constexpr bool BOTH = L.both != 0;
   float* sC = smem;
-  float* sFC = smem + L.oFC;
+  float* sF = smem + L.oF;
   float* sW = smem + L.oW;
   float* sFB = smem + L.oFB;
   float* sX = smem + L.oX;
@@ -233,7 +229,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   const int64_t tile_off = ((int64_t)cidx * H + h) * dv * dk;
   float* base = smem + L.oBase + w * (2 * DT * 256) + 4 * lane;   // + 256 per piece of 16 value rows: M, then I
   const int last = (clen - 1) / kG;
-  float ssum = 0.f;   // wave 0, lanes with bit kG clear: sums of S
+  float ssum = 0.f;   // sum of S over the tile's tokens
 
   const int n0 = R.n0, r0 = R.r0;              // first key column, value row of the launch
   const int nw = n0 + WC * w;                  // of the wave (a lane has DN of its columns, from DN g on)
@@ -354,16 +350,16 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         kt[j] = ok ? x : (TIn)0.f;
       }
     };
-    float M[DT][DN], I[DT][DN];
+    float M[DT][DN], J[DT][DN];   // J = I - Ip
     // state before step `row` (or after token 31) from the base state in LDS
     auto state_at = [&](int row, const bf16_t* T) {
-      const float fb = sFB[row], cI = (1.f - fb) * Ip;
-      f32x4 accM[DT], accI[DT];
+      const float fb = sFB[row];
+      f32x4 accM[DT], accJ[DT];
 #pragma unroll
       for (int x = 0; x < DT; ++x) {
         const f32x4 m = *(const f32x4*)(base + 256 * x), y = *(const f32x4*)(base + 256 * (DT + x));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) { accM[x][r] = fb * m[r]; accI[x][r] = fmaf(fb, y[r], cI); }
+        for (int r = 0; r < 4; ++r) { accM[x][r] = fb * m[r]; accJ[x][r] = fb * y[r]; }
       }
       if (row == kSub || (row & (kSub / 2 - 1)) != 0) {
         const f32x4 w0 = *(const f32x4*)&sW[row * kHalf + 8 * g], w1 = *(const f32x4*)&sW[row * kHalf + 8 * g + 4];
@@ -392,17 +388,17 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           if constexpr (F32) {
             const bf16x8 Vl = *(const bf16x8*)(p + (DS + 16 * x) * kHS), Bl = *(const bf16x8*)(p + (3 * DS + 16 * x) * kHS);
             accM[x] = mfma16_split(K1, K1l, V, Vl, accM[x]);
-            accI[x] = mfma16_split(K2, K2l, B, Bl, accI[x]);
+            accJ[x] = mfma16_split(K2, K2l, B, Bl, accJ[x]);
           } else {
             accM[x] = mfma16(K1, V, accM[x]);
-            accI[x] = mfma16(K2, B, accI[x]);
+            accJ[x] = mfma16(K2, B, accJ[x]);
           }
         }
       }
 #pragma unroll
       for (int x = 0; x < DT; ++x)
 #pragma unroll
-        for (int r = 0; r < DN; ++r) { M[x][r] = accM[x][r]; I[x][r] = accI[x][r]; }
+        for (int r = 0; r < DN; ++r) { M[x][r] = accM[x][r]; J[x][r] = accJ[x][r]; }
     };
     // base state of the first half: the state at the start of the tile
     struct BaseIn { f32x4 m[DT], y[DT]; };
@@ -433,7 +429,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
 #pragma unroll
       for (int x = 0; x < DT; ++x) {
 #pragma unroll
-        for (int r = 0; r < DN; ++r) z.m[x][r] *= z.y[x][r];
+        for (int r = 0; r < DN; ++r) { z.m[x][r] *= z.y[x][r]; z.y[x][r] -= Ip; }
         *(f32x4*)(base + 256 * x) = z.m[x];
         *(f32x4*)(base + 256 * (DT + x)) = z.y[x];
       }
@@ -465,15 +461,15 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         store_vec<4>(flush_at(j, it), (const float*)&x);
       }
     };
-    // wave 0: the waves' sums of a step, lane = 2 kG n + t (t: S of its tokens, then X)
+    // wave 0: a step's gates, of the first token of the step after in the place of its own first
     auto flush_xs = [&](int j) {
-      const float* p = smem + L.oXS + (j & 1) * NBW * 2 * kG + lane;
-      float x = lane < 2 * kG * NBW ? p[0] : 0.f;
-      if constexpr (2 * kG * NBW > 64) x += lane + 64 < 2 * kG * NBW ? p[64] : 0.f;
-      ssum += x;
-      if constexpr (kG == 4) x += row_ror<8>(x);
-      x = rows4_sum(x);
-      if (lane >= kG && lane < 2 * kG) sX[kG * j + lane - kG] += x;
+      if (lane < kG) {
+        const float* p = smem + L.oXS + (j & 1) * NBW * kG + lane;
+        float x = p[0];
+#pragma unroll
+        for (int y = 1; y < NBW; ++y) x += p[y * kG];
+        sX[kG * j + (lane ? lane : kG)] = x;
+      }
     };
 
     // Everything the pass starts from is requested at once.
@@ -497,11 +493,10 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         const float c = wave_inclusive_scan(-gt * gh, lane);
         sC[lane] = c;
         sX[lane] = 0.f;
-        const float f = fast_exp2(-gt * gh);
-        *(f32x2*)&sFC[2 * lane] = f32x2{f, (1.f - f) * Ip};
+        sF[lane] = fast_exp2(-gt * gh);
         if (lane == 63) {
           A.wFtot[(int64_t)cidx * H + h] = c;
-          *(f32x2*)&sFC[2 * kC] = f32x2{1.f, 0.f};
+          sF[kC] = 1.f;
         }
       }
       __syncthreads();
@@ -527,7 +522,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
 #pragma unroll
         for (int x = 0; x < DT; ++x) {
           *(f32x4*)(base + 256 * x) = f32x4{M[x][0], M[x][1], M[x][2], DN == 4 ? M[x][DN - 1] : 0.f};
-          *(f32x4*)(base + 256 * (DT + x)) = f32x4{I[x][0], I[x][1], I[x][2], DN == 4 ? I[x][DN - 1] : 1.f};
+          *(f32x4*)(base + 256 * (DT + x)) = f32x4{J[x][0], J[x][1], J[x][2], DN == 4 ? J[x][DN - 1] : 0.f};
         }
         if constexpr (!BOTH) __syncthreads();
       }
@@ -589,57 +584,42 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       }
       const float* krow = smem + L.oKQ + ((j & 1) * NBW + w) * kG * 32 + 4 * g;
       const float* vrow = smem + L.oVB + (j & 1) * kG * SV + i * DTP;
-      const float* fcs = sFC + 2 * kG * j;
+      const float* fs = sF + kG * j;
       const int o_tok = kG * j * (int)dks;   // (64 tokens of a tile stay within 32 bits)
-      float mu[kG][DT][DN], rI[kG][DT][DN];
-      // ---- forward over the step; a token's operands are requested during the burst of the token before it
+      float sM[kG][DT][DN], sJ[kG][DT][DN];   // state after each token; in reverse mu and 1 / I in their place
+      // ---- forward over the step; a token's operands are requested during the arithmetic of the token before it
       TokFwd<DT> xf[kG], xr[kG];
       TokRev<DT, VAR> yr[kG];
-      xf[0].load(krow, vrow, fcs, plane);
+      xf[0].load(krow, vrow, fs, plane);
 #pragma unroll
       for (int u = 0; u < kG; ++u) {
         const TokFwd<DT>& x = xf[u];
+        __builtin_amdgcn_sched_barrier(0);
+        if (u + 1 < kG) xf[u + 1].load(krow + (u + 1) * 32, vrow + (u + 1) * SV, fs + u + 1, plane);
+        else yr[u].load(krow + u * 32, vrow + u * SV, fs + u, plane);
 #pragma unroll
         for (int r = 0; r < DN; ++r) {
           const float kk = x.k[r] * x.k[r];
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
-            M[d][r] = fmaf(x.v[d], x.k[r], M[d][r] * x.fc[0]);
-            fma3(I[d][r], x.fc[0], x.fc[1]);
-            I[d][r] = fmaf(x.b[d], kk, I[d][r]);
+            sM[u][d][r] = fmaf(x.v[d], x.k[r], (u ? sM[u ? u - 1 : 0][d][r] : M[d][r]) * x.f);
+            sJ[u][d][r] = fmaf(x.b[d], kk, (u ? sJ[u ? u - 1 : 0][d][r] : J[d][r]) * x.f);
           }
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (u + 1 < kG) xf[u + 1].load(krow + (u + 1) * 32, vrow + (u + 1) * SV, fcs + 2 * (u + 1), plane);
-        else yr[u].load(krow + u * 32, vrow + u * SV, fcs + 2 * u, plane);
-        __builtin_amdgcn_s_setprio(3);
-#pragma unroll
-        for (int r = 0; r < DN; ++r)
-#pragma unroll
-          for (int d = 0; d < DT; ++d) {
-            rI[u][d][r] = fast_rcp(I[d][r]);
-            asm volatile("" : "+v"(rI[u][d][r]));   // here, not where the reverse sweep uses it
-          }
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int r = 0; r < DN; ++r)
-#pragma unroll
-          for (int d = 0; d < DT; ++d) {
-            mu[u][d][r] = M[d][r] * rI[u][d][r];
-            asm volatile("" : "+v"(mu[u][d][r]));
-          }
       }
-      // what the gate of the next step's first token sees of the states after this step
+      __builtin_amdgcn_sched_barrier(0);
+      // the gate of the first token of the step after, which saw the state after this one
       float next_gate = 0.f;
 #pragma unroll
       for (int r = 0; r < DN; ++r)
 #pragma unroll
-        for (int d = 0; d < DT; ++d) next_gate = fmaf(dM[d][r], M[d][r], fmaf(dJ[d][r], I[d][r] - Ip, next_gate));
-      next_gate *= fcs[2 * kG];
+        for (int d = 0; d < DT; ++d) next_gate = fmaf(dM[d][r], sM[kG - 1][d][r], fmaf(dJ[d][r], sJ[kG - 1][d][r], next_gate));
+      next_gate *= fs[kG];
+      asm volatile("" : "+v"(next_gate));
+      __builtin_amdgcn_sched_barrier(0);
       // ---- and in reverse
       float* part = smem + L.oPart + ((j & 1) * NBW + w) * (kG * 32 * DT);
-      float xs[kG / 2], oz[kG][2], was[kG][2];
+      float xs[kG / 2], xo, oz[kG][2], was[kG][2], S = 0.f;
       if constexpr (SLICE == 2) acc_load(kG * j + kG - 1, was[kG - 1]);
       TokSums<DT, DN> ts[2];
       auto finish = [&](int u, TokSums<DT, DN>& z) {
@@ -655,8 +635,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         } else {
           if (lane < 32 * DT) pu[lane] = z.p[0];
         }
-        if (u & 1) xs[u >> 1] = z.sx;
-        else xs[u >> 1] = quad_sum(pair_bit2(z.sx, xs[u >> 1]));
+        if (u & 1) xo = z.X;
+        else xs[u >> 1] = pair_bit3(z.X, xo);
       };
 #pragma unroll
       for (int u = kG - 1; u >= 0; --u) {
@@ -664,7 +644,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         if constexpr (SLICE == 2) { if (u > 0) acc_load(kG * j + u - 1, was[u - 1]); }
         const TokFwd<DT>& x = u + 1 < kG ? xr[u] : xf[u];
         const TokRev<DT, VAR>& y = yr[u];
-        float dq[DN], dqv[DN], dkM[DN], dkJ[DN], dvp[DT], dbp[DT], S = 0.f, U = 0.f;
+        float dq[DN], dqv[DN], dkM[DN], dkJ[DN], dvp[DT], dbp[DT], gate = 0.f;
         TokSums<DT, DN>& before = ts[(u + 1) & 1];   // of the token worked before this one
         if (u + 1 < kG) before.stage_a();
 #pragma unroll
@@ -673,19 +653,27 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           if (r == 1 && u + 1 < kG) before.stage_b();
           if (r == 2 && u + 1 < kG) finish(u + 1, before);
           if (r == DN - 2 && u > 0) {   // half of mu, r of this token are dead: room for the next token's operands
-            xr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, fcs + 2 * (u - 1), plane);
-            yr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, fcs + 2 * (u - 1), plane);
+            xr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, fs + u - 1, plane);
+            yr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, fs + u - 1, plane);
           }
+          __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+          for (int d = 0; d < DT; ++d) {
+            sJ[u][d][r] = fast_rcp(sJ[u][d][r] + Ip);
+            asm volatile("" : "+v"(sJ[u][d][r]));
+          }
+          __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+          for (int d = 0; d < DT; ++d) sM[u][d][r] *= sJ[u][d][r];
           const float kk = x.k[r] * x.k[r], q2 = y.q[r] * y.q[r];
 #pragma unroll
           for (int d = 0; d < DT; ++d) {
-            const float p = y.d_o[d] * y.q[r], ri = rI[u][d][r], m = mu[u][d][r];
+            const float p = y.d_o[d] * y.q[r], ri = sJ[u][d][r], m = sM[u][d][r];
             const float dl = p * ri;
             float t;
             if constexpr (VAR) {
               const float go = y.d_ov[d] * q2;
               t = fmaf(go, ri, p * m) * ri;
-              U = fmaf(go, ri, U);
               dqv[r] = d ? fmaf(y.d_ov[d], ri, dqv[r]) : y.d_ov[d] * ri;
             } else {
               t = dl * m;
@@ -693,6 +681,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
             dM[d][r] = fmaf(dM[d][r], y.fn, dl);
             dJ[d][r] = fmaf(dJ[d][r], y.fn, -t);
             S += t;
+            if (u > 0) gate = fmaf(dM[d][r], sM[u ? u - 1 : 0][d][r], fmaf(dJ[d][r], sJ[u ? u - 1 : 0][d][r], gate));
             dq[r] = d ? fmaf(m, y.d_o[d], dq[r]) : m * y.d_o[d];
             dkM[r] = d ? fmaf(dM[d][r], x.v[d], dkM[r]) : dM[d][r] * x.v[d];
             dkJ[r] = d ? fmaf(dJ[d][r], x.b[d], dkJ[r]) : dJ[d][r] * x.b[d];
@@ -701,15 +690,12 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           }
         }
         TokSums<DT, DN>& mine = ts[u & 1];
-        mine.S = S;
-        mine.X = fmaf(Ip, S, u + 1 < kG ? -U : next_gate - U);
+        mine.X = u > 0 ? x.f * gate : next_gate;
+        asm volatile("" : "+v"(S), "+v"(mine.X));
 #pragma unroll
         for (int r = 0; r < DN; ++r) {
           mine.o[r] = VAR ? fmaf(2.f * y.q[r], dqv[r], dq[r]) : dq[r];
-          // <dv, v> + <db, b> = sum over the columns of k (dkM + k dkJ)
-          const float e = fmaf(x.k[r], dkJ[r], dkM[r]);
-          mine.X = fmaf(-x.k[r], e, mine.X);
-          mine.o[DN + r] = fmaf(x.k[r], dkJ[r], e);
+          mine.o[DN + r] = fmaf(2.f * x.k[r], dkJ[r], dkM[r]);
         }
         if constexpr (DT >= 3) {
 #pragma unroll
@@ -750,17 +736,22 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           }
         }
       }
-      // (S, X) by lane bit 3, odd token of a pair by bit 2, pair of tokens by lane row (kG = 4: by bit 5)
-      if constexpr (kG == 4) {
-        float x0 = xs[0], x1 = xs[1];
-        swap_halves(x0, x1);
-        float s = x0 + x1, t = s;
-        swap_rows(s, t);
-        s += t;
-        if ((lane & 19) == 0) smem[L.oXS + ((j & 1) * NBW + w) * 8 + ((lane >> 3) & 1) * 4 + (lane >> 5) * 2 + ((lane >> 2) & 1)] = s;
-      } else {
-        const float s = rows4_sum_x4(xs[0], xs[1], xs[kG / 2 - 2], xs[kG / 2 - 1]);
-        if ((lane & 3) == 0) smem[L.oXS + ((j & 1) * NBW + w) * 16 + ((lane >> 3) & 1) * 8 + (lane >> 4) * 2 + ((lane >> 2) & 1)] = s;
+      ssum += S;
+      // gates: odd token of a pair by lane bit 3, pair of tokens by bit 2 (kG = 8: four of them by bit 5)
+      {
+        float x = quad_sum(pair_bit2(xs[0], xs[1]));
+        if constexpr (kG == 8) {
+          float y = quad_sum(pair_bit2(xs[kG / 2 - 2], xs[kG / 2 - 1]));
+          swap_halves(x, y);
+          x += y;
+          y = x;
+          swap_rows(x, y);
+          x += y;
+        } else {
+          x = rows4_sum(x);
+        }
+        if ((lane & (kG == 8 ? 19 : 51)) == 0)
+          smem[L.oXS + ((j & 1) * NBW + w) * kG + (kG == 8 ? (lane >> 5) * 4 : 0) + ((lane >> 2) & 1) * 2 + ((lane >> 3) & 1)] = x;
       }
       if (j > 0) deposit(j - 1);
       __syncthreads();
@@ -773,8 +764,24 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       for (int it = it0; it < nF; it += NT) { flush_sum(0, it, x, fw); flush_store(0, it, x, fw); }
       if (w == 0) flush_xs(0);
     }
+    // gate of the tile's first token, which saw the state at the start of the tile
+    {
+      float y0 = 0.f;
+#pragma unroll
+      for (int x = 0; x < DT; ++x) {
+        const f32x4 m = *(const f32x4*)(base + 256 * x), y = *(const f32x4*)(base + 256 * (DT + x));
+#pragma unroll
+        for (int r = 0; r < DN; ++r) y0 = fmaf(dM[x][r], m[r], fmaf(dJ[x][r], y[r], y0));
+      }
+      y0 = wave_sum(y0);
+      ssum = wave_sum(ssum);
+      if (lane == 0) {   // (the second buffer of partial sums is free)
+        smem[L.oXS + NBW * kG + w] = y0;
+        smem[L.oXS + NBW * kG + NBW + w] = ssum;
+      }
+    }
     // carry handed to the previous tile
-    const float f_first = sFC[0];
+    const float f_first = sF[0];
     int lx = lane;
     asm volatile("" : "+v"(lx));
     const int ci = lx & 15, cn = nw + DN * (lx >> 4);
@@ -798,14 +805,11 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   }
   __syncthreads();
   if (w == 0) {
-    // gamma_t = sum of X over the tokens of its step from t on; the launches add up
-    float x = sX[lane];
-    const float tot = -wave_sum((lane & kG) ? 0.f : ssum);
+    const float* p = smem + L.oXS + NBW * kG;
+    float x = p[0], tot = -p[NBW];
 #pragma unroll
-    for (int o = 1; o < kG; o <<= 1) {
-      const float y = __shfl_down(x, o);
-      if ((lane & (kG - 1)) + o < kG) x += y;
-    }
+    for (int y = 1; y < NBW; ++y) { x += p[y]; tot -= p[NBW + y]; }
+    x = lane ? sX[lane] : sF[0] * x;
     float* pe = A.wE + (int64_t)h * A.tokens + t0 + lane;
     float* ps = A.wSig + (int64_t)cidx * H + h;
     const bool add = R.flags & (kRectRowsBefore | kRectColsBefore);

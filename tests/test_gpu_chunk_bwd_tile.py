@@ -42,3 +42,32 @@ def test_tile_kernel_launches(gpu_device, dk, dv, rows):
         for n, x in zip(leaves, got):
             err = hp.max_rel(x, ref[n])
             assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (T, var, init, n, err)
+
+
+@pytest.mark.parametrize("dk,dv", [(16, 16), (32, 32), (48, 48), (64, 64), (80, 80), (96, 128)])
+@pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_gate_gradient_of_strongly_decaying_tokens(gpu_device, dk, dv, rows):
+    """dgt_t is f_t times a number of the order of the other gradients (what flows back against the state before the
+    token), however small f_t is: that number is held to the bar of the other gradients, entry by entry.  Where there is
+    no state before a token its gradient is exactly zero."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    H, T = 2, 150
+    inp = hp.rounded(po.make_inputs(1, T, H, dk, dv, seed=dk + dv), rows)
+    inp["g"] = torch.tensor([1.0, 2.0])
+    inp["gt"][:, ::5] = 9.0                     # f = e^-9, e^-18
+    for var in (False, True):
+        gen = torch.Generator().manual_seed(T)
+        o_ref, _, _, _ = hp.oracle_forward(inp, dtype=torch.float64)
+        do = (o_ref - 0.3 * torch.randn(1, T, H, dv, generator=gen)).float()
+        dov = 0.3 * torch.randn(1, T, H, dv, generator=gen) if var else None
+        ref = hp.oracle_grads(inp, do, dov)["gt"]
+        leaves = [inp[n].to(gpu_device).requires_grad_(True) for n in NAMES]
+        out = chunk_palimpsa(*leaves, output_uncertainty=var)
+        loss = ((out[0] if var else out).float() * do.to(gpu_device)).sum()
+        if var:
+            loss = loss + (out[1].float() * dov.to(gpu_device)).sum()
+        dgt = torch.autograd.grad(loss, leaves[4])[0].double().cpu()
+        assert bool((dgt[:, 0] == 0).all())
+        f = torch.exp(-inp["gt"].double() * inp["g"].double())
+        err = hp.max_rel(dgt / f, ref / f)
+        assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (var, err)
