@@ -15,7 +15,8 @@ struct BwdArgs {
   float* wE;              // [H, tokens]  local part of d log f
   float* wInitPart;       // [n_seqs,H,dv*dk/256] partial sums of dJ_0
   float* wDgTile;         // [total_chunks,H] the tiles' shares of dg
-  float* wQK;             // [tokens,H,2,dk] dq, dk summed so far, where a tile takes several slices of value rows (bf16 rows)
+  float* wQK;             // [tokens,H,2,cols] dq, dk of a column group summed so far, where a tile takes several slices of
+                          // value rows (bf16 rows); the column groups follow each other, so one group's worth is kept
   int32_t tokens;
   int32_t apply_alias;     // carry apply: db^carry shares LDS with the bf16 carries (large head dims)
 };

@@ -620,12 +620,12 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 static BwdLayout bwd_layout(const PalDims* d) {
   BwdLayout L;
-  const size_t E = (size_t)d->dv * d->dk;
+  const size_t E = (size_t)d->dv * d->dk, row = d->dtype == PAL_DTYPE_BF16 ? 2 : 4;
   const size_t tiles = (size_t)d->total_chunks * d->n_heads;
   const size_t tokens = (size_t)d->batch * d->seq_len;
   size_t o = 0;
-  L.oDM = o; o = align256(o + tiles * E * 4);
-  L.oDJ = o; o = align256(o + tiles * E * 4);
+  L.oDM = o; o = align256(o + tiles * E * row);
+  L.oDJ = o; o = align256(o + tiles * E * row);
   L.oFtot = o; o = align256(o + tiles * 4);
   L.oSig = o; o = align256(o + tiles * 4);
   L.oE = o; o = align256(o + tokens * d->n_heads * 4);
@@ -633,12 +633,13 @@ static BwdLayout bwd_layout(const PalDims* d) {
   L.oDgTile = o; o = align256(o + tiles * 4);
   L.oDqFull = L.oDkFull = o;
   if (d->n_qk_heads > 0 && d->n_qk_heads != d->n_heads) {
-    const size_t full = tokens * d->n_heads * d->dk * (d->dtype == PAL_DTYPE_BF16 ? 2 : 4);
+    const size_t full = tokens * d->n_heads * d->dk * row;
     L.oDqFull = o; o = align256(o + full);
     L.oDkFull = o; o = align256(o + full);
   }
   L.oQK = o;
-  if (tile_rows(tile_piece(d->dk), d->dv) < d->dv && d->dtype == PAL_DTYPE_BF16) o = align256(o + tokens * d->n_heads * d->dk * 2 * 4);
+  const int cols = tile_piece(d->dk);   // (the first column group, the widest)
+  if (tile_rows(cols, d->dv) < d->dv && d->dtype == PAL_DTYPE_BF16) o = align256(o + tokens * d->n_heads * cols * 2 * 4);
   L.total = o;
   return L;
 }

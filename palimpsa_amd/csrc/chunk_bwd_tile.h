@@ -539,12 +539,14 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     const int oc = nw + DN * (lo >> 4) + 2 * ((lo >> 2) & 1), ow = (lo >> 3) & 1;
     const bool out2 = DN == 4 || (lo & 4) == 0;
     TIn* const po = (TIn*)(ow ? A.dk : A.dq) + tok0 * dk + oc;
-    float* const pacc = A.wQK + tok0 * (2 * dk) + ow * dk + oc;   // bf16 rows: sums over the launches so far
+    // bf16 rows: sums over the launches so far
+    float* const pacc = A.wQK + tok0 * (2 * DNG) + ow * DNG + (oc - n0);
+    const int accs = 2 * DNG * H;   // per token
     const bool out_on = (lane & 3) == 0;
     // SLICE 2: what the launches over earlier value rows left for a token, requested two tokens ahead of its use
     auto acc_load = [&](int t, float* was) {
-      const int o = (t < clen ? t : 0) * (int)dks;
-      const float* acc = F32 ? (const float*)po + o : pacc + 2 * o;
+      t = t < clen ? t : 0;
+      const float* acc = F32 ? (const float*)po + t * (int)dks : pacc + t * accs;
       was[0] = acc[0];
       was[1] = acc[out2 ? 1 : 0];
     };
@@ -719,7 +721,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
             bool done = true;
             if constexpr (SLICE != 0 && !F32) {   // the value rows of the launches add up, in fp32
               if (R.flags & kRectRowsAfter) {
-                float* acc = pacc + 2 * (o_tok + u * (int)dks);
+                float* acc = pacc + (kG * j + u) * accs;
                 acc[0] = oz[u][0];
                 if (out2) acc[1] = oz[u][1];
                 done = false;

@@ -347,3 +347,16 @@ def test_build_covers_the_host_module(monkeypatch):
     monkeypatch.setattr(build, "_host_stamp", lambda: "torch 0")
     with pytest.raises(Ran):
         build.build_host()
+
+
+def test_chunk_bwd_workspace_of_bf16_rows(L):
+    """bf16 rows: two carries per tile and head in the rows' dtype, and where a tile takes several slices of value rows
+    the fp32 sums of dq, dk over them for one group of key columns at a time; a few words per token and tile beside."""
+    lib = L.load()
+    T, H = 32768, 16
+    tiles = T // 64
+    for dk, dv, cols in ((64, 64, 0), (96, 64, 0), (96, 96, 64), (128, 128, 64), (80, 80, 48), (48, 96, 48), (96, 192, 64)):
+        d = _dims(L, batch=1, seq_len=T, n_seqs=1, n_heads=H, dk=dk, dv=dv, total_chunks=tiles)
+        carries, sums, rest = 2 * tiles * H * dk * dv * 2, T * H * 2 * cols * 4, T * H * 4 + 4 * tiles * H * 4 + 16 * 1024
+        need = lib.pal_chunk_bwd_workspace_bytes(d)
+        assert carries + sums <= need <= carries + sums + rest, (dk, dv, need)
