@@ -17,6 +17,9 @@ struct BwdArgs {
   float* wDgTile;         // [total_chunks,H] the tiles' shares of dg
   float* wQK;             // [tokens,H,2,cols] dq, dk of a column group summed so far, where a tile takes several slices of
                           // value rows (bf16 rows); the column groups follow each other, so one group's worth is kept
+  // a small pass: every rectangle's parts, summed by chunk_bwd_parts_sum_kernel
+  float *pQK, *pVB;       // [slices][tokens,H,2,dk] dq, dk; [column groups][tokens,H,2,dv] dv, db
+  float *pE, *pSig;       // [rectangles][H,tokens], [rectangles][total_chunks,H]
   int32_t tokens;
   int32_t apply_alias;     // carry apply: db^carry shares LDS with the bf16 carries (large head dims)
 };
@@ -30,10 +33,48 @@ struct BwdArgs {
 // 32x32), 1.8 (16x16): hence 96 rows as 48 + 48, where neither piece pays for a small one.)
 struct TileRect {
   int n0, cols, r0, flags;
+  int group, groups, slices;   // small pass: first column group, their number (grid z), slices of value rows (grid y)
 };
-constexpr int kRectColsBefore = 1, kRectRowsBefore = 2, kRectRowsAfter = 4;   // launches that came before, come after
+constexpr int kRectColsBefore = 1, kRectRowsBefore = 2, kRectRowsAfter = 4, kRectParts = 8;   // launches that came before, come after; a small pass
 inline int tile_piece(int n) { return n == 80 ? 48 : n >= 64 ? 64 : n; }
 inline int tile_rows(int cols, int n) { return cols == 16 ? (n >= 48 ? 48 : 16) : n == 96 ? 48 : tile_piece(n); }   // (16 columns: one wave's staging)
+
+// A pass with too few tiles to fill the chip: all rectangles of a group width in one launch, side by side, each with
+// outputs of its own that a last kernel adds up in a fixed order.  One after the other they cost a tile's serial latency
+// each, however few workgroups there are.  The slices are small, since it is latency that counts; the group width is one
+// that divides the head, if there is one, so that one launch takes them all.  Measured, in us (tile kernel and sum, one
+// after the other -> side by side), bf16 rows, by tiles x heads:
+//            64          256         384         512         768
+//   80x80    225 -> 100  234 -> 160  288 -> 228  293 -> 280  387 -> 392
+//   96x96    277 ->  69  285 -> 175  356 -> 253  360 -> 330  475 -> 491
+//   96x192   472 -> 103  484 -> 326  625 -> 489  631 -> 649  843 -> 976
+//   128x128  307 ->  72  314 -> 233  417 -> 338  425 -> 449  664 -> 667
+//   112x112  283 -> 104  293 -> 253  382 -> 377  389 -> 477  610 -> 701
+//   48x96    125 ->  55  128 -> 102  163 -> 149  165 -> 173  260 -> 255
+//   128x64   148 ->  57  149 -> 122  205 -> 178  208 -> 231  316 -> 340
+// fp32 rows 96x96 288 -> 70, 301 -> 184, 382 -> 266, 387 -> 355, 631 -> 528.  The line lies at one and a half workgroups per
+// compute unit; at two for fp32 rows and for heads whose pieces come out small (80x80, 96x96), which are the dearest one after the other.
+// It bounds the parts too: 8 bytes per token, head, slice and key column, and per group and value column (190 MB at most at 96x192).
+constexpr int kPartsTiles = 384, kPartsTilesSmall = 512;   // tiles x heads
+struct TileParts {
+  int on, rows, slices, groups;
+};
+inline int parts_cols(int dk, int n0) { return dk % 64 == 0 ? 64 : dk % 48 == 0 ? 48 : dk % 32 == 0 ? 32 : tile_piece(dk - n0); }
+inline TileParts tile_parts(int dk, int dv, bool f32, int64_t tile_heads) {
+  TileParts P;
+  P.rows = dk > 16 && dv % 32 == 0 ? 32 : 16;
+  P.slices = dv / P.rows;
+  P.groups = 0;
+  for (int n0 = 0; n0 < dk; n0 += parts_cols(dk, n0)) ++P.groups;
+  int pieces = 0;   // one after the other
+  for (int n0 = 0, c; n0 < dk; n0 += c) {
+    c = tile_piece(dk - n0);
+    for (int r0 = 0; r0 < dv; r0 += tile_rows(c, dv - r0)) ++pieces;
+  }
+  const bool small = f32 || dk * dv <= pieces * 48 * 48;
+  P.on = pieces > 1 && tile_heads <= (small ? kPartsTilesSmall : kPartsTiles);
+  return P;
+}
 
 constexpr int kHalf = 32;          // tokens of a half tile: the contraction length of one matrix instruction
 constexpr int kHS = kHalf + 8;     // row stride (bf16) of the transposed half tiles: 16-byte reads stay aligned
@@ -76,6 +117,6 @@ __host__ __device__ constexpr TileLds tile_lds(int DT, int DN, int nbw, bool var
 }
 
 template <typename TIn, bool VAR>
-int launch_tile_t(const BwdArgs& A, hipStream_t s);   // chunk_bwd_tile_*.hip
+int launch_tile_t(const BwdArgs& A, const TileParts& P, hipStream_t s);   // chunk_bwd_tile_*.hip
 
 }  // namespace pal

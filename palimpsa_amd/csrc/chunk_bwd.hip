@@ -571,8 +571,46 @@ __global__ __launch_bounds__(64) void chunk_bwd_head_reduce_kernel(BwdArgs A) {
   }
 }
 
+// A small pass: sums the rectangles' parts, slices of value rows for dq and dk, column groups for dv and db, both for the gates
+// and the tiles' sums, each in one order.  A thread takes four consecutive entries of a (token, head) row, or one gate.
+template <typename TIn>
+__global__ __launch_bounds__(256) void chunk_bwd_parts_sum_kernel(BwdArgs A, int slices, int groups) {
+  const int dk = A.c.dk, dv = A.c.dv, H = A.c.H;
+  const int64_t rows = (int64_t)A.tokens * H, tiles = (int64_t)A.c.total_chunks * H;
+  const int per = (dk + dv) >> 1;   // groups of four in the rows of dq, dk, dv, db
+  int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx < rows * per) {
+    const int64_t row = idx / per;
+    const int it = (int)(idx - row * per), vb = it >= dk >> 1;
+    const int len = vb ? dv : dk, e = 4 * (vb ? it - (dk >> 1) : it), second = e >= len;
+    const float* p = (vb ? A.pVB : A.pQK) + row * 2 * len + e;
+    f32x4 x = *(const f32x4*)p;
+    for (int y = 1; y < (vb ? groups : slices); ++y) x += *(const f32x4*)(p + y * rows * 2 * len);
+    TIn* o = (TIn*)(vb ? (second ? A.db : A.dv) : (second ? A.dk : A.dq)) + row * len + (second ? e - len : e);
+    store_vec<4>(o, (const float*)&x);
+    return;
+  }
+  idx -= rows * per;
+  const float* p = idx < rows ? A.pE + idx : A.pSig + (idx - rows);
+  if (idx >= rows + tiles) return;
+  float x = 0.f;
+  for (int y = 0; y < slices * groups; ++y) x += p[y * (idx < rows ? rows : tiles)];
+  if (idx < rows) A.wE[idx] = x;
+  else A.wSig[idx - rows] = x;
+}
+
+static int launch_parts_sum(const BwdArgs& A, const TileParts& P, bool bf16, hipStream_t s) {
+  const int64_t rows = (int64_t)A.tokens * A.c.H;
+  const int64_t blocks = (rows * ((A.c.dk + A.c.dv) / 2) + rows + (int64_t)A.c.total_chunks * A.c.H + 255) / 256;
+  if (blocks > 0x7fffffff) return PAL_E_DIM;
+  if (bf16) PAL_TIMED_LAUNCH(kKernBwdPartsSum, s, chunk_bwd_parts_sum_kernel<bf16_t>, dim3((unsigned)blocks), dim3(256), 0, s, A, P.slices, P.groups);
+  else PAL_TIMED_LAUNCH(kKernBwdPartsSum, s, chunk_bwd_parts_sum_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, s, A, P.slices, P.groups);
+  PAL_HIP_LAUNCH_CHECK();
+  return PAL_OK;
+}
+
 struct BwdLayout {
-  size_t oDM, oDJ, oFtot, oSig, oE, oInit, oDgTile, oDqFull, oDkFull, oQK, total;
+  size_t oDM, oDJ, oFtot, oSig, oE, oInit, oDgTile, oDqFull, oDkFull, oQK, oPQK, oPVB, oPE, oPSig, total;
 };
 
 // dq, dk of a q/k head shared by `rep` value heads: the kernels leave one row per value head ([tokens, H, dk]) in the
@@ -639,7 +677,15 @@ static BwdLayout bwd_layout(const PalDims* d) {
   }
   L.oQK = o;
   const int cols = tile_piece(d->dk);   // (the first column group, the widest)
-  if (tile_rows(cols, d->dv) < d->dv && d->dtype == PAL_DTYPE_BF16) o = align256(o + tokens * d->n_heads * cols * 2 * 4);
+  const TileParts P = tile_parts(d->dk, d->dv, row == 4, (int64_t)tiles);
+  L.oPQK = L.oPVB = L.oPE = L.oPSig = o;
+  if (P.on) {
+    const size_t rows = tokens * d->n_heads, rects = (size_t)P.slices * P.groups;
+    L.oPQK = o; o = align256(o + P.slices * rows * 2 * d->dk * 4);
+    L.oPVB = o; o = align256(o + P.groups * rows * 2 * d->dv * 4);
+    L.oPE = o; o = align256(o + rects * rows * 4);
+    L.oPSig = o; o = align256(o + rects * tiles * 4);
+  } else if (tile_rows(cols, d->dv) < d->dv && d->dtype == PAL_DTYPE_BF16) o = align256(o + tokens * d->n_heads * cols * 2 * 4);
   L.total = o;
   return L;
 }
@@ -747,12 +793,16 @@ extern "C" int pal_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const Pal
   A.wE = (float*)(ws + L.oE); A.wInitPart = (float*)(ws + L.oInit);
   A.wDgTile = (float*)(ws + L.oDgTile);
   A.wQK = (float*)(ws + L.oQK);
+  A.pQK = (float*)(ws + L.oPQK); A.pVB = (float*)(ws + L.oPVB);
+  A.pE = (float*)(ws + L.oPE); A.pSig = (float*)(ws + L.oPSig);
   A.tokens = dd.batch * dd.seq_len;
   hipStream_t s = (hipStream_t)stream;
   const bool bf = dd.dtype == PAL_DTYPE_BF16;
   const bool var = dd.flags & PAL_FLAG_HAS_VAR;
-  rc = bf ? (var ? launch_tile_t<bf16_t, true>(A, s) : launch_tile_t<bf16_t, false>(A, s))
-          : (var ? launch_tile_t<float, true>(A, s) : launch_tile_t<float, false>(A, s));
+  const TileParts parts = tile_parts(dd.dk, dd.dv, !bf, (int64_t)dd.total_chunks * dd.n_heads);
+  rc = bf ? (var ? launch_tile_t<bf16_t, true>(A, parts, s) : launch_tile_t<bf16_t, false>(A, parts, s))
+          : (var ? launch_tile_t<float, true>(A, parts, s) : launch_tile_t<float, false>(A, parts, s));
+  if (!rc && parts.on) rc = launch_parts_sum(A, parts, bf, s);
   if (rc) return rc;
   {
     const int64_t blocks = (int64_t)dd.n_seqs * dd.n_heads * carry_scan_blocks((int64_t)dd.dv * dd.dk);

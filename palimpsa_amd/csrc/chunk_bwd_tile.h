@@ -231,7 +231,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   const int last = (clen - 1) / kG;
   float ssum = 0.f;   // sum of S over the tile's tokens
 
-  const int n0 = R.n0, r0 = R.r0;              // first key column, value row of the launch
+  constexpr bool PARTS = SLICE == 3;           // a small pass: workgroups for every rectangle, outputs of their own
+  const int n0 = R.n0 + (PARTS ? blockIdx.z * DNG : 0), r0 = R.r0 + (PARTS ? blockIdx.y * DS : 0);   // first key column, value row
   const int nw = n0 + WC * w;                  // of the wave (a lane has DN of its columns, from DN g on)
   {
     // Staging items, (token of the step, four columns): the first threads take k and q, the next ones (from a wave of their
@@ -441,7 +442,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       const int tok = kG * j + ((it & (2 * kG - 1)) >> 1), c = 4 * (it / (2 * kG));
       return (TIn*)((it & 1) ? A.db : A.dv) + tok0 * dv + (int64_t)tok * vs + r0 + c;
     };
-    const bool cols_before = R.flags & kRectColsBefore;   // what the columns of the earlier launches gave is added to
+    const bool cols_before = !PARTS && R.flags & kRectColsBefore;   // what the columns of the earlier launches gave is added to
     auto flush_sum = [&](int j, int it, f32x4& x, raw4& was) {
       const float* p = smem + L.oPart + (j & 1) * NBW * (kG * 32 * DT) + (it & (2 * kG - 1)) * DS + 4 * (it / (2 * kG));
       if (cols_before && kG * j + ((it & (2 * kG - 1)) >> 1) < clen) was = *(const raw4*)flush_at(j, it);
@@ -454,6 +455,12 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     };
     auto flush_store = [&](int j, int it, f32x4 x, raw4 was) {
       if (kG * j + ((it & (2 * kG - 1)) >> 1) < clen) {
+        if constexpr (PARTS) {
+          const int tok = kG * j + ((it & (2 * kG - 1)) >> 1), c = 4 * (it / (2 * kG));
+          const int64_t row = ((int64_t)(R.group + blockIdx.z) * A.tokens + t0 + tok) * H + h;
+          *(f32x4*)(A.pVB + (row * 2 + (it & 1)) * dv + r0 + c) = x;
+          return;
+        }
         if (cols_before) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) x[e] += (float)was[e];
@@ -495,7 +502,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         sX[lane] = 0.f;
         sF[lane] = fast_exp2(-gt * gh);
         if (lane == 63) {
-          A.wFtot[(int64_t)cidx * H + h] = c;
+          if (!PARTS || (n0 | r0) == 0) A.wFtot[(int64_t)cidx * H + h] = c;
           sF[kC] = 1.f;
         }
       }
@@ -540,8 +547,9 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     const bool out2 = DN == 4 || (lo & 4) == 0;
     TIn* const po = (TIn*)(ow ? A.dk : A.dq) + tok0 * dk + oc;
     // bf16 rows: sums over the launches so far
-    float* const pacc = A.wQK + tok0 * (2 * DNG) + ow * DNG + (oc - n0);
-    const int accs = 2 * DNG * H;   // per token
+    float* const pacc = PARTS ? A.pQK + ((int64_t)blockIdx.y * A.tokens * H + tok0) * (2 * dk) + ow * dk + oc
+                              : A.wQK + tok0 * (2 * DNG) + ow * DNG + (oc - n0);
+    const int accs = 2 * (PARTS ? dk : DNG) * H;   // per token
     const bool out_on = (lane & 3) == 0;
     // SLICE 2: what the launches over earlier value rows left for a token, requested two tokens ahead of its use
     auto acc_load = [&](int t, float* was) {
@@ -719,8 +727,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           if (kG * j + u < clen) {
             TIn* o = po + (o_tok + u * (int)dks);
             bool done = true;
-            if constexpr (SLICE != 0 && !F32) {   // the value rows of the launches add up, in fp32
-              if (R.flags & kRectRowsAfter) {
+            if constexpr (PARTS || (SLICE != 0 && !F32)) {   // the value rows of the launches add up, in fp32
+              if (PARTS || (R.flags & kRectRowsAfter)) {
                 float* acc = pacc + (kG * j + u) * accs;
                 acc[0] = oz[u][0];
                 if (out2) acc[1] = oz[u][1];
@@ -812,9 +820,10 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
 #pragma unroll
     for (int y = 1; y < NBW; ++y) { x += p[y]; tot -= p[NBW + y]; }
     x = lane ? sX[lane] : sF[0] * x;
-    float* pe = A.wE + (int64_t)h * A.tokens + t0 + lane;
-    float* ps = A.wSig + (int64_t)cidx * H + h;
-    const bool add = R.flags & (kRectRowsBefore | kRectColsBefore);
+    const int rect = PARTS ? (R.group + blockIdx.z) * R.slices + blockIdx.y : 0;
+    float* pe = (PARTS ? A.pE : A.wE) + ((int64_t)rect * H + h) * A.tokens + t0 + lane;
+    float* ps = (PARTS ? A.pSig : A.wSig) + ((int64_t)rect * a.total_chunks + cidx) * H + h;
+    const bool add = !PARTS && (R.flags & (kRectRowsBefore | kRectColsBefore));
     if (lane < clen) *pe = add ? x + *pe : x;
     if (lane == 0) *ps = add ? tot + *ps : tot;
   }
@@ -828,9 +837,16 @@ static int launch_tile_n(const BwdArgs& A, const TileRect& R, hipStream_t s) {
   static_assert(lds <= kMaxLds, "LDS of a compute unit");
   auto go = [&](auto kern) -> int {
     if (int rc = allow_lds((const void*)kern, lds)) return rc;
-    PAL_TIMED_LAUNCH(kKernBwdLocal, s, kern, dim3((unsigned)blocks), dim3(64 * NBW), lds, s, A, R);
+    PAL_TIMED_LAUNCH(kKernBwdLocal, s, kern, dim3((unsigned)blocks, (unsigned)R.slices, (unsigned)R.groups), dim3(64 * NBW), lds, s, A, R);
     return 0;
   };
+  if constexpr (DT <= 2) {
+    if (R.flags & kRectParts) {
+      if (int rc = go(&chunk_bwd_tile_kernel<TIn, DT, DN, NBW, VAR, 3>)) return rc;
+      PAL_HIP_LAUNCH_CHECK();
+      return PAL_OK;
+    }
+  }
   if (int rc = R.flags & kRectRowsBefore  ? go(&chunk_bwd_tile_kernel<TIn, DT, DN, NBW, VAR, 2>)
                : R.flags & kRectRowsAfter ? go(&chunk_bwd_tile_kernel<TIn, DT, DN, NBW, VAR, 1>)
                                           : go(&chunk_bwd_tile_kernel<TIn, DT, DN, NBW, VAR, 0>))
@@ -849,17 +865,21 @@ static int launch_tile_d(const BwdArgs& A, const TileRect& R, hipStream_t s) {
   return PAL_E_HEADDIM;
 }
 
-// The launches that make up the tile kernel: groups of key columns, in each the slices of value rows.
+// The launches that make up the tile kernel: groups of key columns, in each the slices of value rows (a small pass: all of
+// them side by side, a launch for each width that the groups have).
 template <typename TIn, bool VAR>
-int launch_tile_t(const BwdArgs& A, hipStream_t s) {
+int launch_tile_t(const BwdArgs& A, const TileParts& P, hipStream_t s) {
   const int dk = A.c.dk, dv = A.c.dv;
   TileRect R;
-  for (R.n0 = 0; R.n0 < dk; R.n0 += R.cols) {
-    R.cols = tile_piece(dk - R.n0);
+  R.group = 0;
+  for (R.n0 = 0; R.n0 < dk; R.n0 += R.groups * R.cols) {
+    R.cols = P.on ? parts_cols(dk, R.n0) : tile_piece(dk - R.n0);
+    R.groups = P.on && dk % R.cols == 0 ? dk / R.cols : 1;
+    R.slices = P.on ? P.slices : 1;
     int rows;
-    for (R.r0 = 0; R.r0 < dv; R.r0 += rows) {
-      rows = tile_rows(R.cols, dv - R.r0);
-      R.flags = (R.n0 ? kRectColsBefore : 0) | (R.r0 ? kRectRowsBefore : 0) | (R.r0 + rows < dv ? kRectRowsAfter : 0);
+    for (R.r0 = 0; R.r0 < dv; R.r0 += rows * R.slices) {
+      rows = P.on ? P.rows : tile_rows(R.cols, dv - R.r0);
+      R.flags = P.on ? kRectParts : (R.n0 ? kRectColsBefore : 0) | (R.r0 ? kRectRowsBefore : 0) | (R.r0 + rows < dv ? kRectRowsAfter : 0);
       int rc;
       switch (rows) {
         case 16: rc = launch_tile_d<TIn, 1, VAR>(A, R, s); break;
@@ -870,6 +890,7 @@ int launch_tile_t(const BwdArgs& A, hipStream_t s) {
       }
       if (rc) return rc;
     }
+    R.group += R.groups;
   }
   return PAL_OK;
 }

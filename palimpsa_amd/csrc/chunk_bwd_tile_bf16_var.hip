@@ -2,5 +2,5 @@
 #include "chunk_bwd_tile.h"
 
 namespace pal {
-template int launch_tile_t<bf16_t, true>(const BwdArgs&, hipStream_t);
+template int launch_tile_t<bf16_t, true>(const BwdArgs&, const TileParts&, hipStream_t);
 }

@@ -30,6 +30,7 @@ enum KernelId {
   kKernChunkStates,
   kKernGlaBwdStates,
   kKernGlaBwdTile,
+  kKernBwdPartsSum,
   kKernCount
 };
 

@@ -71,3 +71,35 @@ def test_gate_gradient_of_strongly_decaying_tokens(gpu_device, dk, dv, rows):
         f = torch.exp(-inp["gt"].double() * inp["g"].double())
         err = hp.max_rel(dgt / f, ref / f)
         assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (var, err)
+
+
+@pytest.mark.parametrize("dk,dv", [(16, 64), (32, 80), (48, 96), (64, 112), (80, 80), (96, 96), (96, 192), (112, 16), (128, 64), (160, 48),
+                                   (176, 32), (192, 80)])
+@pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_small_passes_agree_with_large_ones(gpu_device, dk, dv, rows):
+    """Few tiles: the rectangles of a wide head side by side, their parts summed by a kernel of its own.  Many tiles: one
+    after the other.  The same rows as a small pass and as the first rows of a large one: the same gradients, up to the
+    rounding of the results and the order of their sums (48 rows of another batch entry per tile stay apart)."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    if rows == torch.float32 and max(dk, dv) > 128:
+        pytest.skip("fp32 rows take head dims up to 128")
+    H, few, many = 4, 1, 24          # 24 tiles of 4 heads a pass of few rows, 576 of many
+    T = 64 * 6 - 11                  # the last tile is ragged
+    inp = hp.to_device(hp.rounded(po.make_inputs(many, T, H, dk, dv, seed=dk + dv), rows), gpu_device)
+    gen = torch.Generator(device=gpu_device).manual_seed(3)
+    do, dov = (torch.randn(many, T, H, dv, generator=gen, device=gpu_device) for _ in range(2))
+    mu0 = 0.1 * torch.randn(many, H, dv, dk, generator=gen, device=gpu_device)
+    I0 = inp["Ip"].view(1, H, 1, 1) + torch.rand(many, H, dv, dk, generator=gen, device=gpu_device)
+    for var, init in ((False, False), (True, True)):
+        got = []
+        for B in (few, many):
+            leaves = [(inp[n][:B] if inp[n].dim() > 1 else inp[n]).clone().requires_grad_(True) for n in NAMES]
+            state = [x[:B].clone().requires_grad_(True) for x in (mu0, I0)] if init else [None, None]
+            out = chunk_palimpsa(*leaves, *state, output_uncertainty=var)
+            out = list(out) if var else [out]
+            got.append(torch.autograd.grad(out, leaves[:5] + [x for x in state if x is not None],
+                                           [g[:B].to(rows) for g in (do, dov)][:len(out)]))
+        for n, x, y in zip(NAMES[:5] + ("mu0", "I0"), *got):
+            # 2 x 2 roundings of operands, and for bf16 results one of 2^-9 on each side
+            bar = 4 * 2.0 ** -17 if rows == torch.float32 else (4 if n == "gt" else 6) * 2.0 ** -9
+            assert hp.max_rel(x, y[:few]) <= bar, (var, init, n, hp.max_rel(x, y[:few]))
