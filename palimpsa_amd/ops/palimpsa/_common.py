@@ -57,6 +57,13 @@ def _pal_dtype(dt: torch.dtype) -> int:
     return L.PAL_DTYPE_BF16 if dt == torch.bfloat16 else L.PAL_DTYPE_F32
 
 
+def _plain(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """x in ``dtype`` and contiguous; no call into torch that would hand x back as it is."""
+    if x.dtype is not dtype:
+        x = x.to(dtype)
+    return x if x.is_contiguous() else x.contiguous()
+
+
 @dataclass
 class Prepared:
     """Kernel-ready views of the operator inputs (contiguous, padded, supported dtypes)."""
@@ -94,15 +101,14 @@ def prepare_inputs(q, k, v, b, gt, g, Ip, initial_mu_state, initial_I_state, cu_
     if g.numel() != H or Ip.numel() != H:
         raise ValueError("g and Ip must have one entry per head")
     # one element type for q,k,v,b: bf16 stays bf16, everything else computes from fp32 rows
-    cd = torch.bfloat16 if all(x.dtype == torch.bfloat16 for x in (q, k, v, b)) else torch.float32
-    q, k, v, b = [x.to(cd).contiguous() for x in (q, k, v, b)]
+    cd = torch.bfloat16 if all([x.dtype == torch.bfloat16 for x in (q, k, v, b)]) else torch.float32
+    q, k, v, b = [_plain(x, cd) for x in (q, k, v, b)]
     if gt.dtype not in (torch.float32, torch.bfloat16):
         gt = gt.float()
     gt = gt.contiguous()
     if gt.data_ptr() % 4:       # a bf16 view that starts on an odd element: the kernels fetch gates as aligned words
         gt = gt.clone()
-    g = g.reshape(H).float().contiguous()
-    Ip = Ip.reshape(H).float().contiguous()
+    g, Ip = [_plain(x if x.dim() == 1 else x.reshape(H), torch.float32) for x in (g, Ip)]
     n_seqs = B
     if cu_seqlens is not None:
         n_seqs = int(cu_seqlens.numel()) - 1
@@ -123,8 +129,8 @@ def prepare_inputs(q, k, v, b, gt, g, Ip, initial_mu_state, initial_I_state, cu_
         if tuple(initial_mu_state.shape) != exp or tuple(initial_I_state.shape) != exp:
             raise ValueError(f"Initial states mismatch: expected {exp}, got "
                              f"{tuple(initial_mu_state.shape)} / {tuple(initial_I_state.shape)}")
-        initial_mu_state = initial_mu_state.float().contiguous()
-        initial_I_state = initial_I_state.float().contiguous()
+        initial_mu_state = _plain(initial_mu_state, torch.float32)
+        initial_I_state = _plain(initial_I_state, torch.float32)
         if dk_p != dk or dv_p != dv:
             pad = (0, dk_p - dk, 0, dv_p - dv)
             initial_mu_state = F.pad(initial_mu_state, pad, value=0.0)
