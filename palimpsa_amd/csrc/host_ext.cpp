@@ -245,6 +245,7 @@ struct ChunkNode : torch::autograd::Function<ChunkNode> {
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["flags"] = flags;
     ctx->saved_data["var"] = var;
+    ctx->saved_data["tiles"] = tiles;
     torch::autograd::variable_list r{out.o, out.fm, out.fI};
     if (var) r.push_back(out.ov);
     return r;
@@ -256,6 +257,14 @@ struct ChunkNode : torch::autograd::Function<ChunkNode> {
                  &cu = s[10], &tile_mu = s[11], &tile_I = s[12];
     const c10::DeviceGuard guard(q.device());
     Call c(q, k, v, &b, gt, g, &Ip, ctx->saved_data["scale"].toDouble(), cu.defined() ? cu.numel() - 1 : 0);
+    // what the forward saved has been through the saved-tensor hooks, which may hand back anything
+    const int64_t tiles = ctx->saved_data["tiles"].toInt();
+    const auto f32_as = [&](const Tensor& t, int64_t n) { return plain(t, q.device(), at::kFloat) && t.numel() == n * c.H * c.dv * c.dk; };
+    const auto i32_as = [&](const Tensor& t, int64_t n) { return plain(t, q.device(), at::kInt) && t.numel() == n; };
+    TORCH_CHECK_VALUE(c.ok && f32_as(tile_mu, tiles) && f32_as(tile_I, tiles) && mu.defined() == I.defined() &&
+                          (!mu.defined() || (f32_as(mu, c.N) && f32_as(I, c.N))) &&
+                          (!cu.defined() || (i32_as(cu, c.N + 1) && i32_as(meta, c.N + 1 + 4 * tiles))),
+                      "chunk_palimpsa backward: a saved tensor came back in another shape, dtype, layout or device");
     Tensor d_o = gr[0].defined() ? gr[0].to(c.rows).contiguous() : at::zeros_like(v);
     Tensor d_ov;
     if (ctx->saved_data["var"].toBool() && gr[3].defined()) d_ov = gr[3].to(c.rows).contiguous();
@@ -265,7 +274,7 @@ struct ChunkNode : torch::autograd::Function<ChunkNode> {
     if (mu.defined()) { dmu = at::empty_like(mu); dI = at::empty_like(I); }
     uint32_t flags = (uint32_t)ctx->saved_data["flags"].toInt() & ~(uint32_t)PAL_FLAG_HAS_VAR;
     if (d_ov.defined()) flags |= PAL_FLAG_HAS_VAR;
-    c.dims.total_chunks = (int32_t)tile_mu.size(0);
+    c.dims.total_chunks = (int32_t)tiles;
     c.dims.var_dtype = c.dims.dtype;
     c.dims.flags = flags;
     PalFwdTensors t{};

@@ -15,10 +15,23 @@ def _strided(x):
     return torch.cat([x, x], -1)[..., : x.shape[-1]]
 
 
+def _taken(host, monkeypatch, name):
+    """A list that grows by one entry per call of the extension's function: whether it served the call."""
+    real, taken = getattr(host, name), []
+
+    def call(*args):
+        r = real(*args)
+        taken.append(r is not None)
+        return r
+
+    monkeypatch.setattr(host, name, call)
+    return taken
+
+
 @pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("T,init,var,cu,bf16_gates", [(1, True, False, None, False), (70, False, True, None, True),
                                                       (150, True, True, [0, 17, 17, 150], False)])
-def test_native_and_python_routes_agree(gpu_device, rows, T, init, var, cu, bf16_gates):
+def test_native_and_python_routes_agree(gpu_device, monkeypatch, rows, T, init, var, cu, bf16_gates):
     from palimpsa_amd import _lib as L
     from palimpsa_amd.ops.palimpsa import chunk_palimpsa, fused_recurrent_palimpsa
     from palimpsa_amd.ops.simple_gla import fused_recurrent_simple_gla
@@ -50,17 +63,21 @@ def test_native_and_python_routes_agree(gpu_device, rows, T, init, var, cu, bf16
         return res
 
     for f, grad in ((chunk_palimpsa, False), (chunk_palimpsa, True), (fused_recurrent_palimpsa, False)):
+        if f is chunk_palimpsa or cu is None:   # (a packed token-serial call is not a plain one)
+            taken = _taken(host, monkeypatch, "chunk_fwd" if f is chunk_palimpsa else "recurrent_fwd")
+            run(f, True, grad)
+            run(f, False, grad)
+            assert taken == [True, False], (f.__name__, grad)
         for a, b in zip(run(f, True, grad), run(f, False, grad)):
             assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), (f.__name__, grad)
     if cu is None:
         g = -x["gt"].float()
         S = torch.randn(N, H, dk, dv, device=gpu_device) if init else None
+        taken = _taken(host, monkeypatch, "gla_recurrent_fwd")
         a = fused_recurrent_simple_gla(x["q"], x["k"], x["v"], g, initial_state=S, output_final_state=True)
         b = fused_recurrent_simple_gla(_strided(x["q"]), x["k"], x["v"], g, initial_state=S, output_final_state=True)
+        assert taken == [True, False]
         assert all(torch.equal(y, z) for y, z in zip(a, b))
-        ipad = (x["q"], x["k"], x["v"], x["b"], x["gt"], x["g"], x["Ip"], 1.0, None, None, False, False, 0)
-        assert host.recurrent_fwd(*ipad) is not None
-        assert host.recurrent_fwd(_strided(x["q"]), *ipad[1:]) is None
 
 
 def _plain_call(dev, T=3, H=2, dk=16, dv=16, grad=()):
@@ -154,3 +171,51 @@ def test_library_codes_raise_what_the_python_route_raises(gpu_device):
     finally:
         host.bind([*addresses.values()], L.check)
     chunk_palimpsa(*x).sum().backward()
+
+
+def test_saved_tensor_hooks(gpu_device):
+    """What a hook hands back is what the backward uses, and nothing that the kernels would misread."""
+    from torch.autograd.graph import save_on_cpu, saved_tensors_hooks
+
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+
+    def grads(hooks):
+        x = _plain_call(gpu_device, T=150, grad=range(7))
+        with hooks:
+            out = chunk_palimpsa(*x, initial_mu_state=s[0], initial_I_state=s[1])
+        assert "ChunkNode" in out.grad_fn.name()
+        return torch.autograd.grad(out.square().sum(), x)
+
+    s = [torch.zeros(1, 2, 16, 16, device=gpu_device), torch.ones(1, 2, 16, 16, device=gpu_device)]
+    seen = []
+    want = grads(saved_tensors_hooks(lambda t: seen.append(t.shape) or t, lambda t: t))
+    assert (3, 2, 16, 16) in seen      # the states at the starts of the tiles among them
+    assert all(torch.equal(a, b) for a, b in zip(grads(save_on_cpu()), want))
+    for change in (lambda t: t.double(), lambda t: t[:1], lambda t: t.cpu(), lambda t: t.transpose(-1, -2)):
+        with pytest.raises(ValueError):
+            grads(saved_tensors_hooks(lambda t: t, lambda t: change(t) if t.shape == (3, 2, 16, 16) else t))
+
+
+def test_calls_on_a_stream_of_their_own(gpu_device):
+    """Kernels, outputs and workspaces of a call belong to the stream that is current for it, those of the backward to the
+    forward's."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa, fused_recurrent_palimpsa
+    x = _plain_call(gpu_device, T=150, grad=range(7))
+    want = chunk_palimpsa(*x)
+    want_g = torch.autograd.grad(want.square().sum(), x)
+    with torch.no_grad():
+        want_r = fused_recurrent_palimpsa(*x)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            big = torch.randn(4096, 4096, device=gpu_device)
+            big = big @ big                                   # keeps the stream busy ahead of the call
+            y = [(t.detach() + 0 * big[0, 0]).requires_grad_(True) for t in x]   # ready on this stream only
+            out = chunk_palimpsa(*y)
+            got_g = torch.autograd.grad(out.square().sum(), y)
+            with torch.no_grad():
+                got_r = fused_recurrent_palimpsa(*y)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(out, want) and torch.equal(got_r, want_r)
+    assert all(torch.equal(a, b) for a, b in zip(got_g, want_g))
