@@ -1,4 +1,4 @@
-// Pieces shared by the kernels of the chunked backward (chunk_bwd.hip, chunk_bwd_tile.hip).
+// Pieces shared by the kernels of the chunked backward (chunk_bwd.hip, chunk_bwd_tile.h).
 #pragma once
 #include "chunk_common.h"
 
@@ -12,7 +12,7 @@ struct BwdArgs {
   void *wDM, *wDJ;        // [total_chunks,H,dv,dk] local carries, then incoming carries, in the dtype of the rows
   float* wFtot;           // [total_chunks,H] log2 of the total decay of a tile
   float* wSig;            // [total_chunks,H] sum over the tile of dJloc
-  float* wE;              // [H, tokens]  local part of d log f
+  float* wE;              // [H,tokens]  local part of d log f
   float* wInitPart;       // [n_seqs,H,dv*dk/256] partial sums of dJ_0
   float* wDgTile;         // [total_chunks,H] the tiles' shares of dg
   float* wQK;             // [tokens,H,2,cols] dq, dk of a column group summed so far, where a tile takes several slices of

@@ -9,7 +9,7 @@
 // (:360-384).  All tiles of 64 tokens are processed in parallel; what crosses a
 // tile boundary is handled by two small extra passes (scan, apply); the gate gradient is finished in the second:
 //
-//  local   per (tile, head): chunk_bwd_tile.hip -- dq, the tile's own parts of dv, db, dk and of the gate gradient, and
+//  local   per (tile, head): chunk_bwd_tile.h -- dq, the tile's own parts of dv, db, dk and of the gate gradient, and
 //          the carry the tile hands to its predecessor, R_loc = f_first * dM^loc_first.
 //  scan    per state entry: R_{c-1} = R_loc,c + F_C,c R_c backwards over the tiles
 //          of a sequence (the role of curr_dM/curr_dI, :429-430); also yields the

@@ -42,23 +42,7 @@
 
 namespace pal {
 
-// Sums over lanes by DPP with a bank mask (an instruction writes only the lanes of its mask); the s_nop covers the wait
-// states a DPP read needs after a VALU write, which the compiler cannot see inside the assembly.
-// x over lane bit 3 where the bit is clear, y where it is set
-__device__ __forceinline__ float pair_bit3(float x, float y) {
-  float r;
-  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-      "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc" : "=&v"(r) : "v"(x), "v"(y));
-  return r;
-}
-// the same with lane bit 2
-__device__ __forceinline__ float pair_bit2(float x, float y) {
-  float r;
-  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-      "v_add_f32_dpp %0, %2, %2 row_shr:4 row_mask:0xf bank_mask:0xa" : "=&v"(r) : "v"(x), "v"(y));
-  return r;
-}
-// The sums of a token over lanes, in three stages so that the next token's arithmetic can be placed between them (each
+// The sums of a token over lanes by DPP with a bank mask (see pair_bit3), in three stages so that the next token's arithmetic can be placed between them (each
 // stage is a chain of dependent instructions).
 //   o[2 DN] (dq, then dk of the lane's columns): over the 16 lanes of a row.  Lane bit 3 selects dq or dk, of which z0 is
 //     the first (lane bit 2 clear) or the third column, z1 the second or the fourth (DN = 3: the second in both).
@@ -134,22 +118,6 @@ struct TokSums {
     if constexpr (DT >= 3) q[0] += q[1];
   }
 };
-template <int CTRL>
-__device__ __forceinline__ float dpp_quad(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float quad_sum(float x) {
-  x += dpp_quad<0xB1>(x);    // quad_perm [1,0,3,2]
-  return x + dpp_quad<0x4E>(x);   // quad_perm [2,3,0,1]
-}
-
-template <typename TIn>
-struct Raw4;
-template <>
-struct Raw4<bf16_t> { typedef bf16x4 type; };
-template <>
-struct Raw4<float> { typedef f32x4 type; };
-
 template <int DT>
 __device__ __forceinline__ void lds_vals(const float* p, float* out) {
   if constexpr (DT >= 3) {
@@ -190,10 +158,10 @@ struct TokRev {
 };
 
 // waves per SIMD that a lane's E state entries leave registers for
-constexpr int tile_waves(int E, bool var) { return E > 4 ? 2 : 3; }
+constexpr int tile_waves(int E) { return E > 4 ? 2 : 3; }
 
 template <typename TIn, int DT, int DN, int NBW, bool VAR, int SLICE>
-__global__ __attribute__((amdgpu_flat_work_group_size(NBW * 64, NBW * 64), amdgpu_waves_per_eu(tile_waves(DT * DN, VAR))))
+__global__ __attribute__((amdgpu_flat_work_group_size(NBW * 64, NBW * 64), amdgpu_waves_per_eu(tile_waves(DT * DN))))
 void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   const ChunkArgs& a = A.c;
   extern __shared__ float smem[];

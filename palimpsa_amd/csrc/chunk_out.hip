@@ -60,8 +60,8 @@ struct OutLanes {
   }
   // sum over lane bits 0, 1 and 4, as far as they belong to the column group; every lane gets the total
   static __device__ __forceinline__ float sum_other(float x) {
-    if constexpr (NG >= 8) x += dpp<0xB1>(x);    // quad_perm [1,0,3,2]
-    if constexpr (NG >= 16) x += dpp<0x4E>(x);   // quad_perm [2,3,0,1]
+    if constexpr (NG >= 8) x += quad_move<0xB1>(x);    // quad_perm [1,0,3,2]
+    if constexpr (NG >= 16) x += quad_move<0x4E>(x);   // quad_perm [2,3,0,1]
     if constexpr (NG == 32) {
       float y = x;
       swap_rows(x, y);
@@ -69,38 +69,11 @@ struct OutLanes {
     }
     return x;
   }
-  template <int CTRL>
-  static __device__ __forceinline__ float dpp(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
-  }
 };
-// lanes with bit 3 clear: x summed over bit 3; set: y.  (DPP with a bank mask: two instructions; the s_nop covers the
-// wait states a DPP read needs after a VALU write, which the compiler cannot see inside the assembly)
-__device__ __forceinline__ float pair_bit3(float x, float y) {
-  float r;
-  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-      "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc" : "=&v"(r) : "v"(x), "v"(y));
-  return r;
-}
-// the same for bit 2
-__device__ __forceinline__ float pair_bit2(float x, float y) {
-  float r;
-  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
-      "v_add_f32_dpp %0, %2, %2 row_shr:4 row_mask:0xf bank_mask:0xa" : "=&v"(r) : "v"(x), "v"(y));
-  return r;
-}
-
 // x <- x f + c in one instruction (the compiler would copy c first and accumulate into the copy)
 __device__ __forceinline__ void fma3(float& x, float f, float c) {
   asm("v_fma_f32 %0, %0, %1, %2" : "+v"(x) : "v"(f), "v"(c));
 }
-
-template <typename TIn>
-struct Raw4;
-template <>
-struct Raw4<bf16_t> { typedef bf16x4 type; };
-template <>
-struct Raw4<float> { typedef f32x4 type; };
 
 // pieces of a lane's DN columns: DN / 4 pieces of four, then two, then one; every piece is contiguous over the lanes
 template <int NG, int DN>

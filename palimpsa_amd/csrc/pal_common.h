@@ -93,6 +93,13 @@ __device__ __forceinline__ void load_vec(const bf16_t* p, float* out) {
     out[0] = (float)*p;
   }
 }
+// four consecutive elements of a row as fetched
+template <typename T>
+struct Raw4;
+template <>
+struct Raw4<bf16_t> { typedef bf16x4 type; };
+template <>
+struct Raw4<float> { typedef f32x4 type; };
 // eight consecutive elements of a row as fetched (two 8- or 16-byte accesses), converted when they are used
 template <typename T>
 struct Raw8;
@@ -188,6 +195,31 @@ __device__ __forceinline__ float row16_sum(float x) {
   x += row_ror<2>(x);
   x += row_ror<1>(x);
   return x;
+}
+// Sums over lane bits 3 and 2 by DPP with a bank mask (an instruction writes only the lanes of its mask); the s_nop covers
+// the wait states a DPP read needs after a VALU write, which the compiler cannot see inside the assembly.
+// x over lane bit 3 where the bit is clear, y where it is set
+__device__ __forceinline__ float pair_bit3(float x, float y) {
+  float r;
+  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc" : "=&v"(r) : "v"(x), "v"(y));
+  return r;
+}
+// the same with lane bit 2
+__device__ __forceinline__ float pair_bit2(float x, float y) {
+  float r;
+  asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %2, %2 row_shr:4 row_mask:0xf bank_mask:0xa" : "=&v"(r) : "v"(x), "v"(y));
+  return r;
+}
+// a lane's value from its quad (DPP quad_perm)
+template <int CTRL>
+__device__ __forceinline__ float quad_move(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float quad_sum(float x) {
+  x += quad_move<0xB1>(x);          // quad_perm [1,0,3,2]
+  return x + quad_move<0x4E>(x);    // quad_perm [2,3,0,1]
 }
 // gfx950 lane swaps run in the VALU; the LDS-routed shuffles they replace cost ~64 cycles of latency each.
 // Written as inline assembly: with hipcc 7.2 the two results of the __builtin_amdgcn_permlane*_swap
