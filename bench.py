@@ -48,8 +48,8 @@ COUNTER_TABLE = os.path.join(ROOT, "profiles", "counter_table.txt")
 
 
 def load_counter_table(path=COUNTER_TABLE):
-    """Per-kernel figures that only the profiler can read (rocprofv3 --pmc, one run per counter): HBM bytes per launch
-    (FETCH_SIZE + WRITE_SIZE, scaled by a copy of known size) and vector-ALU instructions per state entry
+    """Per-kernel figures that only the profiler can read (rocprofv3 --pmc, one run per counter), over all launches of a
+    kernel in a step: HBM bytes (FETCH_SIZE + WRITE_SIZE, scaled by a copy of known size) and vector-ALU instructions per state entry
     (SQ_INSTS_VALU minus the matrix instructions, times 64 lanes, per token x value row x key column).  They are kept in a
     small table under profiles/ next to the summaries they come from, one line per (workload, kernel) with the commit the
     kernels were at when they were collected, so that a stale figure shows in the line this script prints."""
@@ -74,7 +74,7 @@ def counter(workload, kernel, field):
 
 
 def add_traffic(roof, workload, kernel):
-    """Attach the profiler's HBM bytes per launch, and the commit they were measured at, to a roofline entry."""
+    """Attach the profiler's HBM bytes of a kernel in a step, and the commit they were measured at, to a roofline entry."""
     roof["traffic"] = counter(workload, kernel, "traffic")
     roof["traffic_measured_at"] = counter(workload, kernel, "measured_at")
     return roof
@@ -141,29 +141,35 @@ def timed_loop(torch, step, steps, warmup):
     torch.cuda.synchronize()
     kern = L.profile_read()
     L.profile_enable(False)
-    kernels = {k: {"avg_ms": v[0] / v[1], "launches": v[1]} for k, v in kern.items()}
+    kernels = {k: {"avg_ms": v[0] / v[1], "launches": v[1], "ms_per_step": v[0] / steps} for k, v in kern.items()}
     return ms_mean, ms_median, kernels
 
 
-def mfma_roofline(workload, kernel, kernels, flops_per_launch, entries, note):
-    """Roofline entry of a chunked kernel: the bf16 matrix peak priced with the metric's fixed flop formula, and the
-    fp32 vector peak priced with the vector instructions the kernel issues per state entry."""
-    avg_ms = kernels.get(kernel, {"avg_ms": float("nan")})["avg_ms"]
-    achieved = flops_per_launch / (avg_ms * 1e-3) / 1e12
+DENSE_NOTE = ("achieved and frac: the flops of the dense contractions of the chunked algorithm (the metric's fixed formula) "
+              "over the kernel's time in a step, all of its launches; the kernel itself runs the recurrence token by token "
+              "on the vector units and is bound by their issue, see valu")
+
+
+def mfma_roofline(workload, kernel, kernels, flops_per_step, entries, note):
+    """Roofline entry of a chunked kernel over a step, which may take several launches of it: the bf16 matrix peak
+    priced with the metric's fixed flop formula, and the fp32 vector peak priced with the vector instructions the kernel
+    issues per state entry."""
+    k = kernels.get(kernel, {"avg_ms": float("nan"), "launches": 0, "ms_per_step": float("nan")})
+    ms = k["ms_per_step"]
+    achieved = flops_per_step / (ms * 1e-3) / 1e12
     out = {"bound": "mfma", "kernel": kernel, "achieved": achieved, "peak": PEAK_BF16_MFMA_TFLOPS, "unit": "TFLOP/s",
-           "frac": achieved / PEAK_BF16_MFMA_TFLOPS, "traffic": None, "algorithmic_flops_per_launch": flops_per_launch,
-           "avg_launch_ms": avg_ms, "note": note}
+           "frac": achieved / PEAK_BF16_MFMA_TFLOPS, "traffic": None, "algorithmic_flops_per_step": flops_per_step,
+           "kernel_ms_per_step": ms, "avg_launch_ms": k["avg_ms"], "note": DENSE_NOTE + "; " + note}
     add_traffic(out, workload, kernel)
     ops = counter(workload, kernel, "valu_ops_per_entry")
     if ops is not None:
-        valu = ops * entries * 2 / (avg_ms * 1e-3) / 1e12
+        valu = ops * entries * 2 / (ms * 1e-3) / 1e12
         out["valu"] = {"ops_per_entry": ops, "achieved": valu, "peak": PEAK_FP32_VALU_TFLOPS, "unit": "TFLOP/s",
                        "frac": valu / PEAK_FP32_VALU_TFLOPS,
                        "note": "vector (non-matrix) lane instructions per state entry x entries x 2 / time: the fp32 "
                                "rate the vector ALUs would show if every instruction were an FMA; the peak assumes "
                                "packed FMA issue, plain fp32 instructions issue at 0.73 of it on this GPU "
-                               "(profiles/issue_rates.txt), and matrix instructions stall the vector issue of "
-                               "their SIMD for their whole duration"}
+                               "(profiles/issue_rates.txt), and a reciprocal takes the time of three"}
     return out
 
 
@@ -196,15 +202,13 @@ def bench_chunk(torch, dev, steps, warmup, gates="bf16"):
     roofline = mfma_roofline(
         "c1", "chunk_bwd_local_kernel", kernels, flops_local, token_heads * E,
         "flops = 4(C+1)*dk*dv per token-head (recompute + reverse triangular contractions, C=64); step_frac uses "
-        "(6C+14)*dk*dv over the whole fwd+bwd step.  The kernel is bound by fp32 vector issue in the tile epilogues "
-        "(one division per state entry), not by the matrix cores: see roofline.valu and "
-        "profiles/bench_c1.sq_counters_pmc.txt")
+        "(6C+14)*dk*dv over the whole fwd+bwd step; counters in profiles/bench_c1.sq_counters_pmc.txt")
     if "valu" in roofline:      # flat copies: nested objects do not survive every consumer of this line
         roofline["valu_frac"] = roofline["valu"]["frac"]
         roofline["valu_ops_per_entry"] = roofline["valu"]["ops_per_entry"]
     roofline["step_frac"] = flops_step / (ms_per_step * 1e-3) / 1e12 / PEAK_BF16_MFMA_TFLOPS
     out_roof = mfma_roofline("c1", "chunk_out_kernel", kernels, 2 * (CHUNK + 1) * E * token_heads, token_heads * E,
-                             "flops = 2(C+1)*dk*dv per token-head (prefix products of M and J)")
+                             "flops = 2(C+1)*dk*dv per token-head")
     return dict(value=tokens / (ms_per_step * 1e-3), ms_per_step=ms_per_step, ms_per_step_median=ms_median,
                 roofline=roofline, roofline_forward=out_roof, kernels=kernels,
                 config={"workload": f"c1: chunked fwd+bwd B=8 T=2048 H=12 dk=dv=64 bf16 rows {gates} gates fp32 states C=64",
@@ -571,8 +575,8 @@ def bench_c2(torch, dev, steps, warmup):
     ms, med, kernels = timed_loop(torch, step, steps, warmup)
     E, th = d * d, T * H
     roof = mfma_roofline("c2", "chunk_bwd_local_kernel", kernels, 4 * (CHUNK + 1) * E * th, th * E,
-                         "flops = 4(C+1)*dk*dv per token-head; step_frac uses (6C+14)*dk*dv; dk = 96 runs the tile kernel "
-                         "in three passes of two column blocks (two workgroups per compute unit)")
+                         "flops = 4(C+1)*dk*dv per token-head; step_frac uses (6C+14)*dk*dv; a 96 x 96 state takes four "
+                         "launches of the tile kernel, 64 and 32 key columns by 48 value rows each")
     roof["step_frac"] = (6 * CHUNK + 14) * E * th / (ms * 1e-3) / 1e12 / PEAK_BF16_MFMA_TFLOPS
     return {"workload": f"c2: packed varlen chunked fwd+bwd, {len(cu) - 1} documents, 32768 tokens, H=16 dk=dv=96 bf16",
             "documents": len(cu) - 1, "tokens_per_s": T / (ms * 1e-3), "ms_per_step": ms, "ms_per_step_median": med,
@@ -597,12 +601,10 @@ def bench_c4(torch, dev, steps, warmup):
 
     ms, med, kernels = timed_loop(torch, step, steps, warmup)
     E, th = d * d, T * H
-    # the forward runs in windows of tiles: the per-kernel averages are per window, the flops likewise
     n_launch = max(1, kernels.get("chunk_out_kernel", {"launches": steps})["launches"] // steps)
-    roof = mfma_roofline("c4", "chunk_out_kernel", kernels, 2 * (CHUNK + 1) * E * th / n_launch, th * E / n_launch,
-                         f"flops = 2(C+1)*dk*dv per token-head (prefix products of M and J); the sequence is run in "
-                         f"{n_launch} windows of tiles handed through the state, one launch each; step_frac uses "
-                         "(2C+6)*dk*dv over the whole forward")
+    roof = mfma_roofline("c4", "chunk_out_kernel", kernels, 2 * (CHUNK + 1) * E * th, th * E,
+                         f"flops = 2(C+1)*dk*dv per token-head; the sequence is run in {n_launch} windows of tiles handed "
+                         "through the state, one launch each; step_frac uses (2C+6)*dk*dv over the whole forward")
     roof["step_frac"] = (2 * CHUNK + 6) * E * th / (ms * 1e-3) / 1e12 / PEAK_BF16_MFMA_TFLOPS
     return {"workload": "c4: chunked forward B=1 T=65536 H=16 dk=dv=128 bf16, initial and final state",
             "tokens_per_s": T / (ms * 1e-3), "ms_per_step": ms, "ms_per_step_median": med, "kernels": kernels,
