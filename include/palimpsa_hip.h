@@ -256,9 +256,10 @@ int pal_gla_chunk_bwd(const PalDims *dims, const PalFwdTensors *t, const PalBwdT
  * fp32 rows without PAL_FLAG_FP32_FAST keep a second bf16 plane of that tile (8 dk (dv + 8) in the sum above)
  * and take head dims up to 128 (e.g. 96x96, 64x128, 128x64).
  * Workspace: two carries of dk x dv per tile and head in the dtype of the rows; for bf16 rows of a head with more
- * than 64 value rows (48 where dk is 48 or dv 96) also fp32 sums of dq and dk over the slices of value rows, of one
- * group of at most 64 key columns at a time (8 bytes per token, head and column): at 32768 tokens and 16 heads
- * 136 MB for 64x64, 573 MB for 96x96, 808 MB for 128x128. */
+ * than 64 value rows (48 where dk is 16) also fp32 sums of dq and dk over the slices of value rows, of one group
+ * of at most 64 key columns at a time (8 bytes per token, head and column): at 32768 tokens and 16 heads 136 MB
+ * for 64x64, 573 MB for 96x96, 808 MB for 128x128.  A pass of few tiles (at most 384 tiles x heads, or 512) of a
+ * head that takes several pieces keeps the parts of every piece instead: up to 190 MB at 96x192. */
 size_t pal_chunk_bwd_workspace_bytes(const PalDims *dims);
 int pal_chunk_bwd(const PalDims *dims, const PalFwdTensors *t, const PalBwdTensors *gr,
                   void *workspace, size_t workspace_bytes, void *stream);

@@ -28,16 +28,21 @@ struct BwdArgs {
 // Larger heads take several: groups of 64, 48 or 32 key columns (16 for a head of 16), in each of them slices of 64, 48,
 // 32 or 16 value rows.  (96 columns as 64 + 32, 80 as 48 + 32: workgroups of four or two waves, two or four of them to a
 // compute unit.  One workgroup of eight waves has nothing to fill its barriers and its set-up with: 96x96, 32768 packed
-// tokens, 16 heads: 5.5 ms, as rectangles 4.2.  A rectangle costs, in ps per state entry and token at B=8 T=2048 H=16, 0.77
-// (64x64: columns x rows), 0.86 (64x48), 0.87 (64x32), 0.98 (48x64), 1.00 (48x48), 1.12 (48x32), 1.06 (32x64), 0.99 (32x48,
-// 32x32), 1.8 (16x16): hence 96 rows as 48 + 48, where neither piece pays for a small one.)
+// tokens, 16 heads: 5.5 ms, as rectangles 4.2.  A rectangle costs, in ps per state entry and token at B=8 T=2048 H=16, bf16
+// rows, 0.68 (64x64: columns x rows), 0.77 (64x48, 64x32), 0.88 (48x64), 0.92 (48x48), 1.00 (48x32), 0.97 (32x64), 0.87 (32x48),
+// 0.89 (32x32), 1.6 (16x16), and fp32 rows 1.14 (64x64, whose LDS leaves one workgroup to a unit), 0.84 (64x48, 64x32), 1.45 (32x64),
+// 1.66 (32x48): hence 96 rows as 64 + 32 where the group has 64 columns and the rows are bf16 (96x96 B=8 T=2048 H=16: 2155 us
+// with 48 + 48 everywhere, 2055 so; 64x96 1299, 1202), as 48 + 48 otherwise (fp32 rows 96x96 2970 us, 3230 with 64 + 32).)
 struct TileRect {
   int n0, cols, r0, flags;
   int group, groups, slices;   // small pass: first column group, their number (grid z), slices of value rows (grid y)
 };
 constexpr int kRectColsBefore = 1, kRectRowsBefore = 2, kRectRowsAfter = 4, kRectParts = 8;   // launches that came before, come after; a small pass
 inline int tile_piece(int n) { return n == 80 ? 48 : n >= 64 ? 64 : n; }
-inline int tile_rows(int cols, int n) { return cols == 16 ? (n >= 48 ? 48 : 16) : n == 96 ? 48 : tile_piece(n); }   // (16 columns: one wave's staging)
+inline int tile_rows(int cols, int n, bool f32) {
+  if (cols == 16) return n >= 48 ? 48 : 16;   // (one wave's staging)
+  return n == 96 && (f32 || cols < 64) ? 48 : tile_piece(n);
+}
 
 // A pass with too few tiles to fill the chip: all rectangles of a group width in one launch, side by side, each with
 // outputs of its own that a last kernel adds up in a fixed order.  One after the other they cost a tile's serial latency
@@ -46,7 +51,7 @@ inline int tile_rows(int cols, int n) { return cols == 16 ? (n >= 48 ? 48 : 16) 
 // after the other -> side by side), bf16 rows, by tiles x heads:
 //            64          256         384         512         768
 //   80x80    225 -> 100  234 -> 160  288 -> 228  293 -> 280  387 -> 392
-//   96x96    277 ->  69  285 -> 175  356 -> 253  360 -> 330  475 -> 491
+//   96x96    265 ->  69  273 -> 174  343 -> 253  349 -> 328  454 -> 488
 //   96x192   472 -> 103  484 -> 326  625 -> 489  631 -> 649  843 -> 976
 //   128x128  307 ->  72  314 -> 233  417 -> 338  425 -> 449  664 -> 667
 //   112x112  283 -> 104  293 -> 253  382 -> 377  389 -> 477  610 -> 701
@@ -69,7 +74,7 @@ inline TileParts tile_parts(int dk, int dv, bool f32, int64_t tile_heads) {
   int pieces = 0;   // one after the other
   for (int n0 = 0, c; n0 < dk; n0 += c) {
     c = tile_piece(dk - n0);
-    for (int r0 = 0; r0 < dv; r0 += tile_rows(c, dv - r0)) ++pieces;
+    for (int r0 = 0; r0 < dv; r0 += tile_rows(c, dv - r0, f32)) ++pieces;
   }
   const bool small = f32 || dk * dv <= pieces * 48 * 48;
   P.on = pieces > 1 && tile_heads <= (small ? kPartsTilesSmall : kPartsTiles);

@@ -14,16 +14,16 @@
 // most 32 tokens (k weighted by the decay against v, and k^2 against b; bf16 operands, two halves of each for fp32
 // rows), the step's tokens are advanced forward leaving their states in registers, then worked in reverse.
 //
-// What bounds it: vector issue.  Per entry and token 19 fp32 instructions and a reciprocal, and about 8 more for the sums
-// over lanes, the recomputed states, staging and the sums over waves; two waves per SIMD (the registers), each of
-// which issues an instruction per 5.4 cycles.  As products on the matrix cores (12 prefix and 12 suffix instructions of
-// 16 cycles per 16 entries of a lane, operands exchanged through LDS between waves of different roles) the same pass took
-// 822 us at B=8 T=2048 H=12 64x64, this takes 585; 48x48 H=16 736 -> 575, packed 32768 tokens 96x96 4.91 -> 4.22 ms, fp32
-// rows 64x64 B=8 T=2048 H=8 (forward and backward together) 1.53 -> 0.97 ms.
+// What bounds it: vector issue.  Per entry and token 19 fp32 instructions and a reciprocal, and 6 more for the sums over
+// lanes, the recomputed states, staging and the sums over waves (64x64; 9 more in the smaller rectangles of 96x96); two waves per
+// SIMD (the registers), which together issue an instruction per 4 cycles.  As products on the matrix cores (12 prefix and 12
+// suffix instructions of 16 cycles per 16 entries of a lane, operands exchanged through LDS between waves of different roles)
+// the same pass took 822 us at B=8 T=2048 H=12 64x64, this takes 555; 48x48 H=16 736 -> 555, packed 32768 tokens 96x96 4.91 -> 4.1 ms,
+// fp32 rows 64x64 B=8 T=2048 H=8 (forward and backward together) 1.53 -> 0.95 ms.
 // Layout: a wave holds 4 DN columns x 16 DT rows of the state, a lane DN neighbouring columns of DT rows, the layout in
 // which the matrix products leave the state (DN = 3: the fourth operand row of a lane group is empty), so that a head of
 // 48 columns loads all four SIMDs.  As many tokens per step as the registers hold: the fixed cost of a step (about
-// 3000 cycles of a SIMD per wave beside 48 per entry and token) is what small pieces pay.
+// 2600 cycles of a SIMD per wave beside 67 per entry and token of a lane) is what small pieces pay.
 //
 // Gate: gamma_t = f_t (<dM_t, M_{t-1}> + <dJ_t, J_{t-1}>), formed as it stands: where a token decays strongly, what is left of
 // the state is of the order of f_t, and so is gamma.  (The states of the step are in registers, so that it takes two
@@ -846,7 +846,7 @@ int launch_tile_t(const BwdArgs& A, const TileParts& P, hipStream_t s) {
     R.slices = P.on ? P.slices : 1;
     int rows;
     for (R.r0 = 0; R.r0 < dv; R.r0 += rows * R.slices) {
-      rows = P.on ? P.rows : tile_rows(R.cols, dv - R.r0);
+      rows = P.on ? P.rows : tile_rows(R.cols, dv - R.r0, sizeof(TIn) == 4);
       R.flags = P.on ? kRectParts : (R.n0 ? kRectColsBefore : 0) | (R.r0 ? kRectRowsBefore : 0) | (R.r0 + rows < dv ? kRectRowsAfter : 0);
       int rc;
       switch (rows) {
