@@ -11,15 +11,14 @@
 // the four, and rounds the operands.  What bounds the kernel is vector issue: per entry and token six fp32
 // instructions and one reciprocal.
 //
-// How a SIMD of gfx950 issues these (measured with one kind of instruction per wave): a wave issues one instruction per 4.3
-// cycles; two waves can issue an fp32 add / mul / fma each in the same 4 cycles, as can one of these beside an integer,
-// conversion or DPP instruction, but a reciprocal (8.3 cycles) runs with no other vector instruction, and the oldest
-// wave goes first.  So (1) a wave that reaches its reciprocals is starved by the older ones' fp32 instructions, and those
-// then run alone at half rate: the reciprocals of a token are issued as one burst at raised wave priority
+// How a SIMD of gfx950 issues these (profiles/issue_rates.txt): a lone wave issues an fp32 add, mul or fma per 5 cycles; two waves
+// issue one each in the same cycles (2.4 to 2.6 per instruction), a reciprocal takes 8.2 with no other beside it, and the
+// oldest wave goes first.  So (1) a wave that reaches its reciprocals is starved by the older ones' fp32 instructions, and
+// those then run alone at half rate: the reciprocals of a token are issued as one burst at raised wave priority
 // (s_setprio; B=8 T=2048 H=12 64x64: 185 -> 161 us); (2) fp32 instructions with a scalar-register operand do not pair
 // (every operand comes from LDS into vector registers, wave-uniform ones too); (3) an odd number of waves on a
-// SIMD leaves one without a partner (two or four waves, not three: __launch registers <= 128).
-// Ideal by these rates: 6 x 2.15 + 8.3 = 21.2 cycles per entry and wave; measured 25.6 (slope over the batch size).
+// SIMD leaves one without a partner (two or four waves, not three: at most 128 registers).
+// Ideal by these rates: 6 x 2.4 + 8.2 = 22.6 cycles per entry and wave; measured 27.9 (profiles/bench_c1.sq_counters_pmc.txt).
 // Against the earlier kernels on the matrix cores: 64x64 B=8 T=2048 H=12 250 -> 155 us, 128x128 B=2 T=4096 H=16
 // 568 -> 388, 96x96 B=8 T=2048 H=16 0.287 -> 0.202 ps per entry, fp32 rows at 64x64 570 -> 160 us (they ran split operands).
 //
