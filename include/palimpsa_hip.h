@@ -48,10 +48,11 @@ extern "C" {
 /* How the chunked entry points (pal_chunk_fwd, pal_gla_chunk_fwd, pal_gla_chunk_bwd) build the states at the start
  * of every tile; no counterpart in the reference, results agree to rounding.  Neither bit: chosen by shape.
  * Meant for tests and measurements. */
-/* fp32 rows (dtype == PAL_DTYPE_F32) through the chunked entry points: by default every matrix product takes its
- * operands as sums of two bf16 numbers (three matrix instructions per product, fp32 accumulation), which keeps
- * outputs, states and gradients within 1e-4 (relative, max-norm) of the fp32 recurrence.  With this flag the fp32
- * rows are rounded to single bf16 / f16 operands like bf16 rows (errors of 1e-3 .. 1e-2, about twice as fast). */
+/* fp32 rows (dtype == PAL_DTYPE_F32) through the chunked entry points: by default every matrix product (tile states,
+ * carries) takes its operands as sums of two bf16 numbers (three matrix instructions per product, fp32 accumulation),
+ * which keeps outputs, states and gradients within 1e-4 (relative, max-norm) of the fp32 recurrence.  With this flag
+ * those products take single bf16 operands (errors of 1e-3 .. 1e-2, a few per cent faster, and pal_chunk_bwd serves
+ * the head dims of bf16 rows).  Outputs and tile gradients are computed in fp32 either way. */
 #define PAL_FLAG_FP32_FAST 1024u
 #define PAL_FLAG_STATES_TWO_KERNELS 256u /* per-tile contributions by all tiles in parallel, then a scan over
                                             the tiles (any shape and dtype)                                  */
@@ -185,13 +186,7 @@ int pal_recurrent_bwd(const PalDims *dims, const PalFwdTensors *t, const PalBwdT
 /* Chunked forward.  Replaces ChunkPalimpsa.forward + chunk_palimpsa_fwd_kernel
  * (chunk_palimpsa_forgetting_scalar.py:66-218, :441-517).  Fills chunk_mu /
  * chunk_I (the reference's intermediate_mu_state / intermediate_I_state,
- * :187-188) for the backward.  The prefix products of the output kernel use f16
- * operands normalised per 64-token tile by three block exponents (of k, v and b),
- * so results do not depend on the magnitude of the rows; within a tile, entries
- * more than 2^26 below the largest of their tensor lose precision.  The state at
- * the start of a tile enters those products through the operands of the tile's
- * first token (as an f16 number: 11 bits, against the 8 of bf16 rows), and the
- * exponents of v and b are raised where that state is large against the rows.
+ * :187-188) for the backward.  Inside a 64-token tile outputs are computed token by token in fp32.
  * cu_seqlens (varlen) must ascend from 0 to the token count; the kernels clamp
  * every sequence and tile to the token range, so a malformed array cannot make
  * them address memory beyond the tensors (results are then unspecified). */

@@ -198,9 +198,10 @@ def set_state_pass_mode(mode: int) -> None:
     _state_pass_mode = mode
 
 
-# fp32 rows through the chunked entry points: False (default) = operands split into two bf16 halves, results within
-# 1e-4 of the fp32 recurrence; True = single bf16/f16 operands as for bf16 rows (PAL_FLAG_FP32_FAST; about twice as
-# fast, errors of 1e-3 .. 1e-2).  Initial value from the environment variable PALIMPSA_FP32_FAST.
+# fp32 rows through the chunked entry points: False (default) = operands of the matrix products split into two bf16 halves,
+# results within 1e-4 of the fp32 recurrence; True = single bf16 operands (PAL_FLAG_FP32_FAST; a few per cent faster,
+# errors of 1e-3 .. 1e-2, the backward's head dims are those of bf16 rows).  Initial value from the environment variable
+# PALIMPSA_FP32_FAST.
 _fp32_fast = os.environ.get("PALIMPSA_FP32_FAST", "0") not in ("", "0")
 
 
@@ -212,8 +213,8 @@ def set_fp32_fast(on: bool) -> None:
 # Backward of the token-serial entry point: sequences of at least this many tokens on average are handed to the
 # chunked backward kernels (tile-start states from a states-only forward, then pal_chunk_bwd; fp32 rows keep the fp32
 # bar there through split operands), shorter ones run the token-serial backward kernel, which walks a sequence
-# token by token (measured at 196608 token-heads of 64 x 64, fp32 rows: 256 sequences of 64 tokens 4.97 ms token-serial
-# against 2.9 ms chunked, 8 sequences of 2048 tokens 7.05 against 2.93; a tile costs the same however few of its 64
+# token by token (measured at 196608 token-heads of 64 x 64, fp32 rows: 256 sequences of 64 tokens 4.96 ms token-serial
+# against 1.42 ms chunked, 8 sequences of 2048 tokens 7.04 against 1.87; a tile costs the same however few of its 64
 # tokens are real, so below a tile per sequence the token-serial kernel wins).  None = never.  Initial value from the environment variable PALIMPSA_RECURRENT_BWD_CHUNK_MIN.
 _recurrent_bwd_chunk_min = os.environ.get("PALIMPSA_RECURRENT_BWD_CHUNK_MIN", "64")
 _recurrent_bwd_chunk_min = None if _recurrent_bwd_chunk_min in ("", "none", "None") else int(_recurrent_bwd_chunk_min)

@@ -6,8 +6,8 @@
 //   M_t = sum_s L[t,s] v_s k_s^T + F_t M_0          (the associative scan of the
 //   I_t = sum_s L[t,s] b_s (k_s*k_s)^T + F_t (I_0 - Ip) + Ip    reference,
 //                                     chunk_palimpsa_forgetting_scalar.py:190-195)
-// The sums over s are bf16 MFMA contractions with fp32 accumulation; M_0, I_0
-// are the fp32 states at the start of the tile.
+// M_0, I_0 are the fp32 states at the start of the tile.  The kernels that carry the state from tile to tile take the
+// sums over s as bf16 MFMA contractions with fp32 accumulation; those that work inside the tiles run token by token.
 #pragma once
 #include "pal_common.h"
 

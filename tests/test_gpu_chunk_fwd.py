@@ -82,8 +82,8 @@ def test_fp32_inputs_meet_the_fp32_bar(gpu_device, dk, dv):
 
 
 def test_fp32_fast_mode_is_an_opt_in_at_bf16_accuracy(gpu_device):
-    """PAL_FLAG_FP32_FAST (here through the Python knob): fp32 rows rounded to single bf16/f16 operands, the accuracy
-    of the bf16 path, about twice as fast; never the default."""
+    """PAL_FLAG_FP32_FAST (here through the Python knob): single bf16 operands in the products that build the
+    tile states, the accuracy of the bf16 path; never the default."""
     from palimpsa_amd import _lib
     ck, _ = _ops()
     inp = po.make_inputs(2, 100, 2, 32, 48, seed=4)
@@ -158,9 +158,8 @@ def test_error_paths_match_reference(gpu_device):
 @pytest.mark.parametrize("v_scale,k_scale", [(3.0e5, 1.0), (40.0, 30.0), (1.0e-4, 1.0), (1.0e-6, 1.0), (1.0e-8, 1.0),
                                              (1.0, 300.0), (1.0e20, 1.0e-3), (1.0e-20, 1.0e3)])
 def test_block_exponent_of_the_f16_operands(gpu_device, v_scale, k_scale):
-    """Rows far from O(1), in both directions: the output kernel's f16 operands are normalised per tile by block
-    exponents of k, v and b, so the relative error is that of O(1) rows and nothing overflows or flushes
-    (|k| = 300 squares to 9e4, beyond the f16 range without the exponent of k)."""
+    """Rows far from O(1), in both directions: the relative error is that of O(1) rows and nothing overflows or flushes
+    (|k| = 300 squares to 9e4, beyond the range of half-precision operands)."""
     ck, _ = _ops()
     B, T, H, d = 1, 200, 2, 64
     inp = po.make_inputs(B, T, H, d, d, seed=77)
@@ -178,11 +177,10 @@ def test_block_exponent_of_the_f16_operands(gpu_device, v_scale, k_scale):
 @pytest.mark.parametrize("d", [64, 96])
 @pytest.mark.parametrize("case", ["rows_shrink", "large_initial_state", "precision_below_prior", "rows_grow"])
 def test_tile_start_state_in_the_first_token_operands(gpu_device, d, case):
-    """The output kernels add the tile-start state to the f16 operands of a tile's first token and make room for it in
-    the block exponents.  Cases where the state and the rows of a tile are far apart, for both kernel layouts
-    (d = 64: by key columns, d = 96: by value rows): rows that shrink by 1e5 half way (the state then dwarfs them),
-    an initial state 1e4 above the rows, an initial precision far below the prior (I_t = (1 - F_t) Ip + F_t I_0 + ...
-    has no cancelling term), rows that grow by 1e4 (the state is then small against them)."""
+    """Cases where the state at the start of a tile and the rows of the tile are far apart, for two layouts of the output
+    kernel: rows that shrink by 1e5 half way (the state then dwarfs them), an initial state 1e4 above the rows, an
+    initial precision far below the prior (I_t = (1 - F_t) Ip + F_t I_0 + ... has no cancelling term), rows that grow by
+    1e4 (the state is then small against them)."""
     ck, _ = _ops()
     B, T, H = 1, 320, 2
     inp = po.make_inputs(B, T, H, d, d, seed=123)
