@@ -363,13 +363,14 @@ def test_runs_on_the_callers_stream(gpu_device):
     assert torch.isfinite(total)
 
 
-def test_forward_and_backward_replay_in_a_graph(gpu_device):
+@pytest.mark.parametrize("dk,dv", [(64, 64), (80, 96)])   # one piece per head; several, side by side, and their sum
+def test_forward_and_backward_replay_in_a_graph(gpu_device, dk, dv):
     """chunk_palimpsa forward + backward recorded into a HIP graph (the C ABI allocates nothing, synchronises nothing
     and records no memset; the wrapper's buffers come from torch's capture-aware allocator): three replays on new
     input values, with eager work and synchronisations in between, each equal to the eager result."""
     from palimpsa_amd.ops.palimpsa import chunk_palimpsa
     dev = gpu_device
-    B, T, H, dk, dv = 2, 200, 2, 64, 64
+    B, T, H = 2, 200, 2
     names = ("q", "k", "v", "b", "gt", "g", "Ip")
 
     def fresh(seed):

@@ -341,9 +341,8 @@ def test_output_kernel_wave_layouts_with_uncertainty(gpu_device, dk, dv):
 @pytest.mark.parametrize("dk,dv,var", [(112, 112, False), (64, 96, True), (96, 192, False), (48, 80, True),
                                        (16, 64, False), (128, 128, True)])
 def test_output_kernel_row_layout_slices_packed(gpu_device, dk, dv, var):
-    """Head dims whose forward output kernel is laid out by value rows, with slices of unequal size (112 = 64 + 48,
-    80 = 48 + 32 with uncertainty), several slices (192 = 3 x 64), one column block (dk = 16) and eight, on a packed
-    batch with tiles of 1, 2, 63 and 64 tokens and an initial state per document."""
+    """Head dims whose value rows the waves of the output kernel share unevenly (112, 80, 192) and one to eight blocks of key
+    columns, on a packed batch with tiles of 1, 2, 63 and 64 tokens and an initial state per document."""
     ck, _ = _ops()
     H = 2
     cu = [0, 1, 3, 66, 130, 257]
