@@ -219,3 +219,27 @@ def test_calls_on_a_stream_of_their_own(gpu_device):
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(out, want) and torch.equal(got_r, want_r)
     assert all(torch.equal(a, b) for a, b in zip(got_g, want_g))
+
+
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_activation_checkpointing(gpu_device, reentrant):
+    """torch.utils.checkpoint runs the forward again inside the backward and stops it by an exception from a hook."""
+    from torch.utils.checkpoint import checkpoint
+
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    x = _plain_call(gpu_device, T=150, grad=range(7))
+
+    def f(*a):
+        return chunk_palimpsa(*a).square()
+
+    want = torch.autograd.grad(f(*x).sum(), x)
+    y = checkpoint(f, *x, use_reentrant=reentrant)
+    if reentrant:
+        y.sum().backward()
+        got = [t.grad for t in x]
+    else:
+        got = torch.autograd.grad(y.sum(), x)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    with torch.inference_mode():
+        from palimpsa_amd import _lib as L
+        assert L.host().chunk_fwd(*[t.detach() for t in x], None, None, 1.0, False, 0, None, None, 1 << 30) is not None
