@@ -11,6 +11,8 @@
 //
 //  local   per (tile, head): chunk_bwd_tile.h -- dq, the tile's own parts of dv, db, dk and of the gate gradient, and
 //          the carry the tile hands to its predecessor, R_loc = f_first * dM^loc_first.
+//          Heads above 64x64 in several pieces (chunk_bwd.h); a small pass works on them side by side and
+//  sum     adds up their parts.
 //  scan    per state entry: R_{c-1} = R_loc,c + F_C,c R_c backwards over the tiles
 //          of a sequence (the role of curr_dM/curr_dI, :429-430); also yields the
 //          gradients of the initial state.
