@@ -411,3 +411,39 @@ def test_decode_with_the_mean_state_kept_in_bf16(gpu_device):
     assert hp.max_rel(outs["fp32"][1], mu_ref) <= 1e-4 and hp.max_rel(outs["fp32"][2], I_ref) <= 1e-4
     assert hp.max_rel(outs["bf16"][1], mu_ref) <= 2e-2
     assert hp.max_rel(outs["bf16"][2], I_ref) <= 1e-4          # I never sees the rounding of mu
+
+
+@pytest.mark.parametrize("H,dk,dv,lens", [
+    (3, 48, 48, [8]), (3, 32, 32, [15]), (2, 64, 80, [16]), (2, 16, 16, [31]), (2, 32, 48, [32]), (1, 128, 64, [33]),   # 4, 8, 16 waves
+    (2, 256, 64, [49]), (2, 192, 16, [100]),                    # wide keys: 8 at most
+    (8, 96, 192, [64, 65, 70, 64]), (16, 64, 64, [8, 9]),       # more value rows: 4
+    (2, 32, 32, [1, 90, 0, 5, 64]),                             # documents shorter than their segments, and an empty one
+])
+def test_sequences_in_segments(gpu_device, H, dk, dv, lens):
+    """Sequences that a workgroup walks in segments: lengths beside the rule's lines and the segments' ends, initial
+    state, uncertainty and a final state written over the initial one's place in memory."""
+    packed = len(set(lens)) > 1
+    B, T = (1, sum(lens)) if packed else (len(lens), lens[0])
+    N = len(lens)
+    inp = po.make_inputs(B, T, H, dk, dv, seed=dk + dv + T)
+    inp["g"] = torch.linspace(0.05, 6.0, H)
+    gen = torch.Generator().manual_seed(T)
+    mu0 = 0.1 * torch.randn(N, H, dv, dk, generator=gen)
+    I0 = inp["Ip"].view(1, H, 1, 1) + torch.nn.functional.softplus(torch.randn(N, H, dv, dk, generator=gen))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32) if packed else None
+    o_ref, ov_ref, mu_ref, I_ref = hp.oracle_forward(inp, mu0=mu0, I0=I0, cu=cu, want_var=0 not in lens, dtype=torch.float64)
+    d = hp.to_device(inp, gpu_device)
+    rows = [d[n] for n in ("q", "k", "v", "b", "gt", "g", "Ip")]
+    mu0, I0 = mu0.to(gpu_device), I0.to(gpu_device)
+    (o, ov), mu, I = _ops()(*rows, initial_mu_state=mu0, initial_I_state=I0, output_final_state=True,
+                            output_uncertainty=True, cu_seqlens=None if cu is None else cu.to(gpu_device))
+    for x, r in ((o, o_ref), (ov, ov_ref), (mu, mu_ref), (I, I_ref)):
+        if r is None:   # (the oracle has no uncertainty for empty documents)
+            continue
+        assert hp.max_rel(x, r) <= 1e-5   # fp32 sums of up to 100 tokens in any order: a few times 2^-24 per token
+    if not packed:   # the bound step updates its states in place
+        from palimpsa_amd.ops.palimpsa import DecodeStep
+        step = DecodeStep(B, H, dk, dv, gpu_device, torch.float32, tokens=T)
+        step.bind(*rows, mu0, I0)
+        assert hp.max_rel(step.step(), o_ref) <= 1e-5
+        assert hp.max_rel(mu0, mu_ref) <= 1e-5 and hp.max_rel(I0, I_ref) <= 1e-5
