@@ -71,6 +71,12 @@ extern "C" {
  * hands long sequences to pal_chunk_bwd this way.  No counterpart in the reference. */
 #define PAL_FLAG_STATES_ONLY 4096u
 
+/* pal_gla_chunk_fwd and pal_gla_chunk_bwd, bf16 rows: every result is computed in one walk over each sequence with the
+ * running state in registers; no tile states are kept, chunk_mu and chunk_I are NULL (PAL_E_STATE otherwise, and for rows of
+ * fp32 or of 2 GiB and more).  Both calls of a pair are made with the flag or both without it, and the workspace of the
+ * backward is asked for with the flags of its call.  pal_gla_walk_applies tells when it is the faster way. */
+#define PAL_FLAG_GLA_NO_TILES 8192u
+
 /* error codes (negative) */
 #define PAL_OK 0
 #define PAL_E_NULL -1        /* required pointer is NULL                      */
@@ -221,6 +227,10 @@ int pal_chunk_fwd_static(const PalDims *dims, const PalFwdTensors *t, void *stre
  * b, Ip, o_var, init_I, final_I are ignored; PAL_FLAG_HAS_VAR is rejected with
  * PAL_E_STATE.  init_mu / final_mu hold S as [N,H,dv,dk] fp32. */
 int pal_gla_chunk_fwd(const PalDims *dims, const PalFwdTensors *t, void *stream);
+
+/* 1 when pal_gla_chunk_fwd and pal_gla_chunk_bwd of these dims (flags included; longest: tokens of the longest sequence) are
+ * faster with PAL_FLAG_GLA_NO_TILES: bf16 rows, and enough sequences and heads that walks over whole sequences fill the GPU. */
+int pal_gla_walk_applies(const PalDims *dims, int64_t longest);
 
 /* Token-serial forward without the precision state (T >= 1; T == 1 is a decode
  * step).  Replaces fla.ops.simple_gla.fused_recurrent_simple_gla as called at

@@ -18,6 +18,7 @@ PAL_FLAG_VARLEN, PAL_FLAG_HAS_INIT, PAL_FLAG_STORE_FINAL, PAL_FLAG_HAS_VAR = 1, 
 PAL_FLAG_STATES_TWO_KERNELS, PAL_FLAG_STATES_ONE_PASS, PAL_FLAG_FP32_FAST = 256, 512, 1024
 PAL_FLAG_STATE_MU_BF16 = 2048   # pal_recurrent_fwd: mu kept in bf16 between calls (DecodeStep(mu_dtype=torch.bfloat16))
 PAL_FLAG_STATES_ONLY = 4096     # pal_chunk_fwd: tile-start states only, outputs untouched
+PAL_FLAG_GLA_NO_TILES = 8192    # pal_gla_chunk_fwd / bwd: no tile states in memory (see pal_gla_walk_applies)
 PAL_CHUNK = 64
 
 PAL_E_NULL, PAL_E_DIM, PAL_E_HEADDIM, PAL_E_DTYPE, PAL_E_VARLEN_BATCH = -1, -2, -3, -4, -5
@@ -130,6 +131,8 @@ def load() -> C.CDLL:
         fn.argtypes = [P(PalGlueDims)]
     lib.pal_state_pass_applies.restype = C.c_int
     lib.pal_state_pass_applies.argtypes = [P(PalDims), C.c_int]
+    lib.pal_gla_walk_applies.restype = C.c_int
+    lib.pal_gla_walk_applies.argtypes = [P(PalDims), C.c_int64]
     lib.pal_chunk_bwd_supported.restype = C.c_int
     lib.pal_chunk_bwd_supported.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_uint32]
     lib.pal_profile_enable.restype = C.c_int

@@ -74,6 +74,54 @@ __device__ __forceinline__ void seq_lookup(const ChunkArgs& a, int n, int& bos, 
   }
 }
 
+// Workgroups that walk the tiles of a sequence in order, one per (sequence, head, slice): consecutive workgroup ids go to
+// different XCDs, the slices of one (sequence, head) belong on the same one (they read the same rows).
+struct WalkPlan {
+  int32_t n_sl, per_xcd, total;
+  int32_t by_length;   // packed sequences are handed out longest first (see walk_item)
+};
+inline bool walk_plan(const ChunkArgs& a, int n_sl, WalkPlan& p) {
+  const int64_t total = (int64_t)a.n_seqs * a.H * n_sl;
+  int64_t per_xcd = (total + 7) / 8;
+  per_xcd = (per_xcd + n_sl - 1) / n_sl * n_sl;
+  p.by_length = (a.cu_seqlens && a.n_seqs > 1 && a.n_seqs <= 64) ? 1 : 0;
+  if (p.by_length) per_xcd = (int64_t)((a.n_seqs + 7) / 8) * a.H * n_sl;   // whole sequences per XCD
+  if (per_xcd * 8 > 0x7fffffff) return false;
+  p.n_sl = n_sl;
+  p.total = (int32_t)total;
+  p.per_xcd = (int32_t)per_xcd;   // the grid is 8 per_xcd workgroups
+  return true;
+}
+// the workgroup's sequence, head and slice; false: it has none
+__device__ __forceinline__ bool walk_item(const ChunkArgs& a, const WalkPlan& p, int lane, int& n, int& h, int& sl) {
+  const int xcd = (int)blockIdx.x & 7, pos = (int)blockIdx.x >> 3;
+  int m;
+  if (p.by_length) {
+    // Packed sequences of unequal length (at most 64): the walk over a sequence's tiles is serial, so a long sequence
+    // that starts late ends the kernel late.  The sequence of rank r in descending length goes to XCD r mod 8, in
+    // rank order there; every wave finds the sequence of its rank with one lane per sequence.
+    const int rank = (pos / (a.H * p.n_sl)) * 8 + xcd;
+    if (rank >= a.n_seqs) return false;
+    int b_l = 0, len_l = -1;
+    if (lane < a.n_seqs) packed_seq_bounds(a.cu_seqlens, lane, a.T, b_l, len_l);
+    int before = 0;   // sequences ahead of lane's own in the order (longer, or as long with a smaller index)
+    for (int j = 0; j < a.n_seqs; ++j) {
+      const int len_j = __builtin_amdgcn_readlane(len_l, j);
+      before += (len_j > len_l || (len_j == len_l && j < lane)) ? 1 : 0;
+    }
+    const uint64_t hit = __ballot(lane < a.n_seqs && before == rank);
+    n = hit ? (int)__builtin_ctzll(hit) : 0;
+    m = n * a.H * p.n_sl + pos % (a.H * p.n_sl);
+  } else {
+    m = xcd * p.per_xcd + pos;
+    if (m >= p.total) return false;
+    n = (m / p.n_sl) / a.H;
+  }
+  sl = m % p.n_sl;
+  h = (m / p.n_sl) % a.H;
+  return true;
+}
+
 // inclusive prefix sum over the 64 lanes of a wave: four shifted adds inside each row of 16 lanes (DPP
 // row_shr with zero fill), then the totals of the rows before (lane 15 of each, read as scalars)
 template <int N>

@@ -7,8 +7,10 @@
 //     O = ((Q K^T) o L) V + diag(F) Q S_0^T ,      L[t,s] = 2^{c_t - c_s} (s <= t),  F_t = 2^{c_t},
 // so nothing of the [tokens x dv x dk] state has to be materialised per token: the tile-start states
 // come from the same two kernels as in the Palimpsa forward (local contribution + serial scan, both
-// without the J branch) and the kernel below does the rest on the matrix cores.
+// without the J branch) and the kernel below does the rest on the matrix cores.  Where there are enough sequences and heads
+// the states do not exist in memory either: gla_walk.hip.
 #include "chunk_common.h"
+#include "gla_walk.h"
 #include "pal_host.h"
 #include "pal_profile.h"
 
@@ -663,7 +665,12 @@ static int check_gla(const PalDims* d, const PalFwdTensors* t) {
   int rc = pal_validate_dims(d);
   if (rc) return rc;
   if (!t) return PAL_E_NULL;
-  if (!t->q || !t->k || !t->v || !t->gt || !t->g || !t->o || !t->chunk_I) return PAL_E_NULL;
+  if (!t->q || !t->k || !t->v || !t->gt || !t->g || !t->o) return PAL_E_NULL;
+  if (d->flags & PAL_FLAG_GLA_NO_TILES) {
+    if (t->chunk_mu || t->chunk_I || !gla_walk_possible(d)) return PAL_E_STATE;
+  } else if (!t->chunk_I) {
+    return PAL_E_NULL;
+  }
   if (d->flags & PAL_FLAG_HAS_VAR) return PAL_E_STATE;   // no precision state, no output variance
   if (d->flags & PAL_FLAG_STATE_MU_BF16) return PAL_E_STATE;
   if (((d->flags & PAL_FLAG_HAS_INIT) != 0) != (t->init_mu != nullptr)) return PAL_E_STATE;
@@ -762,7 +769,8 @@ __global__ __launch_bounds__(256) void gla_bwd_scan_kernel(ChunkArgs a, const fl
 constexpr int kGateTok = 4;                    // consecutive tokens per thread
 constexpr int kGatePiece = 256 * kGateTok;     // tokens per step of a workgroup
 
-__global__ __launch_bounds__(256) void gla_bwd_gate_kernel(ChunkArgs a, const float* qdq, const float* kdk, float* dgt,
+// (The dot products come in n_dot parts of [H][tokens], one per slice of the columns they sum over.)
+__global__ __launch_bounds__(256) void gla_bwd_gate_kernel(ChunkArgs a, const float* qdq, const float* kdk, int n_dot, float* dgt,
                                                            float* dg_part, int64_t n_tokens) {
   __shared__ float sTot[2][4];
   __shared__ float sAcc[4];
@@ -780,6 +788,10 @@ __global__ __launch_bounds__(256) void gla_bwd_gate_kernel(ChunkArgs a, const fl
     for (int j = 0; j < kGateTok; ++j) {
       const int64_t off = (int64_t)h * n_tokens + bos + tf + j;      // the dot products are stored head-major
       x[j] = (tf + j < len) ? qdq[off] - kdk[off] : 0.f;
+      for (int u = 1; u < n_dot; ++u) {
+        const int64_t part = off + (int64_t)u * a.H * n_tokens;
+        if (tf + j < len) x[j] += qdq[part] - kdk[part];
+      }
     }
     // suffix sums inside the thread, then over the lanes of the wave (exclusive of the thread itself)
 #pragma unroll
@@ -831,17 +843,20 @@ __global__ void gla_bwd_head_reduce_kernel(const float* dg_part, float* dg, int 
 // per-sequence shares of dg
 struct GlaBwdWorkspace {
   size_t d_tiles, g_tiles, qdq, kdk, dg_part, dq_full, dk_full, total;
+  int n_dot;   // parts that the dot products come in
 };
 static GlaBwdWorkspace gla_bwd_layout(const PalDims* d) {
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
   GlaBwdWorkspace w;
   const size_t tokens = (size_t)d->batch * d->seq_len;
-  const size_t entries = (size_t)d->total_chunks * d->n_heads * d->dv * d->dk;
+  const bool walk = d->flags & PAL_FLAG_GLA_NO_TILES;   // no tiles in memory
+  const size_t entries = walk ? 0 : (size_t)d->total_chunks * d->n_heads * d->dv * d->dk;
+  w.n_dot = walk ? gla_walk_slices(d, d->dv, d->dk, 2) : 1;
   w.d_tiles = 0;
   w.g_tiles = w.d_tiles + up(sizeof(float) * entries);
   w.qdq = w.g_tiles + up(sizeof(bf16_t) * entries);
-  w.kdk = w.qdq + up(sizeof(float) * tokens * d->n_heads);
-  w.dg_part = w.kdk + up(sizeof(float) * tokens * d->n_heads);
+  w.kdk = w.qdq + up(sizeof(float) * tokens * d->n_heads * w.n_dot);
+  w.dg_part = w.kdk + up(sizeof(float) * tokens * d->n_heads * w.n_dot);
   w.total = w.dg_part + up(sizeof(float) * (size_t)d->n_seqs * d->n_heads);
   w.dq_full = w.dk_full = w.total;
   if (d->n_qk_heads > 0 && d->n_qk_heads != d->n_heads) {   // one dq, dk row per value head, summed per group at the end
@@ -887,8 +902,27 @@ extern "C" int pal_gla_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const
   const bool grouped = a.Hq != a.H;
   void* dq_out = grouped ? (void*)(ws + w.dq_full) : gr->dq;
   void* dk_out = grouped ? (void*)(ws + w.dk_full) : gr->dk;
-  // D_c = sum_t F_t dO_t q_t^T per tile, then the reverse scan over the tiles of each sequence
-  {
+  const bool walk = d->flags & PAL_FLAG_GLA_NO_TILES;
+  if (walk) {
+    GlaWalkArgs A{};
+    A.c = a;
+    A.n_tokens = (int64_t)d->batch * d->seq_len;
+    // dv: X = k, Y = q, Z = dO, from the end; what is left before the first tile is the gradient of the initial state
+    A.role[0] = GlaWalkRole{(const bf16_t*)t->k, (const bf16_t*)t->q, (const bf16_t*)gr->d_o, nullptr, (bf16_t*)gr->dv, nullptr,
+                            nullptr, gr->d_init_mu, 0, 1, a.scale};
+    A.n_roles = 1;
+    A.dc = d->dk; A.de = d->dv; A.hX = a.Hq; A.hZ = a.H;
+    if (int rc = launch_gla_walk(A, d, kKernGlaDv, s)) return rc;
+    // dq: X = dO, Y = v, Z = k, the state transposed, q . dq on the side; dk: X = v, Y = dO, Z = q, from the end, k . dk
+    A.role[0] = GlaWalkRole{(const bf16_t*)gr->d_o, (const bf16_t*)t->v, (const bf16_t*)t->k, (const bf16_t*)t->q, (bf16_t*)dq_out,
+                            qdq, t->init_mu, nullptr, 1, 0, 0.f};
+    A.role[1] = GlaWalkRole{(const bf16_t*)t->v, (const bf16_t*)gr->d_o, (const bf16_t*)t->q, (const bf16_t*)t->k, (bf16_t*)dk_out,
+                            kdk, nullptr, nullptr, 0, 1, 0.f};
+    A.n_roles = 2;
+    A.dc = d->dv; A.de = d->dk; A.hX = a.H; A.hZ = a.Hq;
+    if (int rc = launch_gla_walk(A, d, kKernGlaDk, s)) return rc;
+  } else {
+    // D_c = sum_t F_t dO_t q_t^T per tile, then the reverse scan over the tiles of each sequence
     ChunkArgs b = a;
     b.k = t->q; b.v = gr->d_o; b.chunk_mu = d_tiles; b.flags |= kFlagDecayFromStart;
     if (state_pass_applies(b, d->dtype, false)) {
@@ -896,15 +930,15 @@ extern "C" int pal_gla_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const
                                      kKernGlaBwdStates, s))
         return rc;
     } else {
-    if (int rc = launch_tile_delta(b, d->dtype, false, s)) return rc;
-    const int64_t blocks = (int64_t)d->n_seqs * d->n_heads * (((int64_t)d->dv * d->dk + 1023) / 1024);
-    if (blocks > 0x7fffffff) return PAL_E_DIM;
-    PAL_TIMED_LAUNCH(kKernGlaBwdScan, s, gla_bwd_scan_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, d_tiles,
-                     g_tiles, gr->d_init_mu);
-    PAL_HIP_LAUNCH_CHECK();
+      if (int rc = launch_tile_delta(b, d->dtype, false, s)) return rc;
+      const int64_t blocks = (int64_t)d->n_seqs * d->n_heads * (((int64_t)d->dv * d->dk + 1023) / 1024);
+      if (blocks > 0x7fffffff) return PAL_E_DIM;
+      PAL_TIMED_LAUNCH(kKernGlaBwdScan, s, gla_bwd_scan_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, d_tiles,
+                       g_tiles, gr->d_init_mu);
+      PAL_HIP_LAUNCH_CHECK();
     }
   }
-  if (gla_bwd_tile_applies(d)) {
+  if (!walk && gla_bwd_tile_applies(d)) {
     GlaBwdTileArgs F{};
     F.c = a;
     F.q = t->q; F.k = t->k; F.v = t->v; F.d_o = gr->d_o;
@@ -912,29 +946,29 @@ extern "C" int pal_gla_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const
     F.dq = dq_out; F.dk = dk_out; F.dv = gr->dv; F.qdq = qdq; F.kdk = kdk;
     F.n_tokens = (int64_t)d->batch * d->seq_len;
     if (int rc = launch_gla_bwd_tile(F, s)) return rc;
-  } else {
-  GlaTileArgs A{};
-  A.c = a;
-  A.n_tokens = (int64_t)d->batch * d->seq_len;
-  // dq: X = dO, Y = v, Z = k, tile-start states read transposed; q . dq on the side
-  A.X = gr->d_o; A.Y = t->v; A.Z = t->k; A.St = (const bf16_t*)t->chunk_I; A.out = dq_out; A.W = t->q; A.dot = qdq;
-  A.dc = d->dv; A.de = d->dk;
-  A.hX = a.H; A.hY = a.H; A.hZ = a.Hq; A.hW = a.Hq;
-  if (int rc = launch_gla_tile_dt(A, d->dtype, kGlaDq, s)) return rc;
-  // dv: X = k, Y = q, Z = dO, tile-end state gradients
-  A.X = t->k; A.Y = t->q; A.Z = gr->d_o; A.St = g_tiles; A.out = gr->dv; A.W = nullptr; A.dot = nullptr;
-  A.dc = d->dk; A.de = d->dv;
-  A.hX = a.Hq; A.hY = a.Hq; A.hZ = a.H; A.hW = a.H;
-  if (int rc = launch_gla_tile_dt(A, d->dtype, kGlaDv, s)) return rc;
-  // dk: X = v, Y = dO, Z = q, tile-end state gradients read transposed; k . dk on the side
-  A.X = t->v; A.Y = gr->d_o; A.Z = t->q; A.St = g_tiles; A.out = dk_out; A.W = t->k; A.dot = kdk;
-  A.dc = d->dv; A.de = d->dk;
-  A.hX = a.H; A.hY = a.H; A.hZ = a.Hq; A.hW = a.Hq;
-  if (int rc = launch_gla_tile_dt(A, d->dtype, kGlaDk, s)) return rc;
+  } else if (!walk) {
+    GlaTileArgs A{};
+    A.c = a;
+    A.n_tokens = (int64_t)d->batch * d->seq_len;
+    // dq: X = dO, Y = v, Z = k, tile-start states read transposed; q . dq on the side
+    A.X = gr->d_o; A.Y = t->v; A.Z = t->k; A.St = (const bf16_t*)t->chunk_I; A.out = dq_out; A.W = t->q; A.dot = qdq;
+    A.dc = d->dv; A.de = d->dk;
+    A.hX = a.H; A.hY = a.H; A.hZ = a.Hq; A.hW = a.Hq;
+    if (int rc = launch_gla_tile_dt(A, d->dtype, kGlaDq, s)) return rc;
+    // dv: X = k, Y = q, Z = dO, tile-end state gradients
+    A.X = t->k; A.Y = t->q; A.Z = gr->d_o; A.St = g_tiles; A.out = gr->dv; A.W = nullptr; A.dot = nullptr;
+    A.dc = d->dk; A.de = d->dv;
+    A.hX = a.Hq; A.hY = a.Hq; A.hZ = a.H; A.hW = a.H;
+    if (int rc = launch_gla_tile_dt(A, d->dtype, kGlaDv, s)) return rc;
+    // dk: X = v, Y = dO, Z = q, tile-end state gradients read transposed; k . dk on the side
+    A.X = t->v; A.Y = gr->d_o; A.Z = t->q; A.St = g_tiles; A.out = dk_out; A.W = t->k; A.dot = kdk;
+    A.dc = d->dv; A.de = d->dk;
+    A.hX = a.H; A.hY = a.H; A.hZ = a.Hq; A.hW = a.Hq;
+    if (int rc = launch_gla_tile_dt(A, d->dtype, kGlaDk, s)) return rc;
   }
   {
     const int64_t blocks = (int64_t)d->n_seqs * d->n_heads;
-    PAL_TIMED_LAUNCH(kKernGlaBwdGate, s, gla_bwd_gate_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, qdq, kdk, gr->dgt,
+    PAL_TIMED_LAUNCH(kKernGlaBwdGate, s, gla_bwd_gate_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a, qdq, kdk, w.n_dot, gr->dgt,
                      dg_part, (int64_t)d->batch * d->seq_len);
     PAL_HIP_LAUNCH_CHECK();
     hipLaunchKernelGGL(gla_bwd_head_reduce_kernel, dim3((d->n_heads + 63) / 64), dim3(64), 0, s, dg_part, gr->dg,
@@ -954,6 +988,15 @@ extern "C" int pal_gla_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void*
   if (int rc = check_gla(d, t)) return rc;
   ChunkArgs a;
   fill_gla_args(a, d, t);
+  if (d->flags & PAL_FLAG_GLA_NO_TILES) {
+    GlaWalkArgs A{};
+    A.c = a;
+    A.role[0] = GlaWalkRole{(const bf16_t*)t->q, (const bf16_t*)t->k, (const bf16_t*)t->v, nullptr, (bf16_t*)t->o, nullptr,
+                            t->init_mu, t->final_mu, 0, 0, 1.f};
+    A.n_roles = 1;
+    A.dc = d->dk; A.de = d->dv; A.hX = a.Hq; A.hZ = a.H;
+    return launch_gla_walk(A, d, kKernGlaOut, (hipStream_t)stream);
+  }
   // the fp32 scratch is only used by the two-kernel form of the tile-start states
   if (!t->chunk_mu && !state_pass_applies(a, d->dtype, false)) return PAL_E_NULL;
   hipStream_t s = (hipStream_t)stream;

@@ -157,13 +157,22 @@ def chunk_meta(cu_seqlens: torch.Tensor, total_tokens: int, device: torch.device
     the copy taken when its entry was made (its memory may be shared with an array that a loader rewrites without
     torch noticing).  For a device tensor the entry relies on torch's version counter: a kernel or extension that
     writes through ``data_ptr()`` must call ``invalidate_chunk_meta()`` (or hand over a new tensor)."""
+    return _chunk_entry(cu_seqlens, total_tokens, device)[:2]
+
+
+def longest_sequence(cu_seqlens: torch.Tensor, total_tokens: int, device: torch.device) -> int:
+    """Tokens of the longest sequence of a packed batch (kept with the chunk bookkeeping of ``chunk_meta``)."""
+    return _chunk_entry(cu_seqlens, total_tokens, device)[2]
+
+
+def _chunk_entry(cu_seqlens: torch.Tensor, total_tokens: int, device: torch.device):
     key = id(cu_seqlens)
     hit = _chunk_meta_cache.get(key)
     if hit is not None:
-        ref, version, tokens, dev, packed, total, host_copy = hit
+        ref, version, tokens, dev, packed, total, longest, host_copy = hit
         if (ref() is cu_seqlens and version == cu_seqlens._version and tokens == total_tokens and dev == device
                 and (host_copy is None or torch.equal(cu_seqlens.detach().to(torch.int64), host_copy))):
-            return packed, total
+            return packed, total, longest
     if cu_seqlens.dim() != 1 or cu_seqlens.numel() < 2:
         raise ValueError(f"cu_seqlens must be a 1-D tensor of at least two entries, got shape {tuple(cu_seqlens.shape)}")
     cu_host = cu_seqlens.detach().to("cpu", torch.int64).numpy()
@@ -174,16 +183,16 @@ def chunk_meta(cu_seqlens: torch.Tensor, total_tokens: int, device: torch.device
             f"decreasing={bool((cu_host[1:] < cu_host[:-1]).any())}")
     table, offsets = L.build_chunk_table(cu_host)
     packed = torch.cat([torch.from_numpy(offsets), torch.from_numpy(table.reshape(-1))]).to(torch.int32).to(device)
-    total = int(table.shape[0])
+    total, longest = int(table.shape[0]), int((cu_host[1:] - cu_host[:-1]).max())
     if len(_chunk_meta_cache) >= _CHUNK_META_CACHE_MAX:
         _chunk_meta_cache.pop(next(iter(_chunk_meta_cache)))
     try:
         ref = weakref.ref(cu_seqlens, lambda _r, k=key: _chunk_meta_cache.pop(k, None))
     except TypeError:
-        return packed, total
+        return packed, total, longest
     host_copy = torch.from_numpy(cu_host).clone() if cu_seqlens.device.type == "cpu" else None
-    _chunk_meta_cache[key] = (ref, cu_seqlens._version, int(total_tokens), device, packed, total, host_copy)
-    return packed, total
+    _chunk_meta_cache[key] = (ref, cu_seqlens._version, int(total_tokens), device, packed, total, longest, host_copy)
+    return packed, total, longest
 
 
 def invalidate_chunk_meta() -> None:

@@ -74,6 +74,11 @@ def _run(op, q, k, v, g, scale, initial_state, output_final_state, cu_seqlens, *
     return out, None
 
 
+def _walks(dims: L.PalDims, longest: int) -> bool:
+    """Whether a call runs as walks over whole sequences (many of them, or many heads) instead of tiles in parallel."""
+    return bool(L.load().pal_gla_walk_applies(dims, longest))
+
+
 class ChunkSimpleGLA(torch.autograd.Function):
     """forward(ctx, q, k, v, g, scale, initial_state, output_final_state, cu_seqlens) -> (o, final_state | None)
     on ``pal_gla_chunk_fwd`` / ``pal_gla_chunk_bwd``.  The state is ``[N, H, dk, dv]`` at this boundary and
@@ -100,16 +105,20 @@ class ChunkSimpleGLA(torch.autograd.Function):
         if p.init_mu is not None:
             flags |= L.PAL_FLAG_HAS_INIT
         o = torch.empty(B, T, H, p.dv_p, dtype=p.compute_dtype, device=dev)
-        # per-tile contributions (fp32, only needed inside the call) and tile-start states (bf16, kept for the backward)
-        tile_S = torch.empty(total_chunks, H, p.dv_p, p.dk_p, dtype=torch.bfloat16, device=dev)
         final = None
         if output_final_state:
             final = torch.empty(p.n_seqs, H, p.dv_p, p.dk_p, dtype=torch.float32, device=dev)
         dims = cm.make_dims(p, scale, flags | (L.PAL_FLAG_STORE_FINAL if output_final_state else 0), total_chunks)
-        # the fp32 scratch (4 bytes per state entry and tile) only exists for the two-kernel form of the tile states
-        scratch = None
-        if not L.load().pal_state_pass_applies(dims, 0):
-            scratch = torch.empty(total_chunks, H, p.dv_p, p.dk_p, dtype=torch.float32, device=dev)
+        tile_S = scratch = None
+        if _walks(dims, T if p.cu_seqlens is None else cm.longest_sequence(cu_seqlens, T, dev)):
+            flags |= L.PAL_FLAG_GLA_NO_TILES       # forward and backward without tile states in memory
+            dims.flags |= L.PAL_FLAG_GLA_NO_TILES
+        else:
+            # tile-start states (bf16, kept for the backward) and per-tile contributions (fp32, only inside the call: 4
+            # bytes per state entry and tile, for the two-kernel form of the tile states)
+            tile_S = torch.empty(total_chunks, H, p.dv_p, p.dk_p, dtype=torch.bfloat16, device=dev)
+            if not L.load().pal_state_pass_applies(dims, 0):
+                scratch = torch.empty(total_chunks, H, p.dv_p, p.dk_p, dtype=torch.float32, device=dev)
         pt = cm._ptr
         tens = L.PalFwdTensors(q=pt(p.q), k=pt(p.k), v=pt(p.v), gt=pt(p.gt), g=pt(p.g), o=pt(o), init_mu=pt(p.init_mu),
                                final_mu=pt(final), cu_seqlens=pt(p.cu_seqlens), chunk_table=pt(table),

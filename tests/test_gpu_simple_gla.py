@@ -719,3 +719,75 @@ def test_shared_qk_heads_are_indexed_not_repeated(gpu_device, dk, dv, dtype):
                     err = hp.max_rel(pk[n].grad[:, a:b_], want)
                     assert err <= hp.BF16_GRAD_NORM_TOL, (n, a, err)
         assert hp.max_abs(o_p.float(), torch.cat(o_parts, dim=1)) <= out_tol
+
+
+@pytest.mark.parametrize("H,Hq,dk,dv,lens", [
+    (2, 2, 16, 16, [64, 64]),                     # one tile; least head dims
+    (2, 1, 48, 96, [1, 63, 0, 65, 130]),          # columns of the contraction that pad a step; shared q/k heads; no tokens
+    (3, 3, 80, 48, [127]),                        # slices with idle waves
+    (2, 2, 96, 192, [200, 70]),                   # one part / two parts of the contraction
+    (1, 1, 128, 128, [129]),
+    (1, 1, 160, 208, [66]),                       # widths beside the compiled ones
+    (2, 2, 256, 240, [100]),
+    (130, 65, 96, 192, [5, 80]),                  # six blocks of columns to a workgroup
+])
+def test_walks_against_closed_form(gpu_device, monkeypatch, H, Hq, dk, dv, lens):
+    """Every result in one walk over each sequence, whatever the rule says of these sizes: outputs, final state and all
+    gradients against the closed form, and the form with the tiles' states in memory at the same bars."""
+    from palimpsa_amd.ops import simple_gla as sg
+    N, T = len(lens), sum(lens)
+    gen = torch.Generator().manual_seed(H + dk + dv)
+    unit = lambda: torch.nn.functional.normalize(torch.randn(1, T, Hq, dk, generator=gen), dim=-1).bfloat16()  # noqa: E731
+    q, k, v = unit(), unit(), torch.randn(1, T, H, dv, generator=gen).bfloat16()
+    g = -torch.nn.functional.softplus(torch.randn(1, T, H, generator=gen)) * torch.linspace(0.05, 2.0, H)
+    S0 = torch.randn(N, H, dk, dv, generator=gen) * 0.2
+    do = torch.randn(1, T, H, dv, generator=gen).bfloat16()
+    ref = [x.double().requires_grad_(True) for x in (q, k, v, g, S0)]
+    o_ref, S_ref, t0 = [], [], 0
+    for n, t in enumerate(lens):
+        if t == 0:
+            S_ref.append(ref[4][n:n + 1])
+            continue
+        rows = [x[:, t0:t0 + t] for x in ref[:4]]
+        rep = [x.repeat_interleave(H // Hq, dim=2) for x in rows[:2]]
+        o, S = _closed_form(*rep, rows[2], rows[3], dk ** -0.5, ref[4][n:n + 1])
+        o_ref.append(o)
+        S_ref.append(S)
+        t0 += t
+    o_ref, S_ref = torch.cat(o_ref, 1), torch.cat(S_ref)
+    g_ref = torch.autograd.grad(o_ref, ref, do.double())
+    cu = torch.tensor([0] + [sum(lens[:n + 1]) for n in range(N)], dtype=torch.int32, device=gpu_device)
+    for walk in (True, False):
+        monkeypatch.setattr(sg, "_walks", lambda dims, longest: walk)
+        leaves = [x.to(gpu_device).requires_grad_(True) for x in (q, k, v, g, S0)]
+        o, S = sg.chunk_simple_gla(q=leaves[0], k=leaves[1], v=leaves[2], g=leaves[3], initial_state=leaves[4],
+                                   output_final_state=True, cu_seqlens=cu if N > 1 else None)
+        assert hp.max_abs(o.float(), o_ref) <= hp.BF16_OUT_ABS_TOL
+        assert hp.max_rel(S, S_ref) <= 1e-2
+        for name, x, r in zip("q k v g S0".split(), torch.autograd.grad(o, leaves, do.to(gpu_device)), g_ref):
+            assert hp.max_rel(x, r) <= hp.BF16_GRAD_NORM_TOL, (name, walk)
+
+
+def test_walk_rule_and_its_flag(gpu_device):
+    """Many heads walk, few do not, one long document among short ones does not; the flag is refused where it cannot be."""
+    from palimpsa_amd import _lib as L
+    lib = L.load()
+
+    def dims(B, T, H, dk, dv, chunks=None, n=None, flags=0, dtype=L.PAL_DTYPE_BF16):
+        return L.PalDims(batch=B, seq_len=T, n_seqs=n or B, n_heads=H, dk=dk, dv=dv, dtype=dtype, flags=flags, scale=1.0,
+                         total_chunks=chunks or B * ((T + 63) // 64))
+
+    assert lib.pal_gla_walk_applies(dims(8, 2048, 16, 96, 192), 2048) == 1
+    assert lib.pal_gla_walk_applies(dims(1, 2048, 16, 96, 192), 2048) == 0
+    assert lib.pal_gla_walk_applies(dims(8, 2048, 16, 96, 192, flags=L.PAL_FLAG_STATES_ONE_PASS), 2048) == 0
+    assert lib.pal_gla_walk_applies(dims(8, 2048, 16, 96, 192, dtype=L.PAL_DTYPE_F32), 2048) == 0
+    packed = dims(1, 32768, 8, 96, 96, chunks=600, n=200, flags=L.PAL_FLAG_VARLEN)
+    assert lib.pal_gla_walk_applies(packed, 512) == 1
+    assert lib.pal_gla_walk_applies(packed, 30000) == 0
+    x = torch.zeros(1 << 16, dtype=torch.bfloat16, device=gpu_device)
+    p = x.data_ptr()
+    tens = dict(q=p, k=p, v=p, gt=p, g=p, o=p)
+    fp32 = dims(1, 64, 1, 16, 16, flags=L.PAL_FLAG_GLA_NO_TILES, dtype=L.PAL_DTYPE_F32)
+    assert lib.pal_gla_chunk_fwd(fp32, L.PalFwdTensors(**tens), None) == L.PAL_E_STATE
+    with_tiles = L.PalFwdTensors(**tens, chunk_I=p)
+    assert lib.pal_gla_chunk_fwd(dims(1, 64, 1, 16, 16, flags=L.PAL_FLAG_GLA_NO_TILES), with_tiles, None) == L.PAL_E_STATE
