@@ -77,6 +77,10 @@ extern "C" {
  * backward is asked for with the flags of its call.  pal_gla_walk_applies tells when it is the faster way. */
 #define PAL_FLAG_GLA_NO_TILES 8192u
 
+/* pal_chunk_fwd only: the tile-start states are not needed after the call (no backward will follow): chunk_mu and chunk_I are
+ * scratch, their contents afterwards are undefined, and a short pass may be run without tiles. */
+#define PAL_FLAG_OUTPUTS_ONLY 16384u
+
 /* error codes (negative) */
 #define PAL_OK 0
 #define PAL_E_NULL -1        /* required pointer is NULL                      */

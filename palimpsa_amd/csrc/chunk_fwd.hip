@@ -14,6 +14,7 @@
 #include "chunk_common.h"
 #include "pal_host.h"
 #include "pal_profile.h"
+#include "recurrent.h"
 
 namespace pal {
 
@@ -476,6 +477,12 @@ extern "C" int pal_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void* str
   }
   int rc = check_chunk_common(d, t);
   if (rc) return rc;
+  constexpr uint32_t forms = PAL_FLAG_STATES_TWO_KERNELS | PAL_FLAG_STATES_ONE_PASS | PAL_FLAG_FP32_FAST;
+  if ((d->flags & PAL_FLAG_OUTPUTS_ONLY) && !(d->flags & forms) && short_pass(d)) {
+    PalDims r = *d;
+    r.flags &= PAL_FLAG_HAS_INIT | PAL_FLAG_STORE_FINAL | PAL_FLAG_HAS_VAR;
+    return pal_recurrent_fwd(&r, t, stream);
+  }
   ChunkArgs a;
   fill_chunk_args(a, d, t);
   hipStream_t s = (hipStream_t)stream;

@@ -332,7 +332,7 @@ py::object chunk_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Te
   }
   ChunkOut out;
   const Tensor none;
-  if (chunk_forward(c, q, k, v, b, gt, g, Ip, mu.value_or(none), I.value_or(none), var, flags, meta.value_or(none), cu.value_or(none),
+  if (chunk_forward(c, q, k, v, b, gt, g, Ip, mu.value_or(none), I.value_or(none), var, flags | PAL_FLAG_OUTPUTS_ONLY, meta.value_or(none), cu.value_or(none),
                     tiles, out))
     return py::none();
   return py::make_tuple(out.o, var ? py::cast(out.ov) : py::none(), out.fm, out.fI);

@@ -13,32 +13,12 @@
 // The sum over dk is a 4-step DPP rotation inside the row.  Memory access is
 // the only cost that matters at T == 1: every lane issues all its state loads
 // up front as 16-byte vectors that are contiguous across the row.
-//
-// A few waves on many tokens leave the chip idle and walk serially: there a workgroup of NW waves shares a sequence, a
-// segment of the tokens each.  M and J are affine in the state a segment starts from (S_end = F S_start + S_local), so
-// every wave first walks its segment from zero without outputs (no reciprocal, no q: half the instructions), leaves S_local
-// and F in LDS, folds the segments before its own in their order and walks again with outputs.  All in fp32, the fold is
-// one fma per entry and segment: errors against float64 as in one walk (1.4e-7 at 256 tokens, both).  B=2 T=256 H=4
-// 32x32 fp32: 41 -> 13.7 us.
 #include "pal_common.h"
 #include "pal_host.h"
 #include "pal_profile.h"
+#include "recurrent.h"
 
 namespace pal {
-
-struct RecArgs {
-  const void *q, *k, *v, *b, *gt;
-  const float *g, *Ip;
-  void *o, *o_var;
-  const float *init_mu, *init_I;
-  float *final_mu, *final_I;
-  const int32_t* cu_seqlens;
-  int32_t T, H, dk, dv, n_seqs;
-  int32_t Hq;   // heads of q and k (H, or a divisor of it: a group of H / Hq value heads shares one)
-  int32_t gate_bf16, var_bf16;
-  uint32_t flags;
-  float scale;
-};
 
 // n index of element e of lane j (j = lane % 16); VW-wide vectors interleaved across the row.
 // WIDE (the bf16 cache format of mu): 8-wide vectors where a lane has 8 entries, so that the bf16 state moves in
@@ -98,45 +78,17 @@ __device__ __forceinline__ void store_n_stream(T* p, const float* in) {
   }
 }
 
-// PF token rows in flight: token t lives in register set t mod PF; it is worked from there and the set requested again for
-// token t + PF (the walk of a segment without outputs).
-template <int NPL, int PF, typename Ask, typename Work>
-__device__ __forceinline__ void walk_tokens(int T, Ask&& ask, Work&& work) {
-  float kb[PF][NPL], vb[PF], bb[PF];
-  unsigned gb[PF];
-#pragma unroll
-  for (int u = 0; u < PF; ++u)
-    if (u < T) ask(kb[u], vb[u], bb[u], gb[u]);
-  int t0 = 0;
-  for (; t0 + 2 * PF <= T; t0 += PF) {
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      work(kb[u], vb[u], bb[u], gb[u]);
-      ask(kb[u], vb[u], bb[u], gb[u]);
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < 2 * PF; ++u) {
-    if (t0 + u < T) {
-      work(kb[u % PF], vb[u % PF], bb[u % PF], gb[u % PF]);
-      if (t0 + u + PF < T) ask(kb[u % PF], vb[u % PF], bb[u % PF], gb[u % PF]);
-    }
-  }
-}
-
 // PF = tokens whose rows are in flight.  PF = 1 (decode): the next token's rows are requested while the current one
 // is processed.  A long token-serial run is bound by the latency of those requests (0.3-0.6 us per token against
 // 0.1-0.2 us of arithmetic), so it keeps PF tokens in registers: a token is processed from its set and the set is
 // reloaded at once with the token PF ahead (always issued, clamped to the last token, so that the number of
 // requests in flight is the same in every iteration and the compiler can wait for exactly the oldest set).
-template <typename TIn, int NPL, int RD, bool MU16, int PF, bool HAS_VAR, int NW>
-__global__ __launch_bounds__(64 * NW) void recurrent_fwd_kernel(RecArgs a) {
-  static_assert(NW == 1 || (RD == 1 && !MU16), "runs in segments: one value row per lane, fp32 states");
+template <typename TIn, int NPL, int RD, bool MU16, int PF, bool HAS_VAR>
+__global__ __launch_bounds__(64) void recurrent_fwd_kernel(RecArgs a) {
   using Map = NMap<NPL, MU16>;
   constexpr int VW = Map::VW;
   constexpr int NV = Map::NV;
-  const int lane = threadIdx.x & 63;
-  const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x;
   const int j = lane & 15;
   const int grp = lane >> 4;
   const int n_dtiles = a.dv / (4 * RD);
@@ -156,11 +108,6 @@ __global__ __launch_bounds__(64 * NW) void recurrent_fwd_kernel(RecArgs a) {
     bos = (int64_t)n * a.T;
     T = a.T;
   }
-  if constexpr (NW > 1) {   // this wave's segment of the sequence (may be empty at the end)
-    const int len = (T + NW - 1) / NW, first = min(w * len, T);
-    bos += first;
-    T = min(len, T - first);
-  }
   const float gh = a.g[h] * kLog2e;
   const float Ip = a.Ip[h];
   const float scale = a.scale;
@@ -171,7 +118,7 @@ __global__ __launch_bounds__(64 * NW) void recurrent_fwd_kernel(RecArgs a) {
   for (int rr = 0; rr < RD; ++rr) drow[rr] = tile * (4 * RD) + rr * 4 + grp;
 
   float M[RD][NPL], J[RD][NPL];
-  if (a.init_mu && w == 0) {
+  if (a.init_mu) {
 #pragma unroll
     for (int rr = 0; rr < RD; ++rr) {
       const int64_t base = ((int64_t)nh * dv + drow[rr]) * dk;
@@ -260,64 +207,6 @@ __global__ __launch_bounds__(64 * NW) void recurrent_fwd_kernel(RecArgs a) {
     var_i += step_v;
   };
 
-  if constexpr (NW > 1) {
-    // First walk: what the segment leaves of its own tokens (the first segment: of the initial state too) and the decay
-    // over it; then every wave folds the segments before its own into the state its outputs start from.
-    extern __shared__ float smem[];
-    float M0[NPL], J0[NPL];
-    if (w == 0) {
-#pragma unroll
-      for (int e = 0; e < NPL; ++e) { M0[e] = M[0][e]; J0[e] = J[0][e]; }
-    }
-    constexpr int kSlot = (2 * NPL + 1) * 64;   // [M, J of a lane, decay][lane]
-    if (w < NW - 1) {
-      const TIn *kq = kp, *vq = vp, *bq = bp;
-      int64_t gq = gt_i, gu = gt_i;
-      float F = 1.f;
-      auto ask = [&](float* kk_, float& vv_, float& bb_, unsigned& gt_) {
-#pragma unroll
-        for (int iv = 0; iv < NV; ++iv) load_n<VW>(at(kq, lane_k[iv]), kk_ + iv * VW);
-        vv_ = to_f32(*at(vq, lane_v[0]));
-        bb_ = to_f32(*at(bq, lane_v[0]));
-        gt_ = load_gate_word(a.gt, gq, a.gate_bf16);
-        kq += step_k; vq += step_v; bq += step_v; gq += H;
-      };
-      auto advance = [&](const float* kc, float vc, float bc, unsigned word) {
-        const float f = fast_exp2(-gate_value(word, gu, a.gate_bf16) * gh);
-        gu += H;
-        F *= f;
-#pragma unroll
-        for (int e = 0; e < NPL; ++e) {
-          M[0][e] = fmaf(f, M[0][e], vc * kc[e]);
-          J[0][e] = fmaf(f, J[0][e], bc * (kc[e] * kc[e]));
-        }
-      };
-      walk_tokens<NPL, PF>(T, ask, advance);
-      float* slot = smem + w * kSlot + lane;
-#pragma unroll
-      for (int e = 0; e < NPL; ++e) { slot[64 * e] = M[0][e]; slot[64 * (NPL + e)] = J[0][e]; }
-      // (a decay beyond the range of fp32 must not turn entries that are zero into NaN)
-      slot[64 * 2 * NPL] = fminf(F, 3.4028235e38f);
-    }
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-      for (int e = 0; e < NPL; ++e) { M[0][e] = M0[e]; J[0][e] = J0[e]; }
-    } else {
-#pragma unroll
-      for (int e = 0; e < NPL; ++e) { M[0][e] = smem[64 * e + lane]; J[0][e] = smem[64 * (NPL + e) + lane]; }
-      for (int u = 1; u < w; ++u) {
-        const float* slot = smem + u * kSlot + lane;
-        const float F = slot[64 * 2 * NPL];
-#pragma unroll
-        for (int e = 0; e < NPL; ++e) {
-          M[0][e] = fmaf(F, M[0][e], slot[64 * e]);
-          J[0][e] = fmaf(F, J[0][e], slot[64 * (NPL + e)]);
-        }
-      }
-    }
-  }
-
   if constexpr (PF == 1) {
     float kc[NPL], qc[NPL], vc[RD], bc[RD];
     unsigned gtc = 0;
@@ -363,7 +252,7 @@ __global__ __launch_bounds__(64 * NW) void recurrent_fwd_kernel(RecArgs a) {
     }
   }
 
-  if (a.final_mu && w == NW - 1) {
+  if (a.final_mu) {
 #pragma unroll
     for (int rr = 0; rr < RD; ++rr) {
       const int64_t base = ((int64_t)nh * dv + drow[rr]) * dk;
@@ -384,80 +273,46 @@ __global__ __launch_bounds__(64 * NW) void recurrent_fwd_kernel(RecArgs a) {
 }
 
 template <typename TIn, int NPL>
-static int launch_npl(const RecArgs& a, int rd, int nw, hipStream_t s) {
+static int launch_npl(const RecArgs& a, int rd, hipStream_t s) {
   const int64_t blocks = (int64_t)a.n_seqs * a.H * (a.dv / (4 * rd));
   if (blocks > 0x7fffffff) return PAL_E_DIM;
   // tokens in flight of a long run: as many as the registers of a wave take without cutting the occupancy it needs
   constexpr int PFL = NPL <= 4 ? 4 : (NPL <= 8 ? 3 : 2);
   const bool serial = a.T > 4;
   const bool var = a.flags & PAL_FLAG_HAS_VAR;
-#define PAL_REC_LAUNCH_VAR(RD_, MU_, PF_, VAR_, NW_)                                                                      \
+#define PAL_REC_LAUNCH(RD_, MU_, PF_)                                                                                     \
   do {                                                                                                                   \
-    constexpr size_t lds = NW_ > 1 ? (NW_ - 1) * (2 * NPL + 1) * 64 * sizeof(float) : 0;                                  \
-    static_assert(lds <= 64 * 1024, "no raised limit of dynamic LDS");                                                   \
-    PAL_TIMED_LAUNCH(kKernRecurrentFwd, s, (recurrent_fwd_kernel<TIn, NPL, RD_, MU_, PF_, VAR_, NW_>), dim3((unsigned)blocks), dim3(64 * NW_), lds, s, a); \
-  } while (0)
-#define PAL_REC_LAUNCH(RD_, MU_, PF_, NW_)                    \
-  do {                                                       \
-    if (var) PAL_REC_LAUNCH_VAR(RD_, MU_, PF_, true, NW_);   \
-    else PAL_REC_LAUNCH_VAR(RD_, MU_, PF_, false, NW_);      \
+    if (var) PAL_TIMED_LAUNCH(kKernRecurrentFwd, s, (recurrent_fwd_kernel<TIn, NPL, RD_, MU_, PF_, true>), dim3((unsigned)blocks), dim3(64), 0, s, a); \
+    else PAL_TIMED_LAUNCH(kKernRecurrentFwd, s, (recurrent_fwd_kernel<TIn, NPL, RD_, MU_, PF_, false>), dim3((unsigned)blocks), dim3(64), 0, s, a); \
   } while (0)
   if (a.flags & PAL_FLAG_STATE_MU_BF16) {
     // the bf16 cache format of mu is a decode format: the small-wave mapping only
-    PAL_REC_LAUNCH(1, true, 1, 1);
+    PAL_REC_LAUNCH(1, true, 1);
   } else if (rd == 4) {
-    PAL_REC_LAUNCH(4, false, PFL, 1);
-  } else if (nw == 4) {
-    PAL_REC_LAUNCH(1, false, PFL, 4);
-  } else if (nw == 8) {
-    PAL_REC_LAUNCH(1, false, PFL, 8);
-  } else if (nw == 16) {
-    if constexpr (NPL <= 8) PAL_REC_LAUNCH(1, false, PFL, 16);
-    else return PAL_E_HEADDIM;   // (segments() asks for 16 up to 128 key columns)
+    PAL_REC_LAUNCH(4, false, PFL);
   } else if (serial) {
-    PAL_REC_LAUNCH(1, false, PFL, 1);
+    PAL_REC_LAUNCH(1, false, PFL);
   } else {
-    PAL_REC_LAUNCH(1, false, 1, 1);
+    PAL_REC_LAUNCH(1, false, 1);
   }
 #undef PAL_REC_LAUNCH
-#undef PAL_REC_LAUNCH_VAR
   PAL_HIP_LAUNCH_CHECK();
   return PAL_OK;
 }
 
 template <typename TIn>
-static int launch_dtype(const RecArgs& a, int rd, int nw, hipStream_t s) {
+static int launch_dtype(const RecArgs& a, int rd, hipStream_t s) {
   switch (a.dk / 16) {
-    case 1: return launch_npl<TIn, 1>(a, rd, nw, s);
-    case 2: return launch_npl<TIn, 2>(a, rd, nw, s);
-    case 3: return launch_npl<TIn, 3>(a, rd, nw, s);
-    case 4: return launch_npl<TIn, 4>(a, rd, nw, s);
-    case 6: return launch_npl<TIn, 6>(a, rd, nw, s);
-    case 8: return launch_npl<TIn, 8>(a, rd, nw, s);
-    case 12: return launch_npl<TIn, 12>(a, rd, nw, s);
-    case 16: return launch_npl<TIn, 16>(a, rd, nw, s);
+    case 1: return launch_npl<TIn, 1>(a, rd, s);
+    case 2: return launch_npl<TIn, 2>(a, rd, s);
+    case 3: return launch_npl<TIn, 3>(a, rd, s);
+    case 4: return launch_npl<TIn, 4>(a, rd, s);
+    case 6: return launch_npl<TIn, 6>(a, rd, s);
+    case 8: return launch_npl<TIn, 8>(a, rd, s);
+    case 12: return launch_npl<TIn, 12>(a, rd, s);
+    case 16: return launch_npl<TIn, 16>(a, rd, s);
     default: return PAL_E_HEADDIM;
   }
-}
-
-// Segments per sequence (waves per workgroup).  One wave walks its tokens one after the other, 0.16 us each (dk = 32 to 64)
-// however empty the chip is; in segments it walks a part of them, twice, the first time without outputs (about half the
-// work), so the segments pay while the chip has room: up to four waves per SIMD, and six for sequences of 64 tokens or more,
-// whose walks outweigh the fold.  Measured, one wave against 4 / 8 / 16 (us a call; below 7 the host is the limit):
-//   64 waves  (B=2 H=4 32x32 fp32)      T=16   7.1:  6.7  7.0  6.6    T=256   41.1:  20.5  15.1  13.7
-//   192 waves (B=1 H=16 48x48)          T=16   7.7:  6.9  6.6  6.9    T=777  179  :  85.7  52.1  41.0
-//   512 waves (B=1 H=16 128x128)        T=32  14.0: 10.0  9.6 15.2    T=512  178  :  94.0  76.9  85.8
-//   768 waves (B=4 H=16 48x48)          T=32  11.1:  9.6 11.0 16.9    T=512  123  :  81.0  74.3  82.3
-//   1536 waves (B=2 H=16 96x192)        T=32  17.1: 18.0 20.8 35.8    T=256  108  :  92.0  95.0 120
-//   2048 waves (B=8 H=16 64x64)         T=32  14.6: 19.3 24.3 42.7    T=512  165  : 173   183   226
-// (from 192 key columns on, eight at most: a lane's registers allow two waves per SIMD).
-static int segments(const PalDims* d) {
-  const int64_t waves = (int64_t)d->n_seqs * d->n_heads * (d->dv / 4);
-  const int64_t len = (d->flags & PAL_FLAG_VARLEN) ? d->seq_len / d->n_seqs : d->seq_len;   // the mean of a packed batch
-  if (len >= 32 && waves <= 256 && d->dk <= 128) return 16;
-  if (len >= 16 && waves <= 512) return 8;
-  if (len >= 8 && waves <= (len >= 64 ? 1536 : 1024)) return 4;
-  return 1;
 }
 
 bool recurrent_dk_supported(int dk) {
@@ -494,8 +349,9 @@ extern "C" int pal_recurrent_fwd(const PalDims* d, const PalFwdTensors* t, void*
   const int64_t waves16 = (int64_t)d->n_seqs * d->n_heads * (d->dv / 16);
   // decode (a handful of tokens) is pure state streaming: many small waves keep more loads in flight
   const int rd = (d->seq_len > 4 && waves16 >= 2048 && !(d->flags & PAL_FLAG_STATE_MU_BF16)) ? 4 : 1;
-  const int nw = (d->flags & PAL_FLAG_STATE_MU_BF16) ? 1 : segments(d);
   hipStream_t s = (hipStream_t)stream;
-  if (d->dtype == PAL_DTYPE_BF16) return launch_dtype<bf16_t>(a, rd, nw, s);
-  return launch_dtype<float>(a, rd, nw, s);
+  if (!(d->flags & PAL_FLAG_STATE_MU_BF16))
+    if (const int nw = recurrent_segments(d); nw > 1) return launch_recurrent_seg(a, d->dtype, nw, s);
+  if (d->dtype == PAL_DTYPE_BF16) return launch_dtype<bf16_t>(a, rd, s);
+  return launch_dtype<float>(a, rd, s);
 }

@@ -47,9 +47,11 @@ if _HAS_CUSTOM_OP:
                   ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """-> (o, o_var | empty, final_mu, final_I, tile_mu, tile_I).  ``mode_flags``: the knob bits of PalDims.flags
         (L.state_pass_flags() when the call was traced); the backward op gets the same value, so a knob changed
-        between the two cannot mix operand modes.  The tile-start states of every tile are always kept (this op does
+        between the two cannot mix operand modes.  The tile-start states of every tile are returned (this op does
         not know whether a backward follows): a long prefill without gradients under a tracer needs
-        total_chunks * H * dv * dk * 8 bytes where the eager entry point runs in windows of 512 MB."""
+        total_chunks * H * dv * dk * 8 bytes where the eager entry point runs in windows of 512 MB.  With
+        PAL_FLAG_OUTPUTS_ONLY among the mode flags (no gradient was wanted when the call was traced) they may be left
+        unfilled; the backward then fills states of its own."""
         p = cm.prepare_inputs(q, k, v, b, gt, g, Ip, init_mu, init_I, cu_seqlens, recurrent=False)
         dev = p.q.device
         B, T, H, _ = p.v.shape
@@ -132,6 +134,15 @@ if _HAS_CUSTOM_OP:
         dIp = torch.empty(H, dtype=torch.float32, device=dev)
         d_mu = torch.empty_like(p.init_mu) if p.init_mu is not None else None
         d_I = torch.empty_like(p.init_I) if p.init_I is not None else None
+        outputs_only, mode_flags = mode_flags & L.PAL_FLAG_OUTPUTS_ONLY, mode_flags & ~L.PAL_FLAG_OUTPUTS_ONLY
+        if outputs_only:
+            # traced without gradients and run with them: the forward may have left the tile-start states out
+            tile_mu, tile_I = torch.empty_like(tile_mu), torch.empty_like(tile_I)
+            dims = cm.make_dims(p, scale, (flags & ~L.PAL_FLAG_HAS_VAR) | L.PAL_FLAG_STATES_ONLY, total_chunks, var_dtype=cd,
+                                mode_flags=mode_flags)
+            tens = cm.make_fwd_tensors(p, do_p, None, None, None, table, offsets, tile_mu, tile_I)
+            with torch.cuda.device(dev):
+                L.check(L.load().pal_chunk_fwd(dims, tens, cm.current_stream_ptr(dev)), "pal_chunk_fwd")
         dims = cm.make_dims(p, scale, flags, total_chunks, var_dtype=cd, mode_flags=mode_flags)
         tens = cm.make_fwd_tensors(p, do_p, None, None, None, table, offsets, tile_mu, tile_I)
         pt = cm._ptr

@@ -137,7 +137,8 @@ class ChunkPalimpsa(torch.autograd.Function):
             flags |= L.PAL_FLAG_HAS_INIT
         if output_uncertainty:
             flags |= L.PAL_FLAG_HAS_VAR
-        dims = cm.make_dims(p, scale, flags, total_chunks, var_dtype=p.compute_dtype)
+        outputs_only = 0 if any(ctx.needs_input_grad[:9]) else L.PAL_FLAG_OUTPUTS_ONLY
+        dims = cm.make_dims(p, scale, flags | outputs_only, total_chunks, var_dtype=p.compute_dtype)
         tens = cm.make_fwd_tensors(p, o, o_var, final_mu, final_I, table, offsets, int_mu, int_I)
         with torch.cuda.device(dev):
             rc = L.load().pal_chunk_fwd(dims, tens, cm.current_stream_ptr(dev))
@@ -268,6 +269,8 @@ def chunk_palimpsa(q, k, v, b, gt, g, Ip, initial_mu_state=None, initial_I_state
                                      L.PAL_DTYPE_BF16 if rows_bf16 else L.PAL_DTYPE_F32, mode_flags)
             if rc != 0:
                 raise ValueError(f"chunk_palimpsa (backward head dims): unsupported by pal_chunk_bwd (code {rc})")
+        else:
+            mode_flags |= L.PAL_FLAG_OUTPUTS_ONLY
         o, o_var, final_mu_state, final_I_state, _, _ = _ops.chunk_fwd(
             q, k, v, b, gt, g, Ip, initial_mu_state, initial_I_state, float(scale), bool(output_uncertainty), cu_seqlens,
             mode_flags)

@@ -243,3 +243,20 @@ def test_activation_checkpointing(gpu_device, reentrant):
     with torch.inference_mode():
         from palimpsa_amd import _lib as L
         assert L.host().chunk_fwd(*[t.detach() for t in x], None, None, 1.0, False, 0, None, None, 1 << 30) is not None
+
+
+@pytest.mark.filterwarnings("ignore")
+def test_call_traced_without_gradients_differentiates(gpu_device):
+    """A short pass traced without gradients keeps no tile states; run with gradients, its backward fills them."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    x = _plain_call(gpu_device)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda *a: chunk_palimpsa(*a), tuple(x), check_trace=False)
+    grads = []
+    for f in (traced, chunk_palimpsa):
+        leaves = [t.detach().clone().requires_grad_(True) for t in x]
+        junk = torch.full((1 << 16,), 1e6, device=gpu_device)   # what unfilled states would be likely to hold
+        del junk
+        grads.append(torch.autograd.grad(f(*leaves).float().square().sum(), leaves))
+    for a, r in zip(*grads):
+        assert (a.float() - r.float()).abs().max() <= 5e-2 * r.float().abs().max()

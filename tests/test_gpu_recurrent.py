@@ -414,9 +414,10 @@ def test_decode_with_the_mean_state_kept_in_bf16(gpu_device):
 
 
 @pytest.mark.parametrize("H,dk,dv,lens", [
-    (3, 48, 48, [8]), (3, 32, 32, [15]), (2, 64, 80, [16]), (2, 16, 16, [31]), (2, 32, 48, [32]), (1, 128, 64, [33]),   # 4, 8, 16 waves
-    (2, 256, 64, [49]), (2, 192, 16, [100]),                    # wide keys: 8 at most
-    (8, 96, 192, [64, 65, 70, 64]), (16, 64, 64, [8, 9]),       # more value rows: 4
+    (3, 48, 48, [8]), (3, 32, 32, [33]), (2, 16, 16, [63]), (1, 64, 80, [15]),      # 4 waves
+    (2, 64, 80, [64]), (2, 32, 48, [191]), (2, 256, 64, [65]), (2, 192, 16, [200]),   # 8: at most for wide keys
+    (1, 128, 64, [192]), (2, 96, 96, [257]), (1, 16, 16, [255]),                      # 16
+    (8, 96, 192, [48, 48, 48, 48]), (16, 64, 64, [64, 65]),                           # 4 for more value rows
     (2, 32, 32, [1, 90, 0, 5, 64]),                             # documents shorter than their segments, and an empty one
 ])
 def test_sequences_in_segments(gpu_device, H, dk, dv, lens):
@@ -447,3 +448,35 @@ def test_sequences_in_segments(gpu_device, H, dk, dv, lens):
         step.bind(*rows, mu0, I0)
         assert hp.max_rel(step.step(), o_ref) <= 1e-5
         assert hp.max_rel(mu0, mu_ref) <= 1e-5 and hp.max_rel(I0, I_ref) <= 1e-5
+
+
+@pytest.mark.parametrize("rows", ["fp32", "bf16"])
+@pytest.mark.parametrize("B,T,H,dk,dv,Hq", [(1, 1, 2, 48, 48, 2), (2, 70, 4, 32, 64, 2), (1, 257, 3, 64, 48, 3), (1, 777, 4, 48, 48, 4)])
+def test_short_chunked_passes_without_tiles(gpu_device, rows, B, T, H, dk, dv, Hq):
+    """chunk_palimpsa without autograd on few tokens runs the token-serial kernels: outputs, uncertainty in the dtype of the rows and
+    final states against the oracle, and with autograd (tiles) at the same bars."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    dt = torch.float32 if rows == "fp32" else torch.bfloat16
+    inp = hp.rounded(po.make_inputs(B, T, H, dk, dv, seed=T), dt)
+    inp["q"], inp["k"] = inp["q"][:, :, :Hq].contiguous(), inp["k"][:, :, :Hq].contiguous()
+    inp["g"] = torch.linspace(0.05, 3.0, H)
+    gen = torch.Generator().manual_seed(T)
+    mu0 = 0.1 * torch.randn(B, H, dv, dk, generator=gen)
+    I0 = inp["Ip"].view(1, H, 1, 1) + torch.nn.functional.softplus(torch.randn(B, H, dv, dk, generator=gen))
+    rep = dict(inp, q=inp["q"].repeat_interleave(H // Hq, 2), k=inp["k"].repeat_interleave(H // Hq, 2))
+    ref = hp.oracle_forward(rep, mu0=mu0, I0=I0, want_var=True, dtype=torch.float64)
+    d = hp.to_device(inp, gpu_device)
+    args = [d[n] for n in ("q", "k", "v", "b", "gt", "g", "Ip")]
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            args[0] = args[0].detach().requires_grad_(grad)
+            (o, ov), mu, I = chunk_palimpsa(*args, mu0.to(gpu_device), I0.to(gpu_device), output_final_state=True,
+                                            output_uncertainty=True)
+        assert o.dtype == ov.dtype == dt and mu.dtype == I.dtype == torch.float32
+        for x, r in ((o, ref[0]), (ov, ref[1])):
+            if rows == "fp32":
+                assert hp.max_rel(x, r) <= hp.CHUNK_FP32_OUT_TOL
+            else:
+                assert hp.max_abs(x.float(), r) <= hp.BF16_OUT_ABS_TOL
+        for x, r in ((mu, ref[2]), (I, ref[3])):
+            assert hp.max_rel(x, r) <= (1e-5 if not grad else hp.CHUNK_FP32_OUT_TOL if rows == "fp32" else 1e-2)
