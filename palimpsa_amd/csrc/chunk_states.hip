@@ -9,10 +9,19 @@
 // the last tile at the end (:214-218).
 //
 // One workgroup of 12 waves per (sequence, head, slice of ds value rows): four hold the state (the slice times
-// dk is at most 6144 entries = 24 blocks of 16x16, up to six per wave), two groups of four stage the rows for them.  The rows of a tile are staged transposed in LDS
-// (token index fastest, two tokens per 32-bit word) as in chunk_delta_kernel.  The serial chain over the tiles
-// is hidden by fetching ahead: rows are fetched into registers three steps before they go to LDS, two LDS
-// buffers hold the current and the next tile, one barrier per tile.
+// dk is at most 6144 entries = 24 blocks of 16x16, up to six per wave), two groups of four stage the rows for them.  The
+// rows of a tile lie in LDS as they lie in memory, v and b times the weight of their token, 16 bytes a write; the matrix
+// cores take the tokens as contraction index, which the transposing LDS reads turn to the front (four bf16 of a column from
+// four rows at once).  The row stride is an odd number of 32-byte pieces, so neither side conflicts.  (Staged transposed, two
+// tokens to a word, the 4-byte writes and their packing were what the feeding waves spent their time on: whole passes over 4 x 2048
+// tokens, 6 heads of 96 x 192 with the precision state 74.6 us against 54.2, 4 x 1000, 12 of 192 x 64 51.4 against 27.3,
+// 8 x 2048, 16 of 48 x 48 52.8 against 47.4; scalar-gated 2 x 2048, 16 of 128 x 128 46 against 24.)
+// The serial chain over the tiles is hidden by fetching ahead: rows are fetched into registers three steps before they
+// go to LDS, two LDS buffers hold the current and the next tile, one barrier per tile.
+// What bounds it with the precision state: writing mu and I (8 bytes an entry) beside reading rows that come from HBM, at
+// 2.5 - 3.3 TB/s together; without the stores the walk takes half the time, and neither fetching further ahead (up to 10
+// tiles), whole 128-byte lines a store nor non-temporal stores gave more than 6 % at any shape without losing as much at
+// another.
 // The same kernel walks a sequence backwards for the gradient of the scalar-gated path (weights from the
 // start of the tile, G_{c-1} = F_c G_c + D_c, the value left after the first tile is the gradient of the
 // initial state).
@@ -26,8 +35,10 @@ namespace pal {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kStTS = 72;          // tokens (bf16) per staged row: 64 + 8 keeps 16-byte reads conflict-free
 constexpr int kStMaxBlocks = 6;    // 16x16 state blocks per wave
+// row stride (bf16) of a staged tile of n columns: an odd number of 32-byte pieces, so that the four rows by 32 bytes of a
+// transposing read lie on different banks in every lane group
+__host__ __device__ constexpr int staged_stride(int n) { return 16 * ((n >> 4) | 1); }
 
 struct StatePassArgs {
   ChunkArgs c;
@@ -41,20 +52,24 @@ struct StatePassArgs {
   float fin_scale;
 };
 
-template <int NIK>
+template <int NIK, int NIV>
 struct StageRegs {
-  u32x4 k[NIK][2];
-  u32x4 v[2], b[2];
+  u32x4 k[NIK], v[NIV];
   uint32_t gt;   // gate of token `lane` as loaded: fp32 bits or a bf16 in the low half (last wave)
 };
 
-template <bool HAS_J, int NIK>
+// NIK: 16-byte pieces of k per feeding thread and tile (32 columns each); DSB: 16 value rows each of the slice
+template <bool HAS_J, int NIK, int DSB>
 __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
+  constexpr int NIV = HAS_J ? DSB : (DSB + 1) / 2;       // pieces of v and b per feeding thread
+  constexpr int NSB = (DSB * NIK + 1) / 2;               // state blocks per wave
+  static_assert(NSB <= kStMaxBlocks, "state blocks of a wave");
   const ChunkArgs& a = A.c;
   extern __shared__ float smem[];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int H = a.H, dk = a.dk, dv = a.dv, ds = A.ds, dks = A.dks;
+  const int H = a.H, dk = a.dk, dv = a.dv, dks = A.dks;
+  constexpr int ds = 16 * DSB;
   // A workgroup owns the state entries (value rows [d0, d0 + ds)) x (key columns [k0, k0 + dks)) of a (sequence, head).
   int n, h, sl;
   if (!walk_item(a, A.plan, lane, n, h, sl)) return;
@@ -66,11 +81,13 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
 
   float* sA = smem;                                   // [3][64] weight of token s in its tile (ring over tiles)
   float* sF = sA + 3 * kC;                            // [3] decay over the whole tile (+1 pad)
-  uint32_t* sKT = (uint32_t*)(sF + 4);                // [2][dks][36] words = [dks][72] bf16
-  uint32_t* sVT = sKT + 2 * dks * (kStTS / 2);        // [2][ds][36]
-  uint32_t* sBT = sVT + 2 * ds * (kStTS / 2);         // [2][ds][36] (HAS_J)
-  const int kbuf = dks * (kStTS / 2), vbuf = ds * (kStTS / 2);
-
+  const int KS = staged_stride(dks);
+  constexpr int VS = staged_stride(ds);
+  bf16_t* sK = (bf16_t*)(sF + 4);                     // [2][64 tokens][KS]
+  bf16_t* sV = sK + 2 * kC * KS;                      // [2][64][VS]: v times the weight of its token
+  bf16_t* sB = sV + 2 * kC * VS;                      // [2][64][VS] (HAS_J)
+  const int kbuf = kC * KS;
+  constexpr int vbuf = kC * VS;
 
   // Waves 0-3 own the state (a 16x16 block per wave and slot), waves 4-11 feed them: a single wave issues an
   // instruction every five to eight cycles, so the kinds of work sit on different waves of each SIMD instead
@@ -80,37 +97,30 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
   // All roles pass the same barriers, one per step; steps -2 and -1 fill the pipeline.
   if (w >= 4) {
     // ---------------------------------------------------------------- staging role
-    // Items of a thread: (token pair, 8 columns).  The key and the value items start at thread 0 of the group,
-    // the items of b follow those of v (wrapping around), and the last wave turns the gates of a tile into its
-    // weights (in the step in which the group stages nothing).  Byte offsets of the two tokens from the first row of a tile and word offsets in the
-    // staging tiles do not change from tile to tile.
+    // Items of a thread: (token, 8 columns), of k, and of v followed by b (which of the two is the same for all of a wave);
+    // the last wave turns the gates of a tile into its weights (in the step in which the group stages nothing).  Byte
+    // offsets from the first row of a tile and places in the staging tiles do not change from tile to tile.
     const int grp = (w - 4) >> 2;           // parity of the tiles this group stages
     const int wg = (w - 4) & 3;             // wave in the group
     const int st = tid - 256 - 256 * grp;
-    const int gk = dks >> 3, gv = ds >> 3;
-    int ksp[NIK];
-    uint32_t koff[NIK][2], kdst[NIK];
-    bool kval[NIK];
+    uint32_t koff[NIK], voff[NIV];
+    int kdst[NIK], vdst[NIV], vtok[NIV];
+    bool kval[NIK], vval[NIV];
 #pragma unroll
     for (int j = 0; j < NIK; ++j) {
-      const int idx = st + 256 * j;
-      kval[j] = idx < 32 * gk;
-      ksp[j] = idx / gk;
-      const int c8 = idx - ksp[j] * gk;
-      koff[j][0] = kval[j] ? (uint32_t)(((2 * ksp[j]) * a.Hq * dk + k0 + 8 * c8) * 2) : 0x80000000u;
-      koff[j][1] = kval[j] ? (uint32_t)(((2 * ksp[j] + 1) * a.Hq * dk + k0 + 8 * c8) * 2) : 0x80000000u;
-      kdst[j] = (uint32_t)(8 * c8 * (kStTS / 2) + ksp[j]);
+      const int per = dks >> 3, idx = st + 256 * j, s = idx / per, c8 = idx - s * per;
+      kval[j] = s < kC;
+      koff[j] = kval[j] ? (uint32_t)((s * a.Hq * dk + k0 + 8 * c8) * 2) : 0x80000000u;
+      kdst[j] = s * KS + 8 * c8;
     }
-    const int vtid = st, btid = (st + 256 - 32 * gv) & 255;
-    const bool vval = vtid < 32 * gv, bval = HAS_J && btid < 32 * gv;
-    const int vsp = vtid / gv, vc8 = vtid - vsp * gv, bsp = btid / gv, bc8 = btid - bsp * gv;
-    uint32_t voff[2], boff[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      voff[u] = vval ? (uint32_t)(((2 * vsp + u) * H * dv + 8 * vc8) * 2) : 0x80000000u;
-      boff[u] = bval ? (uint32_t)(((2 * bsp + u) * H * dv + 8 * bc8) * 2) : 0x80000000u;
+    for (int j = 0; j < NIV; ++j) {
+      const int idx = st + 256 * j, it = idx % (128 * DSB), s = it / (2 * DSB), c8 = it % (2 * DSB);
+      vval[j] = idx < (HAS_J ? 2 : 1) * 128 * DSB;
+      voff[j] = vval[j] ? (uint32_t)((s * H * dv + 8 * c8) * 2) : 0x80000000u;
+      vdst[j] = s * VS + 8 * c8;
+      vtok[j] = s;
     }
-    const uint32_t vdst = (uint32_t)(8 * vc8 * (kStTS / 2) + vsp), bdst = (uint32_t)(8 * bc8 * (kStTS / 2) + bsp);
     // Rows are fetched through buffer descriptors that end with the last row of the sequence: the byte offset
     // of a row piece is a per-thread constant plus the offset of the tile, rows beyond the end of the sequence
     // (the tail of its last tile, tiles past its end) are out of range and read as zero, so no fetch needs a
@@ -132,21 +142,18 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     const float gh = a.g[h] * kLog2e;
     const bool from_start = (a.flags & kFlagDecayFromStart) != 0;
 
-    auto load_stage = [&](StageRegs<NIK>& R, int p) {
+    auto load_stage = [&](StageRegs<NIK, NIV>& R, int p) {
       const int c = A.reverse ? nchunks - 1 - p : p;
       const bool live = p < nchunks;
       // a tile past the end: every offset out of range
       const uint32_t tk = live ? (uint32_t)(c * kC * a.Hq * dk * 2) : 0x80000000u;
       const uint32_t tv = live ? (uint32_t)(c * kC * H * dv * 2) : 0x80000000u;
 #pragma unroll
-      for (int j = 0; j < NIK; ++j) {
-        R.k[j][0] = __builtin_amdgcn_raw_buffer_load_b128(krs, koff[j][0] + tk, 0, 0);
-        R.k[j][1] = __builtin_amdgcn_raw_buffer_load_b128(krs, koff[j][1] + tk, 0, 0);
-      }
+      for (int j = 0; j < NIK; ++j) R.k[j] = __builtin_amdgcn_raw_buffer_load_b128(krs, koff[j] + tk, 0, 0);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        R.v[u] = __builtin_amdgcn_raw_buffer_load_b128(vrs, voff[u] + tv, 0, 0);
-        if (HAS_J) R.b[u] = __builtin_amdgcn_raw_buffer_load_b128(brs, boff[u] + tv, 0, 0);
+      for (int j = 0; j < NIV; ++j) {
+        const bool is_b = HAS_J && 64 * wg + 256 * j >= 128 * DSB;
+        R.v[j] = __builtin_amdgcn_raw_buffer_load_b128(is_b ? brs : vrs, voff[j] + tv, 0, 0);
       }
       if (wg == 3) {
         const uint32_t tg = live ? (uint32_t)(c * kC * H * esz) : 0x80000000u;
@@ -154,36 +161,30 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
                            : __builtin_amdgcn_raw_buffer_load_b32(grs, goff + tg, 0, 0);   // raw; widened below
       }
     };
-    // eight columns of two tokens -> one word (token pair) per column
-    auto put = [&](uint32_t* dst, const u32x4& x0, const u32x4& x1) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-        dst[e * (kStTS / 2)] = __builtin_amdgcn_perm(x1[e >> 1], x0[e >> 1], sel);
-      }
-    };
-    // the same for rows of v and b, which are staged times the weight of their token (the operand the matrix
-    // cores take is a_s v_s, rounded to bf16 once)
-    auto put_weighted = [&](uint32_t* dst, const u32x4& x0, const u32x4& x1, int sp, const float* wts) {
-      const f32x2 a2 = *(const f32x2*)&wts[2 * sp];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t w0 = x0[e >> 1], w1 = x1[e >> 1];
-        const float f0 = __builtin_bit_cast(float, (e & 1) ? (w0 & 0xffff0000u) : (w0 << 16));
-        const float f1 = __builtin_bit_cast(float, (e & 1) ? (w1 & 0xffff0000u) : (w1 << 16));
-        *(bf16x2*)&dst[e * (kStTS / 2)] = pack2(f0 * a2[0], f1 * a2[1]);
-      }
-    };
-    auto store_stage = [&](const StageRegs<NIK>& R, int buf, int p) {
+    // v and b are staged times the weight of their token (the operand the matrix cores take is a_s v_s, rounded to bf16 once)
+    auto store_stage = [&](const StageRegs<NIK, NIV>& R, int buf, int p) {
 #pragma unroll
       for (int j = 0; j < NIK; ++j)
-        if (kval[j]) put(sKT + buf * kbuf + kdst[j], R.k[j][0], R.k[j][1]);
+        if (kval[j]) *(u32x4*)&sK[buf * kbuf + kdst[j]] = R.k[j];
       const float* wts = sA + (p % 3) * kC;
-      if (vval) put_weighted(sVT + buf * vbuf + vdst, R.v[0], R.v[1], vsp, wts);
-      if (HAS_J && bval) put_weighted(sBT + buf * vbuf + bdst, R.b[0], R.b[1], bsp, wts);
+#pragma unroll
+      for (int j = 0; j < NIV; ++j) {
+        if (vval[j]) {
+          const float wt = wts[vtok[j]];
+          u32x4 x;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t word = R.v[j][e];
+            const bf16x2 y = pack2(wt * __builtin_bit_cast(float, word << 16), wt * __builtin_bit_cast(float, word & 0xffff0000u));
+            x[e] = __builtin_bit_cast(uint32_t, y);
+          }
+          const bool is_b = HAS_J && 64 * wg + 256 * j >= 128 * DSB;
+          *(u32x4*)&(is_b ? sB : sV)[buf * vbuf + vdst[j]] = x;
+        }
+      }
     };
     // weights of the tokens of tile p and the decay over the whole tile, one step before its rows are staged
-    auto scan_stage = [&](const StageRegs<NIK>& R, int p) {
+    auto scan_stage = [&](const StageRegs<NIK, NIV>& R, int p) {
       if (wg == 3) {
         const float gt = __builtin_bit_cast(float, a.gate_bf16 ? R.gt << 16 : R.gt);   // zero beyond the sequence
         const float cs = wave_inclusive_scan(-gt * gh, lane);
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     // with a run-time test it has to wait for all of them, which throws the fetching ahead away.)
     auto run = [&](auto parity) {
       constexpr int G = decltype(parity)::value;
-      StageRegs<NIK> R[2];
+      StageRegs<NIK, NIV> R[2];
       load_stage(R[0], G);
       for (int p0 = -2; p0 < nchunks; p0 += 4) {
 #pragma unroll
@@ -225,20 +226,20 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
 
   // ------------------------------------------------------------------ state role
   // state blocks of this wave: block sb = w + 4 jj -> (value rows 16 db.., key columns 16 nb..)
-  const int NB = dks >> 4, NSB = (ds >> 4) * NB;
-  int ldk[kStMaxBlocks], ldv[kStMaxBlocks], goff[kStMaxBlocks];   // operand rows in the staging tiles, entry in a state
-  bool sval[kStMaxBlocks];
-  f32x4 accM[kStMaxBlocks], accJ[kStMaxBlocks];
+  const int NB = dks >> 4, blocks = DSB * NB;
+  int ldk[NSB], ldv[NSB], goff[NSB];   // operands in the staging tiles, entry in a state
+  bool sval[NSB];
+  f32x4 accM[NSB], accJ[NSB];
   const int64_t E = (int64_t)dv * dk;
   const float Ip = HAS_J ? a.Ip[h] : 0.f;
 #pragma unroll
-  for (int jj = 0; jj < kStMaxBlocks; ++jj) {
+  for (int jj = 0; jj < NSB; ++jj) {
     const int sb = w + 4 * jj;
-    sval[jj] = sb < NSB;
-    const int db = sb / NB, nb = sb - db * NB;
+    sval[jj] = sb < blocks;
+    const int db = sval[jj] ? sb / NB : 0, nb = sval[jj] ? sb - db * NB : 0;
     // rows n = 16 nb + 4 g + r (four consecutive key columns), column d = d0 + 16 db + i
-    ldk[jj] = (16 * nb + i) * kStTS + 8 * g;
-    ldv[jj] = (16 * db + i) * kStTS + 8 * g;
+    ldk[jj] = (4 * g + (i >> 2)) * KS + 16 * nb + 4 * (i & 3);
+    ldv[jj] = (4 * g + (i >> 2)) * VS + 16 * db + 4 * (i & 3);
     goff[jj] = (d0 + 16 * db + i) * dk + k0 + 16 * nb + 4 * g;
     accM[jj] = f32x4{0.f, 0.f, 0.f, 0.f};
     accJ[jj] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -261,41 +262,59 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     const int c = A.reverse ? nchunks - 1 - p : p;
     const int64_t slot = ((int64_t)(cbase + c) * H + h) * E;
     const float F = sF[p % 3];
-    const bf16_t* kt = (const bf16_t*)(sKT + buf * kbuf);
-    const bf16_t* vt = (const bf16_t*)(sVT + buf * vbuf);
-    const bf16_t* bt = (const bf16_t*)(sBT + buf * vbuf);
+    const bf16_t* kt = sK + buf * kbuf;
+    const bf16_t* vt = sV + buf * vbuf;
+    const bf16_t* bt = sB + buf * vbuf;
+    // operands, the tokens as contraction index (g, j) -> 32 ks + 16 (j / 4) + 4 g + j % 4; those of the next block are read
+    // while a block is worked
+    struct Ops { bf16x8 k[2], v[2], b[2]; } x[2];
+    auto read = [&](int jj, Ops& y) {
 #pragma unroll
-    for (int jj = 0; jj < kStMaxBlocks; ++jj) {
-      if (!sval[jj]) continue;
+      for (int ks = 0; ks < 2; ++ks) {
+        const bf16_t* pk = kt + ldk[jj] + 32 * ks * KS;
+        const bf16_t* pv = vt + ldv[jj] + 32 * ks * VS;
+        const bf16_t* pb = bt + ldv[jj] + 32 * ks * VS;
+        y.k[ks] = join(lds_read_tr(pk), lds_read_tr(pk + 16 * KS));
+        y.v[ks] = join(lds_read_tr(pv), lds_read_tr(pv + 16 * VS));
+        if (HAS_J) y.b[ks] = join(lds_read_tr(pb), lds_read_tr(pb + 16 * VS));
+      }
+    };
+    read(0, x[0]);
+#pragma unroll
+    for (int jj = 0; jj < NSB; ++jj) {
+      if (jj > 0 && !sval[jj]) break;
+      if (jj + 1 < NSB) read(jj + 1, x[(jj + 1) & 1]);   // (a block that the wave has not repeats the first one's)
+      __builtin_amdgcn_sched_barrier(0);
+      const Ops& y = x[jj & 1];
       const int64_t off = slot + goff[jj];
-      if (HAS_J) {
-        f32x4 mu, I;
+      if (sval[jj]) {
+        if (HAS_J) {
+          f32x4 mu, I;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) { I[r] = accJ[jj][r] + Ip; mu[r] = accM[jj][r] * fast_rcp(I[r]); }
-        *(f32x4*)((float*)A.tiles_a + off) = mu;
-        *(f32x4*)(A.tiles_b + off) = I;
-      } else {
-        store_vec<4>((bf16_t*)A.tiles_a + off, (const float*)&accM[jj]);
+          for (int r = 0; r < 4; ++r) { I[r] = accJ[jj][r] + Ip; mu[r] = accM[jj][r] * fast_rcp(I[r]); }
+          *(f32x4*)((float*)A.tiles_a + off) = mu;
+          *(f32x4*)(A.tiles_b + off) = I;
+        } else {
+          store_vec<4>((bf16_t*)A.tiles_a + off, (const float*)&accM[jj]);
+        }
       }
       f32x4 M = accM[jj] * F, J = accJ[jj] * F;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const bf16x8 BK = *(const bf16x8*)&kt[ldk[jj] + 32 * ks];
-        const bf16x8 AM = *(const bf16x8*)&vt[ldv[jj] + 32 * ks];
-        M = mfma16(BK, AM, M);
+        M = mfma16(y.k[ks], y.v[ks], M);
         if (HAS_J) {
-          const bf16x8 AJ = *(const bf16x8*)&bt[ldv[jj] + 32 * ks];
-          bf16x8 BKK;
+          bf16x8 kk;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
-            const float kf = (float)BK[j];
-            BKK[j] = (bf16_t)(kf * kf);
+            const float kf = (float)y.k[ks][j];
+            kk[j] = (bf16_t)(kf * kf);
           }
-          J = mfma16(BKK, AJ, J);
+          J = mfma16(kk, y.b[ks], J);
         }
       }
       accM[jj] = M;
       accJ[jj] = J;
+      __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
   }
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
 
   if (A.fin_a) {
 #pragma unroll
-    for (int jj = 0; jj < kStMaxBlocks; ++jj) {
+    for (int jj = 0; jj < NSB; ++jj) {
       if (!sval[jj]) continue;
       const int64_t off = (int64_t)nh * E + goff[jj];
       if (HAS_J) {
@@ -320,21 +339,35 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
   }
 }
 
-template <bool HAS_J, int NIK>
+template <bool HAS_J, int NIK, int DSB>
 static int launch_state_pass_t(const StatePassArgs& A, int kern_id, unsigned grid, size_t lds, hipStream_t s) {
-  if (int rc = allow_lds((const void*)&chunk_states_kernel<HAS_J, NIK>, lds)) return rc;
-  PAL_TIMED_LAUNCH(kern_id, s, (chunk_states_kernel<HAS_J, NIK>), dim3(grid), dim3(768), lds, s, A);
+  if (int rc = allow_lds((const void*)&chunk_states_kernel<HAS_J, NIK, DSB>, lds)) return rc;
+  PAL_TIMED_LAUNCH(kern_id, s, (chunk_states_kernel<HAS_J, NIK, DSB>), dim3(grid), dim3(768), lds, s, A);
   PAL_HIP_LAUNCH_CHECK();
   return PAL_OK;
 }
 
+template <bool HAS_J, int DSB>
+static int launch_state_pass_d(const StatePassArgs& A, int kern_id, unsigned grid, size_t lds, hipStream_t s) {
+  const int nik = (A.dks + 31) / 32;
+  if (nik <= 2) return launch_state_pass_t<HAS_J, 2, DSB>(A, kern_id, grid, lds, s);
+  if (nik == 3) return launch_state_pass_t<HAS_J, 3, DSB>(A, kern_id, grid, lds, s);
+  if constexpr (DSB <= 3) {
+    if (nik == 4) return launch_state_pass_t<HAS_J, 4, DSB>(A, kern_id, grid, lds, s);
+  }
+  if constexpr (DSB <= 2) {
+    if (nik <= 6) return launch_state_pass_t<HAS_J, 6, DSB>(A, kern_id, grid, lds, s);
+  }
+  if constexpr (DSB == 1) return launch_state_pass_t<HAS_J, 8, DSB>(A, kern_id, grid, lds, s);
+  return PAL_E_HEADDIM;   // (launch_state_pass keeps ds dks within the state waves' blocks)
+}
 template <bool HAS_J>
 static int launch_state_pass_j(const StatePassArgs& A, int kern_id, unsigned grid, size_t lds, hipStream_t s) {
-  switch ((A.dks + 63) / 64) {
-    case 1: return launch_state_pass_t<HAS_J, 1>(A, kern_id, grid, lds, s);
-    case 2: return launch_state_pass_t<HAS_J, 2>(A, kern_id, grid, lds, s);
-    case 3: return launch_state_pass_t<HAS_J, 3>(A, kern_id, grid, lds, s);
-    case 4: return launch_state_pass_t<HAS_J, 4>(A, kern_id, grid, lds, s);
+  switch (A.ds) {
+    case 16: return launch_state_pass_d<HAS_J, 1>(A, kern_id, grid, lds, s);
+    case 32: return launch_state_pass_d<HAS_J, 2>(A, kern_id, grid, lds, s);
+    case 48: return launch_state_pass_d<HAS_J, 3>(A, kern_id, grid, lds, s);
+    case 64: return launch_state_pass_d<HAS_J, 4>(A, kern_id, grid, lds, s);
     default: return PAL_E_HEADDIM;
   }
 }
@@ -388,7 +421,8 @@ int launch_state_pass(const ChunkArgs& a, bool has_j, void* tiles_a, float* tile
   A.ksplit = a.dk / dks;
   if ((int64_t)a.n_seqs * a.H <= 0) return PAL_OK;
   if (!walk_plan(a, a.dv / ds * A.ksplit, A.plan)) return PAL_E_DIM;
-  const size_t lds = sizeof(float) * (3 * kC + 4) + (size_t)2 * 2 * kStTS * (dks + ds * (has_j ? 2 : 1));
+  const size_t lds = sizeof(float) * (3 * kC + 4) +
+                     sizeof(bf16_t) * 2 * kC * (size_t)(staged_stride(dks) + staged_stride(ds) * (has_j ? 2 : 1));
   if (lds > kMaxLds) return PAL_E_HEADDIM;
   const unsigned grid = (unsigned)A.plan.per_xcd * 8;
   return has_j ? launch_state_pass_j<true>(A, kern_id, grid, lds, s) : launch_state_pass_j<false>(A, kern_id, grid, lds, s);

@@ -306,6 +306,19 @@ __device__ __forceinline__ void store_vec(bf16_t* p, const float* in) {
   }
 }
 
+// ------------------------------------------------------------------- transposing LDS reads
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// Four rows by 16 columns of a bf16 tile in LDS, transposed on their way out: of the 16 lanes of a row, lane l hands over
+// the address of four consecutive elements of row l / 4 (columns 4 (l % 4) .. of whatever the addresses say), and lane i
+// receives column i of the four rows.
+__device__ __forceinline__ bf16x4 lds_read_tr(const bf16_t* p) {
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
+}
+__device__ __forceinline__ bf16x8 join(bf16x4 a, bf16x4 b) {
+  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
 // ------------------------------------------------------------------ host
 #define PAL_HIP_LAUNCH_CHECK()                 \
   do {                                         \

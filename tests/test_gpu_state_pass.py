@@ -83,6 +83,19 @@ def test_palimpsa_forms_agree(gpu_device, state_pass_mode, case):
     assert hp.max_rel(b[1], fmu_ref) <= 2e-2 and hp.max_rel(b[2], fI_ref) <= 2e-2
 
 
+@pytest.mark.parametrize("dk,dv", [(16, 64), (48, 48), (80, 64), (96, 32), (128, 48), (176, 32), (192, 16), (256, 16)])
+def test_wide_value_slices_agree(gpu_device, state_pass_mode, dk, dv):
+    """Enough heads that a workgroup takes several blocks of value rows, over the widths of the staged key rows; two tiles
+    and a ragged third. Tolerances as above: the forms differ in the order of fp32 sums."""
+    inp = _pal_inputs(2, 129 + dk % 7, 96, dk, dv, dk + dv, gpu_device)
+    state_pass_mode(1)
+    a = _run_palimpsa(inp, None, None, None, False)
+    state_pass_mode(2)
+    b = _run_palimpsa(inp, None, None, None, False)
+    assert hp.max_abs(a[0].float(), b[0].float()) <= 1e-2
+    assert hp.max_rel(a[1], b[1]) <= 1e-4 and hp.max_rel(a[2], b[2]) <= 1e-4
+
+
 def _gla_inputs(B, T, H, dk, dv, seed):
     gen = torch.Generator().manual_seed(seed)
     q = torch.nn.functional.normalize(torch.randn(B, T, H, dk, generator=gen), dim=-1).bfloat16()
