@@ -9,7 +9,20 @@
 // Why not on the matrix cores: a state entry costs four plain fp32 instructions to advance (two per branch).  As prefix
 // products it costs 12 matrix instructions of 16 cycles per 16 entries of a lane plus the operands, more issue time than
 // the four, and rounds the operands.  What bounds the kernel is vector issue: per entry and token six fp32
-// instructions and one reciprocal.
+// instructions and one reciprocal, or (scaled form) six and half a reciprocal.
+//
+// Scaled form (bf16 rows without the uncertainty output): with F_t the decay since the start of a staging step of
+// eight tokens, M = F M', I - Ip = F J':
+//   M' <- M' + (v_t / F_t) k_t^T,   J' <- J' + (b_t / F_t) (k_t*k_t)^T,   M / I = M' / (J' + Ip / F_t)
+// so that the decay costs an addition per entry and token instead of two products and one addition, v / F and b / F once a
+// row; two entries share a reciprocal, n1/x1 + n2/x2 = (n1 x2 + n2 x1) / (x1 x2).  Against a float64 recurrence the outputs
+// are as exact as in plain form to three digits (bf16 rounding is all of the error); in fp32 the error of the outputs would
+// be up to 0.5 % larger and that of the uncertainty 15 %, so fp32 rows and the uncertainty keep the plain form.  A tile
+// takes it where every step decays by less than 2^48, and is worked again in plain form if a total is not finite
+// (precisions beyond 1e15 or so, or inputs that were not finite).  8 x 2048 tokens, 12 heads of 64x64 160 -> 148 us; 65536 of
+// 16 heads of 128x128 3060 -> 2870; 32768 of 16 of 96x96 945 -> 888.  (The issue rates below promise 22.6 -> 18.1 cycles; 26.1
+// of 27.9 are left: LDS reads of the operands 2.3, the totals over the lanes 2.  Four rows a lane halve both, but leave two
+// waves per SIMD: 193 us at 64x64.)
 //
 // How a SIMD of gfx950 issues these (profiles/issue_rates.txt): a lone wave issues an fp32 add, mul or fma per 5 cycles; two waves
 // issue one each in the same cycles (2.4 to 2.6 per instruction), a reciprocal takes 8.2 with no other beside it, and the
@@ -18,7 +31,7 @@
 // (s_setprio; B=8 T=2048 H=12 64x64: 185 -> 161 us); (2) fp32 instructions with a scalar-register operand do not pair
 // (every operand comes from LDS into vector registers, wave-uniform ones too); (3) an odd number of waves on a
 // SIMD leaves one without a partner (two or four waves, not three: at most 128 registers).
-// Ideal by these rates: 6 x 2.4 + 8.2 = 22.6 cycles per entry and wave; measured 27.9 (profiles/bench_c1.sq_counters_pmc.txt).
+// Ideal by these rates in plain form: 6 x 2.4 + 8.2 = 22.6 cycles per entry and wave; measured 27.9 (profiles/bench_c1.sq_counters_pmc.txt).
 // Against the earlier kernels on the matrix cores: 64x64 B=8 T=2048 H=12 250 -> 155 us, 128x128 B=2 T=4096 H=16
 // 568 -> 388, 96x96 B=8 T=2048 H=16 0.287 -> 0.202 ps per entry, fp32 rows at 64x64 570 -> 160 us (they ran split operands).
 //
@@ -34,6 +47,9 @@
 
 namespace pal {
 
+// Least decay over a staging step for the scaled form: M / F stays far inside fp32, and so does a product of two precisions
+// up to 4e4 each.  Steps that decay more are rare (gates of 0.5 at a rate of 2: 2^-12) and gain least from it.
+constexpr float kMinDecay = 0x1p-48f;
 constexpr int kOT = 8;   // tokens per staging step: two buffers of them let four workgroups of four waves share a unit's LDS
 
 template <int DD>
@@ -68,6 +84,11 @@ struct OutRow {
   }
 };
 
+template <int N>
+__device__ __forceinline__ float dpp_shr(float x) {   // lane i of a row of 16 takes lane i - N
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x110 + N, 0xf, 0xf, true));
+}
+
 template <typename TIn, int NG, int DN, int DD, bool HAS_VAR>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(HAS_VAR ? 2 : 4)))
 void chunk_out_kernel(ChunkArgs a, int W) {
@@ -76,6 +97,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   constexpr int DKP = NG * DN;              // key columns of the lanes (dk, or up to 16 more that stay zero)
   constexpr int ROWS = (64 / NG) * DD;      // value rows of a wave
   constexpr int TU = 4 / DD;                // tokens per iteration
+  constexpr bool kMayScale = std::is_same<TIn, bf16_t>::value && !HAS_VAR;
   const int NT = W * 64, VR = W * ROWS;     // threads and value rows of the workgroup
   constexpr int oK = 4, oKK = oK + DKP, oQ = oKK + DKP, oVB = oQ + DKP;
   const int STRIDE = oVB + 2 * VR;          // floats per staged token: f, c, -, -, k, k*k, q, (v, b) of every row
@@ -85,8 +107,9 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   const int r0 = (int)blockIdx.y * VR;
   int seq, t0, clen, cis;
   chunk_lookup(a, cidx, seq, t0, clen, cis);
-  float* sFC = smem;                        // [64][2] f_t, (1 - f_t) Ip
-  float* sRow = sFC + 2 * kC;               // [2][kOT][STRIDE]
+  float* sFC = smem;                        // [64][4] f_t (at the end of a step in scaled form: F), c_t, factor of v and b
+  int* sForm = (int*)(sFC + 4 * kC);        // whether the tile is worked in scaled form
+  float* sRow = sFC + 4 * kC + 4;               // [2][kOT][STRIDE]
   const float Ip = a.Ip[h];
   // every fetch of the set-up is issued before the first is used
   const float gt = (w == 0 && lane < clen) ? load_gate(a.gt, (int64_t)(t0 + lane) * H + h, a.gate_bf16) : 0.f;
@@ -120,12 +143,13 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   };
   auto deposit = [&](int s0, int buf) {
     float* base = sRow + buf * kOT * STRIDE;
-    if (tid < kOT) *(f32x2*)&base[tid * STRIDE] = *(const f32x2*)&sFC[2 * (s0 + tid)];   // s0 + tid < 64
+    if (tid < kOT) *(f32x2*)&base[tid * STRIDE] = *(const f32x2*)&sFC[4 * (s0 + tid)];   // s0 + tid < 64
     if (s_kq < kOT && s0 + s_kq < clen) put_kq(base + s_kq * STRIDE, c_kq, rk, rq);
     if (s_vb < kOT && s0 + s_vb < clen) {
       float* p = &base[s_vb * STRIDE + oVB + 8 * c_vb];
-      *(f32x4*)p = f32x4{(float)rv[0], (float)rb[0], (float)rv[1], (float)rb[1]};
-      *(f32x4*)(p + 4) = f32x4{(float)rv[2], (float)rb[2], (float)rv[3], (float)rb[3]};
+      const float u = sFC[4 * (s0 + s_vb) + 2];
+      *(f32x4*)p = f32x4{u * (float)rv[0], u * (float)rb[0], u * (float)rv[1], u * (float)rb[1]};
+      *(f32x4*)(p + 4) = f32x4{u * (float)rv[2], u * (float)rb[2], u * (float)rv[3], u * (float)rb[3]};
     }
     // wide keys on few waves: the items of k, q beyond the fetched ones
     for (int idx = tid + NT; idx < kOT * nk4; idx += NT) {
@@ -135,48 +159,8 @@ void chunk_out_kernel(ChunkArgs a, int W) {
                *(const raw4*)(qp + (int64_t)(s0 + s) * qs + 4 * c));
     }
   };
-  fetch(0);
   const int ng = OutLanes<NG>::col(lane), dg = OutLanes<NG>::row(lane);
   const int d0 = w * ROWS + dg * DD;        // first value row of the lane inside the workgroup
-  float M[DD][DN], I[DD][DN];
-  {
-    const float* mu = a.chunk_mu + (((int64_t)cidx * H + h) * dv + r0) * dk;
-    const float* Is = a.chunk_I + (((int64_t)cidx * H + h) * dv + r0) * dk;
-#pragma unroll
-    for (int j = 0; j < DD; ++j) {
-      const bool on = r0 + d0 + j < dv;
-      const int64_t ro = (int64_t)(on ? d0 + j : 0) * dk;
-      auto piece = [&](auto width, int i) {
-        constexpr int VW = decltype(width)::value;
-        const int c = col_of<NG, DN>(i, ng);
-        float x[VW], y[VW];
-        const bool in = DKP == 0 || c < dk;
-        load_vec<VW>(mu + ro + (in ? c : 0), x);
-        load_vec<VW>(Is + ro + (in ? c : 0), y);
-#pragma unroll
-        for (int e = 0; e < VW; ++e) {
-          M[j][i + e] = on && in ? x[e] * y[e] : 0.f;
-          I[j][i + e] = on && in ? y[e] : 1.f;
-        }
-      };
-#pragma unroll
-      for (int p = 0; p < DN / 4; ++p) piece(std::integral_constant<int, 4>{}, 4 * p);
-      if constexpr ((DN & 3) >= 2) piece(std::integral_constant<int, 2>{}, 4 * (DN / 4));
-      if constexpr (DN & 1) piece(std::integral_constant<int, 1>{}, DN - 1);
-    }
-  }
-  if (w == 0) {
-    const float f = fast_exp2(-gt * gh);
-    *(f32x2*)&sFC[2 * lane] = f32x2{f, (1.f - f) * Ip};
-  }
-  // rows and columns beyond the head dims stay zero in both buffers
-  if (DKP != dk || VR > dv - r0) {
-    for (int idx = tid; idx < 2 * kOT * STRIDE; idx += NT) sRow[idx] = 0.f;
-  }
-  __syncthreads();
-  deposit(0, 0);
-  __syncthreads();
-
   // The totals of DD rows x TU tokens are reduced together: four values, of which lane bits 3 and 2 select one
   const int sel = 2 * ((lane >> 3) & 1) + ((lane >> 2) & 1);
   const int dsel = sel % DD, tsel = sel / DD;
@@ -186,65 +170,157 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   };
   const int64_t orow = ((int64_t)t0 * H + h) * dv + r0 + d0 + dsel;
 
-  OutRow<NG, DN, DD> x;
-  for (int s0 = 0; s0 < clen; s0 += kOT) {
-    const int buf = (s0 / kOT) & 1;
-    const bool more = s0 + kOT < clen;
-    if (more) fetch(s0 + kOT);
-    const int nt = min(kOT, clen - s0);
-    const float* row = sRow + buf * kOT * STRIDE;
-    x.load(row, ng, d0);
-#pragma unroll 1
-    for (int tt = 0; tt < nt; tt += TU, row += TU * STRIDE) {
-      float acc[4], accv[4];
-#pragma unroll
-      for (int u = 0; u < TU; ++u) {
-        float r[DD][DN], qc[DN];
-#pragma unroll
-        for (int i = 0; i < DN; ++i) {
-#pragma unroll
-          for (int j = 0; j < DD; ++j) {
-            M[j][i] = fmaf(x.vb[2 * j], x.k[i], M[j][i] * x.fc[0]);
-            fma3(I[j][i], x.fc[0], x.fc[1]);
-            I[j][i] = fmaf(x.vb[2 * j + 1], x.kk[i], I[j][i]);
-          }
-          qc[i] = x.q[i];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        // the next token's operands are requested here: the burst of reciprocals hides their latency (after the last
-        // token of a step: rows of the other buffer or, at its end, not yet written; they are read again below)
-        x.load(row + (u + 1) * STRIDE, ng, d0);
-        __builtin_amdgcn_s_setprio(3);
-#pragma unroll
-        for (int i = 0; i < DN; ++i)
-#pragma unroll
-          for (int j = 0; j < DD; ++j) r[j][i] = fast_rcp(I[j][i]);
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < DD; ++j) { acc[u * DD + j] = 0.f; accv[u * DD + j] = 0.f; }
-#pragma unroll
-        for (int i = 0; i < DN; ++i)
-#pragma unroll
-          for (int j = 0; j < DD; ++j) {
-            float& y = acc[u * DD + j];
-            y = fmaf(M[j][i] * r[j][i], qc[i], y);
-            if constexpr (HAS_VAR) accv[u * DD + j] = fmaf(qc[i] * qc[i], r[j][i], accv[u * DD + j]);
-          }
-      }
-      const int t = s0 + tt + tsel;
-      const bool wr = writer && t < clen;
-      const int64_t oo = orow + (int64_t)t * vs;
-      const float out = reduce(acc);
-      if (wr) ((TIn*)a.o)[oo] = from_f32<TIn>(out * a.scale);
-      if constexpr (HAS_VAR) {
-        const float outv = reduce(accv);
-        if (wr) store_rt(a.o_var, oo, outv * a.scale, a.var_bf16);
-      }
+  const float f = fast_exp2(-gt * gh);
+  float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
+  if (kMayScale) {
+    if (w == 0) {
+      const int s = lane & (kOT - 1);
+      // (each shift before its select: a lane that is switched off hands nothing on)
+      float y = dpp_shr<1>(F);
+      F = s >= 1 ? F * y : F;
+      y = dpp_shr<2>(F);
+      F = s >= 2 ? F * y : F;
+      y = dpp_shr<4>(F);
+      F = s >= 4 ? F * y : F;
+      const bool ok = __all(F >= kMinDecay && F <= 1.f);
+      if (lane == 0) *sForm = ok;
     }
-    if (more) deposit(s0 + kOT, buf ^ 1);
     __syncthreads();
   }
+
+  // The tile in scaled or plain form (see above); whether a total of the scaled form is not finite.
+  auto walk_tile = [&](auto form) -> bool {
+    constexpr bool SCALED = decltype(form)::value;
+    constexpr int NR = SCALED ? (DN + 1) / 2 : DN;   // reciprocals of a row and token
+    fetch(0);
+    float M[DD][DN], I[DD][DN];   // SCALED: M / F and (I - Ip) / F
+    {
+      const float* mu = a.chunk_mu + (((int64_t)cidx * H + h) * dv + r0) * dk;
+      const float* Is = a.chunk_I + (((int64_t)cidx * H + h) * dv + r0) * dk;
+#pragma unroll
+      for (int j = 0; j < DD; ++j) {
+        const bool on = r0 + d0 + j < dv;
+        const int64_t ro = (int64_t)(on ? d0 + j : 0) * dk;
+        auto piece = [&](auto width, int i) {
+          constexpr int VW = decltype(width)::value;
+          const int c = col_of<NG, DN>(i, ng);
+          float x[VW], y[VW];
+          const bool in = DKP == 0 || c < dk;
+          load_vec<VW>(mu + ro + (in ? c : 0), x);
+          load_vec<VW>(Is + ro + (in ? c : 0), y);
+#pragma unroll
+          for (int e = 0; e < VW; ++e) {
+            M[j][i + e] = on && in ? x[e] * y[e] : 0.f;
+            I[j][i + e] = on && in ? (SCALED ? y[e] - Ip : y[e]) : 1.f;
+          }
+        };
+#pragma unroll
+        for (int p = 0; p < DN / 4; ++p) piece(std::integral_constant<int, 4>{}, 4 * p);
+        if constexpr ((DN & 3) >= 2) piece(std::integral_constant<int, 2>{}, 4 * (DN / 4));
+        if constexpr (DN & 1) piece(std::integral_constant<int, 1>{}, DN - 1);
+      }
+    }
+    if (w == 0) {
+      const float inv = SCALED ? fast_rcp(F) : 1.f;
+      *(f32x4*)&sFC[4 * lane] = f32x4{SCALED ? F : f, SCALED ? Ip * inv : (1.f - f) * Ip, inv, 0.f};
+    }
+    // rows and columns beyond the head dims stay zero in both buffers
+    if (DKP != dk || VR > dv - r0) {
+      for (int idx = tid; idx < 2 * kOT * STRIDE; idx += NT) sRow[idx] = 0.f;
+    }
+    __syncthreads();
+    deposit(0, 0);
+    __syncthreads();
+
+    bool bad = false;
+    OutRow<NG, DN, DD> x;
+    for (int s0 = 0; s0 < clen; s0 += kOT) {
+      const int buf = (s0 / kOT) & 1;
+      const bool more = s0 + kOT < clen;
+      if (more) fetch(s0 + kOT);
+      const int nt = min(kOT, clen - s0);
+      const float* row = sRow + buf * kOT * STRIDE;
+      x.load(row, ng, d0);
+#pragma unroll 1
+      for (int tt = 0; tt < nt; tt += TU, row += TU * STRIDE) {
+        float acc[4], accv[4];
+#pragma unroll
+        for (int u = 0; u < TU; ++u) {
+          float num[DD][NR], numv[DD][NR], den[DD][NR];
+#pragma unroll
+          for (int i = 0; i < DN; ++i)
+#pragma unroll
+            for (int j = 0; j < DD; ++j) {
+              if constexpr (SCALED) {
+                M[j][i] = fmaf(x.vb[2 * j], x.k[i], M[j][i]);
+                I[j][i] = fmaf(x.vb[2 * j + 1], x.kk[i], I[j][i]);
+                if (i & 1) {   // n1 / x1 + n2 / x2 = (n1 x2 + n2 x1) / (x1 x2)
+                  const float x1 = I[j][i - 1] + x.fc[1], x2 = I[j][i] + x.fc[1];
+                  num[j][i / 2] = fmaf(M[j][i] * x.q[i], x1, M[j][i - 1] * x.q[i - 1] * x2);
+                  den[j][i / 2] = x1 * x2;
+                } else if (i == DN - 1) {
+                  num[j][i / 2] = M[j][i] * x.q[i];
+                  den[j][i / 2] = I[j][i] + x.fc[1];
+                }
+              } else {
+                M[j][i] = fmaf(x.vb[2 * j], x.k[i], M[j][i] * x.fc[0]);
+                fma3(I[j][i], x.fc[0], x.fc[1]);
+                I[j][i] = fmaf(x.vb[2 * j + 1], x.kk[i], I[j][i]);
+                num[j][i] = x.q[i];
+                if constexpr (HAS_VAR) numv[j][i] = x.q[i] * x.q[i];
+                den[j][i] = I[j][i];
+              }
+            }
+          __builtin_amdgcn_sched_barrier(0);
+          // the next token's operands are requested here: the burst of reciprocals hides their latency (after the last
+          // token of a step: rows of the other buffer or, at its end, not yet written; they are read again below)
+          x.load(row + (u + 1) * STRIDE, ng, d0);
+          __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+          for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int j = 0; j < DD; ++j) den[j][i] = fast_rcp(den[j][i]);
+          __builtin_amdgcn_s_setprio(0);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < DD; ++j) { acc[u * DD + j] = 0.f; accv[u * DD + j] = 0.f; }
+#pragma unroll
+          for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int j = 0; j < DD; ++j) {
+              float& y = acc[u * DD + j];
+              if constexpr (SCALED) y = fmaf(num[j][i], den[j][i], y);
+              else y = fmaf(M[j][i] * den[j][i], num[j][i], y);
+              if constexpr (HAS_VAR) accv[u * DD + j] = fmaf(numv[j][i], den[j][i], accv[u * DD + j]);
+            }
+        }
+        const int t = s0 + tt + tsel;
+        const bool wr = writer && t < clen;
+        const int64_t oo = orow + (int64_t)t * vs;
+        const float out = reduce(acc);
+        if (wr) ((TIn*)a.o)[oo] = from_f32<TIn>(out * a.scale);
+        if (SCALED) bad |= wr && !(__builtin_fabsf(out) < __builtin_inff());
+        if constexpr (HAS_VAR) {
+          const float outv = reduce(accv);
+          if (wr) store_rt(a.o_var, oo, outv * a.scale, a.var_bf16);
+        }
+      }
+      if (SCALED && more) {
+        const float Fe = sFC[4 * (s0 + kOT - 1)];
+#pragma unroll
+        for (int i = 0; i < DN; ++i)
+#pragma unroll
+          for (int j = 0; j < DD; ++j) { M[j][i] *= Fe; I[j][i] *= Fe; }
+      }
+      if (more) deposit(s0 + kOT, buf ^ 1);
+      __syncthreads();
+    }
+    return bad;
+  };
+  if constexpr (kMayScale) {
+    if (*sForm && !__syncthreads_or(walk_tile(std::true_type{}))) return;
+  }
+  walk_tile(std::false_type{});
 }
 
 // Waves per workgroup for nw waves of value rows: the hardware deals the waves of a workgroup out to the four SIMDs in
@@ -266,7 +342,7 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
   const int W = out_waves(nw), slices = (nw + W - 1) / W;
   const int64_t blocks = (int64_t)a.total_chunks * a.H;
   if (blocks > 0x7fffffff) return PAL_E_DIM;
-  const size_t lds = sizeof(float) * (2 * kC + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
+  const size_t lds = sizeof(float) * (4 * kC + 4 + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
   if (lds > kMaxLds) return PAL_E_HEADDIM;
   auto go = [&](auto kern) -> int {
     if (int rc = allow_lds((const void*)kern, lds)) return rc;

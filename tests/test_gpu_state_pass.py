@@ -96,6 +96,34 @@ def test_wide_value_slices_agree(gpu_device, state_pass_mode, dk, dv):
     assert hp.max_rel(a[1], b[1]) <= 1e-4 and hp.max_rel(a[2], b[2]) <= 1e-4
 
 
+@pytest.mark.parametrize("dk,dv", [(64, 64), (48, 20), (80, 48)])       # even and odd numbers of columns per lane
+@pytest.mark.parametrize("case", ["usual", "no_decay", "strong", "mixed", "growth", "huge", "nan"])
+def test_scaled_and_plain_tiles(gpu_device, state_pass_mode, dk, dv, case):
+    """Outputs of the tiles over what decides between their two forms, and over what makes the scaled one start again,
+    against the oracle in float64: bf16 rows, so the results' rounding is the tolerance."""
+    inp = _pal_inputs(2, 150, 3, dk, dv, dk, "cpu")
+    gen = torch.Generator().manual_seed(dv)
+    mu0 = torch.randn(2, 3, dv, dk, generator=gen) * 0.3
+    I0 = torch.rand(2, 3, dv, dk, generator=gen) + inp["Ip"][None, :, None, None]
+    if case == "no_decay":
+        inp["g"] = torch.zeros(3)
+    elif case == "strong":            # 2^-60 and less over eight tokens, a gate that leaves nothing among them
+        inp["g"] = torch.tensor([40.0, 80.0, 2000.0])
+    elif case == "mixed":             # one step of one tile decays too much
+        inp["gt"][:, 70] = 30.0
+    elif case == "growth":
+        inp["gt"][:, 20:30] *= -0.2
+    elif case == "huge":              # the product of two precisions overflows, the quotients do not
+        I0 *= 1e24
+    elif case == "nan":
+        inp["v"][0, 40, 1, 3] = float("nan")
+    state_pass_mode(2)
+    o = _run_palimpsa(hp.to_device(inp, gpu_device), mu0.to(gpu_device), I0.to(gpu_device), None, False)[0].float().cpu()
+    o_ref = hp.oracle_forward(inp, mu0=mu0, I0=I0, dtype=torch.float64)[0].float()
+    assert torch.equal(torch.isnan(o), torch.isnan(o_ref))
+    assert hp.max_abs(o.nan_to_num(), o_ref.nan_to_num()) <= hp.BF16_OUT_ABS_TOL
+
+
 def _gla_inputs(B, T, H, dk, dv, seed):
     gen = torch.Generator().manual_seed(seed)
     q = torch.nn.functional.normalize(torch.randn(B, T, H, dk, generator=gen), dim=-1).bfloat16()
