@@ -31,6 +31,7 @@ struct ChunkArgs {
   int32_t T, H, dk, dv, n_seqs, total_chunks;
   int32_t Hq;   // heads of q and k: H, or a divisor of it when a group of H / Hq value heads shares one q/k head
   int32_t gate_bf16, var_bf16;
+  int32_t every;   // tiles per tile-start state that is kept: 1, or more where the output kernel walks that many from one
   uint32_t flags;
   float scale;
 };

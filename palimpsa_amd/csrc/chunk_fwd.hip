@@ -206,8 +206,9 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(ChunkArgs a) {
 #pragma unroll
     for (int x = 0; x < 4; ++x) { SM[x] = mu[x] * I[x]; SJ[x] = I[x] - Ip; }
   }
-  // the slot of a tile: its Delta is read, the state at its start (mu, I) written, the state advanced
-  auto advance = [&](int64_t off, const f32x4& dM, const f32x4& dJ, float F) {
+  // the slot of a tile: its Delta is read, the state at its start (mu, I) written if it is kept, the state advanced
+  auto advance = [&](int c, const f32x4& dM, const f32x4& dJ, float F) {
+    const int64_t off = ((int64_t)(cbase + c) * a.H + h) * E + e;
     f32x4 mu, I;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -216,8 +217,10 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(ChunkArgs a) {
       SM[x] = fmaf(F, SM[x], dM[x]);
       SJ[x] = fmaf(F, SJ[x], dJ[x]);
     }
-    *(f32x4*)(a.chunk_mu + off) = mu;
-    *(f32x4*)(a.chunk_I + off) = I;
+    if ((c & (a.every - 1)) == 0) {
+      *(f32x4*)(a.chunk_mu + off) = mu;
+      *(f32x4*)(a.chunk_I + off) = I;
+    }
   };
   for (int c0 = 0; c0 < nchunks; c0 += kScanTiles) {
     const int cn = min(kScanTiles, nchunks - c0);
@@ -240,12 +243,12 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(ChunkArgs a) {
         dJ[u] = *(const f32x4*)(a.chunk_I + off);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) advance(((int64_t)(cbase + c0 + c + u) * a.H + h) * E + e, dM[u], dJ[u], sF[c + u]);
+      for (int u = 0; u < 4; ++u) advance(c0 + c + u, dM[u], dJ[u], sF[c + u]);
     }
     for (; c < cn; ++c) {
       const int64_t off = ((int64_t)(cbase + c0 + c) * a.H + h) * E + e;
       const f32x4 dM = *(const f32x4*)(a.chunk_mu + off), dJ = *(const f32x4*)(a.chunk_I + off);
-      advance(off, dM, dJ, sF[c]);
+      advance(c0 + c, dM, dJ, sF[c]);
     }
   }
   if (a.final_mu && on) {
@@ -329,6 +332,7 @@ void fill_chunk_args(ChunkArgs& a, const PalDims* d, const PalFwdTensors* t) {
   a.n_seqs = d->n_seqs; a.total_chunks = d->total_chunks;
   a.gate_bf16 = d->gate_dtype == PAL_DTYPE_BF16;
   a.var_bf16 = d->var_dtype == PAL_DTYPE_BF16;
+  a.every = 1;
   a.flags = d->flags;
   a.scale = d->scale;
 }
@@ -336,7 +340,8 @@ void fill_chunk_args(ChunkArgs& a, const PalDims* d, const PalFwdTensors* t) {
 }  // namespace pal
 
 namespace pal {
-// the outputs from the tile-start states (chunk_out.hip)
+// the outputs from the tile-start states, and how many tiles it walks from one where no one else reads them (chunk_out.hip)
+int out_tiles_per_state(const ChunkArgs& a);
 int launch_out(const ChunkArgs& a, int dtype, hipStream_t s);
 // the one-pass form of chunk_states.hip
 bool state_pass_applies(const ChunkArgs& a, int dtype, bool has_j);
@@ -454,6 +459,7 @@ extern "C" int pal_chunk_fwd_static(const PalDims* d, const PalFwdTensors* t, vo
   tt.chunk_I = base + PAL_STATIC_SCRATCH_BYTES / (2 * sizeof(float));
   ChunkArgs a;
   fill_chunk_args(a, d, &tt);
+  a.every = out_tiles_per_state(a);
   hipStream_t s = (hipStream_t)stream;
   // every slot the output kernel reads is written by the state kernels of this call first: nothing has to start at zero
   if (int rc2 = launch_tile_states(a, d->dtype, true, s)) return rc2;
@@ -485,6 +491,7 @@ extern "C" int pal_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void* str
   }
   ChunkArgs a;
   fill_chunk_args(a, d, t);
+  if (d->flags & PAL_FLAG_OUTPUTS_ONLY) a.every = out_tiles_per_state(a);
   hipStream_t s = (hipStream_t)stream;
   if (int rc2 = launch_tile_states(a, d->dtype, true, s)) return rc2;
   return launch_out(a, d->dtype, s);

@@ -1,7 +1,8 @@
 // Chunked Palimpsa forward, outputs: chunk_out_kernel.
 //
 // From the state at the start of every tile (chunk_states.hip, or the two kernels of chunk_fwd.hip) all tiles of 64
-// tokens are worked in parallel.  Inside a tile the recurrence is run token by token on the vector units in fp32,
+// tokens are worked in parallel (large passes that keep no states: walks of up to four tiles, see out_tiles_per_state).
+// Inside a tile the recurrence is run token by token on the vector units in fp32,
 //   M <- f_t M + v_t k_t^T,   I <- f_t I + b_t (k_t*k_t)^T + (1 - f_t) Ip,   o_t = scale (M / I) q_t
 // (the naive recurrence, chunk_palimpsa_forgetting_scalar.py:712-717 of the reference; its associative scan over a
 // register tile, :190-207, is what the chunked kernel of the reference does instead).
@@ -17,9 +18,9 @@
 // so that the decay costs an addition per entry and token instead of two products and one addition, v / F and b / F once a
 // row; two entries share a reciprocal, n1/x1 + n2/x2 = (n1 x2 + n2 x1) / (x1 x2).  Against a float64 recurrence the outputs
 // are as exact as in plain form to three digits (bf16 rounding is all of the error); in fp32 the error of the outputs would
-// be up to 0.5 % larger and that of the uncertainty 15 %, so fp32 rows and the uncertainty keep the plain form.  A tile
-// takes it where every step decays by less than 2^48, and is worked again in plain form if a total is not finite
-// (precisions beyond 1e15 or so, or inputs that were not finite).  8 x 2048 tokens, 12 heads of 64x64 160 -> 148 us; 65536 of
+// be up to 0.5 % larger and that of the uncertainty 15 %, so fp32 rows and the uncertainty keep the plain form.  A walk
+// takes it where every step decays by less than 2^48, and is done again in plain form if a total is not finite
+// or a precision over F beyond 2^61 (then a product of two may have no reciprocal).  8 x 2048 tokens, 12 heads of 64x64 160 -> 148 us; 65536 of
 // 16 heads of 128x128 3060 -> 2870; 32768 of 16 of 96x96 945 -> 888.  (The issue rates below promise 22.6 -> 18.1 cycles; 26.1
 // of 27.9 are left: LDS reads of the operands 2.3, the totals over the lanes 2.  Four rows a lane halve both, but leave two
 // waves per SIMD: 193 us at 64x64.)
@@ -47,9 +48,9 @@
 
 namespace pal {
 
-// Least decay over a staging step for the scaled form: M / F stays far inside fp32, and so does a product of two precisions
-// up to 4e4 each.  Steps that decay more are rare (gates of 0.5 at a rate of 2: 2^-12) and gain least from it.
-constexpr float kMinDecay = 0x1p-48f;
+// Least decay over a staging step for the scaled form, and largest precision over F: the product of two of the latter still
+// has a reciprocal in fp32.  Steps that decay more are rare (gates of 0.5 at a rate of 2: 2^-12) and gain least from it.
+constexpr float kMinDecay = 0x1p-48f, kMaxScaled = 0x1p61f;
 constexpr int kOT = 8;   // tokens per staging step: two buffers of them let four workgroups of four waves share a unit's LDS
 
 template <int DD>
@@ -103,16 +104,26 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   const int STRIDE = oVB + 2 * VR;          // floats per staged token: f, c, -, -, k, k*k, q, (v, b) of every row
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int H = a.H, dk = a.dk, dv = a.dv;
-  const int cidx = (int)(blockIdx.x / H), h = (int)(blockIdx.x % H);
+  int cidx = (int)(blockIdx.x / H);
+  const int h = (int)(blockIdx.x % H);
   const int r0 = (int)blockIdx.y * VR;
   int seq, t0, clen, cis;
-  chunk_lookup(a, cidx, seq, t0, clen, cis);
-  float* sFC = smem;                        // [64][4] f_t (at the end of a step in scaled form: F), c_t, factor of v and b
-  int* sForm = (int*)(sFC + 4 * kC);        // whether the tile is worked in scaled form
-  float* sRow = sFC + 4 * kC + 4;               // [2][kOT][STRIDE]
+  if (a.every > 1) {   // batched sequences of one length, `every` tiles from one state
+    const int tiles = (a.T + kC - 1) / kC, per = (tiles + a.every - 1) / a.every;
+    seq = cidx / per;
+    cis = (cidx - seq * per) * a.every;
+    cidx = seq * tiles + cis;
+    t0 = seq * a.T + cis * kC;
+    clen = min(a.every * kC, a.T - cis * kC);
+  } else {
+    chunk_lookup(a, cidx, seq, t0, clen, cis);
+  }
+  float* sFC = smem;                        // [tokens][4] f_t (scaled form: F_t), c_t, factor of v and b, f_t
+  int* sForm = (int*)(sFC + 4 * kC * a.every);   // whether the tiles are worked in scaled form
+  float* sRow = sFC + 4 * kC * a.every + 4;               // [2][kOT][STRIDE]
   const float Ip = a.Ip[h];
   // every fetch of the set-up is issued before the first is used
-  const float gt = (w == 0 && lane < clen) ? load_gate(a.gt, (int64_t)(t0 + lane) * H + h, a.gate_bf16) : 0.f;
+  const float gt = 64 * w + lane < clen ? load_gate(a.gt, (int64_t)(t0 + 64 * w + lane) * H + h, a.gate_bf16) : 0.f;
   const float gh = a.g[h] * kLog2e;
   const TIn* kp = (const TIn*)a.k + qk_row(a, t0, h);
   const TIn* qp = (const TIn*)a.q + qk_row(a, t0, h);
@@ -143,7 +154,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   };
   auto deposit = [&](int s0, int buf) {
     float* base = sRow + buf * kOT * STRIDE;
-    if (tid < kOT) *(f32x2*)&base[tid * STRIDE] = *(const f32x2*)&sFC[4 * (s0 + tid)];   // s0 + tid < 64
+    if (tid < kOT) *(f32x2*)&base[tid * STRIDE] = *(const f32x2*)&sFC[4 * (s0 + tid)];   // (inside the last tile)
     if (s_kq < kOT && s0 + s_kq < clen) put_kq(base + s_kq * STRIDE, c_kq, rk, rq);
     if (s_vb < kOT && s0 + s_vb < clen) {
       float* p = &base[s_vb * STRIDE + oVB + 8 * c_vb];
@@ -170,10 +181,16 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   };
   const int64_t orow = ((int64_t)t0 * H + h) * dv + r0 + d0 + dsel;
 
-  const float f = fast_exp2(-gt * gh);
-  float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
+  // each wave: the decays of its tiles
   if (kMayScale) {
-    if (w == 0) {
+    if (tid == 0) *sForm = 1;
+    __syncthreads();
+  }
+  for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {
+    const float x = t == tid ? gt : t < clen ? load_gate(a.gt, (int64_t)(t0 + t) * H + h, a.gate_bf16) : 0.f;
+    const float f = fast_exp2(-x * gh);
+    float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
+    if (kMayScale) {
       const int s = lane & (kOT - 1);
       // (each shift before its select: a lane that is switched off hands nothing on)
       float y = dpp_shr<1>(F);
@@ -182,13 +199,14 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       F = s >= 2 ? F * y : F;
       y = dpp_shr<4>(F);
       F = s >= 4 ? F * y : F;
-      const bool ok = __all(F >= kMinDecay && F <= 1.f);
-      if (lane == 0) *sForm = ok;
+      if (!__all(F >= kMinDecay && F <= 1.f && Ip <= kMinDecay * kMaxScaled)) *sForm = 0;
     }
-    __syncthreads();
+    sFC[4 * t] = F;
+    sFC[4 * t + 3] = f;
   }
+  if (kMayScale) __syncthreads();
 
-  // The tile in scaled or plain form (see above); whether a total of the scaled form is not finite.
+  // The tiles in scaled or plain form (see above); whether the scaled form left its range.
   auto walk_tile = [&](auto form) -> bool {
     constexpr bool SCALED = decltype(form)::value;
     constexpr int NR = SCALED ? (DN + 1) / 2 : DN;   // reciprocals of a row and token
@@ -220,9 +238,9 @@ void chunk_out_kernel(ChunkArgs a, int W) {
         if constexpr (DN & 1) piece(std::integral_constant<int, 1>{}, DN - 1);
       }
     }
-    if (w == 0) {
-      const float inv = SCALED ? fast_rcp(F) : 1.f;
-      *(f32x4*)&sFC[4 * lane] = f32x4{SCALED ? F : f, SCALED ? Ip * inv : (1.f - f) * Ip, inv, 0.f};
+    for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {   // (the thread that left f and F there)
+      const float F = sFC[4 * t], f = sFC[4 * t + 3], inv = SCALED ? fast_rcp(F) : 1.f;
+      *(f32x4*)&sFC[4 * t] = f32x4{SCALED ? F : f, SCALED ? Ip * inv : (1.f - f) * Ip, inv, f};
     }
     // rows and columns beyond the head dims stay zero in both buffers
     if (DKP != dk || VR > dv - r0) {
@@ -233,6 +251,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
     __syncthreads();
 
     bool bad = false;
+    float big = 0.f;   // SCALED: the largest |I - Ip| / F
     OutRow<NG, DN, DD> x;
     for (int s0 = 0; s0 < clen; s0 += kOT) {
       const int buf = (s0 / kOT) & 1;
@@ -305,6 +324,12 @@ void chunk_out_kernel(ChunkArgs a, int W) {
           if (wr) store_rt(a.o_var, oo, outv * a.scale, a.var_bf16);
         }
       }
+      if constexpr (SCALED) {   // (b and Ip are not negative: a step's precisions over F are largest at its end)
+#pragma unroll
+        for (int i = 0; i < DN; ++i)
+#pragma unroll
+          for (int j = 0; j < DD; ++j) big = fmaxf(big, __builtin_fabsf(I[j][i]));
+      }
       if (SCALED && more) {
         const float Fe = sFC[4 * (s0 + kOT - 1)];
 #pragma unroll
@@ -315,7 +340,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       if (more) deposit(s0 + kOT, buf ^ 1);
       __syncthreads();
     }
-    return bad;
+    return bad || !(big <= kMaxScaled);
   };
   if constexpr (kMayScale) {
     if (*sForm && !__syncthreads_or(walk_tile(std::true_type{}))) return;
@@ -340,9 +365,10 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
   static_assert(ROWS <= 32, "one staging item of v, b per thread");
   const int nw = (a.dv + ROWS - 1) / ROWS;            // waves over the value rows
   const int W = out_waves(nw), slices = (nw + W - 1) / W;
-  const int64_t blocks = (int64_t)a.total_chunks * a.H;
+  const int64_t walks = a.every > 1 ? (int64_t)a.n_seqs * (((a.T + kC - 1) / kC + a.every - 1) / a.every) : a.total_chunks;
+  const int64_t blocks = walks * a.H;
   if (blocks > 0x7fffffff) return PAL_E_DIM;
-  const size_t lds = sizeof(float) * (4 * kC + 4 + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
+  const size_t lds = sizeof(float) * (4 * kC * a.every + 4 + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
   if (lds > kMaxLds) return PAL_E_HEADDIM;
   auto go = [&](auto kern) -> int {
     if (int rc = allow_lds((const void*)kern, lds)) return rc;
@@ -360,7 +386,7 @@ static int launch_out_dn(const ChunkArgs& a, hipStream_t s) {
   // Two value rows per lane where that still gives every SIMD two waves; below, one row: half the work per wave and
   // twice the waves (one sequence of 777 tokens, 16 heads of 64x64: 28 us with two rows, 23 with one; B=2 T=2048 H=12 64x64,
   // three waves per SIMD: 49.6 against 51.0).
-  const int64_t waves = (int64_t)a.total_chunks * a.H * ((a.dv * NG + 127) / 128);
+  const int64_t waves = (int64_t)a.total_chunks / a.every * a.H * ((a.dv * NG + 127) / 128);
   if (waves <= 2048) return launch_out_dd<TIn, NG, DN, 1>(a, s);
   return launch_out_dd<TIn, NG, DN, 2>(a, s);
 }
@@ -382,6 +408,21 @@ static int launch_out_t(const ChunkArgs& a, hipStream_t s) {
     case 15: case 16: return launch_out_dn<TIn, 32, 8>(a, s);
     default: return PAL_E_HEADDIM;
   }
+}
+
+// Tiles that a walk of the output kernel takes from one state, where nothing else reads the states between: as many, up to
+// four, as leave one and a half rounds of waves (four per SIMD, about 1024 state entries each).  What it saves is the state
+// pass's writes and this kernel's reads; what it costs is the serial length.  States and outputs together, in us, with 1, 2, 4
+// and 8 tiles to a state: 65536 tokens, 16 heads of 128x128 (65536 waves a window) 3925, 3663, 3524, 3534; 2 x 4096, 16 of
+// 128x128 (32768) 478, 424, 410, 424; 8 x 2048, 12 of 64x64 (12288) 182, 177, 188, 216; 4 x 2048, 6 of 96x192 (13824) 240,
+// 235, 263, 304; 16 x 512, 24 of 48x48 (6912) 137, 142, 159, 193.
+int out_tiles_per_state(const ChunkArgs& a) {
+  if (a.flags & PAL_FLAG_VARLEN) return 1;
+  const int64_t tiles = (a.T + kC - 1) / kC;
+  auto waves = [&](int every) {
+    return (int64_t)a.n_seqs * ((tiles + every - 1) / every) * a.H * ((int64_t)a.dk * a.dv) / 1024;
+  };
+  return waves(4) >= 6144 ? 4 : waves(2) >= 6144 ? 2 : 1;
 }
 
 int launch_out(const ChunkArgs& a, int dtype, hipStream_t s) {

@@ -18,7 +18,7 @@
 // 8 x 2048, 16 of 48 x 48 52.8 against 47.4; scalar-gated 2 x 2048, 16 of 128 x 128 46 against 24.)
 // The serial chain over the tiles is hidden by fetching ahead: rows are fetched into registers three steps before they
 // go to LDS, two LDS buffers hold the current and the next tile, one barrier per tile.
-// What bounds it with the precision state: writing mu and I (8 bytes an entry) beside reading rows that come from HBM, at
+// What bounds it with the precision state, where every tile's is kept: writing mu and I (8 bytes an entry) beside reading rows that come from HBM, at
 // 2.5 - 3.3 TB/s together; without the stores the walk takes half the time, and neither fetching further ahead (up to 10
 // tiles), whole 128-byte lines a store nor non-temporal stores gave more than 6 % at any shape without losing as much at
 // another.
@@ -265,6 +265,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     const bf16_t* kt = sK + buf * kbuf;
     const bf16_t* vt = sV + buf * vbuf;
     const bf16_t* bt = sB + buf * vbuf;
+    const bool kept = !HAS_J || (c & (a.every - 1)) == 0;
     // operands, the tokens as contraction index (g, j) -> 32 ks + 16 (j / 4) + 4 g + j % 4; those of the next block are read
     // while a block is worked
     struct Ops { bf16x8 k[2], v[2], b[2]; } x[2];
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
       __builtin_amdgcn_sched_barrier(0);
       const Ops& y = x[jj & 1];
       const int64_t off = slot + goff[jj];
-      if (sval[jj]) {
+      if (sval[jj] && kept) {
         if (HAS_J) {
           f32x4 mu, I;
 #pragma unroll

@@ -41,6 +41,9 @@ def _count_chunks(T: int, B: int) -> int:
 _WINDOW_STATE_BYTES = 512 << 20
 
 
+_SHORT_PASS = 1024   # tokens up to which pal_chunk_fwd may run a pass without gradients token by token
+
+
 def _window_tiles(H: int, dv: int, dk: int) -> int:
     return max(16, _WINDOW_STATE_BYTES // (2 * 4 * H * dv * dk))
 
@@ -67,6 +70,8 @@ def _windowed_forward(p, scale, output_uncertainty, o, o_var, final_mu, final_I,
             s, e = j * seg, min(T, (j + 1) * seg)
             out_mu, out_I = (final_mu, final_I) if (n_seg - 1 - j) % 2 == 0 else scratch
             flags = L.PAL_FLAG_STORE_FINAL | L.state_pass_flags()
+            if e - s > _SHORT_PASS:   # (a shorter one would take the token-serial kernel and round its state differently)
+                flags |= L.PAL_FLAG_OUTPUTS_ONLY
             if cur_mu is not None:
                 flags |= L.PAL_FLAG_HAS_INIT
             if output_uncertainty:
