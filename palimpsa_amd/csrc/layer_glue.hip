@@ -8,8 +8,8 @@
 //   epilogue (:355-363): y = rmsnorm over all heads of a token of ((o + x * D) * swish(gate)) * weight.
 // All of it is bound by HBM: every row is read once and written once.  A row of d elements is handled
 // by a group of GL lanes (the power of two >= d/8), eight consecutive elements per lane (16-byte
-// accesses for bf16 rows); a workgroup of 256 threads owns one head and a range of tokens, so that the
-// per-head sums of the backward are accumulated in a fixed order (no atomics).
+// accesses for bf16 rows); a workgroup of 256 threads owns a few neighbouring heads and a range of tokens, a row slot one
+// head, so that the per-head sums of the backward are accumulated in a fixed order (no atomics).
 #include <type_traits>
 
 #include "pal_common.h"
@@ -18,11 +18,13 @@
 
 namespace pal {
 
-constexpr int kGlueIter = 8;   // rows per row slot of a workgroup
+constexpr int kGlueIter = 4;   // rows per row slot of a workgroup (8: 64 x 64 shapes 2 - 4 us a kernel slower, 48 x 48 the same)
 // rows of a slot that are fetched before the first of them is used: a thread has one or two 16-byte fetches per row and
 // tensor, and taken one row at a time each fetch waits for the stores of the row before it (the kernels ran at
-// 3.3-3.7 TB/s that way).  Four rows in the forward kernels; two in the backward ones, which hold twice the tensors
-// per row (with four they need 200 registers and lose more to the occupancy than they gain).
+// 3.3-3.7 TB/s that way).  Rows are held as fetched (Row8) and converted when they are used: in fp32 they took twice the
+// registers, and the occupancy that costs (same sizes as below: prologue 49 -> 45 us, 4.4 TB/s, its backward 70 -> 58, 5.2,
+// epilogue 35 -> 23, 4.3, its backward 47 -> 35, 5.0).  Four rows in the forward kernels; two in the backward ones, which
+// hold twice the tensors per row (with four: 58 -> 62, 35 -> 40).
 constexpr int kGlueBatch = 4;
 constexpr int kGlueBatchBwd = 2;
 
@@ -40,6 +42,13 @@ __device__ __forceinline__ void store8(T* p, const float* x) {
 struct F32x8 {
   f32x4 lo, hi;
   __device__ __forceinline__ float operator[](int e) const { return e < 4 ? lo[e & 3] : hi[e & 3]; }
+};
+// eight elements as fetched, converted when they are used
+template <typename T>
+struct Row8 {
+  typename std::conditional<sizeof(T) == 2, bf16x8, F32x8>::type v;
+  __device__ __forceinline__ void load(const T* p) { v = *(const decltype(v)*)p; }
+  __device__ __forceinline__ float get(int e) const { return (float)v[e]; }
 };
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float x) {
@@ -69,62 +78,82 @@ __device__ __forceinline__ float softplusf_(float x) { return x > 20.f ? x : log
 template <typename T>
 __device__ __forceinline__ float round_to(float x) { return to_f32(from_f32<T>(x)); }
 
-struct GlueGeom {
-  int GLk, GLv;     // lanes per q/k row and per v row
-  int tok_per_block;
+// The rows of a pass, [tokens, H] of them GL lanes each: the row slots of a workgroup take `heads` neighbouring heads of
+// `tokens` consecutive tokens at a time, kGlueIter times.  As many heads as divide both H and the slots: neighbouring rows
+// share cache lines where a row is no multiple of a line, and a workgroup that takes one head reads and writes every line
+// in two parts (8 x 2048 tokens, 16 heads of 48 bf16, whose rows are 96 bytes: prologue 54 -> 49 us, its backward 78 -> 70,
+// epilogue 38 -> 35, its backward 56 -> 47; rows of whole lines gain nothing and lose nothing).
+struct RowGeom {
+  int GL, heads, tokens, groups;   // groups of `heads` heads
+  int64_t blocks;                  // workgroups: token ranges x groups, the groups of a range next to each other
+  __host__ __device__ int per_block() const { return tokens * kGlueIter; }
 };
-static GlueGeom glue_geom(const PalGlueDims* d) {
-  auto pow2 = [](int n) { int p = 1; while (p < n) p <<= 1; return p; };
-  GlueGeom g;
-  g.GLk = pow2(d->dk / 8);
-  g.GLv = pow2(d->dv / 8);
-  const int GLmax = g.GLk > g.GLv ? g.GLk : g.GLv;
-  g.tok_per_block = (256 / GLmax) * kGlueIter;
+static RowGeom row_geom(int d, int H, int tokens) {
+  RowGeom g;
+  g.GL = 1;
+  while (g.GL < d / 8) g.GL <<= 1;
+  const int slots = 256 / g.GL, pow2 = H & -H;
+  g.heads = pow2 < slots ? pow2 : slots;
+  g.tokens = slots / g.heads;
+  g.groups = H / g.heads;
+  g.blocks = ((int64_t)tokens + g.per_block() - 1) / g.per_block() * g.groups;
   return g;
 }
+// a thread's place: head, first token and end of its walk (steps of g.tokens), lane in the row, row slot, range of tokens
+struct RowAt {
+  int h, tok, end, l, slot, range;
+  __device__ RowAt(const RowGeom& g, int block, int tokens) {
+    range = block / g.groups;
+    slot = (int)threadIdx.x / g.GL;
+    l = (int)threadIdx.x % g.GL;
+    h = (block - range * g.groups) * g.heads + slot % g.heads;
+    const int t0 = range * g.per_block();
+    tok = t0 + slot / g.heads;
+    end = min(tokens, t0 + g.per_block());
+  }
+};
 
 // ------------------------------------------------------------------ prologue
 struct PrologueArgs {
   PalPrologueTensors t;
   PalPrologueGrads g;
-  float* part;          // backward: [H][n_token_blocks][2] partial sums (ddt_bias, db_scale)
-  int tokens, H, Hqk, dk, dv, GLk, GLv, tok_per_block;
+  float* part;          // backward: [H][token ranges][2] partial sums (ddt_bias, db_scale)
+  int tokens, H, Hqk, dk, dv;
+  RowGeom qk, vb;       // rows of q_raw, k_raw; rows of x, b_raw
   float eps;
   int mamba;            // the multiplier of x and b is gt itself, clamped to [dt_min, dt_max] (no bs_raw)
   int task0;            // first task of the grid's z axis (2 when there are no q, k rows)
   float dt_min, dt_max;
 };
 
-// grid (token blocks, heads, 3): z = 0 rows of q, z = 1 rows of k (heads of q_raw / k_raw), z = 2 rows of v, b and gt
+// grid (workgroups, 1, 3): z = 0 rows of q, z = 1 rows of k (heads of q_raw / k_raw), z = 2 rows of v, b and gt
 template <typename T>
 __global__ __launch_bounds__(256) void prologue_fwd_kernel(PrologueArgs A) {
-  const int tid = threadIdx.x, task = blockIdx.z + A.task0, h = blockIdx.y;
-  const int tok0 = blockIdx.x * A.tok_per_block;
-  const int tok1 = min(A.tokens, tok0 + A.tok_per_block);
+  const int task = blockIdx.z + A.task0;
+  const RowGeom& G = task < 2 ? A.qk : A.vb;
+  if (blockIdx.x >= G.blocks) return;
+  const RowAt at(G, blockIdx.x, A.tokens);
+  const int GL = G.GL, l = at.l, h = at.h, rows = G.tokens, tok1 = at.end;
   if (task < 2) {
-    if (h >= A.Hqk) return;
-    const int GL = A.GLk, d = A.dk, rep = A.H / A.Hqk;
-    const int slot = tid / GL, l = tid % GL, rows = 256 / GL;
+    const int d = A.dk, rep = A.H / A.Hqk;
     const T* src = (const T*)(task ? A.t.k_raw : A.t.q_raw);
     T* dst = (T*)(task ? A.t.k : A.t.q);
     const bool on = 8 * l < d;
-    for (int tb = tok0 + slot; tb < tok1; tb += kGlueBatch * rows) {
-      float xb[kGlueBatch][8];
+    const int lc = on ? 8 * l : 0;   // (lanes beyond the row, and rows beyond the range, fetch what exists)
+    for (int tb = at.tok; tb < tok1; tb += kGlueBatch * rows) {
+      Row8<T> xb[kGlueBatch];
+#pragma unroll
+      for (int u = 0; u < kGlueBatch; ++u) xb[u].load(src + ((int64_t)min(tb + u * rows, tok1 - 1) * A.Hqk + h) * d + lc);
 #pragma unroll
       for (int u = 0; u < kGlueBatch; ++u) {
         const int tok = tb + u * rows;
+        float x[8], ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xb[u][e] = 0.f;
-        if (on && tok < tok1) load8(src + ((int64_t)tok * A.Hqk + h) * d + 8 * l, xb[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kGlueBatch; ++u) {
-        const int tok = tb + u * rows;
-        float* x = xb[u];
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
-        ss = group_sum(ss, GL);
+        for (int e = 0; e < 8; ++e) {
+          x[e] = xb[u].get(e);
+          ss = fmaf(x[e], x[e], ss);
+        }
+        ss = group_sum(on ? ss : 0.f, GL);
         const float inv = rcpf_(fmaxf(__builtin_amdgcn_sqrtf(ss), A.eps));
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] *= inv;
@@ -133,50 +162,45 @@ __global__ __launch_bounds__(256) void prologue_fwd_kernel(PrologueArgs A) {
       }
     }
   } else {
-    const int GL = A.GLv, d = A.dv;
-    const int slot = tid / GL, l = tid % GL, rows = 256 / GL;
+    const int d = A.dv;
     const bool on = 8 * l < d;
+    const int lc = on ? 8 * l : 0;   // (lanes beyond the row, and rows beyond the range, fetch what exists)
     const float sp = A.t.b_raw ? softplusf_(A.t.b_scale[h]) : 0.f;
     const float bias = A.t.dt_bias[h];
     const bool has_b = A.t.b_raw != nullptr;
-    for (int tb = tok0 + slot; tb < tok1; tb += kGlueBatch * rows) {
-      float xb[kGlueBatch][8], bb[kGlueBatch][8], dtr[kGlueBatch], bsr[kGlueBatch];
+    for (int tb = at.tok; tb < tok1; tb += kGlueBatch * rows) {
+      Row8<T> xb[kGlueBatch], bb[kGlueBatch];
+      T dtr[kGlueBatch], bsr[kGlueBatch];
 #pragma unroll
       for (int u = 0; u < kGlueBatch; ++u) {
-        const int tok = tb + u * rows;
-        dtr[u] = bsr[u] = 0.f;
-        if (tok < tok1) {
-          const int64_t th = (int64_t)tok * A.H + h;
-          dtr[u] = to_f32(((const T*)A.t.dt_raw)[th]);
-          if (!A.mamba) bsr[u] = to_f32(((const T*)A.t.bs_raw)[th]);
-          if (on) {
-            load8((const T*)A.t.x + th * d + 8 * l, xb[u]);
-            if (has_b) load8((const T*)A.t.b_raw + th * d + 8 * l, bb[u]);
-          }
-        }
+        const int64_t th = (int64_t)min(tb + u * rows, tok1 - 1) * A.H + h;
+        dtr[u] = ((const T*)A.t.dt_raw)[th];
+        if (!A.mamba) bsr[u] = ((const T*)A.t.bs_raw)[th];
+        xb[u].load((const T*)A.t.x + th * d + lc);
+        if (has_b) bb[u].load((const T*)A.t.b_raw + th * d + lc);
       }
 #pragma unroll
       for (int u = 0; u < kGlueBatch; ++u) {
         const int tok = tb + u * rows;
         if (tok >= tok1) break;
         const int64_t th = (int64_t)tok * A.H + h;
-        float gtv = softplusf_(dtr[u] + bias), bs;
+        float gtv = softplusf_(to_f32(dtr[u]) + bias), bs;
         if (A.mamba) {
           gtv = fminf(fmaxf(gtv, A.dt_min), A.dt_max);
           bs = gtv;
         } else {
-          bs = round_to<T>(sigmoidf_(bsr[u]));
+          bs = round_to<T>(sigmoidf_(to_f32(bsr[u])));
         }
         if (l == 0) A.t.gt[th] = gtv;
         if (!on) continue;
-        float* x = xb[u];
+        float x[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] *= bs;
+        for (int e = 0; e < 8; ++e) x[e] = xb[u].get(e) * bs;
         store8((T*)A.t.v + th * d + 8 * l, x);
         if (has_b) {
-          float* br = bb[u];
+          float br[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) br[e] = sigmoidf_(br[e]) * sp * bs;
+          for (int e = 0; e < 8; ++e) br[e] = sigmoidf_(bb[u].get(e)) * sp * bs;
           store8((T*)A.t.b + th * d + 8 * l, br);
         }
       }
@@ -186,46 +210,50 @@ __global__ __launch_bounds__(256) void prologue_fwd_kernel(PrologueArgs A) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void prologue_bwd_kernel(PrologueArgs A) {
-  __shared__ float sRed[4][2];
-  const int tid = threadIdx.x, task = blockIdx.z + A.task0, h = blockIdx.y;
-  const int tok0 = blockIdx.x * A.tok_per_block;
-  const int tok1 = min(A.tokens, tok0 + A.tok_per_block);
+  __shared__ float sRed[256][2];
+  const int task = blockIdx.z + A.task0;
+  const RowGeom& G = task < 2 ? A.qk : A.vb;
+  if (blockIdx.x >= G.blocks) return;
+  const RowAt at(G, blockIdx.x, A.tokens);
+  const int GL = G.GL, l = at.l, h = at.h, rows = G.tokens, tok1 = at.end;
   if (task < 2) {
-    if (h >= A.Hqk) return;
     // y = x / n, n = max(|x|, eps):  dx = (s - y (y . s)) / n with s the sum of the gradients of the repeated heads
     // (for |x| < eps the norm is the constant eps and dx = s / eps)
-    const int GL = A.GLk, d = A.dk, rep = A.H / A.Hqk;
-    const int slot = tid / GL, l = tid % GL, rows = 256 / GL;
+    const int d = A.dk, rep = A.H / A.Hqk;
     const T* src = (const T*)(task ? A.t.k_raw : A.t.q_raw);
     const T* gsrc = (const T*)(task ? A.g.dk : A.g.dq);
     T* dst = (T*)(task ? A.g.dk_raw : A.g.dq_raw);
     const bool on = 8 * l < d;
-    for (int tb = tok0 + slot; tb < tok1; tb += kGlueBatchBwd * rows) {
-      float xb[kGlueBatchBwd][8], sb[kGlueBatchBwd][8];
+    const int lc = on ? 8 * l : 0;   // (lanes beyond the row, and rows beyond the range, fetch what exists)
+    for (int tb = at.tok; tb < tok1; tb += kGlueBatchBwd * rows) {
+      Row8<T> xb[kGlueBatchBwd], sb[kGlueBatchBwd], sb2[kGlueBatchBwd];   // x, gradients of the first two repeated heads
 #pragma unroll
       for (int u = 0; u < kGlueBatchBwd; ++u) {
-        const int tok = tb + u * rows;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xb[u][e] = sb[u][e] = 0.f;
-        if (on && tok < tok1) {
-          load8(src + ((int64_t)tok * A.Hqk + h) * d + 8 * l, xb[u]);
-          for (int r = 0; r < rep; ++r) {
-            float gy[8];
-            load8(gsrc + ((int64_t)tok * A.H + h * rep + r) * d + 8 * l, gy);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) sb[u][e] += gy[e];
-          }
-        }
+        const int64_t tok = min(tb + u * rows, tok1 - 1);
+        xb[u].load(src + (tok * A.Hqk + h) * d + lc);
+        sb[u].load(gsrc + (tok * A.H + h * rep) * d + lc);
+        if (rep > 1) sb2[u].load(gsrc + (tok * A.H + h * rep + 1) * d + lc);
       }
 #pragma unroll
       for (int u = 0; u < kGlueBatchBwd; ++u) {
         const int tok = tb + u * rows;
-        const float *x = xb[u], *s = sb[u];
-        float ss = 0.f, xs = 0.f;
+        float x[8], s[8], ss = 0.f, xs = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { x[e] = xb[u].get(e); s[e] = sb[u].get(e); }
+        if (rep > 1) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s[e] += sb2[u].get(e);
+          for (int r = 2; r < rep; ++r) {
+            float gy[8];
+            load8(gsrc + ((int64_t)min(tok, tok1 - 1) * A.H + h * rep + r) * d + lc, gy);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += gy[e];
+          }
+        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) { ss = fmaf(x[e], x[e], ss); xs = fmaf(x[e], s[e], xs); }
-        ss = group_sum(ss, GL);
-        xs = group_sum(xs, GL);
+        ss = group_sum(on ? ss : 0.f, GL);
+        xs = group_sum(on ? xs : 0.f, GL);
         const float nrm = __builtin_amdgcn_sqrtf(ss);
         const bool clamped = nrm < A.eps;
         const float inv = rcpf_(fmaxf(nrm, A.eps));
@@ -237,33 +265,28 @@ __global__ __launch_bounds__(256) void prologue_bwd_kernel(PrologueArgs A) {
       }
     }
   } else {
-    const int GL = A.GLv, d = A.dv;
-    const int slot = tid / GL, l = tid % GL, rows = 256 / GL;
+    const int d = A.dv;
     const bool on = 8 * l < d;
+    const int lc = on ? 8 * l : 0;   // (lanes beyond the row, and rows beyond the range, fetch what exists)
     const bool has_b = A.t.b_raw != nullptr;
     const float sp = has_b ? softplusf_(A.t.b_scale[h]) : 0.f;
     const float bias = A.t.dt_bias[h];
     float acc_dt = 0.f, acc_bs = 0.f;   // this thread's share of ddt_bias[h] and of sum db * sigmoid(b_raw) * bs
-    for (int tb = tok0 + slot; tb < tok1; tb += kGlueBatchBwd * rows) {
-      float xb[kGlueBatchBwd][8], gvb[kGlueBatchBwd][8], brb[kGlueBatchBwd][8], gbb[kGlueBatchBwd][8];
-      float dtr[kGlueBatchBwd], bsr[kGlueBatchBwd], dgr[kGlueBatchBwd];
+    for (int tb = at.tok; tb < tok1; tb += kGlueBatchBwd * rows) {
+      Row8<T> xb[kGlueBatchBwd], gvb[kGlueBatchBwd], brb[kGlueBatchBwd], gbb[kGlueBatchBwd];
+      T dtr[kGlueBatchBwd], bsr[kGlueBatchBwd];
+      float dgr[kGlueBatchBwd];
 #pragma unroll
       for (int u = 0; u < kGlueBatchBwd; ++u) {
-        const int tok = tb + u * rows;
-        dtr[u] = bsr[u] = dgr[u] = 0.f;
-        if (tok < tok1) {
-          const int64_t th = (int64_t)tok * A.H + h;
-          dtr[u] = to_f32(((const T*)A.t.dt_raw)[th]);
-          if (!A.mamba) bsr[u] = to_f32(((const T*)A.t.bs_raw)[th]);
-          if (l == 0) dgr[u] = A.g.dgt[th];
-          if (on) {
-            load8((const T*)A.t.x + th * d + 8 * l, xb[u]);
-            load8((const T*)A.g.dv + th * d + 8 * l, gvb[u]);
-            if (has_b) {
-              load8((const T*)A.t.b_raw + th * d + 8 * l, brb[u]);
-              load8((const T*)A.g.db + th * d + 8 * l, gbb[u]);
-            }
-          }
+        const int64_t th = (int64_t)min(tb + u * rows, tok1 - 1) * A.H + h;
+        dtr[u] = ((const T*)A.t.dt_raw)[th];
+        if (!A.mamba) bsr[u] = ((const T*)A.t.bs_raw)[th];
+        dgr[u] = A.g.dgt[th];
+        xb[u].load((const T*)A.t.x + th * d + lc);
+        gvb[u].load((const T*)A.g.dv + th * d + lc);
+        if (has_b) {
+          brb[u].load((const T*)A.t.b_raw + th * d + lc);
+          gbb[u].load((const T*)A.g.db + th * d + lc);
         }
       }
 #pragma unroll
@@ -271,7 +294,7 @@ __global__ __launch_bounds__(256) void prologue_bwd_kernel(PrologueArgs A) {
         const int tok = tb + u * rows;
         if (tok >= tok1) break;   // the lanes of a row leave together
         const int64_t th = (int64_t)tok * A.H + h;
-        const float pre = dtr[u] + bias;
+        const float pre = to_f32(dtr[u]) + bias;
         float sg = 0.f, bs;
         bool pass = true;     // mamba: the clamp lets the gradient through (bounds included, as torch.clamp)
         if (A.mamba) {
@@ -279,24 +302,26 @@ __global__ __launch_bounds__(256) void prologue_bwd_kernel(PrologueArgs A) {
           pass = spd >= A.dt_min && spd <= A.dt_max;
           bs = fminf(fmaxf(spd, A.dt_min), A.dt_max);
         } else {
-          sg = sigmoidf_(bsr[u]);
+          sg = sigmoidf_(to_f32(bsr[u]));
           bs = round_to<T>(sg);
         }
         float dbs = 0.f, dsp = 0.f;
         if (on) {
-          const float *x = xb[u], *gv = gvb[u];
           float dx[8];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) { dx[e] = gv[e] * bs; dbs = fmaf(gv[e], x[e], dbs); }
+          for (int e = 0; e < 8; ++e) {
+            const float gv = gvb[u].get(e);
+            dx[e] = gv * bs;
+            dbs = fmaf(gv, xb[u].get(e), dbs);
+          }
           store8((T*)A.g.dx + th * d + 8 * l, dx);
           if (has_b) {
-            const float *br = brb[u], *gb = gbb[u];
             float out[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-              const float s = sigmoidf_(br[e]);
-              out[e] = gb[e] * sp * bs * s * (1.f - s);
-              dsp = fmaf(gb[e], s, dsp);
+              const float s = sigmoidf_(brb[u].get(e)), gb = gbb[u].get(e);
+              out[e] = gb * sp * bs * s * (1.f - s);
+              dsp = fmaf(gb, s, dsp);
             }
             store8((T*)A.g.db_raw + th * d + 8 * l, out);
           }
@@ -317,30 +342,46 @@ __global__ __launch_bounds__(256) void prologue_bwd_kernel(PrologueArgs A) {
         acc_bs = fmaf(dsp, bs, acc_bs);
       }
     }
-    // workgroup totals in a fixed order: lanes, then waves
-    acc_dt = wave_sum(acc_dt);
-    acc_bs = wave_sum(acc_bs);
-    if ((tid & 63) == 0) { sRed[tid >> 6][0] = acc_dt; sRed[tid >> 6][1] = acc_bs; }
+    // totals of a head in a fixed order: the lanes of a row, then the head's row slots
+    acc_bs = group_sum(acc_bs, GL);
+    if (l == 0) { sRed[at.slot][0] = acc_dt; sRed[at.slot][1] = acc_bs; }
     __syncthreads();
-    if (tid == 0) {
-      float* p = A.part + ((int64_t)h * gridDim.x + blockIdx.x) * 2;
-      p[0] = sRed[0][0] + sRed[1][0] + sRed[2][0] + sRed[3][0];
-      p[1] = sRed[0][1] + sRed[1][1] + sRed[2][1] + sRed[3][1];
+    if ((int)threadIdx.x < 2 * G.heads) {
+      const int hs = threadIdx.x >> 1, which = threadIdx.x & 1;
+      float sum = 0.f;
+      for (int x = 0; x < G.tokens; ++x) sum += sRed[x * G.heads + hs][which];
+      const int64_t head = (blockIdx.x - at.range * G.groups) * G.heads + hs;
+      A.part[(head * (G.blocks / G.groups) + at.range) * 2 + which] = sum;
     }
   }
 }
 
+// The partial sums are added by 16 waves of a workgroup, each its share in order, then the waves' in order: the result does
+// not depend on timing.
+constexpr int kRedWaves = 16;
+__device__ __forceinline__ float reduce_block(float x, float* s /* [kRedWaves] */) {
+  x = wave_sum(x);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = x;
+  __syncthreads();
+  float t = s[0];
+#pragma unroll
+  for (int w = 1; w < kRedWaves; ++w) t += s[w];
+  return t;
+}
+
 // ddt_bias[h], db_scale[h] from the per-workgroup partial sums; db_scale picks up softplus'(b_scale) = sigmoid(b_scale)
-__global__ void prologue_bwd_reduce_kernel(PrologueArgs A, int n_blocks) {
-  const int h = blockIdx.x, lane = threadIdx.x;
+__global__ __launch_bounds__(64 * kRedWaves) void prologue_bwd_reduce_kernel(PrologueArgs A) {
+  __shared__ float sA[kRedWaves], sB[kRedWaves];
+  const int n_blocks = (int)(A.vb.blocks / A.vb.groups);
+  const int h = blockIdx.x;
   float a = 0.f, b = 0.f;
-  for (int j = lane; j < n_blocks; j += 64) {
+  for (int j = threadIdx.x; j < n_blocks; j += 64 * kRedWaves) {
     a += A.part[((int64_t)h * n_blocks + j) * 2];
     b += A.part[((int64_t)h * n_blocks + j) * 2 + 1];
   }
-  a = wave_sum(a);
-  b = wave_sum(b);
-  if (lane == 0) {
+  a = reduce_block(a, sA);
+  b = reduce_block(b, sB);
+  if (threadIdx.x == 0) {
     A.g.ddt_bias[h] = a;
     if (A.g.db_scale) A.g.db_scale[h] = A.t.b_raw ? b * sigmoidf_(A.t.b_scale[h]) : 0.f;
   }
@@ -350,51 +391,45 @@ __global__ void prologue_bwd_reduce_kernel(PrologueArgs A, int n_blocks) {
 struct EpilogueArgs {
   PalEpilogueTensors t;
   PalEpilogueGrads g;
-  float* part_w;        // backward: [H][n_token_blocks][dv] partial sums of dweight
-  float* part_D;        // backward: [H][n_token_blocks]
-  int tokens, H, dv, GL, tok_per_block;
+  float* part_w;        // backward: [workgroups][dv] partial sums of dweight
+  float* part_D;        // backward: [H][token ranges]
+  int tokens, H, dv;
+  int heads_iter;       // norm over all heads, backward: tokens per wave
+  RowGeom rows;
   float eps;
 };
 
 template <typename T>
 __global__ __launch_bounds__(256) void epilogue_fwd_kernel(EpilogueArgs A) {
-  const int tid = threadIdx.x, h = blockIdx.y;
-  const int tok0 = blockIdx.x * A.tok_per_block;
-  const int tok1 = min(A.tokens, tok0 + A.tok_per_block);
-  const int GL = A.GL, d = A.dv;
-  const int slot = tid / GL, l = tid % GL, rows = 256 / GL;
+  const RowAt at(A.rows, blockIdx.x, A.tokens);
+  const int GL = A.rows.GL, d = A.dv, l = at.l, h = at.h, rows = A.rows.tokens, tok1 = at.end;
   const bool on = 8 * l < d;
+  const int lc = on ? 8 * l : 0;   // (lanes beyond the row, and rows beyond the range, fetch what exists)
   const float Dh = A.t.x ? A.t.D[h] : 0.f;
   float w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (on) load8(A.t.weight + 8 * l, w);
   const float inv_d = 1.f / (float)d;
   const bool has_x = A.t.x != nullptr, has_gate = A.t.gate != nullptr;
-  for (int tb = tok0 + slot; tb < tok1; tb += kGlueBatch * rows) {
-    float rb[kGlueBatch][8], xb[kGlueBatch][8], gb[kGlueBatch][8];
+  for (int tb = at.tok; tb < tok1; tb += kGlueBatch * rows) {
+    Row8<T> rb[kGlueBatch], xb[kGlueBatch], gb[kGlueBatch];
 #pragma unroll
     for (int u = 0; u < kGlueBatch; ++u) {
-      const int tok = tb + u * rows;
-      const int64_t th = (int64_t)tok * A.H + h;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) rb[u][e] = xb[u][e] = gb[u][e] = 0.f;
-      if (on && tok < tok1) {
-        load8((const T*)A.t.o + th * d + 8 * l, rb[u]);
-        if (has_x) load8((const T*)A.t.x + th * d + 8 * l, xb[u]);
-        if (has_gate) load8((const T*)A.t.gate + th * d + 8 * l, gb[u]);
-      }
+      const int64_t th = (int64_t)min(tb + u * rows, tok1 - 1) * A.H + h;
+      rb[u].load((const T*)A.t.o + th * d + lc);
+      if (has_x) xb[u].load((const T*)A.t.x + th * d + lc);
+      if (has_gate) gb[u].load((const T*)A.t.gate + th * d + lc);
     }
 #pragma unroll
     for (int u = 0; u < kGlueBatch; ++u) {
       const int tok = tb + u * rows;
       if (tok >= tok1) break;   // the lanes of a row leave together
       const int64_t th = (int64_t)tok * A.H + h;
-      float* r = rb[u];
+      float r[8], ss = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[e] = fmaf(xb[u][e], Dh, r[e]);
-      float ss = 0.f;
+      for (int e = 0; e < 8; ++e) r[e] = has_x ? fmaf(xb[u].get(e), Dh, rb[u].get(e)) : rb[u].get(e);
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss = fmaf(r[e], r[e], ss);
-      ss = group_sum(ss, GL);
+      ss = group_sum(on ? ss : 0.f, GL);
       const float rstd = rsqrtf(ss * inv_d + A.eps);
       if (l == 0) A.t.rstd[th] = rstd;
       if (!on) continue;
@@ -403,7 +438,10 @@ __global__ __launch_bounds__(256) void epilogue_fwd_kernel(EpilogueArgs A) {
       for (int e = 0; e < 8; ++e) y[e] = r[e] * rstd * w[e];
       if (has_gate) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] *= gb[u][e] * sigmoidf_(gb[u][e]);
+        for (int e = 0; e < 8; ++e) {
+          const float z = gb[u].get(e);
+          y[e] *= z * sigmoidf_(z);
+        }
       }
       store8((T*)A.t.y + th * d + 8 * l, y);
     }
@@ -412,14 +450,12 @@ __global__ __launch_bounds__(256) void epilogue_fwd_kernel(EpilogueArgs A) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void epilogue_bwd_kernel(EpilogueArgs A) {
-  extern __shared__ float sW[];   // [rows][dv padded to 8 GL] dweight shares of the row slots
-  __shared__ float sRed[4];
-  const int tid = threadIdx.x, h = blockIdx.y;
-  const int tok0 = blockIdx.x * A.tok_per_block;
-  const int tok1 = min(A.tokens, tok0 + A.tok_per_block);
-  const int GL = A.GL, d = A.dv;
-  const int slot = tid / GL, l = tid % GL, rows = 256 / GL;
+  extern __shared__ float sW[];   // [row slots][dv padded to 8 GL] dweight shares of the row slots
+  __shared__ float sRed[256];
+  const RowAt at(A.rows, blockIdx.x, A.tokens);
+  const int GL = A.rows.GL, d = A.dv, l = at.l, h = at.h, rows = A.rows.tokens, tok1 = at.end;
   const bool on = 8 * l < d;
+  const int lc = on ? 8 * l : 0;   // (lanes beyond the row, and rows beyond the range, fetch what exists)
   const float Dh = A.t.x ? A.t.D[h] : 0.f;
   float w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (on) load8(A.t.weight + 8 * l, w);
@@ -427,40 +463,33 @@ __global__ __launch_bounds__(256) void epilogue_bwd_kernel(EpilogueArgs A) {
   float dw[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float accD = 0.f;
   const bool has_x = A.t.x != nullptr, has_gate = A.t.gate != nullptr;
-  for (int tb = tok0 + slot; tb < tok1; tb += kGlueBatchBwd * rows) {
-    float rb[kGlueBatchBwd][8], xb[kGlueBatchBwd][8], gyb[kGlueBatchBwd][8], gtb[kGlueBatchBwd][8], rsb[kGlueBatchBwd];
+  for (int tb = at.tok; tb < tok1; tb += kGlueBatchBwd * rows) {
+    Row8<T> rb[kGlueBatchBwd], xb[kGlueBatchBwd], gyb[kGlueBatchBwd], gtb[kGlueBatchBwd];
+    float rsb[kGlueBatchBwd];
 #pragma unroll
     for (int u = 0; u < kGlueBatchBwd; ++u) {
-      const int tok = tb + u * rows;
-      const int64_t th = (int64_t)tok * A.H + h;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) rb[u][e] = xb[u][e] = gyb[u][e] = gtb[u][e] = 0.f;
-      rsb[u] = 0.f;
-      if (tok < tok1) {
-        rsb[u] = A.t.rstd[th];
-        if (on) {
-          load8((const T*)A.t.o + th * d + 8 * l, rb[u]);
-          load8((const T*)A.g.dy + th * d + 8 * l, gyb[u]);
-          if (has_x) load8((const T*)A.t.x + th * d + 8 * l, xb[u]);
-          if (has_gate) load8((const T*)A.t.gate + th * d + 8 * l, gtb[u]);
-        }
-      }
+      const int64_t th = (int64_t)min(tb + u * rows, tok1 - 1) * A.H + h;
+      rsb[u] = A.t.rstd[th];
+      rb[u].load((const T*)A.t.o + th * d + lc);
+      gyb[u].load((const T*)A.g.dy + th * d + lc);
+      if (has_x) xb[u].load((const T*)A.t.x + th * d + lc);
+      if (has_gate) gtb[u].load((const T*)A.t.gate + th * d + lc);
     }
 #pragma unroll
     for (int u = 0; u < kGlueBatchBwd; ++u) {
       const int tok = tb + u * rows;
       if (tok >= tok1) break;   // the lanes of a row leave together
       const int64_t th = (int64_t)tok * A.H + h;
-      float* r = rb[u];
-      const float *x = xb[u], *gy = gyb[u];
-      float sw[8], dsw[8];   // swish(gate) and its derivative
+      float r[8], x[8], gy[8], sw[8], dsw[8];   // swish(gate) and its derivative
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        r[e] = fmaf(x[e], Dh, r[e]);
+        x[e] = has_x ? xb[u].get(e) : 0.f;
+        gy[e] = on ? gyb[u].get(e) : 0.f;
+        r[e] = fmaf(x[e], Dh, rb[u].get(e));
         sw[e] = 1.f;
         dsw[e] = 0.f;
         if (has_gate) {
-          const float z = gtb[u][e], s = sigmoidf_(z);
+          const float z = gtb[u].get(e), s = sigmoidf_(z);
           sw[e] = z * s;
           dsw[e] = s * (1.f + z * (1.f - s));
         }
@@ -498,95 +527,135 @@ __global__ __launch_bounds__(256) void epilogue_bwd_kernel(EpilogueArgs A) {
   // dweight: the row slots' shares are added in slot order
   const int dpad = 8 * GL;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) sW[slot * dpad + 8 * l + e] = dw[e];
-  accD = wave_sum(accD);
-  if ((tid & 63) == 0) sRed[tid >> 6] = accD;
+  for (int e = 0; e < 8; ++e) sW[at.slot * dpad + 8 * l + e] = dw[e];
+  accD = group_sum(accD, GL);
+  if (l == 0) sRed[at.slot] = accD;
   __syncthreads();
-  const int64_t blk = (int64_t)h * gridDim.x + blockIdx.x;
-  for (int c = tid; c < d; c += 256) {
+  for (int c = threadIdx.x; c < d; c += 256) {
     float s = 0.f;
-    for (int r = 0; r < rows; ++r) s += sW[r * dpad + c];
-    A.part_w[blk * d + c] = s;
+    for (int r = 0; r < 256 / GL; ++r) s += sW[r * dpad + c];
+    A.part_w[(int64_t)blockIdx.x * d + c] = s;
   }
-  if (tid == 0 && A.t.x) A.part_D[blk] = sRed[0] + sRed[1] + sRed[2] + sRed[3];
+  const int hs = threadIdx.x;
+  if (hs < A.rows.heads && A.t.x) {   // a head's row slots in order
+    float s = 0.f;
+    for (int x = 0; x < rows; ++x) s += sRed[x * A.rows.heads + hs];
+    const int64_t head = (blockIdx.x - at.range * A.rows.groups) * A.rows.heads + hs;
+    A.part_D[head * (A.rows.blocks / A.rows.groups) + at.range] = s;
+  }
 }
 
-// dweight[c] = sum over heads and token blocks; dD[h] = sum over token blocks (fixed order)
-__global__ void epilogue_bwd_reduce_kernel(EpilogueArgs A, int n_blocks) {
-  const int lane = threadIdx.x;
+// dweight[c] = sum over the workgroups; dD[h] = sum over the token ranges (fixed order)
+__global__ __launch_bounds__(64 * kRedWaves) void epilogue_bwd_reduce_kernel(EpilogueArgs A) {
+  __shared__ float sRed[kRedWaves];
+  const int n_blocks = (int)(A.rows.blocks / A.rows.groups);
   if ((int)blockIdx.x < A.dv) {
     const int c = blockIdx.x;
     float s = 0.f;
-    for (int64_t j = lane; j < (int64_t)A.H * n_blocks; j += 64) s += A.part_w[j * A.dv + c];
-    s = wave_sum(s);
-    if (lane == 0) A.g.dweight[c] = s;
+    for (int64_t j = threadIdx.x; j < A.rows.blocks; j += 64 * kRedWaves) s += A.part_w[j * A.dv + c];
+    s = reduce_block(s, sRed);
+    if (threadIdx.x == 0) A.g.dweight[c] = s;
   } else if (A.t.x) {
     const int h = blockIdx.x - A.dv;
     float s = 0.f;
-    for (int j = lane; j < n_blocks; j += 64) s += A.part_D[(int64_t)h * n_blocks + j];
-    s = wave_sum(s);
-    if (lane == 0) A.g.dD[h] = s;
+    for (int j = threadIdx.x; j < n_blocks; j += 64 * kRedWaves) s += A.part_D[(int64_t)h * n_blocks + j];
+    s = reduce_block(s, sRed);
+    if (threadIdx.x == 0) A.g.dD[h] = s;
   }
 }
 
 // ------------------------------------------------------------------ epilogue over all heads of a token
 // y = rmsnorm_{H dv}((o + x D) swish(gate)) weight  (palimpsa/layers/meta_mamba2.py:355-363: the gate is applied before
 // a norm that runs over the whole token).  One wave per token, 512 elements per pass (eight per lane, inside one head
-// since dv is a multiple of 8); a wave takes kHeadsIter tokens in turn and the four waves of a workgroup add their sums
-// over tokens (dweight, dD of the backward) in LDS, so that a workgroup leaves one partial row per 16 tokens.
-constexpr int kHeadsIter = 4;      // tokens per wave (a workgroup of four waves takes 16)
+// since dv is a multiple of 8); a wave of the backward takes up to four tokens in turn and the four waves of a
+// workgroup add their sums over tokens (dweight, dD) in LDS, so that a workgroup leaves one partial row per 4 to 16 tokens.
+// Tokens per wave of the backward kernel: few tokens are spread over more waves, many leave fewer partial rows (16 heads of
+// 96, in us, with one, two and four: 1024 tokens 12, 16, 24, 6124 tokens 32, 31, 33; 16384 tokens of 16 heads of 128, the
+// sums over the partial rows included, 205, 184, 165).
+static int heads_iter(int tokens) {
+  const int n = (tokens + 3072) / 4096;
+  return n < 1 ? 1 : n > 4 ? 4 : n;
+}
 constexpr int kHeadsMaxCh = 8;     // passes of 512 elements: H dv <= 4096
 
-template <typename T>
+// NCH as in the backward kernel below: every fetch of the token is in flight before the first is used.  One token per wave, as
+// nothing is summed over tokens (4 x 1531 tokens, 16 heads of 96: four tokens in turn, fetched a pass at a time, 31 us, so 17.5).
+template <typename T, int NCH>
 __global__ __launch_bounds__(256) void epilogue_heads_fwd_kernel(EpilogueArgs A) {
+  constexpr bool KEEP = NCH > 0;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int dv = A.dv, HD = A.H * dv, nch = (HD + 511) >> 9;
+  const int dv = A.dv, HD = A.H * dv, nch = KEEP ? NCH : (HD + 511) >> 9;
   const float inv_n = 1.f / (float)HD;
-  for (int it = 0; it < kHeadsIter; ++it) {
-    const int tok = ((int)blockIdx.x * 4 + w) * kHeadsIter + it;
-    if (tok >= A.tokens) break;
-    const int64_t row = (int64_t)tok * HD;
-    float r[kHeadsMaxCh][8];
-    float ss = 0.f;
+  const int64_t tok = (int64_t)blockIdx.x * 4 + w;
+  if (tok >= A.tokens) return;
+  const bool has_x = A.t.x != nullptr, has_gate = A.t.gate != nullptr;
+  const int64_t row = tok * HD;
+  constexpr int N = KEEP ? NCH : kHeadsMaxCh;
+  Row8<T> o[KEEP ? N : 1], x[KEEP ? N : 1], z[KEEP ? N : 1];
+  auto fetch = [&](int c, int e0) {
+    const int k = KEEP ? c : 0;
+    o[k].load((const T*)A.t.o + row + e0);
+    if (has_x) x[k].load((const T*)A.t.x + row + e0);
+    if (has_gate) z[k].load((const T*)A.t.gate + row + e0);
+  };
+  if constexpr (KEEP) {
 #pragma unroll
-    for (int c = 0; c < kHeadsMaxCh; ++c) {
+    for (int c = 0; c < N; ++c) {
       const int e0 = 512 * c + 8 * lane;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) r[c][e] = 0.f;
-      if (c < nch && e0 < HD) {
-        load8((const T*)A.t.o + row + e0, r[c]);
-        if (A.t.x) {
-          float x[8];
-          load8((const T*)A.t.x + row + e0, x);
-          const float Dh = A.t.D[e0 / dv];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) r[c][e] = fmaf(x[e], Dh, r[c][e]);
-        }
-        if (A.t.gate) {
-          float z[8];
-          load8((const T*)A.t.gate + row + e0, z);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) r[c][e] *= z[e] * sigmoidf_(z[e]);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss = fmaf(r[c][e], r[c][e], ss);
-      }
+      if (e0 < HD) fetch(c, e0);
     }
-    ss = wave_sum(ss);
-    const float rstd = rsqrtf(ss * inv_n + A.eps);
-    if (lane == 0) A.t.rstd[tok] = rstd;
+  }
+  float r[N][8];
+  float ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < kHeadsMaxCh; ++c) {
-      const int e0 = 512 * c + 8 * lane;
-      if (c < nch && e0 < HD) {
-        float wv[8], y[8];
-        load8(A.t.weight + e0, wv);
+  for (int c = 0; c < N; ++c) {
+    const int e0 = 512 * c + 8 * lane;
+    if (c < nch && e0 < HD) {
+      if constexpr (!KEEP) fetch(c, e0);
+      const int k = KEEP ? c : 0;
+      const float Dh = has_x ? A.t.D[e0 / dv] : 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] = r[c][e] * rstd * wv[e];
-        store8((T*)A.t.y + row + e0, y);
+      for (int e = 0; e < 8; ++e) {
+        float y = o[k].get(e);
+        if (has_x) y = fmaf(x[k].get(e), Dh, y);
+        if (has_gate) {
+          const float g = z[k].get(e);
+          y *= g * sigmoidf_(g);
+        }
+        ss = fmaf(y, y, ss);
+        r[c][e] = y;
       }
     }
   }
+  ss = wave_sum(ss);
+  const float rstd = rsqrtf(ss * inv_n + A.eps);
+  if (lane == 0) A.t.rstd[tok] = rstd;
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    const int e0 = 512 * c + 8 * lane;
+    if (c < nch && e0 < HD) {
+      float wv[8], y[8];
+      load8(A.t.weight + e0, wv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = r[c][e] * rstd * wv[e];
+      store8((T*)A.t.y + row + e0, y);
+    }
+  }
+}
+template <typename T>
+static void launch_heads_fwd(const EpilogueArgs& A, hipStream_t s) {
+  const int nch = (A.H * A.dv + 511) / 512;
+  const dim3 grid((unsigned)((A.tokens + 3) / 4));
+  auto go = [&](auto kern) { PAL_TIMED_LAUNCH(kKernEpilogueFwd, s, kern, grid, dim3(256), 0, s, A); };
+  if constexpr (sizeof(T) == 2) {
+    switch (nch) {
+      case 1: return go(&epilogue_heads_fwd_kernel<T, 1>);
+      case 2: return go(&epilogue_heads_fwd_kernel<T, 2>);
+      case 3: return go(&epilogue_heads_fwd_kernel<T, 3>);
+      case 4: return go(&epilogue_heads_fwd_kernel<T, 4>);
+    }
+  }
+  go(&epilogue_heads_fwd_kernel<T, 0>);
 }
 
 // r = u s, u = o + x D, s = swish(gate);  n = r rstd;  y = n w;  g = dy w;  dr = rstd (g - n mean(g n));
@@ -620,8 +689,8 @@ void epilogue_heads_bwd_kernel(EpilogueArgs A) {
     if (has_x) R.x = *(const Raw*)((const T*)A.t.x + off);
     if (has_gate) R.z = *(const Raw*)((const T*)A.t.gate + off);
   };
-  for (int it = 0; it < kHeadsIter; ++it) {
-    const int tok = (int)wave_id * kHeadsIter + it;
+  for (int it = 0; it < A.heads_iter; ++it) {
+    const int tok = (int)wave_id * A.heads_iter + it;
     if (tok >= A.tokens) break;
     const int64_t row = (int64_t)tok * HD;
     const float rstd = A.t.rstd[tok];
@@ -742,7 +811,6 @@ static int launch_heads_bwd_nch(int nch, const EpilogueArgs& A, int nblk, size_t
 // the backward kernel.  16 waves per block: wave w adds the rows j = w (mod 16) in order, four loads in flight, and
 // the waves' sums are added in order, so the result does not depend on timing (one wave per block walked the rows
 // alone before: 0.24 ms at 1024 partial rows).
-constexpr int kRedWaves = 16;
 __global__ __launch_bounds__(64 * kRedWaves) void epilogue_heads_reduce_kernel(EpilogueArgs A, int n_waves /* partial rows */) {
   __shared__ float sPart[kRedWaves][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -788,7 +856,7 @@ __global__ __launch_bounds__(64 * kRedWaves) void epilogue_heads_reduce_kernel(E
   }
 }
 
-static int heads_waves(const PalGlueDims* d) { return (d->tokens + kHeadsIter - 1) / kHeadsIter; }
+static int heads_waves(const PalGlueDims* d) { return (d->tokens + heads_iter(d->tokens) - 1) / heads_iter(d->tokens); }
 
 static int check_glue_dims(const PalGlueDims* d) {
   if (!d) return PAL_E_NULL;
@@ -819,15 +887,20 @@ static int check_prologue(const PalGlueDims* d, const PalPrologueTensors* t) {
 }
 
 static void fill_prologue(PrologueArgs& A, const PalGlueDims* d, const PalPrologueTensors* t) {
-  const GlueGeom g = glue_geom(d);
   A.t = *t;
   A.tokens = d->tokens; A.H = d->n_heads; A.Hqk = d->n_qk_heads; A.dk = d->dk; A.dv = d->dv;
-  A.GLk = g.GLk; A.GLv = g.GLv; A.tok_per_block = g.tok_per_block;
+  A.qk = row_geom(d->dk, d->n_qk_heads, d->tokens);
+  A.vb = row_geom(d->dv, d->n_heads, d->tokens);
   A.eps = d->eps;
   A.part = nullptr;
   A.mamba = t->bs_raw == nullptr;
   A.task0 = t->q_raw ? 0 : 2;
   A.dt_min = d->dt_min; A.dt_max = d->dt_max;
+}
+
+static dim3 prologue_grid(const PrologueArgs& A) {
+  const int64_t n = A.task0 ? 0 : A.qk.blocks;
+  return dim3((unsigned)(n > A.vb.blocks ? n : A.vb.blocks), 1, 3 - A.task0);
 }
 
 static int check_epilogue(const PalGlueDims* d, const PalEpilogueTensors* t) {
@@ -842,10 +915,10 @@ static int check_epilogue(const PalGlueDims* d, const PalEpilogueTensors* t) {
 }
 
 static void fill_epilogue(EpilogueArgs& A, const PalGlueDims* d, const PalEpilogueTensors* t) {
-  const GlueGeom g = glue_geom(d);
   A.t = *t;
   A.tokens = d->tokens; A.H = d->n_heads; A.dv = d->dv;
-  A.GL = g.GLv; A.tok_per_block = (256 / g.GLv) * kGlueIter;
+  A.rows = row_geom(d->dv, d->n_heads, d->tokens);
+  A.heads_iter = heads_iter(d->tokens);
   A.eps = d->eps;
   A.part_w = nullptr; A.part_D = nullptr;
 }
@@ -860,7 +933,7 @@ extern "C" int pal_prologue_fwd(const PalGlueDims* d, const PalPrologueTensors* 
   PrologueArgs A{};
   fill_prologue(A, d, t);
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((d->tokens + A.tok_per_block - 1) / A.tok_per_block, d->n_heads, 3 - A.task0);
+  const dim3 grid = prologue_grid(A);
   if (d->dtype == PAL_DTYPE_BF16) PAL_TIMED_LAUNCH(kKernPrologueFwd, s, prologue_fwd_kernel<bf16_t>, grid, dim3(256), 0, s, A);
   else PAL_TIMED_LAUNCH(kKernPrologueFwd, s, prologue_fwd_kernel<float>, grid, dim3(256), 0, s, A);
   PAL_HIP_LAUNCH_CHECK();
@@ -870,9 +943,8 @@ extern "C" int pal_prologue_fwd(const PalGlueDims* d, const PalPrologueTensors* 
 extern "C" size_t pal_prologue_bwd_workspace_bytes(const PalGlueDims* d) {
   using namespace pal;
   if (check_glue_dims(d) != PAL_OK) return 0;
-  const GlueGeom g = glue_geom(d);
-  const size_t nb = (d->tokens + g.tok_per_block - 1) / g.tok_per_block;
-  return up256(sizeof(float) * 2 * nb * d->n_heads);
+  const RowGeom g = row_geom(d->dv, d->n_heads, d->tokens);
+  return up256(sizeof(float) * 2 * (size_t)(g.blocks / g.groups) * d->n_heads);
 }
 
 extern "C" int pal_prologue_bwd(const PalGlueDims* d, const PalPrologueTensors* t, const PalPrologueGrads* gr,
@@ -893,12 +965,11 @@ extern "C" int pal_prologue_bwd(const PalGlueDims* d, const PalPrologueTensors* 
   A.g = *gr;
   A.part = (float*)workspace;
   hipStream_t s = (hipStream_t)stream;
-  const int nb = (d->tokens + A.tok_per_block - 1) / A.tok_per_block;
-  const dim3 grid(nb, d->n_heads, 3 - A.task0);
+  const dim3 grid = prologue_grid(A);
   if (d->dtype == PAL_DTYPE_BF16) PAL_TIMED_LAUNCH(kKernPrologueBwd, s, prologue_bwd_kernel<bf16_t>, grid, dim3(256), 0, s, A);
   else PAL_TIMED_LAUNCH(kKernPrologueBwd, s, prologue_bwd_kernel<float>, grid, dim3(256), 0, s, A);
   PAL_HIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(prologue_bwd_reduce_kernel, dim3(d->n_heads), dim3(64), 0, s, A, nb);
+  hipLaunchKernelGGL(prologue_bwd_reduce_kernel, dim3(d->n_heads), dim3(64 * kRedWaves), 0, s, A);
   PAL_HIP_LAUNCH_CHECK();
   return PAL_OK;
 }
@@ -910,13 +981,12 @@ extern "C" int pal_epilogue_fwd(const PalGlueDims* d, const PalEpilogueTensors* 
   fill_epilogue(A, d, t);
   hipStream_t s = (hipStream_t)stream;
   if (d->norm_over_heads) {
-    const dim3 hgrid((heads_waves(d) + 3) / 4);
-    if (d->dtype == PAL_DTYPE_BF16) PAL_TIMED_LAUNCH(kKernEpilogueFwd, s, epilogue_heads_fwd_kernel<bf16_t>, hgrid, dim3(256), 0, s, A);
-    else PAL_TIMED_LAUNCH(kKernEpilogueFwd, s, epilogue_heads_fwd_kernel<float>, hgrid, dim3(256), 0, s, A);
+    if (d->dtype == PAL_DTYPE_BF16) launch_heads_fwd<bf16_t>(A, s);
+    else launch_heads_fwd<float>(A, s);
     PAL_HIP_LAUNCH_CHECK();
     return PAL_OK;
   }
-  const dim3 grid((d->tokens + A.tok_per_block - 1) / A.tok_per_block, d->n_heads);
+  const dim3 grid((unsigned)A.rows.blocks);
   if (d->dtype == PAL_DTYPE_BF16) PAL_TIMED_LAUNCH(kKernEpilogueFwd, s, epilogue_fwd_kernel<bf16_t>, grid, dim3(256), 0, s, A);
   else PAL_TIMED_LAUNCH(kKernEpilogueFwd, s, epilogue_fwd_kernel<float>, grid, dim3(256), 0, s, A);
   PAL_HIP_LAUNCH_CHECK();
@@ -930,10 +1000,8 @@ extern "C" size_t pal_epilogue_bwd_workspace_bytes(const PalGlueDims* d) {
     const size_t HD = (size_t)d->n_heads * d->dv, nblk = (size_t)((heads_waves(d) + 3) / 4);
     return up256(sizeof(float) * nblk * HD) + up256(sizeof(float) * nblk * (HD / 8));
   }
-  const GlueGeom g = glue_geom(d);
-  const int tpb = (256 / g.GLv) * kGlueIter;
-  const size_t nb = (d->tokens + tpb - 1) / tpb;
-  return up256(sizeof(float) * nb * d->n_heads * d->dv) + up256(sizeof(float) * nb * d->n_heads);
+  const RowGeom g = row_geom(d->dv, d->n_heads, d->tokens);
+  return up256(sizeof(float) * (size_t)g.blocks * d->dv) + up256(sizeof(float) * (size_t)(g.blocks / g.groups) * d->n_heads);
 }
 
 extern "C" int pal_epilogue_bwd(const PalGlueDims* d, const PalEpilogueTensors* t, const PalEpilogueGrads* gr,
@@ -967,16 +1035,15 @@ extern "C" int pal_epilogue_bwd(const PalGlueDims* d, const PalEpilogueTensors* 
     PAL_HIP_LAUNCH_CHECK();
     return PAL_OK;
   }
-  const int nb = (d->tokens + A.tok_per_block - 1) / A.tok_per_block;
   A.part_w = (float*)workspace;
-  A.part_D = (float*)((char*)workspace + up256(sizeof(float) * (size_t)nb * d->n_heads * d->dv));
+  A.part_D = (float*)((char*)workspace + up256(sizeof(float) * (size_t)A.rows.blocks * d->dv));
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(nb, d->n_heads);
-  const size_t lds = sizeof(float) * (256 / A.GL) * 8 * A.GL;   // = 8 KB
+  const dim3 grid((unsigned)A.rows.blocks);
+  const size_t lds = sizeof(float) * 256 * 8;
   if (d->dtype == PAL_DTYPE_BF16) PAL_TIMED_LAUNCH(kKernEpilogueBwd, s, epilogue_bwd_kernel<bf16_t>, grid, dim3(256), lds, s, A);
   else PAL_TIMED_LAUNCH(kKernEpilogueBwd, s, epilogue_bwd_kernel<float>, grid, dim3(256), lds, s, A);
   PAL_HIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(epilogue_bwd_reduce_kernel, dim3(d->dv + d->n_heads), dim3(64), 0, s, A, nb);
+  hipLaunchKernelGGL(epilogue_bwd_reduce_kernel, dim3(d->dv + d->n_heads), dim3(64 * kRedWaves), 0, s, A);
   PAL_HIP_LAUNCH_CHECK();
   return PAL_OK;
 }

@@ -382,3 +382,23 @@ def test_mamba_layer_slice_end_to_end(gpu_device):
     for n in vals:
         err = hp.max_rel(lv[n].grad, rl[n].grad)
         assert err <= hp.BF16_GRAD_NORM_TOL, (n, err)
+
+
+# ------------------------------------------------------------------ how rows are dealt out
+@pytest.mark.parametrize("lead,Hqk,H,dk,dv", [
+    ((1,), 16, 16, 48, 48),       # one token: most row slots are empty
+    ((9,), 16, 16, 48, 48),       # a workgroup's tokens and one more
+    ((300,), 24, 24, 48, 96),     # groups of eight heads, rows of two widths
+    ((3, 41), 4, 16, 64, 64),     # q, k of four heads each: the third and fourth gradient are fetched late
+    ((77,), 5, 40, 16, 16),       # an odd number of q, k heads beside groups of eight
+    ((130,), 64, 64, 8, 16),      # more heads than row slots
+])
+def test_rows_over_heads_and_tokens(gpu_device, lead, Hqk, H, dk, dv):
+    test_prologue_forward_backward(gpu_device, lead, Hqk, H, dk, dv, torch.bfloat16, True)
+    test_epilogue_forward_backward(gpu_device, lead, H, dv, torch.bfloat16, True, True)
+
+
+@pytest.mark.parametrize("tokens", [1, 4097, 5121, 13315])       # one, one, two and four tokens per wave, a ragged end
+def test_mamba_epilogue_tokens_per_wave(gpu_device, tokens):
+    test_mamba_epilogue_forward_backward(gpu_device, (tokens,), 2, 16, torch.float32, True, True)
+    test_mamba_epilogue_forward_backward(gpu_device, (tokens,), 4, 152, torch.bfloat16, True, True)
