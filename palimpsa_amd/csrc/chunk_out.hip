@@ -158,7 +158,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
     if (s_kq < kOT && s0 + s_kq < clen) put_kq(base + s_kq * STRIDE, c_kq, rk, rq);
     if (s_vb < kOT && s0 + s_vb < clen) {
       float* p = &base[s_vb * STRIDE + oVB + 8 * c_vb];
-      const float u = sFC[4 * (s0 + s_vb) + 2];
+      const float u = kMayScale ? sFC[4 * (s0 + s_vb) + 2] : 1.f;
       *(f32x4*)p = f32x4{u * (float)rv[0], u * (float)rb[0], u * (float)rv[1], u * (float)rb[1]};
       *(f32x4*)(p + 4) = f32x4{u * (float)rv[2], u * (float)rb[2], u * (float)rv[3], u * (float)rb[3]};
     }
@@ -181,16 +181,16 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   };
   const int64_t orow = ((int64_t)t0 * H + h) * dv + r0 + d0 + dsel;
 
-  // each wave: the decays of its tiles
-  if (kMayScale) {
+  auto decay_of = [&](int t) {
+    const float x = t == tid ? gt : t < clen ? load_gate(a.gt, (int64_t)(t0 + t) * H + h, a.gate_bf16) : 0.f;
+    return fast_exp2(-x * gh);
+  };
+  if constexpr (kMayScale) {   // each wave: the decays of its tiles
     if (tid == 0) *sForm = 1;
     __syncthreads();
-  }
-  for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {
-    const float x = t == tid ? gt : t < clen ? load_gate(a.gt, (int64_t)(t0 + t) * H + h, a.gate_bf16) : 0.f;
-    const float f = fast_exp2(-x * gh);
-    float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
-    if (kMayScale) {
+    for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {
+      const float f = decay_of(t);
+      float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
       const int s = lane & (kOT - 1);
       // (each shift before its select: a lane that is switched off hands nothing on)
       float y = dpp_shr<1>(F);
@@ -200,11 +200,11 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       y = dpp_shr<4>(F);
       F = s >= 4 ? F * y : F;
       if (!__all(F >= kMinDecay && F <= 1.f && Ip <= kMinDecay * kMaxScaled)) *sForm = 0;
+      sFC[4 * t] = F;
+      sFC[4 * t + 3] = f;
     }
-    sFC[4 * t] = F;
-    sFC[4 * t + 3] = f;
+    __syncthreads();
   }
-  if (kMayScale) __syncthreads();
 
   // The tiles in scaled or plain form (see above); whether the scaled form left its range.
   auto walk_tile = [&](auto form) -> bool {
@@ -239,8 +239,8 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       }
     }
     for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {   // (the thread that left f and F there)
-      const float F = sFC[4 * t], f = sFC[4 * t + 3], inv = SCALED ? fast_rcp(F) : 1.f;
-      *(f32x4*)&sFC[4 * t] = f32x4{SCALED ? F : f, SCALED ? Ip * inv : (1.f - f) * Ip, inv, f};
+      const float f = kMayScale ? sFC[4 * t + 3] : decay_of(t), F = SCALED ? sFC[4 * t] : f, inv = SCALED ? fast_rcp(F) : 1.f;
+      *(f32x4*)&sFC[4 * t] = f32x4{F, SCALED ? Ip * inv : (1.f - f) * Ip, inv, f};
     }
     // rows and columns beyond the head dims stay zero in both buffers
     if (DKP != dk || VR > dv - r0) {
