@@ -145,7 +145,8 @@ __global__ __launch_bounds__(256, 2) void chunk_bwd_carry_apply_kernel(BwdArgs A
   bf16_t* sRTl = sRT + 2 * dk * RS;        // PREC: [2][dk][dv + 8] lo halves
   const int OS = dmax + 4;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = lane & 15, g = lane >> 4;
-  const int cidx = blockIdx.x / H, h = blockIdx.x % H;
+  int cidx, h;
+  if (!tile_head(a.total_chunks, H, blockIdx.x, cidx, h)) return;
   int seq, t0, clen, cis;
   chunk_lookup(a, cidx, seq, t0, clen, cis);
   int bos, len, cbase;
@@ -814,7 +815,7 @@ extern "C" int pal_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const Pal
     PAL_HIP_LAUNCH_CHECK();
   }
   {
-    const unsigned blocks = (unsigned)((int64_t)dd.total_chunks * dd.n_heads);
+    const unsigned blocks = (unsigned)tile_head_blocks(dd.total_chunks, dd.n_heads);
     A.apply_alias = P.apply_alias;
     rc = bf     ? launch_carry_apply<bf16_t, false>(A, P.apply_ksmax, P.apply_seq != 0, blocks, P.lds_apply, s)
          : prec ? launch_carry_apply<float, true>(A, P.apply_ksmax, P.apply_seq != 0, blocks, P.lds_apply, s)

@@ -182,7 +182,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.H, dk = a.dk, dv = a.dv;
-  const int cidx = (int)(blockIdx.x / H), h = (int)(blockIdx.x % H);
+  int cidx, h;
+  if (!tile_head(a.total_chunks, H, (int)blockIdx.x, cidx, h)) return;
   int seq, t0, clen, cis;
   chunk_lookup(a, cidx, seq, t0, clen, cis);
   const float Ip = a.Ip[h], scale = a.scale;
@@ -799,7 +800,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
 
 template <typename TIn, int DT, int DN, int NBW, bool VAR>
 static int launch_tile_n(const BwdArgs& A, const TileRect& R, hipStream_t s) {
-  const int64_t blocks = (int64_t)A.c.total_chunks * A.c.H;
+  const int64_t blocks = tile_head_blocks(A.c.total_chunks, A.c.H);
   if (blocks > 0x7fffffff) return PAL_E_DIM;
   constexpr size_t lds = sizeof(float) * (size_t)tile_lds(DT, DN, NBW, VAR, sizeof(TIn) == 4).total;
   static_assert(lds <= kMaxLds, "LDS of a compute unit");

@@ -75,6 +75,22 @@ __device__ __forceinline__ void seq_lookup(const ChunkArgs& a, int n, int& bos, 
   }
 }
 
+// A workgroup per (tile, head).  Consecutive workgroup ids go to different XCDs: the heads of a tile are dealt to one of them
+// side by side, since rows that are no multiple of a cache line leave lines to two heads.
+__host__ __device__ inline bool tiles_by_xcd(int64_t tiles) { return tiles >= 64; }
+inline int64_t tile_head_blocks(int64_t tiles, int H) { return (tiles_by_xcd(tiles) ? (tiles + 7) / 8 * 8 : tiles) * H; }
+__device__ __forceinline__ bool tile_head(int tiles, int H, int block, int& tile, int& h) {
+  if (tiles_by_xcd(tiles)) {
+    const int l = block >> 3, t = l / H;
+    tile = t * 8 + (block & 7);
+    h = l - t * H;
+    return tile < tiles;
+  }
+  tile = block / H;
+  h = block - tile * H;
+  return true;
+}
+
 // Workgroups that walk the tiles of a sequence in order, one per (sequence, head, slice): consecutive workgroup ids go to
 // different XCDs, the slices of one (sequence, head) belong on the same one (they read the same rows).
 struct WalkPlan {

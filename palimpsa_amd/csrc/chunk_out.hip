@@ -104,8 +104,9 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   const int STRIDE = oVB + 2 * VR;          // floats per staged token: f, c, -, -, k, k*k, q, (v, b) of every row
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int H = a.H, dk = a.dk, dv = a.dv;
-  int cidx = (int)(blockIdx.x / H);
-  const int h = (int)(blockIdx.x % H);
+  const int walks = a.every > 1 ? a.n_seqs * (((a.T + kC - 1) / kC + a.every - 1) / a.every) : a.total_chunks;
+  int cidx, h;
+  if (!tile_head(walks, H, (int)blockIdx.x, cidx, h)) return;
   const int r0 = (int)blockIdx.y * VR;
   int seq, t0, clen, cis;
   if (a.every > 1) {   // batched sequences of one length, `every` tiles from one state
@@ -366,7 +367,7 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
   const int nw = (a.dv + ROWS - 1) / ROWS;            // waves over the value rows
   const int W = out_waves(nw), slices = (nw + W - 1) / W;
   const int64_t walks = a.every > 1 ? (int64_t)a.n_seqs * (((a.T + kC - 1) / kC + a.every - 1) / a.every) : a.total_chunks;
-  const int64_t blocks = walks * a.H;
+  const int64_t blocks = tile_head_blocks(walks, a.H);
   if (blocks > 0x7fffffff) return PAL_E_DIM;
   const size_t lds = sizeof(float) * (4 * kC * a.every + 4 + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
   if (lds > kMaxLds) return PAL_E_HEADDIM;
