@@ -21,7 +21,7 @@ struct BwdArgs {
   float *pQK, *pVB;       // [slices][tokens,H,2,dk] dq, dk; [column groups][tokens,H,2,dv] dv, db
   float *pE, *pSig;       // [rectangles][H,tokens], [rectangles][total_chunks,H]
   int32_t tokens;
-  int32_t apply_alias;     // carry apply: db^carry shares LDS with the bf16 carries (large head dims)
+  int32_t apply_stride;    // carry apply: row stride of the carries in LDS
 };
 
 // A launch of the tile kernel covers a rectangle of the state: `cols` key columns from n0 on, and value rows from r0 on.

@@ -111,39 +111,34 @@ __global__ __launch_bounds__(256) void chunk_bwd_carry_scan_kernel(BwdArgs A) {
 
 // ---------------------------------------------------------------- carry apply
 // dv_s += a_s R_M k_s ; db_s += a_s R_J k_s^2 ; dk_s += a_s (R_M^T v_s + 2 k_s * R_J^T b_s)
-// One workgroup of 4 waves per (tile, head); wave w owns tokens [16w, 16w+16).  The four products
-// run on the matrix cores (bf16 operands, fp32 accumulate); their results are parked in LDS and then
-// added to the tile-local gradients with 16-byte loads/stores that are contiguous along the head dim.
-// KSMAX = operand registers per product (32 contraction indices each: head dims up to 32 KSMAX).  With
-// SEQ the dv and db products take turns in one result buffer: less LDS, so that more workgroups share
-// a compute unit (the kernel is a chain of dependent load, product and store phases, and it is the
-// number of resident workgroups that hides them).
-// PREC (fp32 rows): operands as two bf16 halves, three matrix instructions per product; the transposed copy of the
-// carries then holds a second plane with the lo halves (never shared with a result buffer).
-// (second launch bound: at most 256 registers per lane, so matrix results stay in ordinary vector registers)
-// The kernel is a chain of phases, each of which starts with fetches from global memory (the carries, the operand
-// rows, the gradients it adds to); taken in turn their latencies add up to most of the kernel's time.  So every fetch
-// is issued as early as its address is known: the operand rows of all four products before the carries are staged,
-// the gradients that a phase adds to before the matrix instructions of that phase.  Every wave scans the gates
-// itself (the decay a_s of its own token rows), so the operands do not wait for another wave.
-template <typename TIn, int KSMAX, bool SEQ, bool PREC>
-__global__ __launch_bounds__(256, 2) void chunk_bwd_carry_apply_kernel(BwdArgs A) {
+// One workgroup of 4 waves per (tile, head); wave w owns tokens [16w, 16w+16).  The four products run on the matrix cores
+// (bf16 operands, fp32 accumulate) with the tokens as columns: a lane's four results are neighbours in the row of its
+// token, and in every product the operand of a lane is the same four-element pieces of that token's row, so that a
+// row is fetched once, serves as operand and as the factor of the results, and the sums go back to memory from the
+// registers.  Bound by HBM traffic (the rows, the gradients in and out, the carries, and the states for the boundary
+// term: 375 MB at 8 x 2048 tokens, 12 heads of 64x64) and by the latency that few workgroups hide: every fetch
+// is issued before the first is used, and there is one barrier between them and the results.  (With results parked in
+// LDS, phase by phase with a barrier and fetches in each, 112 us at that size, now 108; 16 heads of 48x48 120, 95; 32768 packed
+// tokens, 16 of 96x96 660, 527; 4 x 2048, 8 of 128x128 182, 96; fp32 rows 2 x 2048, 8 of 128x64 62, 39.)
+// KSMAX = operand registers per product (32 contraction indices each: head dims up to 32 KSMAX).
+// PREC (fp32 rows): operands as two bf16 halves, three matrix instructions per product; the copy of the carries in LDS
+// then holds a second plane with the lo halves.
+// Every wave scans the gates itself (the decay a_s of its own token rows), so the operands do not wait for another wave.
+// waves per SIMD: what the rows, gradients and operands leave (64x64 squeezed into 128 registers for four: 116 us)
+constexpr int apply_waves(int KSMAX, bool f32) { return f32 ? (KSMAX == 1 ? 3 : 2) : KSMAX == 1 ? 4 : KSMAX <= 3 ? 3 : 2; }
+template <typename TIn, int KSMAX, bool PREC>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(apply_waves(KSMAX, sizeof(TIn) == 4))))
+void chunk_bwd_carry_apply_kernel(BwdArgs A) {
   const ChunkArgs& a = A.c;
   extern __shared__ float smem[];
   const int H = a.H, dk = a.dk, dv = a.dv;
-  const int dmax = dk > dv ? dk : dv;
-  float* sW4 = smem + kC;                  // [8]
-  float* sBt = sW4 + 8;                    // [64][dv/8] beta of the carry terms, one slot per work item
-  float* sO1 = sBt + kC * (dv >> 3);       // [64][OS] dk^carry, later dv^carry
-  float* sO2 = SEQ ? sO1 : sO1 + kC * (dmax + 4);   // [64][OS] db^carry (SEQ: after dv^carry has been applied)
-  // [2][dk][dv + 8] R_M^T, R_J^T in bf16, operand source of all four products.  When both do not fit the LDS
-  // (large head dims) the bf16 copy shares its bytes with db^carry and the dv/db products read the fp32
-  // carries from global memory instead.
-  const bool alias = !SEQ && A.apply_alias != 0;
-  bf16_t* sRT = (bf16_t*)(alias ? sO2 : sO2 + kC * (dmax + 4));
-  const int RS = dv + 8;
-  bf16_t* sRTl = sRT + 2 * dk * RS;        // PREC: [2][dk][dv + 8] lo halves
-  const int OS = dmax + 4;
+  float* sW4 = smem;                       // [4] shares of the boundary term
+  float* sBt = smem + 4;                   // [64] beta of the carry terms
+  // [2][dv][RS] R_M, R_J in bf16 as they lie in memory, operand source of all four products: the ones that contract over
+  // the key columns read pieces of a row, the ones over the value rows four rows at once, transposed on their way out
+  bf16_t* sR = (bf16_t*)(smem + 4 + kC);
+  const int RS = A.apply_stride;
+  bf16_t* sRl = sR + 2 * dv * RS;          // PREC: [2][dv][RS] lo halves
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = lane & 15, g = lane >> 4;
   int cidx, h;
   if (!tile_head(a.total_chunks, H, blockIdx.x, cidx, h)) return;
@@ -176,94 +171,59 @@ __global__ __launch_bounds__(256, 2) void chunk_bwd_carry_apply_kernel(BwdArgs A
     return;
   }
   const float gh = a.g[h] * kLog2e;
-  const int srow = 16 * w + i;            // operand row (token) of this lane
+  const int srow = 16 * w + i;            // this lane's token
   const bool row_ok = srow < clen;
+  typedef typename Raw4<TIn>::type raw4;
+  constexpr int NB = 2 * KSMAX;           // blocks of 16 columns
+  // where the registers are there, the gradients are fetched with everything else; where they are not even there for the
+  // rows, these are fetched again
+  constexpr bool AHEAD = KSMAX * sizeof(TIn) <= 8, KEEP = KSMAX * sizeof(TIn) <= 12;
+  const int64_t tokA = (int64_t)(t0 + (row_ok ? srow : 0)) * H + h;
+  const TIn* vp = (const TIn*)a.v + tokA * dv + 4 * g;
+  const TIn* bp = (const TIn*)a.b + tokA * dv + 4 * g;
+  const TIn* kp = (const TIn*)a.k + qk_row(a, t0 + (row_ok ? srow : 0), h) + 4 * g;
+  TIn* dkp = (TIn*)A.dk + tokA * dk + 4 * g;
+  TIn* dvp = (TIn*)A.dv + tokA * dv + 4 * g;
+  TIn* dbp = (TIn*)A.db + tokA * dv + 4 * g;
+  auto load = [&](const TIn* p, int nb) { return *(const raw4*)(p + 16 * nb); };
+  constexpr int NK = KEEP ? NB : 1, NA = AHEAD ? NB : 1;
+  raw4 vr[NK], br[NK], kr[NK], dkr[NA], dvr[NA], dbr[NA];   // columns 16 nb + 4 g .. of the token's rows
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (16 * nb < dv) {
+        vr[nb] = load(vp, nb);
+        br[nb] = load(bp, nb);
+      }
+      if (16 * nb < dk) kr[nb] = load(kp, nb);
+    }
+  }
+  auto v_of = [&](int nb) { if constexpr (KEEP) return vr[nb]; else return load(vp, nb); };
+  auto b_of = [&](int nb) { if constexpr (KEEP) return br[nb]; else return load(bp, nb); };
+  auto k_of = [&](int nb) { if constexpr (KEEP) return kr[nb]; else return load(kp, nb); };
+  auto fetch_grads = [&]() {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (16 * nb < dk) dkr[nb] = load(dkp, nb);
+      if (16 * nb < dv) {
+        dvr[nb] = load(dvp, nb);
+        dbr[nb] = load(dbp, nb);
+      }
+    }
+  };
   float as, Ftot;                         // decay from token srow to the end of the tile, and over the whole tile
   {
     const float c = wave_inclusive_scan(-gt_l * gh, lane);
     const float tot = __shfl(c, 63);
-    as = fast_exp2(tot - __shfl(c, srow));
+    as = row_ok ? fast_exp2(tot - __shfl(c, srow)) : 0.f;
     Ftot = fast_exp2(tot);
   }
-  const int64_t tokA = ((int64_t)(t0 + (row_ok ? srow : 0)) * H + h);
-  const int64_t tok0 = ((int64_t)t0 * H + h);
-
-  // operands of the four products: rows a_s v_s, a_s b_s (contraction over the value rows) and a_s k_s, a_s k_s^2
-  // (over the key columns) of this lane's token.  EARLY: built before anything else (the registers are there).
-  constexpr bool EARLY = (PREC ? 2 : 1) * KSMAX <= 4;
-  bf16x8 A3[KSMAX], A4[KSMAX], A1[KSMAX], A2[KSMAX];
-  bf16x8 A3l[PREC ? KSMAX : 1], A4l[PREC ? KSMAX : 1], A1l[PREC ? KSMAX : 1], A2l[PREC ? KSMAX : 1];
-  auto build_vb = [&]() {
-    const int KS = (dv + 31) / 32;
-    const TIn* vp = (const TIn*)a.v + tokA * dv;
-    const TIn* bp = (const TIn*)a.b + tokA * dv;
-#pragma unroll
-    for (int ks = 0; ks < KSMAX; ++ks) {
-      if (ks < KS) {
-        const int d0 = 8 * g + 32 * ks;
-        float vv[8], bb[8];
-        if (row_ok && d0 < dv) {
-          load_vec<4>(vp + d0, vv); load_vec<4>(vp + d0 + 4, vv + 4);
-          load_vec<4>(bp + d0, bb); load_vec<4>(bp + d0 + 4, bb + 4);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) { vv[j] = 0.f; bb[j] = 0.f; }
-        }
-        if constexpr (PREC) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) { vv[j] *= as; bb[j] *= as; }
-          split_bf16(vv, A3[ks], A3l[ks]);
-          split_bf16(bb, A4[ks], A4l[ks]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            A3[ks][j] = (bf16_t)(as * vv[j]);
-            A4[ks][j] = (bf16_t)(as * bb[j]);
-          }
-        }
-      }
-    }
-  };
-  auto build_k = [&]() {
-    const int KS = (dk + 31) / 32;
-    const TIn* kp = (const TIn*)a.k + qk_row(a, t0 + (row_ok ? srow : 0), h);
-#pragma unroll
-    for (int ks = 0; ks < KSMAX; ++ks) {
-      if (ks < KS) {
-        const int n0 = 8 * g + 32 * ks;
-        float kv[8];
-        if (row_ok && n0 < dk) {
-          load_vec<4>(kp + n0, kv);
-          load_vec<4>(kp + n0 + 4, kv + 4);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) kv[j] = 0.f;
-        }
-        if constexpr (PREC) {
-          float k1[8], k2[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) { k1[j] = as * kv[j]; k2[j] = k1[j] * kv[j]; }
-          split_bf16(k1, A1[ks], A1l[ks]);
-          split_bf16(k2, A2[ks], A2l[ks]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            A1[ks][j] = (bf16_t)(as * kv[j]);
-            A2[ks][j] = (bf16_t)(as * kv[j] * kv[j]);
-          }
-        }
-      }
-    }
-  };
-  build_vb();
-  if constexpr (EARLY) build_k();
-
   const int64_t E = (int64_t)dv * dk;
   const TIn* RM = (const TIn*)A.wDM + ((int64_t)cidx * H + h) * E;
   const TIn* RJ = (const TIn*)A.wDJ + ((int64_t)cidx * H + h) * E;
   {
     // F_C (<R_M, M_0> + <R_J, J_0>) with (M_0, J_0) the state at the start of this tile; the same
-    // pass leaves R^T in LDS for the products that contract over the value rows
+    // pass leaves R in LDS for the products
     const float* smu = a.chunk_mu + ((int64_t)cidx * H + h) * E;
     const float* sI = a.chunk_I + ((int64_t)cidx * H + h) * E;
     const float Ipb = a.Ip[h];
@@ -273,35 +233,45 @@ __global__ __launch_bounds__(256, 2) void chunk_bwd_carry_apply_kernel(BwdArgs A
     // four blocks are fetched before the first is used
     const int nc = dk >> 4, nblk = (dv >> 4) * nc, per = (nblk + 3) >> 2;
     for (int j0 = 0; j0 < per; j0 += 4) {
-      float rm[4][4], rj[4][4];
+      raw4 rm[4], rj[4];
       f32x4 mu[4], I[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int blk = w * per + j0 + u;
         if (j0 + u < per && blk < nblk) {
           const int64_t e = (int64_t)(16 * (blk / nc) + i) * dk + 4 * (4 * (blk % nc) + g);
-          load_vec<4>(RM + e, rm[u]);
-          load_vec<4>(RJ + e, rj[u]);
+          rm[u] = *(const raw4*)(RM + e);
+          rj[u] = *(const raw4*)(RJ + e);
           mu[u] = *(const f32x4*)(smu + e);
           I[u] = *(const f32x4*)(sI + e);
         }
+      }
+      if constexpr (AHEAD) {
+        if (j0 == 0) fetch_grads();
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int blk = w * per + j0 + u;
         if (j0 + u < per && blk < nblk) {
-          const int d = 16 * (blk / nc) + i, c4 = 4 * (blk % nc) + g;
+          const int o = (16 * (blk / nc) + i) * RS + 4 * (4 * (blk % nc) + g);
+          bf16x4 mh, jh, ml, jl;
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
-            acc = fmaf(rm[u][x], mu[u][x] * I[u][x], acc);
-            acc = fmaf(rj[u][x], I[u][x] - Ipb, acc);
-            const bf16_t mh = (bf16_t)rm[u][x], jh = (bf16_t)rj[u][x];
-            sRT[(4 * c4 + x) * RS + d] = mh;
-            sRT[(dk + 4 * c4 + x) * RS + d] = jh;
+            const float m = (float)rm[u][x], y = (float)rj[u][x];
+            acc = fmaf(m, mu[u][x] * I[u][x], acc);
+            acc = fmaf(y, I[u][x] - Ipb, acc);
+            mh[x] = (bf16_t)m;
+            jh[x] = (bf16_t)y;
             if constexpr (PREC) {
-              sRTl[(4 * c4 + x) * RS + d] = (bf16_t)(rm[u][x] - (float)mh);
-              sRTl[(dk + 4 * c4 + x) * RS + d] = (bf16_t)(rj[u][x] - (float)jh);
+              ml[x] = (bf16_t)(m - (float)mh[x]);
+              jl[x] = (bf16_t)(y - (float)jh[x]);
             }
+          }
+          *(bf16x4*)&sR[o] = mh;
+          *(bf16x4*)&sR[dv * RS + o] = jh;
+          if constexpr (PREC) {
+            *(bf16x4*)&sRl[o] = ml;
+            *(bf16x4*)&sRl[dv * RS + o] = jl;
           }
         }
       }
@@ -309,240 +279,128 @@ __global__ __launch_bounds__(256, 2) void chunk_bwd_carry_apply_kernel(BwdArgs A
     acc = wave_sum(acc);
     if (lane == 0) sW4[w] = acc;
   }
-  // gradients this kernel adds to, as fetched: item m of a thread is (token s, eight consecutive entries c8) with
-  // s * groups + c8 = tid + 256 m; a row has at most 4 KSMAX groups of eight, so a thread has at most KSMAX items
-  // PRE: fetched a phase ahead, where the registers are there for it (else right before they are used)
-  constexpr bool PRE = KSMAX <= 2 || (KSMAX == 4 && SEQ && !PREC && sizeof(TIn) == 2);
-  Raw8<TIn> old1[KSMAX], old2[KSMAX], in1[KSMAX], in2[KSMAX];
-  auto fetch_items = [&](const TIn* p, int groups, int row_len, Raw8<TIn>* dst) {
+  // Operands: contraction index (g, j) -> 32 ks + 16 (j / 4) + 4 g + j % 4, rows times the decay of their token (PREC: hi, lo)
+  struct Opnd { bf16x8 hi, lo; };
+  auto operand = [&](const float* x) {
+    Opnd y;
+    if constexpr (PREC) {
+      split_bf16(x, y.hi, y.lo);
+    } else {
 #pragma unroll
-    for (int m = 0; m < KSMAX; ++m) {
-      const int idx = tid + 256 * m, c8 = idx % groups, s = idx / groups;
-      if (idx < kC * groups && s < clen) dst[m].load(p + (int64_t)s * H * row_len + 8 * c8);
+      for (int j = 0; j < 8; ++j) y.hi[j] = (bf16_t)x[j];
     }
+    return y;
   };
-  TIn* dko = (TIn*)A.dk + tok0 * dk;
-  if constexpr (PRE) fetch_items(dko, dk >> 3, dk, old1);
-  __syncthreads();
-  const float bnd = Ftot * (sW4[0] + sW4[1] + sW4[2] + sW4[3]);   // every thread; the slots are not written again
-
-  // ---- dk: out[s, n] = sum_d (a_s v_s[d]) R_M[d, n] + 2 k_s[n] sum_d (a_s b_s[d]) R_J[d, n]
-  {
-    const int KS = (dv + 31) / 32;
-    const TIn* kin = (const TIn*)a.k + qk_row(a, t0, h);
-    // k of the result entries (row s = 16w + 4g + r, column n = 16nbk + i), fetched one step ahead
-    auto load_k4 = [&](int nbk, float* kv) {
+  auto mac = [&](const Opnd& r, const Opnd& t, f32x4 acc) {
+    if constexpr (PREC) return mfma16_split(r.hi, r.lo, t.hi, t.lo, acc);
+    else return mfma16(r.hi, t.hi, acc);
+  };
+  const bf16x4 none = {(bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f};
+  Opnd X[KSMAX], Y[KSMAX];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int s = 16 * w + 4 * g + r;
-        kv[r] = (s < clen) ? to_f32(kin[(int64_t)s * qk_stride(a) + 16 * nbk + i]) : 0.f;
+  for (int ks = 0; ks < KSMAX; ++ks) {
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (16 * (2 * ks + q) < dv) {
+        const raw4 vv = v_of(2 * ks + q), bb = b_of(2 * ks + q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { x[4 * q + j] = as * (float)vv[j]; y[4 * q + j] = as * (float)bb[j]; }
       }
-    };
-    float kcur[4], knext[4] = {0.f, 0.f, 0.f, 0.f};
-    load_k4(0, kcur);
-    const int NBK = dk / 16;
-    for (int nbk = 0; nbk < NBK; ++nbk) {
-      if (nbk + 1 < NBK) load_k4(nbk + 1, knext);
+    }
+    X[ks] = operand(x);
+    Y[ks] = operand(y);
+  }
+  __syncthreads();
+  const float bnd = Ftot * (sW4[0] + sW4[1] + sW4[2] + sW4[3]);   // every thread
+
+  // ---- dk: out[n, s] = sum_d R_M[d, n] (a_s v_s[d]) + 2 k_s[n] sum_d R_J[d, n] (a_s b_s[d])
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    if (16 * nb < dk) {
       f32x4 accM = {0.f, 0.f, 0.f, 0.f}, accJ = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KSMAX; ++ks) {
-        if (ks < KS) {
-          const int d0 = 8 * g + 32 * ks;
-          bf16x8 B3, B4;
-          if (d0 < dv) {
-            B3 = *(const bf16x8*)&sRT[(16 * nbk + i) * RS + d0];
-            B4 = *(const bf16x8*)&sRT[(dk + 16 * nbk + i) * RS + d0];
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) { B3[j] = (bf16_t)0.f; B4[j] = (bf16_t)0.f; }
-          }
-          if constexpr (PREC) {
-            bf16x8 B3l = B3, B4l = B4;   // zero beyond dv
-            if (d0 < dv) {
-              B3l = *(const bf16x8*)&sRTl[(16 * nbk + i) * RS + d0];
-              B4l = *(const bf16x8*)&sRTl[(dk + 16 * nbk + i) * RS + d0];
-            }
-            accM = mfma16_split(A3[ks], A3l[ks], B3, B3l, accM);
-            accJ = mfma16_split(A4[ks], A4l[ks], B4, B4l, accJ);
-          } else {
-            accM = mfma16(A3[ks], B3, accM);
-            accJ = mfma16(A4[ks], B4, accJ);
-          }
+        if (32 * ks < dv) {
+          // rows 32 ks + 4 g + i / 4 and 16 further on, columns 16 nb + 4 (i % 4) ..
+          const int o = (32 * ks + 4 * g + (i >> 2)) * RS + 16 * nb + 4 * (i & 3);
+          const bool two = 32 * ks + 16 < dv;
+          auto rows = [&](int at) {
+            Opnd y;
+            y.hi = join(lds_read_tr(sR + at), two ? lds_read_tr(sR + at + 16 * RS) : none);
+            if constexpr (PREC) y.lo = join(lds_read_tr(sRl + at), two ? lds_read_tr(sRl + at + 16 * RS) : none);
+            return y;
+          };
+          accM = mac(rows(o), X[ks], accM);
+          accJ = mac(rows(dv * RS + o), Y[ks], accJ);
         }
       }
-      // rows s = 16w + 4g + r, column n = 16nbk + i
+      float y[4];
+      const raw4 kk = k_of(nb), was = AHEAD ? dkr[AHEAD ? nb : 0] : load(dkp, nb);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = (float)was[r] + fmaf(2.f * (float)kk[r], accJ[r], accM[r]);
+      if (row_ok) store_vec<4>(dkp + 16 * nb, y);
+    }
+  }
+  // ---- dv, db: out[d, s] = sum_n R[d, n] (a_s k_s[n]), (a_s k_s[n]^2);  beta_s = <v_s, dv^carry_s> + <b_s, db^carry_s>
+#pragma unroll
+  for (int ks = 0; ks < KSMAX; ++ks) {
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      if (16 * (2 * ks + q) < dk) {
+        const raw4 kk = k_of(2 * ks + q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float kv = (float)kk[j];
+          x[4 * q + j] = as * kv;
+          y[4 * q + j] = as * kv * kv;
+        }
+      }
+    }
+    X[ks] = operand(x);
+    Y[ks] = operand(y);
+  }
+  float beta = 0.f;
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    if (16 * nb < dv) {
+      f32x4 accV = {0.f, 0.f, 0.f, 0.f}, accB = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KSMAX; ++ks) {
+        if (32 * ks < dk) {
+          const int o = (16 * nb + i) * RS + 32 * ks + 4 * g;
+          const bool two = 32 * ks + 16 < dk;
+          auto row = [&](int at) {
+            Opnd y;
+            y.hi = join(*(const bf16x4*)(sR + at), two ? *(const bf16x4*)(sR + at + 16) : none);
+            if constexpr (PREC) y.lo = join(*(const bf16x4*)(sRl + at), two ? *(const bf16x4*)(sRl + at + 16) : none);
+            return y;
+          };
+          accV = mac(row(o), X[ks], accV);
+          accB = mac(row(dv * RS + o), Y[ks], accB);
+        }
+      }
+      float x[4], y[4];
+      const raw4 vv = v_of(nb), bb = b_of(nb);
+      const raw4 was_v = AHEAD ? dvr[AHEAD ? nb : 0] : load(dvp, nb), was_b = AHEAD ? dbr[AHEAD ? nb : 0] : load(dbp, nb);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int s = 16 * w + 4 * g + r;
-        sO1[s * OS + 16 * nbk + i] = fmaf(2.f * kcur[r], accJ[r], accM[r]);
-        kcur[r] = knext[r];
+        beta = fmaf((float)vv[r], accV[r], beta);
+        beta = fmaf((float)bb[r], accB[r], beta);
+        x[r] = (float)was_v[r] + accV[r];
+        y[r] = (float)was_b[r] + accB[r];
+      }
+      if (row_ok) {
+        store_vec<4>(dvp + 16 * nb, x);
+        store_vec<4>(dbp + 16 * nb, y);
       }
     }
   }
-  if constexpr (!EARLY) build_k();
-  const int vgroups = dv >> 3;   // work item = (token, 8 value rows); the items of a token sit in adjacent lanes
-  const TIn* vin = (const TIn*)a.v + tok0 * dv;
-  const TIn* bin = (const TIn*)a.b + tok0 * dv;
-  TIn* dvo = (TIn*)A.dv + tok0 * dv;
-  TIn* dbo = (TIn*)A.db + tok0 * dv;
-  // dv and its v rows for the next phase (SEQ: db and b before the second pass)
-  if constexpr (PRE) {
-    fetch_items(vin, vgroups, dv, in1);
-    fetch_items(dvo, vgroups, dv, old2);
-  }
+  beta = rows4_sum(beta);
+  if (g == 0) sBt[srow] = row_ok ? beta : 0.f;
   __syncthreads();
-  {
-    const int groups = dk >> 3;
-    auto item = [&](int m) {
-      const int idx = tid + 256 * m, c8 = idx % groups, s = idx / groups;
-      if (idx < kC * groups && s < clen) {
-        TIn* o = dko + (int64_t)s * H * dk + 8 * c8;
-        Raw8<TIn> now;
-        if constexpr (!PRE) now.load(o);
-        const Raw8<TIn>& was = PRE ? old1[m] : now;
-        float gk[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) gk[e] = was.get(e) + sO1[s * OS + 8 * c8 + e];
-        store_vec<4>(o, gk); store_vec<4>(o + 4, gk + 4);
-      }
-    };
-    if constexpr (PRE) {
-#pragma unroll
-      for (int m = 0; m < KSMAX; ++m) item(m);
-    } else {
-#pragma unroll 1
-      for (int m = 0; m < KSMAX; ++m) item(m);
-    }
-  }
-  if constexpr (PRE && !SEQ) {
-    fetch_items(bin, vgroups, dv, in2);
-    fetch_items(dbo, vgroups, dv, old1);
-  }
-  __syncthreads();   // sO1 is free again
-
-  // ---- dv, db: out[s, d] = sum_n (a_s k_s[n]) R_M[d, n]
-  {
-    const int KS = (dk + 31) / 32;
-    const int groups = vgroups;
-    constexpr int NPASS = SEQ ? 2 : 1;
-#pragma unroll
-    for (int pass = 0; pass < NPASS; ++pass) {
-      const bool doV = !SEQ || pass == 0, doB = !SEQ || pass == 1;
-      for (int db_ = 0; db_ < dv / 16; ++db_) {
-        f32x4 accV = {0.f, 0.f, 0.f, 0.f}, accB = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KSMAX; ++ks) {
-          if (ks < KS) {
-            const int n0 = 8 * g + 32 * ks;
-            bf16x8 B1, B2;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) { B1[j] = (bf16_t)0.f; B2[j] = (bf16_t)0.f; }
-            bf16x8 B1l = B1, B2l = B2;
-            if constexpr (PREC) {
-              if (n0 < dk) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                  if (doV) { B1[j] = sRT[(n0 + j) * RS + 16 * db_ + i]; B1l[j] = sRTl[(n0 + j) * RS + 16 * db_ + i]; }
-                  if (doB) { B2[j] = sRT[(dk + n0 + j) * RS + 16 * db_ + i]; B2l[j] = sRTl[(dk + n0 + j) * RS + 16 * db_ + i]; }
-                }
-              }
-              if (doV) accV = mfma16_split(A1[ks], A1l[ks], B1, B1l, accV);
-              if (doB) accB = mfma16_split(A2[ks], A2l[ks], B2, B2l, accB);
-              continue;
-            }
-            if (n0 < dk && !alias) {
-              // 8 consecutive key columns of value row d = 16db_ + i: a column walk through the transposed
-              // bf16 copy in LDS (the fp32 carries in global memory would miss L2 on this second read)
-#pragma unroll
-              for (int j = 0; j < 8; ++j) {
-                if (doV) B1[j] = sRT[(n0 + j) * RS + 16 * db_ + i];
-                if (doB) B2[j] = sRT[(dk + n0 + j) * RS + 16 * db_ + i];
-              }
-            } else if (n0 < dk) {
-              const TIn* r1 = RM + (int64_t)(16 * db_ + i) * dk + n0;
-              const TIn* r2 = RJ + (int64_t)(16 * db_ + i) * dk + n0;
-              float x[8], y[8];
-              load_vec<4>(r1, x); load_vec<4>(r1 + 4, x + 4);
-              load_vec<4>(r2, y); load_vec<4>(r2 + 4, y + 4);
-#pragma unroll
-              for (int j = 0; j < 8; ++j) {
-                B1[j] = (bf16_t)x[j];
-                B2[j] = (bf16_t)y[j];
-              }
-            }
-            if (doV) accV = mfma16(A1[ks], B1, accV);
-            if (doB) accB = mfma16(A2[ks], B2, accB);
-          }
-        }
-        // accumulator layout: rows s = 16w + 4g + r, column d = 16db_ + i
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (doV) sO1[(16 * w + 4 * g + r) * OS + 16 * db_ + i] = accV[r];
-          if (doB) sO2[(16 * w + 4 * g + r) * OS + 16 * db_ + i] = accB[r];
-        }
-      }
-      __syncthreads();
-      // add to the tile-local dv, db; beta_s = <v_s, dv^carry_s> + <b_s, db^carry_s>
-      // (SEQ: the rows of the pass are in in1/old2; else v, dv in in1/old2 and b, db in in2/old1)
-      auto item = [&](int m) {
-        const int idx = tid + 256 * m, c8 = idx % groups, s = idx / groups;
-        if (idx < kC * groups) {
-          float beta = 0.f;
-          if (s < clen) {
-            const int64_t off = (int64_t)s * H * dv + 8 * c8;
-            if (doV) {
-              Raw8<TIn> x_now, g_now;
-              if constexpr (!PRE) { x_now.load(vin + off); g_now.load(dvo + off); }
-              const Raw8<TIn>& xv = PRE ? in1[m] : x_now;
-              const Raw8<TIn>& gvo = PRE ? old2[m] : g_now;
-              float gv[8];
-#pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const float cv = sO1[s * OS + 8 * c8 + e];
-                beta = fmaf(xv.get(e), cv, beta);
-                gv[e] = gvo.get(e) + cv;
-              }
-              store_vec<4>(dvo + off, gv); store_vec<4>(dvo + off + 4, gv + 4);
-            }
-            if (doB) {
-              Raw8<TIn> x_now, g_now;
-              if constexpr (!PRE) { x_now.load(bin + off); g_now.load(dbo + off); }
-              const Raw8<TIn>& xb = PRE ? (SEQ ? in1[m] : in2[m]) : x_now;
-              const Raw8<TIn>& gbo = PRE ? (SEQ ? old2[m] : old1[m]) : g_now;
-              float gb[8];
-#pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const float cb = sO2[s * OS + 8 * c8 + e];
-                beta = fmaf(xb.get(e), cb, beta);
-                gb[e] = gbo.get(e) + cb;
-              }
-              store_vec<4>(dbo + off, gb); store_vec<4>(dbo + off + 4, gb + 4);
-            }
-          }
-          // the second pass of SEQ adds to the share the same thread left in the first
-          sBt[idx] = (SEQ && pass == 1) ? sBt[idx] + beta : beta;
-        }
-      };
-      if constexpr (PRE) {
-#pragma unroll
-        for (int m = 0; m < KSMAX; ++m) item(m);
-      } else {
-#pragma unroll 1
-        for (int m = 0; m < KSMAX; ++m) item(m);
-      }
-      if (PRE && SEQ && pass == 0) {
-        fetch_items(bin, groups, dv, in1);
-        fetch_items(dbo, groups, dv, old2);
-      }
-      __syncthreads();   // SEQ: the result buffer is free for the next pass; last pass: sBt is complete
-    }
-    if (w == 0) {
-      float bsum = 0.f;
-      if (tok_ok)
-        for (int c8 = 0; c8 < groups; ++c8) bsum += sBt[lane * groups + c8];   // fixed order
-      gate_grad(bsum, bnd);
-    }
-  }
+  if (w == 0) gate_grad(sBt[lane], bnd);
 }
 
 // ----------------------------------------------------------------- head sums
@@ -697,44 +555,41 @@ static BwdLayout bwd_layout(const PalDims* d) {
 // backward cannot serve is refused while nothing has been enqueued.
 struct BwdPlan {
   size_t lds_apply;
-  int apply_alias, apply_seq, apply_ksmax;
+  int apply_stride;
 };
 
 // prec: the fp32-accurate variants (fp32 rows without PAL_FLAG_FP32_FAST)
 static int bwd_plan(int dk, int dv, bool prec, BwdPlan& P) {
   const int dmax = dk > dv ? dk : dv;
-  const size_t rt_bytes = (prec ? 2 : 1) * 2 * (size_t)2 * dk * (dv + 8), o_bytes = sizeof(float) * kC * (dmax + 4);
   if (prec && dmax > 128) return PAL_E_HEADDIM;
-  const size_t lds_fixed = sizeof(float) * (kC + 8 + kC * (dv >> 3)) + o_bytes;
-  size_t lds = lds_fixed + o_bytes + rt_bytes;
-  P.apply_alias = 0;
-  if (lds > kMaxLds && !prec) {
-    P.apply_alias = 1;
-    lds = lds_fixed + (rt_bytes > o_bytes ? rt_bytes : o_bytes);
-  }
-  // one result buffer used twice when that lets more workgroups share a compute unit
-  const size_t lds_seq = lds_fixed + rt_bytes;
-  P.apply_seq = lds_seq <= kMaxLds && kMaxLds / lds_seq > (lds > kMaxLds ? 0 : kMaxLds / lds);
-  if (P.apply_seq) { lds = lds_seq; P.apply_alias = 0; }
-  if (lds > kMaxLds) return PAL_E_HEADDIM;
-  P.lds_apply = lds;
-  P.apply_ksmax = dmax <= 64 ? 2 : dmax <= 128 ? 4 : 8;
-  return PAL_OK;
+  // The head dims that are served: those whose carries (as columns of dv + 8 entries) fit the LDS beside a result buffer.
+  const size_t planes = prec ? 2 : 1, cols = planes * 4 * (size_t)dk * (dv + 8), out = sizeof(float) * kC * (dmax + 4);
+  const size_t fixed = sizeof(float) * (kC + 8 + kC * (dv >> 3)) + out;
+  if (fixed + cols > kMaxLds) return PAL_E_HEADDIM;
+  // row stride of the carries in LDS: an odd number of 32-byte pieces, for both kinds of reads and for the writes, where that fits
+  auto lds = [&](int stride) { return sizeof(float) * (4 + kC) + planes * 4 * (size_t)dv * stride; };
+  P.apply_stride = 16 * ((dk >> 4) | 1);
+  if (lds(P.apply_stride) > kMaxLds) P.apply_stride = dk;
+  P.lds_apply = lds(P.apply_stride);
+  return P.lds_apply <= kMaxLds ? PAL_OK : PAL_E_HEADDIM;
 }
 
-template <typename TIn, int KSMAX, bool SEQ, bool PREC>
+template <typename TIn, int KSMAX, bool PREC>
 static int launch_carry_apply_t(const BwdArgs& A, unsigned blocks, size_t lds, hipStream_t s) {
-  if (int rc = allow_lds((const void*)&chunk_bwd_carry_apply_kernel<TIn, KSMAX, SEQ, PREC>, lds)) return rc;
-  PAL_TIMED_LAUNCH(kKernBwdCarryApply, s, (chunk_bwd_carry_apply_kernel<TIn, KSMAX, SEQ, PREC>), dim3(blocks), dim3(256), lds, s, A);
+  if (int rc = allow_lds((const void*)&chunk_bwd_carry_apply_kernel<TIn, KSMAX, PREC>, lds)) return rc;
+  PAL_TIMED_LAUNCH(kKernBwdCarryApply, s, (chunk_bwd_carry_apply_kernel<TIn, KSMAX, PREC>), dim3(blocks), dim3(256), lds, s, A);
   PAL_HIP_LAUNCH_CHECK();
   return PAL_OK;
 }
 template <typename TIn, bool PREC>
-static int launch_carry_apply(const BwdArgs& A, int ksmax, bool seq, unsigned blocks, size_t lds, hipStream_t s) {
-  if (ksmax == 2) return seq ? launch_carry_apply_t<TIn, 2, true, PREC>(A, blocks, lds, s) : launch_carry_apply_t<TIn, 2, false, PREC>(A, blocks, lds, s);
-  if (ksmax == 4) return seq ? launch_carry_apply_t<TIn, 4, true, PREC>(A, blocks, lds, s) : launch_carry_apply_t<TIn, 4, false, PREC>(A, blocks, lds, s);
+static int launch_carry_apply(const BwdArgs& A, unsigned blocks, size_t lds, hipStream_t s) {
+  const int dmax = A.c.dk > A.c.dv ? A.c.dk : A.c.dv;
+  if (dmax <= 32) return launch_carry_apply_t<TIn, 1, PREC>(A, blocks, lds, s);
+  if (dmax <= 64) return launch_carry_apply_t<TIn, 2, PREC>(A, blocks, lds, s);
+  if (dmax <= 96) return launch_carry_apply_t<TIn, 3, PREC>(A, blocks, lds, s);
+  if (dmax <= 128) return launch_carry_apply_t<TIn, 4, PREC>(A, blocks, lds, s);
   if constexpr (PREC) return PAL_E_HEADDIM;   // the split operands of 256-wide heads do not fit the registers
-  else return seq ? launch_carry_apply_t<TIn, 8, true, false>(A, blocks, lds, s) : launch_carry_apply_t<TIn, 8, false, false>(A, blocks, lds, s);
+  else return dmax <= 192 ? launch_carry_apply_t<TIn, 6, false>(A, blocks, lds, s) : launch_carry_apply_t<TIn, 8, false>(A, blocks, lds, s);
 }
 
 }  // namespace pal
@@ -816,10 +671,10 @@ extern "C" int pal_chunk_bwd(const PalDims* d, const PalFwdTensors* t, const Pal
   }
   {
     const unsigned blocks = (unsigned)tile_head_blocks(dd.total_chunks, dd.n_heads);
-    A.apply_alias = P.apply_alias;
-    rc = bf     ? launch_carry_apply<bf16_t, false>(A, P.apply_ksmax, P.apply_seq != 0, blocks, P.lds_apply, s)
-         : prec ? launch_carry_apply<float, true>(A, P.apply_ksmax, P.apply_seq != 0, blocks, P.lds_apply, s)
-                : launch_carry_apply<float, false>(A, P.apply_ksmax, P.apply_seq != 0, blocks, P.lds_apply, s);
+    A.apply_stride = P.apply_stride;
+    rc = bf     ? launch_carry_apply<bf16_t, false>(A, blocks, P.lds_apply, s)
+         : prec ? launch_carry_apply<float, true>(A, blocks, P.lds_apply, s)
+                : launch_carry_apply<float, false>(A, blocks, P.lds_apply, s);
     if (rc) return rc;
     PAL_HIP_LAUNCH_CHECK();
   }

@@ -363,6 +363,34 @@ def test_runs_on_the_callers_stream(gpu_device):
     assert torch.isfinite(total)
 
 
+@pytest.mark.parametrize("dk,dv,rows", [(16, 16, "bf16"), (112, 48, "bf16"), (16, 176, "bf16"), (176, 80, "bf16"), (208, 32, "bf16"),
+                                        (240, 64, "bf16"), (96, 224, "bf16"), (112, 80, "fp32"), (48, 112, "fp32"), (144, 64, "fast"),
+                                        (208, 48, "fast")])
+def test_carries_over_the_head_dims(gpu_device, dk, dv, rows):
+    """What flows into a tile from the later ones, at the numbers of 16-column blocks that the carry kernel is built for, odd
+    ones too, and the rows it holds in registers or fetches again; nothing else reaches the first tiles' dv, db, dk."""
+    from palimpsa_amd import _lib
+    T, H = 150, 2
+    inp = po.make_inputs(1, T, H, dk, dv, seed=dk + dv)
+    if rows == "bf16":
+        inp = hp.rounded(inp, torch.bfloat16)
+    inp["g"] = torch.tensor([0.02, 0.2])
+    o_ref, _, _, _ = hp.oracle_forward(inp, dtype=torch.float64)
+    do = torch.zeros(1, T, H, dv)
+    do[:, 128:] = (o_ref[:, 128:] - 0.3 * torch.randn(1, T - 128, H, dv, generator=torch.Generator().manual_seed(dk))).float()
+    ref = hp.oracle_grads(inp, do)
+    try:
+        _lib.set_fp32_fast(rows == "fast")
+        grads = _run_bwd(inp, gpu_device, do)
+    finally:
+        _lib.set_fp32_fast(False)
+    first = lambda x: x[:, :128]   # noqa: E731
+    tol = hp.CHUNK_FP32_GRAD_TOL if rows == "fp32" else hp.BF16_GRAD_NORM_TOL
+    for n in ("k", "v", "b", "gt"):
+        assert hp.max_rel(first(grads[n]), first(ref[n])) <= tol, n
+    _compare(grads, ref, NAMES, tol=tol, inp=inp, dg_l1=True)
+
+
 @pytest.mark.parametrize("dk,dv", [(64, 64), (80, 96)])   # one piece per head; several, side by side, and their sum
 def test_forward_and_backward_replay_in_a_graph(gpu_device, dk, dv):
     """chunk_palimpsa forward + backward recorded into a HIP graph (the C ABI allocates nothing, synchronises nothing
