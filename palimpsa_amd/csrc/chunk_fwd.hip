@@ -180,90 +180,90 @@ __global__ __launch_bounds__(256) void chunk_delta_kernel(ChunkArgs a, int dvn) 
 
 // ------------------------------------------------------------------ kernel 1b
 // Serial part of the forward: S_c = F_c S_{c-1} + Delta_c per state entry, fp32, pure streaming.
-// One thread per four consecutive state entries of a (sequence, head), 1024 entries per block.  Each slot of
+// blocks of a (sequence, head) at vw entries per thread
+__host__ __device__ inline int scan_blocks(int64_t E, int vw) { return (int)((E + 256 * vw - 1) / (256 * vw)); }
+
+// One thread per VW consecutive state entries of a (sequence, head), 256 VW entries per block.  Each slot of
 // chunk_mu / chunk_I is overwritten with the state at the START of its tile in (mu, I) form
 // (what the reference stores as intermediate_*_state, chunk_palimpsa_forgetting_scalar.py:187-188);
 // the state after the last tile goes to final_mu / final_I (:214-218).
+template <int VW>
 __global__ __launch_bounds__(256) void chunk_scan_kernel(ChunkArgs a) {
   __shared__ float sF[kScanTiles];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t E = (int64_t)a.dv * a.dk;
-  const int nblk = (int)((E + 1023) / 1024);     // four consecutive entries per thread
+  const int nblk = scan_blocks(E, VW);
   const int blk = blockIdx.x % nblk;
   const int nh = blockIdx.x / nblk;
   const int h = nh % a.H, n = nh / a.H;
-  const int64_t e = ((int64_t)blk * 256 + tid) * 4;
+  const int64_t e = ((int64_t)blk * 256 + tid) * VW;
   const bool on = e < E;
   int bos, len, cbase;
   seq_lookup(a, n, bos, len, cbase);
   const int nchunks = (len + kC - 1) / kC;
   const float Ip = a.Ip[h];
   const float gh = a.g[h] * kLog2e;
-  f32x4 SM = {0.f, 0.f, 0.f, 0.f}, SJ = {0.f, 0.f, 0.f, 0.f};
+  float SM[VW], SJ[VW];
+#pragma unroll
+  for (int x = 0; x < VW; ++x) SM[x] = SJ[x] = 0.f;
   const int64_t so = (int64_t)nh * E + e;
   if (a.init_mu && on) {
-    const f32x4 mu = *(const f32x4*)(a.init_mu + so), I = *(const f32x4*)(a.init_I + so);
+    float mu[VW], I[VW];
+    load_vec<VW>(a.init_mu + so, mu);
+    load_vec<VW>(a.init_I + so, I);
 #pragma unroll
-    for (int x = 0; x < 4; ++x) { SM[x] = mu[x] * I[x]; SJ[x] = I[x] - Ip; }
+    for (int x = 0; x < VW; ++x) { SM[x] = mu[x] * I[x]; SJ[x] = I[x] - Ip; }
   }
-  // the slot of a tile: its Delta is read, the state at its start (mu, I) written if it is kept, the state advanced
-  auto advance = [&](int64_t off, const f32x4& dM, const f32x4& dJ, float F, bool kept) {
-    f32x4 mu, I;
+  auto store_state = [&](float* dst_mu, float* dst_I) {
+    float mu[VW], I[VW];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      I[x] = SJ[x] + Ip;
-      mu[x] = SM[x] * fast_rcp(I[x]);
+    for (int x = 0; x < VW; ++x) { I[x] = SJ[x] + Ip; mu[x] = SM[x] * fast_rcp(I[x]); }
+    store_vec<VW>(dst_mu, mu);
+    store_vec<VW>(dst_I, I);
+  };
+  // the slot of a tile: its Delta is read, the state at its start (mu, I) written if it is kept, the state advanced
+  auto advance = [&](int64_t off, const float* dM, const float* dJ, float F, bool kept) {
+    if (kept) store_state(a.chunk_mu + off, a.chunk_I + off);
+#pragma unroll
+    for (int x = 0; x < VW; ++x) {
       SM[x] = fmaf(F, SM[x], dM[x]);
       SJ[x] = fmaf(F, SJ[x], dJ[x]);
     }
-    if (kept) {
-      *(f32x4*)(a.chunk_mu + off) = mu;
-      *(f32x4*)(a.chunk_I + off) = I;
-    }
   };
+  constexpr int U = VW == 1 ? 8 : 4;   // tiles in flight
   for (int c0 = 0; c0 < nchunks; c0 += kScanTiles) {
     const int cn = min(kScanTiles, nchunks - c0);
     __syncthreads();
-    for (int c = w; c < cn; c += 4) {
-      const int t = (c0 + c) * kC + lane;
-      const float gt = (t < len) ? load_gate(a.gt, (int64_t)(bos + t) * a.H + h, a.gate_bf16) : 0.f;
-      const float tot = wave_sum(-gt * gh);
-      if (lane == 0) sF[c] = fast_exp2(tot);
-    }
+    tile_decays(a, c0, cn, bos, len, h, gh, w, lane, sF);
     __syncthreads();
     if (!on) continue;
     int c = 0;
+    auto at = [&](int u) { return ((int64_t)(cbase + c0 + c + u) * a.H + h) * E + e; };
     // (a copy of the loop without conditions: with them in it a batch's loads wait for the stores of the one before, 65x31
     // 2 x 9079 tokens, 2 heads 42 -> 54 us)
     auto batches = [&](auto all) {
-      for (; c + 4 <= cn; c += 4) {
-        f32x4 dM[4], dJ[4];
-        auto at = [&](int u) { return ((int64_t)(cbase + c0 + c + u) * a.H + h) * E + e; };
+      for (; c + U <= cn; c += U) {
+        float dM[U][VW], dJ[U][VW];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          dM[u] = *(const f32x4*)(a.chunk_mu + at(u));
-          dJ[u] = *(const f32x4*)(a.chunk_I + at(u));
+        for (int u = 0; u < U; ++u) {
+          load_vec<VW>(a.chunk_mu + at(u), dM[u]);
+          load_vec<VW>(a.chunk_I + at(u), dJ[u]);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          advance(at(u), dM[u], dJ[u], sF[c + u], decltype(all)::value || u == 0 || (u == 2 && a.every == 2));   // every: 1, 2 or 4
+        for (int u = 0; u < U; ++u)   // every: 1, 2 or 4
+          advance(at(u), dM[u], dJ[u], sF[c + u], decltype(all)::value || u % 4 == 0 || (u % 4 == 2 && a.every == 2));
       }
     };
     if (a.every == 1) batches(std::true_type{});
     else batches(std::false_type{});
     for (; c < cn; ++c) {
-      const int64_t off = ((int64_t)(cbase + c0 + c) * a.H + h) * E + e;
-      const f32x4 dM = *(const f32x4*)(a.chunk_mu + off), dJ = *(const f32x4*)(a.chunk_I + off);
-      advance(off, dM, dJ, sF[c], (c & (a.every - 1)) == 0);
+      float dM[VW], dJ[VW];
+      load_vec<VW>(a.chunk_mu + at(0), dM);
+      load_vec<VW>(a.chunk_I + at(0), dJ);
+      advance(at(0), dM, dJ, sF[c], (c & (a.every - 1)) == 0);
     }
   }
-  if (a.final_mu && on) {
-    f32x4 mu, I;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) { I[x] = SJ[x] + Ip; mu[x] = SM[x] * fast_rcp(I[x]); }
-    *(f32x4*)(a.final_mu + so) = mu;
-    *(f32x4*)(a.final_I + so) = I;
-  }
+  if (a.final_mu && on) store_state(a.final_mu + so, a.final_I + so);
 }
 
 // The same scan without the precision state: S_c = F_c S_{c-1} + Delta_c with Delta_c read from chunk_mu (fp32).
@@ -290,12 +290,7 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(ChunkArgs a) {
   for (int c0 = 0; c0 < nchunks; c0 += kScanTiles) {
     const int cn = min(kScanTiles, nchunks - c0);
     __syncthreads();
-    for (int c = w; c < cn; c += 4) {
-      const int t = (c0 + c) * kC + lane;
-      const float gt = (t < len) ? load_gate(a.gt, (int64_t)(bos + t) * a.H + h, a.gate_bf16) : 0.f;
-      const float tot = wave_sum(-gt * gh);
-      if (lane == 0) sF[c] = fast_exp2(tot);
-    }
+    tile_decays(a, c0, cn, bos, len, h, gh, w, lane, sF);
     __syncthreads();
     if (!on) continue;
     int c = 0;
@@ -403,10 +398,13 @@ int launch_tile_states(const ChunkArgs& a, int dtype, bool has_j, hipStream_t s)
                              a.init_I, a.final_mu, a.final_I, false, 1.f, kKernChunkStates, s);
   if (int rc = launch_tile_delta(a, dtype, has_j, s)) return rc;
   {
-    const int64_t E = (int64_t)a.dv * a.dk;
-    const int64_t blocks = (int64_t)a.n_seqs * a.H * ((E + 1023) / 1024);
-    if (blocks > 0x7fffffff) return PAL_E_DIM;
-    if (has_j) PAL_TIMED_LAUNCH(kKernChunkScan, s, chunk_scan_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+    const int64_t E = (int64_t)a.dv * a.dk, nh = (int64_t)a.n_seqs * a.H;
+    const int64_t blocks = nh * scan_blocks(E, 4);
+    if (nh * scan_blocks(E, 1) > 0x7fffffff) return PAL_E_DIM;
+    // few blocks: one entry per thread spreads them over more compute units, each of which moves only so much
+    // (1 x 16384 tokens, 4 heads of 48x48, 12 blocks: 59 -> 37 us; 1 x 8192, 16 of 64x64, 64 blocks: 37 -> 31)
+    if (has_j && blocks < 256) PAL_TIMED_LAUNCH(kKernChunkScan, s, chunk_scan_kernel<1>, dim3((unsigned)(nh * scan_blocks(E, 1))), dim3(256), 0, s, a);
+    else if (has_j) PAL_TIMED_LAUNCH(kKernChunkScan, s, chunk_scan_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, s, a);
     else PAL_TIMED_LAUNCH(kKernChunkScan, s, gla_scan_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
     PAL_HIP_LAUNCH_CHECK();
   }

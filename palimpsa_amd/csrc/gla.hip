@@ -723,12 +723,7 @@ __global__ __launch_bounds__(256) void gla_bwd_scan_kernel(ChunkArgs a, const fl
   for (int c_hi = nchunks; c_hi > 0; c_hi -= kScanTiles) {
     const int c0 = max(0, c_hi - kScanTiles), cn = c_hi - c0;
     __syncthreads();
-    for (int c = w; c < cn; c += 4) {
-      const int t = (c0 + c) * kC + lane;
-      const float gt = (t < len) ? load_gate(a.gt, (int64_t)(bos + t) * a.H + h, a.gate_bf16) : 0.f;
-      const float tot = wave_sum(-gt * gh);
-      if (lane == 0) sF[c] = fast_exp2(tot);
-    }
+    tile_decays(a, c0, cn, bos, len, h, gh, w, lane, sF);
     __syncthreads();
     if (!on) continue;
     int c = cn;
