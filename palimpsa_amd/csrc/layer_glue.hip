@@ -394,7 +394,6 @@ struct EpilogueArgs {
   float* part_w;        // backward: [workgroups][dv] partial sums of dweight
   float* part_D;        // backward: [H][token ranges]
   int tokens, H, dv;
-  int heads_iter;       // norm over all heads, backward: tokens per wave
   RowGeom rows;
   float eps;
 };
@@ -567,15 +566,12 @@ __global__ __launch_bounds__(64 * kRedWaves) void epilogue_bwd_reduce_kernel(Epi
 // ------------------------------------------------------------------ epilogue over all heads of a token
 // y = rmsnorm_{H dv}((o + x D) swish(gate)) weight  (palimpsa/layers/meta_mamba2.py:355-363: the gate is applied before
 // a norm that runs over the whole token).  One wave per token, 512 elements per pass (eight per lane, inside one head
-// since dv is a multiple of 8); a wave of the backward takes up to four tokens in turn and the four waves of a
-// workgroup add their sums over tokens (dweight, dD) in LDS, so that a workgroup leaves one partial row per 4 to 16 tokens.
-// Tokens per wave of the backward kernel: few tokens are spread over more waves, many leave fewer partial rows (16 heads of
-// 96, in us, with one, two and four: 1024 tokens 12, 16, 24, 6124 tokens 32, 31, 33; 16384 tokens of 16 heads of 128, the
-// sums over the partial rows included, 205, 184, 165).
-static int heads_iter(int tokens) {
-  const int n = (tokens + 3072) / 4096;
-  return n < 1 ? 1 : n > 4 ? 4 : n;
-}
+// since dv is a multiple of 8); a wave of the backward takes four tokens in turn and the four waves of a
+// workgroup add their sums over tokens (dweight, dD) in LDS, so that a workgroup leaves one partial row per 16 tokens.
+// (Tokens per wave of the backward kernel, 16 heads of 96, in us with one, two and four: 1024 tokens 12, 16, 24, 6124 tokens
+// 32, 31, 33; 16384 tokens of 16 heads of 128, the sums over the partial rows included, 205, 184, 165.  Four everywhere, as the
+// partial rows are memory that callers ask the size of and keep.)
+constexpr int kHeadsIter = 4;
 constexpr int kHeadsMaxCh = 8;     // passes of 512 elements: H dv <= 4096
 
 // NCH as in the backward kernel below: every fetch of the token is in flight before the first is used.  One token per wave, as
@@ -689,8 +685,8 @@ void epilogue_heads_bwd_kernel(EpilogueArgs A) {
     if (has_x) R.x = *(const Raw*)((const T*)A.t.x + off);
     if (has_gate) R.z = *(const Raw*)((const T*)A.t.gate + off);
   };
-  for (int it = 0; it < A.heads_iter; ++it) {
-    const int tok = (int)wave_id * A.heads_iter + it;
+  for (int it = 0; it < kHeadsIter; ++it) {
+    const int tok = (int)wave_id * kHeadsIter + it;
     if (tok >= A.tokens) break;
     const int64_t row = (int64_t)tok * HD;
     const float rstd = A.t.rstd[tok];
@@ -856,7 +852,7 @@ __global__ __launch_bounds__(64 * kRedWaves) void epilogue_heads_reduce_kernel(E
   }
 }
 
-static int heads_waves(const PalGlueDims* d) { return (d->tokens + heads_iter(d->tokens) - 1) / heads_iter(d->tokens); }
+static int heads_waves(const PalGlueDims* d) { return (d->tokens + kHeadsIter - 1) / kHeadsIter; }
 
 static int check_glue_dims(const PalGlueDims* d) {
   if (!d) return PAL_E_NULL;
@@ -918,7 +914,6 @@ static void fill_epilogue(EpilogueArgs& A, const PalGlueDims* d, const PalEpilog
   A.t = *t;
   A.tokens = d->tokens; A.H = d->n_heads; A.dv = d->dv;
   A.rows = row_geom(d->dv, d->n_heads, d->tokens);
-  A.heads_iter = heads_iter(d->tokens);
   A.eps = d->eps;
   A.part_w = nullptr; A.part_D = nullptr;
 }
