@@ -81,6 +81,12 @@ extern "C" {
  * scratch, their contents afterwards are undefined, and a short pass may be run without tiles. */
 #define PAL_FLAG_OUTPUTS_ONLY 16384u
 
+/* pal_chunk_fwd only: chunk_mu and chunk_I are scratch as well, and large passes over sequences of one length may keep the state
+ * of every second or fourth tile and walk on from it.  The results then differ, within the rounding of the states between,
+ * from those of a pass that keeps every tile's: for passes that nobody expects to equal another grouping of the same
+ * sequences bit for bit, such as the windows of one long sequence. */
+#define PAL_FLAG_SPARSE_STATES 32768u
+
 /* error codes (negative) */
 #define PAL_OK 0
 #define PAL_E_NULL -1        /* required pointer is NULL                      */

@@ -20,6 +20,7 @@ PAL_FLAG_STATE_MU_BF16 = 2048   # pal_recurrent_fwd: mu kept in bf16 between cal
 PAL_FLAG_STATES_ONLY = 4096     # pal_chunk_fwd: tile-start states only, outputs untouched
 PAL_FLAG_GLA_NO_TILES = 8192    # pal_gla_chunk_fwd / bwd: no tile states in memory (see pal_gla_walk_applies)
 PAL_FLAG_OUTPUTS_ONLY = 16384   # pal_chunk_fwd: the tile-start states are not needed afterwards
+PAL_FLAG_SPARSE_STATES = 32768  # pal_chunk_fwd: nor need every tile's be kept during the call
 PAL_CHUNK = 64
 
 PAL_E_NULL, PAL_E_DIM, PAL_E_HEADDIM, PAL_E_DTYPE, PAL_E_VARLEN_BATCH = -1, -2, -3, -4, -5

@@ -463,7 +463,6 @@ extern "C" int pal_chunk_fwd_static(const PalDims* d, const PalFwdTensors* t, vo
   tt.chunk_I = base + PAL_STATIC_SCRATCH_BYTES / (2 * sizeof(float));
   ChunkArgs a;
   fill_chunk_args(a, d, &tt);
-  a.every = out_tiles_per_state(a);
   hipStream_t s = (hipStream_t)stream;
   // every slot the output kernel reads is written by the state kernels of this call first: nothing has to start at zero
   if (int rc2 = launch_tile_states(a, d->dtype, true, s)) return rc2;
@@ -495,7 +494,7 @@ extern "C" int pal_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void* str
   }
   ChunkArgs a;
   fill_chunk_args(a, d, t);
-  if (d->flags & PAL_FLAG_OUTPUTS_ONLY) a.every = out_tiles_per_state(a);
+  if (d->flags & PAL_FLAG_SPARSE_STATES) a.every = out_tiles_per_state(a);
   hipStream_t s = (hipStream_t)stream;
   if (int rc2 = launch_tile_states(a, d->dtype, true, s)) return rc2;
   return launch_out(a, d->dtype, s);

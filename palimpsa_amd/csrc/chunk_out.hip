@@ -1,7 +1,7 @@
 // Chunked Palimpsa forward, outputs: chunk_out_kernel.
 //
 // From the state at the start of every tile (chunk_states.hip, or the two kernels of chunk_fwd.hip) all tiles of 64
-// tokens are worked in parallel (large passes that keep no states: walks of up to four tiles, see out_tiles_per_state).
+// tokens are worked in parallel (PAL_FLAG_SPARSE_STATES: walks of up to four tiles, see out_tiles_per_state).
 // Inside a tile the recurrence is run token by token on the vector units in fp32,
 //   M <- f_t M + v_t k_t^T,   I <- f_t I + b_t (k_t*k_t)^T + (1 - f_t) Ip,   o_t = scale (M / I) q_t
 // (the naive recurrence, chunk_palimpsa_forgetting_scalar.py:712-717 of the reference; its associative scan over a
@@ -416,7 +416,8 @@ static int launch_out_t(const ChunkArgs& a, hipStream_t s) {
 // pass's writes and this kernel's reads; what it costs is the serial length.  States and outputs together, in us, with 1, 2, 4
 // and 8 tiles to a state: 65536 tokens, 16 heads of 128x128 (65536 waves a window) 3925, 3663, 3524, 3534; 2 x 4096, 16 of
 // 128x128 (32768) 478, 424, 410, 424; 8 x 2048, 12 of 64x64 (12288) 182, 177, 188, 216; 4 x 2048, 6 of 96x192 (13824) 240,
-// 235, 263, 304; 16 x 512, 24 of 48x48 (6912) 137, 142, 159, 193.
+// 235, 263, 304; 16 x 512, 24 of 48x48 (6912) 137, 142, 159, 193.  A walk carries the state on unrounded where a kept one went
+// through (mu, I), so only callers that ask for it get walks: a document alone otherwise gives the bits that it gives in a pack.
 int out_tiles_per_state(const ChunkArgs& a) {
   if (a.flags & PAL_FLAG_VARLEN) return 1;
   const int64_t tiles = (a.T + kC - 1) / kC;

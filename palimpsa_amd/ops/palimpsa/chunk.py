@@ -41,9 +41,6 @@ def _count_chunks(T: int, B: int) -> int:
 _WINDOW_STATE_BYTES = 512 << 20
 
 
-_SHORT_PASS = 1024   # tokens up to which pal_chunk_fwd may run a pass without gradients token by token
-
-
 def _window_tiles(H: int, dv: int, dk: int) -> int:
     return max(16, _WINDOW_STATE_BYTES // (2 * 4 * H * dv * dk))
 
@@ -51,7 +48,8 @@ def _window_tiles(H: int, dv: int, dk: int) -> int:
 def _windowed_forward(p, scale, output_uncertainty, o, o_var, final_mu, final_I, window: int) -> None:
     """Forward of one sequence (B == 1) in segments of ``window`` tiles, each started from the final
     state of the one before.  Same kernels and same tiles as the single call; the state crosses a
-    segment boundary as (mu, I), which costs one fp32 rounding per boundary."""
+    segment boundary as (mu, I), which costs one fp32 rounding per boundary, and inside a segment only the states of every
+    second or fourth tile may be kept."""
     dev = p.q.device
     _, T, H, _ = p.v.shape
     seg = window * L.PAL_CHUNK
@@ -69,9 +67,7 @@ def _windowed_forward(p, scale, output_uncertainty, o, o_var, final_mu, final_I,
         for j in range(n_seg):
             s, e = j * seg, min(T, (j + 1) * seg)
             out_mu, out_I = (final_mu, final_I) if (n_seg - 1 - j) % 2 == 0 else scratch
-            flags = L.PAL_FLAG_STORE_FINAL | L.state_pass_flags()
-            if e - s > _SHORT_PASS:   # (a shorter one would take the token-serial kernel and round its state differently)
-                flags |= L.PAL_FLAG_OUTPUTS_ONLY
+            flags = L.PAL_FLAG_STORE_FINAL | L.PAL_FLAG_SPARSE_STATES | L.state_pass_flags()
             if cur_mu is not None:
                 flags |= L.PAL_FLAG_HAS_INIT
             if output_uncertainty:

@@ -124,31 +124,36 @@ def test_scaled_and_plain_tiles(gpu_device, state_pass_mode, dk, dv, case):
     assert hp.max_abs(o.nan_to_num(), o_ref.nan_to_num()) <= hp.BF16_OUT_ABS_TOL
 
 
-@pytest.mark.parametrize("B,dtype,case", [(16, torch.bfloat16, "usual"), (8, torch.bfloat16, "usual"), (16, torch.bfloat16, "strong"),
-                                          (16, torch.bfloat16, "huge"), (16, torch.bfloat16, "uncertainty"), (16, torch.float32, "usual")])
-def test_walks_over_several_tiles(gpu_device, B, dtype, case):
-    """Large passes without gradients keep the state of every fourth (second) tile only and walk on from it; a pass that
-    keeps all of them gives the same final states, and the outputs up to what the states between are rounded to."""
-    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
-    H, d, T = 24, 64, 1100     # a ragged last tile in a walk of its own two tiles
-    inp = _pal_inputs(B, T, H, d, d, 31, gpu_device)
+@pytest.mark.parametrize("tiles,dtype,case", [(257, torch.bfloat16, "usual"), (129, torch.bfloat16, "usual"),
+                                              (257, torch.bfloat16, "strong"), (257, torch.bfloat16, "huge"),
+                                              (257, torch.bfloat16, "uncertainty"), (257, torch.float32, "usual")])
+def test_walks_over_several_tiles(gpu_device, monkeypatch, tiles, dtype, case):
+    """The windows of a long sequence keep the state of every fourth (second) tile only and walk on from it; windows that
+    keep all of them give the same final states, and the outputs up to what the states between are rounded to."""
+    from palimpsa_amd import _lib
+    from palimpsa_amd.ops.palimpsa import chunk as chunk_mod, chunk_palimpsa
+    H, d = 24, 64
+    T = 64 * (2 * tiles - 1) - 20     # the last window ends in a ragged tile; a walk of one or two tiles ends the first
+    monkeypatch.setattr(chunk_mod, "_WINDOW_STATE_BYTES", tiles * 2 * 4 * H * d * d)
+    inp = _pal_inputs(1, T, H, d, d, 31, gpu_device)
     inp = {n: x.to(dtype) if n in "qkvb" else x for n, x in inp.items()}
     if case == "strong":
         inp["g"] = torch.linspace(0.5, 90.0, H, device=gpu_device)
     gen = torch.Generator().manual_seed(32)
-    mu0 = (torch.randn(B, H, d, d, generator=gen) * 0.2).to(gpu_device)
-    I0 = (torch.rand(B, H, d, d, generator=gen) + 0.5).to(gpu_device) * (1e24 if case == "huge" else 1.0)
+    mu0 = (torch.randn(1, H, d, d, generator=gen) * 0.2).to(gpu_device)
+    I0 = (torch.rand(1, H, d, d, generator=gen) + 0.5).to(gpu_device) * (1e24 if case == "huge" else 1.0)
     kw = dict(initial_mu_state=mu0, initial_I_state=I0, output_final_state=True, output_uncertainty=case == "uncertainty")
     with torch.no_grad():
         o, mu, I = chunk_palimpsa(**inp, **kw)
-    v = inp.pop("v").requires_grad_(True)
-    o_all, mu_all, I_all = chunk_palimpsa(v=v, **inp, **kw)
+        monkeypatch.setattr(_lib, "PAL_FLAG_SPARSE_STATES", 0)
+        o_all, mu_all, I_all = chunk_palimpsa(**inp, **kw)
     assert torch.equal(mu, mu_all) and torch.equal(I, I_all)
-    for x, y in zip(*((z if isinstance(z, tuple) else (z,)) for z in (o, o_all))):
+    o, o_all = ((z if isinstance(z, tuple) else (z,)) for z in (o, o_all))
+    for x, y in zip(o, o_all):
         if dtype == torch.float32:
             assert hp.max_rel(x, y) <= hp.FP32_REL_TOL
         else:
-            assert hp.max_abs(x.float(), y.detach().float()) <= hp.BF16_OUT_ABS_TOL
+            assert hp.max_abs(x.float(), y.float()) <= hp.BF16_OUT_ABS_TOL
 
 
 @pytest.mark.parametrize("T", [64, 64 * 9 + 5, 64 * 21])
