@@ -157,23 +157,25 @@ __device__ __forceinline__ float wave_inclusive_scan(float x, int lane) {
   return x + (row == 0 ? 0.f : row == 1 ? t0 : row == 2 ? t0 + t1 : (t0 + t1) + t2);
 }
 
-// Decays over the tiles [c0, c0 + cn) of a sequence, by the four waves of a scan's workgroup.  Eight tiles' gates are fetched
-// before the first is used: one at a time, this set-up is a chain of fetches that took longer than the scan itself (1 x 16384
+// Decays over the tiles [c0, c0 + cn) of a sequence, by the four waves of a scan's workgroup in turn.  A wave fetches eight tiles'
+// gates before the first is used: one at a time, this set-up is a chain of fetches that took longer than the scan itself (1 x 16384
 // tokens, 4 heads of 48x48: 72 us, so 59).
 __device__ __forceinline__ void tile_decays(const ChunkArgs& a, int c0, int cn, int bos, int len, int h, float gh, int w, int lane,
                                             float* sF) {
   constexpr int N = 8;
-  for (int c = N * w; c < cn; c += 4 * N) {
+  for (int c = w; c < cn; c += 4 * N) {
     float gt[N];
 #pragma unroll
     for (int u = 0; u < N; ++u) {
-      const int t = (c0 + c + u) * kC + lane;
+      const int t = (c0 + c + 4 * u) * kC + lane;
       gt[u] = t < len ? load_gate(a.gt, (int64_t)(bos + t) * a.H + h, a.gate_bf16) : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < N; ++u) {
-      const float tot = wave_sum(-gt[u] * gh);
-      if (lane == 0 && c + u < cn) sF[c + u] = fast_exp2(tot);
+      if (c + 4 * u < cn) {
+        const float tot = wave_sum(-gt[u] * gh);
+        if (lane == 0) sF[c + 4 * u] = fast_exp2(tot);
+      }
     }
   }
 }

@@ -256,11 +256,17 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(ChunkArgs a) {
     };
     if (a.every == 1) batches(std::true_type{});
     else batches(std::false_type{});
-    for (; c < cn; ++c) {
-      float dM[VW], dJ[VW];
-      load_vec<VW>(a.chunk_mu + at(0), dM);
-      load_vec<VW>(a.chunk_I + at(0), dJ);
-      advance(at(0), dM, dJ, sF[c], (c & (a.every - 1)) == 0);
+    if (const int rest = cn - c; rest > 0) {   // fetched together too
+      float dM[U - 1][VW], dJ[U - 1][VW];
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (u < rest) {
+          load_vec<VW>(a.chunk_mu + at(u), dM[u]);
+          load_vec<VW>(a.chunk_I + at(u), dJ[u]);
+        }
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (u < rest) advance(at(u), dM[u], dJ[u], sF[c + u], ((c + u) & (a.every - 1)) == 0);
     }
   }
   if (a.final_mu && on) store_state(a.final_mu + so, a.final_I + so);
