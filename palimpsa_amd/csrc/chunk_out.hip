@@ -182,15 +182,16 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   };
   const int64_t orow = ((int64_t)t0 * H + h) * dv + r0 + d0 + dsel;
 
-  auto decay_of = [&](int t) {
-    const float x = t == tid ? gt : t < clen ? load_gate(a.gt, (int64_t)(t0 + t) * H + h, a.gate_bf16) : 0.f;
-    return fast_exp2(-x * gh);
+  // fn(t, f_t) for the tokens of this thread, whole tiles; only walks of several tiles have more than the one whose gate is there
+  auto tokens = [&](auto fn) {
+    if (tid < a.every * kC && tid - lane < clen) fn(tid, fast_exp2(-gt * gh));
+    for (int t = tid + NT; t < a.every * kC && t - lane < clen; t += NT)
+      fn(t, fast_exp2(-(t < clen ? load_gate(a.gt, (int64_t)(t0 + t) * H + h, a.gate_bf16) : 0.f) * gh));
   };
   if constexpr (kMayScale) {   // each wave: the decays of its tiles
     if (tid == 0) *sForm = 1;
     __syncthreads();
-    for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {
-      const float f = decay_of(t);
+    tokens([&](int t, float f) {
       float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
       const int s = lane & (kOT - 1);
       // (each shift before its select: a lane that is switched off hands nothing on)
@@ -203,7 +204,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       if (!__all(F >= kMinDecay && F <= 1.f && Ip <= kMinDecay * kMaxScaled)) *sForm = 0;
       sFC[4 * t] = F;
       sFC[4 * t + 3] = f;
-    }
+    });
     __syncthreads();
   }
 
@@ -239,9 +240,13 @@ void chunk_out_kernel(ChunkArgs a, int W) {
         if constexpr (DN & 1) piece(std::integral_constant<int, 1>{}, DN - 1);
       }
     }
-    for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {   // (the thread that left f and F there)
-      const float f = kMayScale ? sFC[4 * t + 3] : decay_of(t), F = SCALED ? sFC[4 * t] : f, inv = SCALED ? fast_rcp(F) : 1.f;
-      *(f32x4*)&sFC[4 * t] = f32x4{F, SCALED ? Ip * inv : (1.f - f) * Ip, inv, f};
+    if constexpr (kMayScale) {
+      for (int t = tid; t < a.every * kC && t - lane < clen; t += NT) {   // (the thread that left f and F there)
+        const float f = sFC[4 * t + 3], F = SCALED ? sFC[4 * t] : f, inv = SCALED ? fast_rcp(F) : 1.f;
+        *(f32x4*)&sFC[4 * t] = f32x4{F, SCALED ? Ip * inv : (1.f - f) * Ip, inv, f};
+      }
+    } else {
+      tokens([&](int t, float f) { *(f32x2*)&sFC[4 * t] = f32x2{f, (1.f - f) * Ip}; });
     }
     // rows and columns beyond the head dims stay zero in both buffers
     if (DKP != dk || VR > dv - r0) {
