@@ -346,8 +346,8 @@ __global__ __launch_bounds__(256) void prologue_bwd_kernel(PrologueArgs A) {
     acc_bs = group_sum(acc_bs, GL);
     if (l == 0) { sRed[at.slot][0] = acc_dt; sRed[at.slot][1] = acc_bs; }
     __syncthreads();
-    if ((int)threadIdx.x < 2 * G.heads) {
-      const int hs = threadIdx.x >> 1, which = threadIdx.x & 1;
+    for (int x2 = threadIdx.x; x2 < 2 * G.heads; x2 += 256) {   // (rows of eight elements: up to 256 heads, two sums each)
+      const int hs = x2 >> 1, which = x2 & 1;
       float sum = 0.f;
       for (int x = 0; x < G.tokens; ++x) sum += sRed[x * G.heads + hs][which];
       const int64_t head = (blockIdx.x - at.range * G.groups) * G.heads + hs;

@@ -392,6 +392,8 @@ def test_mamba_layer_slice_end_to_end(gpu_device):
     ((3, 41), 4, 16, 64, 64),     # q, k of four heads each: the third and fourth gradient are fetched late
     ((77,), 5, 40, 16, 16),       # an odd number of q, k heads beside groups of eight
     ((130,), 64, 64, 8, 16),      # more heads than row slots
+    ((40,), 256, 256, 8, 8),      # a head to every thread: more sums per head than threads
+    ((9,), 4, 512, 16, 8),        # two groups of them
 ])
 def test_rows_over_heads_and_tokens(gpu_device, lead, Hqk, H, dk, dv):
     test_prologue_forward_backward(gpu_device, lead, Hqk, H, dk, dv, torch.bfloat16, True)
