@@ -139,6 +139,11 @@ __device__ __forceinline__ bool walk_item(const ChunkArgs& a, const WalkPlan& p,
   return true;
 }
 
+// lane l of a row of 16 gets lane l + N's value, zero from beyond the row
+template <int N>
+__device__ __forceinline__ float row_shl_zero(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x100 + N, 0xf, 0xf, true));
+}
 // inclusive prefix sum over the 64 lanes of a wave: four shifted adds inside each row of 16 lanes (DPP
 // row_shr with zero fill), then the totals of the rows before (lane 15 of each, read as scalars)
 template <int N>

@@ -8,9 +8,11 @@
 // What bounds it is vector issue: a workgroup's 16 waves sit on one compute unit.  So
 // * a wave stages its rows through LDS of its own (no barrier) in pieces of P tokens: 16-byte requests and one conversion per
 //   element in place of 2- to 8-byte requests of every lane for itself, four lane groups over;
-// * the first walk takes the tokens of a piece times their decay to its end (a scan over the piece's gates), so that an entry costs
-//   three instructions a token, k*k included, and the decay itself two per piece;
+// * the first walk takes the tokens of a piece times their decay to its end (a scan from there over the piece's gates), so that an
+//   entry costs three instructions a token, k*k included, and the decay itself two per piece;
 // * outputs of four tokens are summed over the lanes together.
+// Errors against float64 are those of the walk of one wave: outputs 1.0e-7 rms, precision state 3.5e-8 to 5e-8, for decay rates
+// of 0.5 to 16 a token (T = 200 to 512, 32x32 to 128x128); B=2 T=256 H=4 32x32 fp32 40.4 -> 8.9 us.
 #include <type_traits>
 
 #include "chunk_common.h"
@@ -112,17 +114,21 @@ __global__ __launch_bounds__(64 * NW) void recurrent_seg_kernel(RecArgs a) {
   if (w < NW - 1) {
     float tot = 0.f;
     for (int t0 = 0; t0 < T; t0 += P) {
-      float c = gate(t0);
-      c += row_shr_zero<1>(c);
-      c += row_shr_zero<2>(c);
-      c += row_shr_zero<4>(c);
-      if constexpr (P > 8) c += row_shr_zero<8>(c);
-      const float end = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), P - 1));
+      const float c = gate(t0);
+      // log2 of the decay after a token to the end of the piece: the tokens after it alone.  (As the difference of two sums from
+      // the start of the piece it carried the rounding of all of them: 1e-4 of the weight behind a token of decay e^-1e4, NaN
+      // behind one of zero.)
+      float after = row_shl_zero<1>(c);
+      after += row_shl_zero<1>(after);
+      after += row_shl_zero<2>(after);
+      after += row_shl_zero<4>(after);
+      if constexpr (P > 8) after += row_shl_zero<8>(after);
+      const float end = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, after + c)));
       tot += end;
       staged();
       put(false);
       if (lane < P) {
-        const float wt = fast_exp2(end - c);
+        const float wt = fast_exp2(after);
 #pragma unroll
         for (int r = 0; r < 4; ++r) *(f32x2*)&sw[lane * STRIDE + oR + 2 * r] = f32x2{wt * (float)rv[r], wt * (float)rb[r]};
       }
@@ -152,8 +158,9 @@ __global__ __launch_bounds__(64 * NW) void recurrent_seg_kernel(RecArgs a) {
     float* end = sw + lane;
 #pragma unroll
     for (int e = 0; e < NPL; ++e) { end[64 * e] = M[e]; end[64 * (NPL + e)] = J[e]; }
-    // (a growth beyond fp32 must not turn entries that are zero into NaN)
-    if (lane == 0) sF[w] = fminf(fast_exp2(tot), 3.4028235e38f);
+    // (a growth beyond fp32 must not turn entries that are zero into NaN; a NaN stays one)
+    const float F = fast_exp2(tot);
+    if (lane == 0) sF[w] = F > 3.4028235e38f ? 3.4028235e38f : F;
     request(0, true);
   }
   const int64_t so = ((int64_t)nh * dv + 4 * tile + grp) * DK;

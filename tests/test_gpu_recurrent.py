@@ -450,6 +450,43 @@ def test_sequences_in_segments(gpu_device, H, dk, dv, lens):
         assert hp.max_rel(mu0, mu_ref) <= 1e-5 and hp.max_rel(I0, I_ref) <= 1e-5
 
 
+def _state_behind_a_border(gpu_device, H, dk, dv, T, gt):
+    """(outputs, mu, I) of a run in segments and the oracle's, from a weak prior: the tokens after the last border start from
+    what the folded segments left."""
+    inp = po.make_inputs(1, T, H, dk, dv, seed=dk + T)
+    inp["gt"], inp["g"], inp["Ip"] = gt, torch.ones(H), torch.full((H,), 1e-3)
+    ref = hp.oracle_forward(inp, dtype=torch.float64)
+    d = hp.to_device(inp, gpu_device)
+    out = _ops()(*[d[n] for n in ("q", "k", "v", "b", "gt", "g", "Ip")], output_final_state=True)
+    return out, (ref[0], ref[2], ref[3])
+
+
+# 16 segments of 16 tokens and a last one of a single token, staged by 16 and by 8 tokens; 8 of 15 and a last one of 8
+@pytest.mark.parametrize("decay", [1e4, 1e6, 1e9, float("inf"), float("nan")])
+@pytest.mark.parametrize("H,dk,dv,T,border", [(4, 32, 32, 241, 240), (4, 96, 64, 241, 240), (8, 192, 64, 113, 105)])
+def test_resets_before_a_segment_border(gpu_device, H, dk, dv, T, border, decay):
+    """A token that forgets everything, two tokens before the last border, among tokens that forget little."""
+    gt = 0.02 * torch.rand(1, T, H, generator=torch.Generator().manual_seed(T))
+    gt[:, border - 3] = decay
+    (o, mu, I), (o_ref, mu_ref, I_ref) = _state_behind_a_border(gpu_device, H, dk, dv, T, gt)
+    for x, r in ((o[:, border:], o_ref[:, border:]), (mu, mu_ref), (I, I_ref)):
+        x = x.cpu()
+        assert torch.equal(torch.isnan(x), torch.isnan(r))
+        assert hp.max_rel(x.nan_to_num(), r.nan_to_num()) <= 1e-5   # fp32 sums of the few tokens since
+
+
+@pytest.mark.parametrize("rate", [0.5, 2.0, 6.0])
+@pytest.mark.parametrize("H,dk,dv", [(4, 32, 32), (4, 96, 64)])
+def test_segments_keep_the_precision_of_one_walk(gpu_device, H, dk, dv, rate):
+    """The precision state of ordinary gates, one token after a border: a token's weight carries the rounding of the decays
+    after it alone, whose sum is small where the weight counts (a sum over all of its piece is not)."""
+    T = 241
+    gt = 2 * rate * torch.rand(1, T, H, generator=torch.Generator().manual_seed(T))
+    (_, _, I), (_, _, r) = _state_behind_a_border(gpu_device, H, dk, dv, T, gt)
+    # a few roundings of 2^-25 rms each for a token's product and decay: below one of 2^-23
+    assert (I.double().cpu() - r).norm() <= 2.0 ** -23 * r.norm()
+
+
 @pytest.mark.parametrize("rows", ["fp32", "bf16"])
 @pytest.mark.parametrize("B,T,H,dk,dv,Hq", [(1, 1, 2, 48, 48, 2), (2, 70, 4, 32, 64, 2), (1, 257, 3, 64, 48, 3), (1, 777, 4, 48, 48, 4)])
 def test_short_chunked_passes_without_tiles(gpu_device, rows, B, T, H, dk, dv, Hq):
