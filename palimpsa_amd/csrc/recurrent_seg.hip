@@ -319,12 +319,22 @@ int launch_recurrent_seg(const RecArgs& a, int dtype, int waves, hipStream_t s) 
 //   1536 (B=2 H=16 96x192)                 T=32   17.3:  15.5  22.3  49.8     T=256  107  :  73.0  73.9  95.3
 //   2048 (B=8 H=16 64x64)                  T=32   14.5:  15.4  25.2  58.6     T=256   84.0:  63.4  68.3  95.3
 //   4096 (B=16 H=16 64x64 fp32)            T=32   21.3:  30.6  55.0 129       T=256  123  : 140   150   206
+// Four segments of two tokens cost more than they save, and so do segments whose workgroups (34 KB of LDS at 128 key columns, 67 at
+// 256) do not all find room at once, until the walk is long: the line grows with waves times columns (us of the kernel alone).
+//   784 (64 columns)                       T=8     5.6:   7.2     1024    T=13    7.0:   7.7
+//   576 (B=6 H=4 256x96 fp32)              T=10    8.2:  17.9
+//   576 (B=3 H=16 256x48 fp32)             T=34   22.2:  29.6
+//   768 (B=4 H=12 256x64)                  T=120  73.2:  59.1
+//   1920 (B=5 H=16 128x96 fp32)            T=54   31.6:  39.5
+//   1920 (B=30 H=8 128x32)                 T=111  62.3:  58.4
+// Over 1500 drawn calls (16 to 256 columns, 4 to 1448 tokens, up to 2048 waves) 1091 are more than a fifth faster than with one wave
+// and 12 more than 5 % slower, 1.27 times at most; with a line at 8 and 48 tokens for all columns it was 124, 2.33 times at most.
 int recurrent_segments(const PalDims* d) {
   const int64_t waves = (int64_t)d->n_seqs * d->n_heads * (d->dv / 4);
   const int64_t len = (d->flags & PAL_FLAG_VARLEN) ? d->seq_len / d->n_seqs : d->seq_len;   // the mean of a packed batch
   if (waves <= 256 && len >= 192 && d->dk <= 128) return 16;
   if (waves <= 512 && len >= 64) return 8;
-  if (waves <= 2048 && len >= (waves <= 1024 ? 8 : 48)) return 4;
+  if (waves <= 2048 && len >= 12 && 4000 * len >= waves * d->dk) return 4;
   return 1;
 }
 

@@ -414,10 +414,11 @@ def test_decode_with_the_mean_state_kept_in_bf16(gpu_device):
 
 
 @pytest.mark.parametrize("H,dk,dv,lens", [
-    (3, 48, 48, [8]), (3, 32, 32, [33]), (2, 16, 16, [63]), (1, 64, 80, [15]),      # 4 waves
+    (3, 48, 48, [8]), (3, 32, 32, [33]), (2, 16, 16, [63]), (1, 64, 80, [15]),      # 1 and 4 waves
     (2, 64, 80, [64]), (2, 32, 48, [191]), (2, 256, 64, [65]), (2, 192, 16, [200]),   # 8: at most for wide keys
     (1, 128, 64, [192]), (2, 96, 96, [257]), (1, 16, 16, [255]),                      # 16
     (8, 96, 192, [48, 48, 48, 48]), (16, 64, 64, [64, 65]),                           # 4 for more value rows
+    (3, 48, 48, [11]), (3, 48, 48, [12]), (40, 256, 64, [40]), (40, 256, 64, [41]),   # beside the line, narrow and wide keys
     (2, 32, 32, [1, 90, 0, 5, 64]),                             # documents shorter than their segments, and an empty one
 ])
 def test_sequences_in_segments(gpu_device, H, dk, dv, lens):
