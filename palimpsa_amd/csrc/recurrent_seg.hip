@@ -338,13 +338,29 @@ int recurrent_segments(const PalDims* d) {
   return 1;
 }
 
-// Outputs and final states of a short pass (pal_chunk_fwd): its three kernels take 13 us for 8 tokens and 25 for 64 to 256, most of
-// it the 64 tokens of a tile one after the other.  The walk in segments costs by the token, so the line is one of work, and of 1024
-// tokens, beyond which a segment is as long as a tile (walk / tiles, us: H=16 48x48 T=256 12.2 / 25.6, T=777 29.1 / 32.8, T=1536 45.4 /
-// 42.2; 128x128 T=128 19.7 / 24.4, T=256 34.8 / 31.3; B=8 H=16 64x64 T=64 22.0 / 25.2, T=128 36.2 / 30.9).
+// Whether outputs and final states of a short pass (pal_chunk_fwd) come from the walk: its three kernels take 13 us for 8 tokens and
+// 25 for 64 to 256, most of it the 64 tokens of a tile one after the other, the walk costs by the token.  Both are estimated in us.
+// The walk is the longer of its chain (the waves of a sequence share a compute unit's issue, so segments do not shorten it much:
+// 0.5 ns a token and key column; workgroups of eight waves with 100 KB of LDS take turns beyond 256 of them) and of the chip's issue
+// (33 ps a token and wave and 2 ps for each key column, more with the uncertainty output, most in the form of many rows per
+// wave); the tiles are a tile's chain, the traffic of their states and their issue.
+// Walk / tiles, us: H=16 48x48 T=256 12.2 / 25.6, T=777 29.1 / 32.8, T=1536 45.4 / 42.2; 128x128 T=128 19.7 / 24.4, T=256 34.8 / 31.3;
+// B=8 H=16 64x64 T=64 22.0 / 25.2, T=128 36.2 / 30.9; one wave a sequence: 74 x 2 heads 16x64 fp32 T=232 60.9 / 34.1, 129 x 1 32x64 T=111
+// 37.5 / 30.7, 61 x 12 heads 256x64 fp32 T=4 45.6 / 138; uncertainty: 23 x 12 heads 16x128 T=21 51.1 / 24.9.
+// Over 5000 drawn calls (16 to 256 key columns, 4 to 1024 tokens, 5e4 to 1e7 entries) 4120 are more than a fifth faster than by tiles
+// and 38 more than 5 % slower, 1.35 times at most (by work alone, up to 1e7 entries, 299, 3.1 times at most).  Not beyond 1024 tokens and
+// 1e7 entries, where nothing was measured.
 bool short_pass(const PalDims* d) {
   if (!recurrent_dk_supported(d->dk) || (d->flags & PAL_FLAG_VARLEN) || d->seq_len > 1024) return false;
-  return (int64_t)d->seq_len * d->n_seqs * d->n_heads * (d->dv / 4) * d->dk <= 10000000;
+  const int T = d->seq_len, dk = d->dk, segments = recurrent_segments(d), tiles = (T + PAL_CHUNK - 1) / PAL_CHUNK;
+  const int64_t waves = (int64_t)d->n_seqs * d->n_heads * (d->dv / 4);
+  if (waves * T * dk > 10000000) return false;
+  double chain = 5e-4 * T * dk + 0.03 * T / segments;
+  if (segments == 8 && dk > 128 && waves > 256) chain *= 2;
+  const double uncertainty = !(d->flags & PAL_FLAG_HAS_VAR) ? 0.0 : segments == 1 ? 83e-6 : 23e-6;
+  const double issue = (33e-6 + 2e-6 * dk + uncertainty) * waves * T;
+  const double by_tiles = 10 + 0.16 * (T < PAL_CHUNK ? T : PAL_CHUNK) + 0.4 * tiles + (0.6e-6 * T + 13e-6 * (1 + tiles)) * waves * dk;
+  return 6.7 + (chain > issue ? chain : issue) <= by_tiles;
 }
 
 }  // namespace pal

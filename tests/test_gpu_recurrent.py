@@ -489,7 +489,8 @@ def test_segments_keep_the_precision_of_one_walk(gpu_device, H, dk, dv, rate):
 
 
 @pytest.mark.parametrize("rows", ["fp32", "bf16"])
-@pytest.mark.parametrize("B,T,H,dk,dv,Hq", [(1, 1, 2, 48, 48, 2), (2, 70, 4, 32, 64, 2), (1, 257, 3, 64, 48, 3), (1, 777, 4, 48, 48, 4)])
+@pytest.mark.parametrize("B,T,H,dk,dv,Hq", [(1, 1, 2, 48, 48, 2), (2, 70, 4, 32, 64, 2), (1, 257, 3, 64, 48, 3), (1, 777, 4, 48, 48, 4),
+                                            (1, 777, 16, 48, 48, 16)])
 def test_short_chunked_passes_without_tiles(gpu_device, rows, B, T, H, dk, dv, Hq):
     """chunk_palimpsa without autograd on few tokens runs the token-serial kernels: outputs, uncertainty in the dtype of the rows and
     final states against the oracle, and with autograd (tiles) at the same bars."""
