@@ -78,7 +78,8 @@ extern "C" {
 #define PAL_FLAG_GLA_NO_TILES 8192u
 
 /* pal_chunk_fwd only: the tile-start states are not needed after the call (no backward will follow): chunk_mu and chunk_I are
- * scratch, their contents afterwards are undefined, and a short pass may be run without tiles. */
+ * scratch, their contents afterwards are undefined, and a short pass may be run without tiles (its results then differ from
+ * those by tiles within the rounding of the rows). */
 #define PAL_FLAG_OUTPUTS_ONLY 16384u
 
 /* pal_chunk_fwd only: chunk_mu and chunk_I are scratch as well, and large passes over sequences of one length may keep the state

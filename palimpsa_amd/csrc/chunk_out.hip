@@ -422,7 +422,8 @@ static int launch_out_t(const ChunkArgs& a, hipStream_t s) {
 // and 8 tiles to a state: 65536 tokens, 16 heads of 128x128 (65536 waves a window) 3925, 3663, 3524, 3534; 2 x 4096, 16 of
 // 128x128 (32768) 478, 424, 410, 424; 8 x 2048, 12 of 64x64 (12288) 182, 177, 188, 216; 4 x 2048, 6 of 96x192 (13824) 240,
 // 235, 263, 304; 16 x 512, 24 of 48x48 (6912) 137, 142, 159, 193.  A walk carries the state on unrounded where a kept one went
-// through (mu, I), so only callers that ask for it get walks: a document alone otherwise gives the bits that it gives in a pack.
+// through (mu, I), so how many sequences share a call would show in the last bits of all of them (a document of a large packed pass
+// and the same one alone otherwise agree to 1e-6): only the windows of one sequence, which the library itself cuts, ask for walks.
 int out_tiles_per_state(const ChunkArgs& a) {
   if (a.flags & PAL_FLAG_VARLEN) return 1;
   const int64_t tiles = (a.T + kC - 1) / kC;

@@ -448,7 +448,8 @@ bool gla_walk_possible(const PalDims* d) {
 // meet: heads that are walked at a time, times columns.  Tiles / walks, us of kernels, T=2048 (96x192: 225 / 282 with 32 heads
 // in all, 408 / 285 with 64, 827 / 365 with 128; 96x96: 261 / 258 with 64, 493 / 287 with 128; 48x96: 197 / 236, 340 / 242).
 // Up to 64x64 one kernel forms the three gradients and walks are faster from 192 heads on only (194 / 224 with 128, T=512 149 / 111
-// with 384): not taken, so that a call's results do not depend on how many sequences it has.
+// with 384): not taken.  The line would lie in the middle of ordinary batch sizes, and a large batch of such heads agrees with its
+// sequences in small ones to 1e-6, which walks, whose states are rounded at other places, would end; wider heads do pay that.
 bool gla_walk_applies(const PalDims* d, int64_t longest) {
   if (!gla_walk_possible(d) || (d->flags & (PAL_FLAG_STATES_TWO_KERNELS | PAL_FLAG_STATES_ONE_PASS))) return false;
   const int64_t tiles = (longest + PAL_CHUNK - 1) / PAL_CHUNK;

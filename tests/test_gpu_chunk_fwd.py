@@ -307,6 +307,39 @@ def test_entry_points_compile_without_a_graph_break(gpu_device, backend, case):
         assert hp.max_rel(b_, a) <= 1e-6
 
 
+@pytest.mark.parametrize("rows", ["fp32", "bf16"])
+@pytest.mark.parametrize("lens", [[777, 30, 300], [9, 1100]])
+def test_equal_calls_give_equal_bits(gpu_device, rows, lens):
+    """A document alone (walked token by token where it is short), in a pack and with gradients takes different kernels: the
+    results agree to the rounding of the rows, and each of the calls repeats its own bits."""
+    ck, _ = _ops()
+    H, dk, dv = 4, 48, 64
+    dt = torch.float32 if rows == "fp32" else torch.bfloat16
+    d = hp.to_device(hp.rounded(po.make_inputs(1, sum(lens), H, dk, dv, seed=3), dt), gpu_device)
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0)], dtype=torch.int32, device=gpu_device)
+
+    def run(x, grad, **kw):
+        outs = []
+        for _ in range(2):
+            with torch.set_grad_enabled(grad):
+                y = dict(x, q=x["q"].detach().requires_grad_(grad))
+                outs.append([t.detach() for t in _call(ck, y, output_final_state=True, **kw)])
+        assert all(torch.equal(a, b) for a, b in zip(*outs))
+        return outs[0]
+
+    packs = [run(d, grad, cu_seqlens=cu) for grad in (False, True)]
+    for n, (a, b) in enumerate(zip(cu.tolist(), cu.tolist()[1:])):
+        doc = {k: (v[:, a:b].contiguous() if v.dim() > 1 else v) for k, v in d.items()}
+        alone = [run(doc, grad) for grad in (False, True)]
+        for o, mu, I in [[p[0][:, a:b], p[1][n:n + 1], p[2][n:n + 1]] for p in packs] + alone[1:]:
+            if rows == "fp32":
+                assert hp.max_rel(o, alone[0][0]) <= hp.CHUNK_FP32_OUT_TOL
+            else:
+                assert hp.max_abs(o.float(), alone[0][0].float()) <= hp.BF16_OUT_ABS_TOL
+            for x, r in ((mu, alone[0][1]), (I, alone[0][2])):
+                assert hp.max_rel(x, r) <= (hp.CHUNK_FP32_OUT_TOL if rows == "fp32" else STATE_REL_TOL)
+
+
 def test_library_ops_pass_opcheck(gpu_device):
     """torch.library.opcheck on the four ops: schema, fake implementation against the real one, autograd registration."""
     from palimpsa_amd.ops.palimpsa import _custom_ops as ops
