@@ -535,14 +535,14 @@ def bench_c0(torch, dev, steps, warmup, with_cpu):
 
     ms, med, kernels = timed_loop(torch, step, steps, warmup)
     bytes_alg = B * T * H * (4 * (2 * d + 2 * d) + 4 + 4 * d) + 2 * B * H * d * d * 4
-    k_ms = kernels.get("recurrent_fwd_kernel", {"avg_ms": float("nan")})["avg_ms"]
+    k_ms = kernels.get("recurrent_seg_kernel", {"avg_ms": float("nan")})["avg_ms"]
     out = {"workload": "c0: fused-recurrent forward fp32 B=2 T=256 H=4 dk=dv=32, final states",
            "tokens_per_s": B * T / (ms * 1e-3), "ms_per_step": ms, "ms_per_step_median": med, "kernels": kernels,
-           "roofline": {"bound": "hbm", "kernel": "recurrent_fwd_kernel", "achieved": bytes_alg / (k_ms * 1e-3) / 1e9,
+           "roofline": {"bound": "hbm", "kernel": "recurrent_seg_kernel", "achieved": bytes_alg / (k_ms * 1e-3) / 1e9,
                         "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": bytes_alg / (k_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
                         "traffic": None, "algorithmic_bytes_per_launch": bytes_alg, "avg_launch_ms": k_ms,
-                        "note": "256 dependent token steps on 64 waves: the launch is bound by serial latency "
-                                "(about 0.2 us per token), not by any throughput roofline"}}
+                        "note": "64 workgroups of 16 waves, a segment of 16 tokens walked twice by each wave: the call is bound by "
+                                "the launch and the host path, then by that chain, not by any throughput roofline"}}
     if with_cpu:
         from oracle import palimpsa_oracle as po
         t0 = time.perf_counter()
@@ -663,9 +663,9 @@ def bench_recurrent(torch, dev, steps, warmup):
 
     return {"workload": "token-serial forward, and forward+backward, B=8 T=2048 H=12 dk=dv=64 fp32 rows",
             "forward": {"tokens_per_s": B * T / (ms_f * 1e-3), "ms_per_step": ms_f, "ms_per_step_median": med_f, "kernels": k_f,
-                        "roofline": roof("recurrent_fwd_kernel", k_f, bytes_f,
-                                         "rows in, outputs out; 2048 dependent steps per wave with the state in registers: "
-                                         "bound by fp32 vector work and serial latency, not by HBM")},
+                        "roofline": roof("recurrent_seg_kernel", k_f, bytes_f,
+                                         "rows in, outputs out; four segments of 512 dependent steps, walked twice, with the "
+                                         "state in registers: bound by fp32 vector work and serial latency, not by HBM")},
             "forward_backward": {"tokens_per_s": B * T / (ms_fb * 1e-3), "ms_per_step": ms_fb, "ms_per_step_median": med_fb,
                                  "kernels": k_fb,
                                  "note": "sequences of 64 tokens or more: the backward of this entry point runs the "

@@ -31,6 +31,7 @@ enum KernelId {
   kKernGlaBwdStates,
   kKernGlaBwdTile,
   kKernBwdPartsSum,
+  kKernRecurrentSeg,
   kKernCount
 };
 

@@ -271,7 +271,7 @@ static int launch_nw(const RecArgs& a, hipStream_t s) {
   constexpr size_t lds = SegShape<NPL, NW>::lds;
   auto go = [&](auto kern) -> int {
     if (int rc = allow_lds((const void*)kern, lds)) return rc;
-    PAL_TIMED_LAUNCH(kKernRecurrentFwd, s, kern, dim3((unsigned)blocks), dim3(64 * NW), lds, s, a);
+    PAL_TIMED_LAUNCH(kKernRecurrentSeg, s, kern, dim3((unsigned)blocks), dim3(64 * NW), lds, s, a);
     return 0;
   };
   const int rc = (a.flags & PAL_FLAG_HAS_VAR) ? go(&recurrent_seg_kernel<TIn, NPL, NW, true>) : go(&recurrent_seg_kernel<TIn, NPL, NW, false>);
@@ -346,7 +346,7 @@ int recurrent_segments(const PalDims* d) {
 // wave); the tiles are a tile's chain, the traffic of their states and their issue.
 // Walk / tiles, us: H=16 48x48 T=256 12.2 / 25.6, T=777 29.1 / 32.8, T=1536 45.4 / 42.2; 128x128 T=128 19.7 / 24.4, T=256 34.8 / 31.3;
 // B=8 H=16 64x64 T=64 22.0 / 25.2, T=128 36.2 / 30.9; one wave a sequence: 74 x 2 heads 16x64 fp32 T=232 60.9 / 34.1, 129 x 1 32x64 T=111
-// 37.5 / 30.7, 61 x 12 heads 256x64 fp32 T=4 45.6 / 138; uncertainty: 23 x 12 heads 16x128 T=21 51.1 / 24.9.
+// 37.5 / 30.7, 9 x 1 256x96 fp32 T=137 30.0 / 52.7; uncertainty: 23 x 12 heads 16x128 T=21 51.1 / 24.9.
 // Over 5000 drawn calls (16 to 256 key columns, 4 to 1024 tokens, 5e4 to 1e7 entries) 4120 are more than a fifth faster than by tiles
 // and 38 more than 5 % slower, 1.35 times at most (by work alone, up to 1e7 entries, 299, 3.1 times at most).  Not beyond 1024 tokens and
 // 1e7 entries, where nothing was measured.
