@@ -179,10 +179,10 @@ __global__ __launch_bounds__(256) void chunk_delta_kernel(ChunkArgs a, int dvn) 
 }
 
 // ------------------------------------------------------------------ kernel 1b
-// Serial part of the forward: S_c = F_c S_{c-1} + Delta_c per state entry, fp32, pure streaming.
 // blocks of a (sequence, head) at vw entries per thread
 __host__ __device__ inline int scan_blocks(int64_t E, int vw) { return (int)((E + 256 * vw - 1) / (256 * vw)); }
 
+// Serial part of the forward: S_c = F_c S_{c-1} + Delta_c per state entry, fp32, pure streaming.
 // One thread per VW consecutive state entries of a (sequence, head), 256 VW entries per block.  Each slot of
 // chunk_mu / chunk_I is overwritten with the state at the START of its tile in (mu, I) form
 // (what the reference stores as intermediate_*_state, chunk_palimpsa_forgetting_scalar.py:187-188);

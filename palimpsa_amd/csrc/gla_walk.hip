@@ -6,7 +6,9 @@
 // (dv: k, q, dO; dk: v, dO, q, transposed), S in fp32.  With the tiles' states in memory this takes a pass that writes them
 // and a kernel that reads them per result, 37 KB a tile and head at 96x192: 1.3 GB of a training step's 2 GB.  Here S never leaves
 // the registers of the wave that uses it, the rows are read once per result, and dq needs no states kept from the forward.
-// B=8 T=2048 H=16 96x192, forward and backward: 813 -> 365 us, 1.3 GB at 3.6 TB/s.
+// B=8 T=2048 H=16 96x192, forward and backward: 813 -> 365 us, 1.3 GB at 3.6 TB/s.  Errors against float64 are those of the
+// kernels with tile states to three digits for o, dq, dk and dv, and to the scatter of a badly conditioned sum for the gate's
+// gradient (96x192, 32 seeds: 1.11e-2 both; 96x96 1.04e-2 / 8.8e-3, 128x128 8.6e-3 / 9.2e-3).
 //
 // One workgroup per (sequence, head, slice of 16 NE columns e).  A wave holds S for 16 of the columns and all c, as the
 // accumulators of 16x16 products with row c and column e: two of them, rounded, are the operand of the state term, so S takes
@@ -403,8 +405,10 @@ void gla_walk_kernel(GlaWalkArgs A) {
 
 // Blocks of 16 output columns per workgroup, four or six.  Six share the rows and scores of a tile among more columns, but leave
 // fewer workgroups: taken where four would give the GPU more than a workgroup per compute unit and the columns divide (four / six,
-// us a walk, B=8 T=2048 H=16: 96x192 forward 104 / 86, dq and dk 246 / 179; with 64 heads in all 76 / 77 and 123 / 150; up to
-// 64 columns of contraction, where staging is cheap, four is never behind: 48x96 with 384 heads 34 / 42).
+// us a walk, B=8 T=2048 H=16: 96x192 forward 104 / 86, dq and dk 246 / 179; with 64 heads in all 76 / 77 and 123 / 150; all
+// walks of a step: 96x96 299 / 283, 192x96 450 / 428, 192x192 796 / 604, 160x192 807 / 668, 80x96 of 16 sequences 486 / 440, 96x96 of
+// 32 x 512 253 / 227).  Up to 64 columns of contraction, where staging is cheap, four is never behind (48x96 with 384 heads
+// 34 / 42); 97 to 128 and more than 192 columns have no instance with six.
 static int walk_blocks(const PalDims* d, int dc, int de, int n_roles) {
   const int ks = (dc + 31) / 32;
   const bool six = de % 96 == 0 && (ks == 3 || ks == 5 || ks == 6) &&

@@ -400,7 +400,7 @@ def test_rows_over_heads_and_tokens(gpu_device, lead, Hqk, H, dk, dv):
     test_epilogue_forward_backward(gpu_device, lead, H, dv, torch.bfloat16, True, True)
 
 
-@pytest.mark.parametrize("tokens", [1, 4097, 5121, 13315])       # one, one, two and four tokens per wave, a ragged end
+@pytest.mark.parametrize("tokens", [1, 4097, 5121, 13315])       # four tokens a wave: ragged ends of one and of three
 def test_mamba_epilogue_tokens_per_wave(gpu_device, tokens):
     test_mamba_epilogue_forward_backward(gpu_device, (tokens,), 2, 16, torch.float32, True, True)
     test_mamba_epilogue_forward_backward(gpu_device, (tokens,), 4, 152, torch.bfloat16, True, True)
