@@ -89,19 +89,19 @@ __host__ __device__ constexpr int tile_g(int DT, int DN) { return DT * DN <= 9 ?
 __host__ __device__ constexpr int rows_pad(int DT) { return DT == 3 ? 4 : DT; }
 __host__ __device__ constexpr int vb_stride(int DT, bool var) { return (var ? 4 : 3) * 16 * rows_pad(DT) + 4; }
 
-// LDS (floats): running decay, f per token, decay weights of every step's state, their factors of the base state,
+// LDS (floats): running decay, decays of every token (and which tokens rule scaled form out), decay weights of every step's state, their factors of the base state,
 // gamma_t, its partial sums; base states; transposed v, b of both halves (of one, and the first half's in the
 // partial sums' memory at the start, where that lets two workgroups share a compute unit); two buffers of staged rows
 // and of partial dv, db
 struct TileLds {
-  int oF, oW, oFB, oX, oXS, oBase, oT, oKQ, oVB, oPart, both, total;
+  int oDec, oW, oFB, oX, oXS, oBase, oT, oKQ, oVB, oPart, both, total;
 };
 __host__ __device__ constexpr TileLds tile_lds(int DT, int DN, int nbw, bool var, bool f32) {
   TileLds L = {};
   const int G = tile_g(DT, DN), half = (f32 ? 2 : 1) * 16 * DT * kHS;   // (two tensors of bf16)
   for (int both = 1; both >= 0; --both) {
     int o = kC;
-    L.oF = o; o += kC + 4;
+    L.oDec = o; o += 4 * kC + 8;
     L.oW = o; o += (kC / G + 1) * kHalf;
     L.oFB = o; o += kC / G + 4;
     L.oX = o; o += kC + 4;

@@ -14,25 +14,36 @@
 // most 32 tokens (k weighted by the decay against v, and k^2 against b; bf16 operands, two halves of each for fp32
 // rows), the step's tokens are advanced forward leaving their states in registers, then worked in reverse.
 //
-// What bounds it: vector issue.  Per entry and token 19 fp32 instructions and a reciprocal, and 6 more for the sums over
-// lanes, the recomputed states, staging and the sums over waves (64x64; 9 more in the smaller rectangles of 96x96); two waves per
-// SIMD (the registers), which together issue an instruction per 4 cycles.  As products on the matrix cores (12 prefix and 12
-// suffix instructions of 16 cycles per 16 entries of a lane, operands exchanged through LDS between waves of different roles)
-// the same pass took 822 us at B=8 T=2048 H=12 64x64, this takes 555; 48x48 H=16 736 -> 555, packed 32768 tokens 96x96 4.91 -> 4.1 ms,
-// fp32 rows 64x64 B=8 T=2048 H=8 (forward and backward together) 1.53 -> 0.95 ms.
+// Scaled form: with F_t the decay since the start of the step, M = F M', J = F J' and dM' = F dM, dJ' = F dJ
+//   M' <- M' + (v_t / F_t) k_t    J' <- J' + (b_t / F_t) k_t^2    r' = 1 / (J' + Ip / F_t) = F_t r    mu = M' r'
+//   dM' <- dM' + (do_t r') q_t    dJ' <- dJ' - (do_t r' mu) q_t    dv = (1 / F_t) sum_n dM' k,  dk = sum_d dM' (v / F) + ...
+// so that a decay costs nothing per entry (17 instructions instead of 20; dM, dJ take the step's whole decay once), v / F and
+// b / F are formed where the rows are staged, and F dM of the step's first token is the carry that the step before it takes.
+// Rounding is that of the plain form but for one more of 2^-24 in v / F, b / F and 1 / F.  A tile is worked in plain form
+// where a step decays below 2^-56, a token grows (f > 1), or a row's entry is above 2^20 or a state or Ip above 2^66: then nothing
+// over F leaves fp32's range.  (Two copies of the loop: both forms of a step in one loop keep too many registers.)
+//
+// What bounds it: vector issue, of waves that are two to a SIMD (the registers).  By the counters 24 instructions per entry and
+// token at 64x64, 16 of them fp32 arithmetic of the entry and one a reciprocal, 7 for the sums over lanes, the recomputed states,
+// staging and the sums over waves; a wave alone issues one per 5 cycles, and waits (reads of LDS, barriers, what the other
+// wave has in the way) for two fifths of its time.  B=8 T=2048 H=12 64x64 564 -> 528 us, 48x48 H=16 549 -> 513, 48x96 4 x 1531 456 -> 406,
+// packed 32768 tokens 96x96 4060 -> 3780, fp32 rows 64x64 H=8 604 -> 586 (plain form throughout -> this, with the fetches and stores
+// below).  As products on the matrix cores (12 prefix and 12 suffix instructions of 16 cycles per 16 entries of a lane, operands
+// exchanged through LDS between waves of different roles) the same pass took 822 us at 64x64.
+// Waits that the compiler places (counted in order, for loads and stores alike) cost more than instructions here: rows are
+// fetched by every wave on one path, nothing is stored between a fetch and its use, and a token's dq, dk leave from the four
+// lanes of a quad that would otherwise hold the same sum, four tokens a store.
 // Layout: a wave holds 4 DN columns x 16 DT rows of the state, a lane DN neighbouring columns of DT rows, the layout in
 // which the matrix products leave the state (DN = 3: the fourth operand row of a lane group is empty), so that a head of
-// 48 columns loads all four SIMDs.  As many tokens per step as the registers hold: the fixed cost of a step (about
-// 2600 cycles of a SIMD per wave beside 67 per entry and token of a lane) is what small pieces pay.
+// 48 columns loads all four SIMDs.  As many tokens per step as the registers hold: the fixed cost of a step is what small
+// pieces pay (profiles/tile_kernel_pieces.txt).
 //
-// Gate: gamma_t = f_t (<dM_t, M_{t-1}> + <dJ_t, J_{t-1}>), formed as it stands: where a token decays strongly, what is left of
-// the state is of the order of f_t, and so is gamma.  (The states of the step are in registers, so that it takes two
-// instructions per entry and token and the one that makes I out of J.  gamma_{t+1} + Ip sum(G r mu) - <dv_t, v_t> - <db_t, b_t>
-// is the same number for one addition, but as a difference of terms of order 1: with every fifth token at f = e^-18 the
-// gradients of these tokens were off by 200 times their size in fp32.  The definition costs 531 -> 555 us at B=8 T=2048 H=12
-// 64x64; fp32 rows B=8 T=2048 H=8 64x64 went from 636 to 612, since the reciprocals of a token are now taken beside its
-// products instead of with the forward sweep.)  The first token of a step sees the state after the step before it in time:
-// its gamma is formed there, that of the tile's first token from the state at the start of the tile.
+// Gate: gamma_t = f_t (<dM_t, M_{t-1}> + <dJ_t, J_{t-1}>) = <dM'_t, M'_{t-1}> + <dJ'_t, J'_{t-1}>, formed as it stands: where a
+// token decays strongly, what is left of the state is of the order of f_t, and so is gamma.  (gamma_{t+1} + Ip sum(G r mu) -
+// <dv_t, v_t> - <db_t, b_t> is the same number for one addition, but as a difference of terms of order 1: with every fifth token
+// at f = e^-18 the gradients of these tokens were off by 200 times their size in fp32.)  The first token of a step sees the
+// state after the step before it in time: its gamma is formed there, that of the tile's first token from the state at
+// the start of the tile.
 #pragma once
 #include <type_traits>
 
@@ -44,8 +55,9 @@ namespace pal {
 
 // The sums of a token over lanes by DPP with a bank mask (see pair_bit3), in three stages so that the next token's arithmetic can be placed between them (each
 // stage is a chain of dependent instructions).
-//   o[2 DN] (dq, then dk of the lane's columns): over the 16 lanes of a row.  Lane bit 3 selects dq or dk, of which z0 is
-//     the first (lane bit 2 clear) or the third column, z1 the second or the fourth (DN = 3: the second in both).
+//   o[2 DN] (dq, then dk of the lane's columns): over the 16 lanes of a row but for its quads, over which four tokens are
+//     summed together (quad_tokens).  Lane bit 3 selects dq or dk, of which z0 is the first (lane bit 2 clear) or the third
+//     column, z1 the second or the fourth (DN = 3: the second in both).
 //   p[4], q[4] (dv, db of the lane's rows; DT < 3: dv0, dv1 or 0, db0, db1 or 0 in p): over the four rows of lanes, the
 //     lanes of row g get p_g and q_g.
 template <int DT, int DN>
@@ -107,17 +119,16 @@ struct TokSums {
     }
   }
   __device__ __forceinline__ void stage_c() {
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 0\n\t"
-        "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
-        : "+v"(z0), "+v"(z1));
     p[0] += p[1];
     if constexpr (DT >= 3) q[0] += q[1];
   }
 };
+// the values of four tokens, each summed over the quad: lane u of the quad gets token u's
+__device__ __forceinline__ float quad_tokens(int lane, float z0, float z1, float z2, float z3) {
+  const bool b0 = lane & 1, b1 = lane & 2;
+  const float x = (b0 ? z1 : z0) + quad_move<0xB1>(b0 ? z0 : z1), y = (b0 ? z3 : z2) + quad_move<0xB1>(b0 ? z2 : z3);
+  return (b1 ? y : x) + quad_move<0x4E>(b1 ? x : y);
+}
 template <int DT>
 __device__ __forceinline__ void lds_vals(const float* p, float* out) {
   if constexpr (DT >= 3) {
@@ -132,30 +143,34 @@ __device__ __forceinline__ void lds_vals(const float* p, float* out) {
   }
 }
 
-// what both sweeps read of a token: its k, v, b and f
-template <int DT>
+// what both sweeps read of a token: its k, v and b (over F in scaled form), and in plain form f
+template <int DT, bool SCALED>
 struct TokFwd {
   f32x4 k;
   float v[DT], b[DT], f;
-  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* pf, int plane) {
-    f = *pf;
+  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* dec, int plane) {
+    if constexpr (!SCALED) f = dec[3];
     k = *(const f32x4*)kq;
     lds_vals<DT>(vb, v);
     lds_vals<DT>(vb + plane, b);
   }
 };
-// and the reverse sweep: q, do, (dovar), the next token's f
-template <int DT, bool VAR>
+// and the reverse sweep: q, do, (dovar), Ip and 1 / F or, in plain form, the next token's f
+template <int DT, bool VAR, bool SCALED>
 struct TokRev {
   f32x4 q;
-  float d_o[DT], d_ov[VAR ? DT : 1], fn;
-  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* pf, int plane) {
+  float d_o[DT], d_ov[VAR ? DT : 1], ip, inv;
+  __device__ __forceinline__ void load(const float* kq, const float* vb, const float* dec, float Ip, int plane) {
     q = *(const f32x4*)(kq + 16);
     lds_vals<DT>(vb + 2 * plane, d_o);
     if constexpr (VAR) lds_vals<DT>(vb + 3 * plane, d_ov);
-    fn = pf[1];
+    ip = SCALED ? dec[0] : Ip;
+    inv = dec[SCALED ? 1 : 7];
   }
 };
+
+// Least decay over a step, and largest row entries and states, for the scaled form: then nothing over F leaves fp32's range.
+constexpr float kMinStepDecay = 0x1p-56f, kMaxRow = 0x1p20f, kMaxState = 0x1p66f;
 
 // waves per SIMD that a lane's E state entries leave registers for
 constexpr int tile_waves(int E) { return E > 4 ? 2 : 3; }
@@ -175,7 +190,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   constexpr int kG = tile_g(DT, DN), kSub = kC / kG;   // tokens per step, steps per tile
   constexpr bool BOTH = L.both != 0;
   float* sC = smem;
-  float* sF = smem + L.oF;
+  float* sDec = smem + L.oDec;   // [64] Ip / F_t, 1 / F_t, F_t, f_t
+  int* sPlain = (int*)(smem + L.oDec + 4 * kC);   // whether the tile is worked in plain form
   float* sW = smem + L.oW;
   float* sFB = smem + L.oFB;
   float* sX = smem + L.oX;
@@ -210,45 +226,83 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     constexpr int nKQ = kG * DNG / 4, nVB = kG * DS / 4;
     constexpr int offV = ((nKQ + 63) & ~63) + nVB <= NT ? (nKQ + 63) & ~63 : nKQ;
     static_assert(nKQ + nVB <= NT, "one staging item per thread");
+    // Where a wave stages rows of one kind, it fetches through descriptors that end with the step's last valid row: tokens beyond the
+    // end read as zero, without a branch, a select or a register to clear (which would wait for all that is in flight).
+    constexpr bool kByWave = offV % 64 == 0;
+    constexpr int kStagers = (offV + nVB + 63) / 64;
     raw4 r1, r2, r3;
     float rdv[VAR ? 4 : 1];
+    const bool kq_wave = w < offV / 64;
+    const int64_t f_stride = kq_wave ? qks : vs;
+    const TIn* f1 = (kq_wave ? kp + n0 : vp + r0) + kG * last * f_stride;   // of the step that is fetched next
+    const TIn* f2 = (kq_wave ? qp + n0 : bp + r0) + kG * last * f_stride;
+    const TIn* f3 = dop + r0 + kG * last * vs;
+    const int f_width = kq_wave ? DNG : DS;
+    const int f_full = w < kStagers ? (int)(((kG - 1) * (int)f_stride + f_width) * sizeof(TIn)) : 0;
+    unsigned f_off = 0xf0000000u;
+    if constexpr (kByWave) {
+      const int it = kq_wave ? tid : tid - offV, t = it & (kG - 1), c = 4 * (it / kG);
+      if (c < f_width) f_off = (unsigned)((t * (int)f_stride + c) * (int)sizeof(TIn));
+    }
     auto fetch = [&](int j) {
-      int tx = tid;
-      asm volatile("" : "+v"(tx));
-      const int s = kG * j;
-      const bool kq = offV % 64 == 0 ? w < offV / 64 : tx < offV;
-      const int it = kq ? tx : tx - offV, t = it & (kG - 1), c = 4 * (it / kG);
-      if (s + t < clen && c < (kq ? DNG : DS)) {
-        const unsigned o = (unsigned)((s + t) * (int)(kq ? qks : vs) + (kq ? n0 : r0) + c);
-        r1 = *(const raw4*)((kq ? kp : vp) + o);
-        r2 = *(const raw4*)((kq ? qp : bp) + o);
-        if (!kq) {
-          r3 = *(const raw4*)(dop + o);
-          if constexpr (VAR) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) rdv[e] = load_rt(A.d_o_var, tok0 * dv + o + e, a.var_bf16);
+      const int ntok = j < 0 ? 0 : min(kG, clen - kG * j);
+      if constexpr (kByWave) {
+        const int bytes = j < 0 ? 0 : ntok == kG || f_full == 0 ? f_full : (int)(((ntok - 1) * (int)f_stride + f_width) * sizeof(TIn));
+        auto take = [&](const TIn* p, int n) {
+          const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, n, 0x00020000);
+          if constexpr (F32) return __builtin_bit_cast(raw4, __builtin_amdgcn_raw_buffer_load_b128(rs, f_off, 0, 0));
+          else return __builtin_bit_cast(raw4, __builtin_amdgcn_raw_buffer_load_b64(rs, f_off, 0, 0));
+        };
+        r1 = take(f1, bytes);
+        r2 = take(f2, bytes);
+        r3 = take(f3, kq_wave ? 0 : bytes);
+        f1 -= kG * f_stride;
+        f2 -= kG * f_stride;
+        f3 -= kG * vs;
+      }
+      if (!kByWave || VAR) {
+        int tx = tid;
+        asm volatile("" : "+v"(tx));
+        const int s = kG * j;
+        const bool kq = kByWave ? kq_wave : tx < offV;
+        const int it = kq ? tx : tx - offV, t = it & (kG - 1), c = 4 * (it / kG);
+        if constexpr (!kByWave) {
+          const bool on = t < ntok && c < (kq ? DNG : DS);
+          if (ntok > 0) {
+            const int64_t o = kq ? (int64_t)n0 + (on ? s * qks + t * qks + c : 0) : (int64_t)r0 + (on ? s * vs + t * vs + c : 0);
+            r1 = *(const raw4*)((kq ? kp : vp) + o);
+            r2 = *(const raw4*)((kq ? qp : bp) + o);
+            r3 = *(const raw4*)(dop + (kq ? (int64_t)r0 : o));
           }
+        }
+        if (VAR && ntok > 0) {
+          const int64_t o = tok0 * dv + r0 + s * vs + (!kq && t < ntok && c < DS ? t * (int)vs + c : 0);
+#pragma unroll
+          for (int e = 0; e < (VAR ? 4 : 0); ++e) rdv[e] = load_rt(A.d_o_var, o + e, a.var_bf16);
         }
       }
     };
-    // value rows are staged with the DT rows of a lane next to each other; tokens beyond the end are zero
+    // value rows are staged with the DT rows of a lane next to each other; v, b and dovar over F
+    bool plain = false;
     auto deposit = [&](int j) {
       int tx = tid;
       asm volatile("" : "+v"(tx));
-      const int s = kG * j;
-      if (offV % 64 == 0 ? w < offV / 64 : tx < offV) {
-        const int t = tx & (kG - 1), c4 = tx / kG;
-        const bool ok = s + t < clen;
-        if (4 * c4 < DNG) {
+      // (in every wave the fetched rows' registers are theirs until here: one that is reused earlier makes its wave wait for the fetch)
+      asm volatile("" : "+v"(r1), "+v"(r2), "+v"(r3));
+      const bool kq = kByWave ? w < offV / 64 : tx < offV;
+      const int it = kq ? tx : tx - offV, t = it & (kG - 1), c = 4 * (it / kG);
+      const bool ok = kByWave || kG * j + t < clen;
+      if (kq) {
+        if (c < DNG) {
           f32x4 x, y;
 #pragma unroll
           for (int e = 0; e < 4; ++e) { x[e] = ok ? (float)r1[e] : 0.f; y[e] = ok ? (float)r2[e] : 0.f; }
           if constexpr (DN == 4) {
-            float* p = smem + L.oKQ + (((j & 1) * NBW + (c4 >> 2)) * kG + t) * 32 + 4 * (c4 & 3);
+            float* p = smem + L.oKQ + (((j & 1) * NBW + (c >> 4)) * kG + t) * 32 + (c & 15);
             *(f32x4*)p = x;
             *(f32x4*)(p + 16) = y;
           } else {   // lane groups of three columns, four words apart
-            const int wv = c4 / 3, c12 = 4 * (c4 - 3 * wv);
+            const int wv = c / 12, c12 = c - 12 * wv;
             float* p = smem + L.oKQ + (((j & 1) * NBW + wv) * kG + t) * 32;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -258,18 +312,15 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
             }
           }
         }
-      } else {
-        const int it = tx - offV, t = it & (kG - 1), d = 4 * (it / kG);
-        const bool ok = s + t < clen;
-        float* p = smem + L.oVB + ((j & 1) * kG + t) * SV + (d & 15) * DTP + (d >> 4);
-        if (d < DS) {
+      } else if (c < DS) {
+        float* p = smem + L.oVB + ((j & 1) * kG + t) * SV + (c & 15) * DTP + (c >> 4);
+        const float inv = plain ? 1.f : sDec[4 * (kG * j + t) + 1];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            p[e * DTP] = ok ? (float)r1[e] : 0.f;
-            p[e * DTP + plane] = ok ? (float)r2[e] : 0.f;
-            p[e * DTP + 2 * plane] = ok ? scale * (float)r3[e] : 0.f;
-            if constexpr (VAR) p[e * DTP + 3 * plane] = ok ? scale * rdv[e] : 0.f;
-          }
+        for (int e = 0; e < 4; ++e) {
+          p[e * DTP] = ok ? inv * (float)r1[e] : 0.f;
+          p[e * DTP + plane] = ok ? inv * (float)r2[e] : 0.f;
+          p[e * DTP + 2 * plane] = ok ? scale * (float)r3[e] : 0.f;
+          if constexpr (VAR) p[e * DTP + 3 * plane] = kG * j + t < clen ? (inv * scale) * rdv[e] : 0.f;
         }
       }
     };
@@ -307,7 +358,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     };
     // the wave's k in operand layout (tokens 8g + j of the half; operand row i is column i & 3 of lane group i >> 2)
     TIn kt[8];
-    auto load_kt = [&](int hf) {
+    auto load_kt = [&](int hf, TIn* kt) {
       int lx = lane;
       asm volatile("" : "+v"(lx));
       const int i = lx & 15, g = lx >> 4;
@@ -455,13 +506,16 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       asm volatile("" : "+v"(tp));
       BaseIn bs;
       HalfItem y0, y1;
+      float big = 0.f;   // the largest of v, b and k
       bf16_t* const sT0 = BOTH || !two ? sT : (bf16_t*)(smem + L.oPart);
       bf16_t* const sT1 = BOTH ? sT + 2 * PL * DS * kHS : sT;
       fetch(last);
       half_fetch(0, min(tp, HI - 1), y0);
       half_fetch(two, min(tp, HI - 1), y1);
       base_fetch(bs);
-      load_kt(0);
+      TIn kt1[8];
+      load_kt(0, kt);
+      load_kt(two, kt1);
       {
       if (w == 0) {
         const float gh = a.g[h] * kLog2e;
@@ -469,11 +523,23 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         const float c = wave_inclusive_scan(-gt * gh, lane);
         sC[lane] = c;
         sX[lane] = 0.f;
-        sF[lane] = fast_exp2(-gt * gh);
-        if (lane == 63) {
-          if (!PARTS || (n0 | r0) == 0) A.wFtot[(int64_t)cidx * H + h] = c;
-          sF[kC] = 1.f;
+        if (lane == 63 && (!PARTS || (n0 | r0) == 0)) A.wFtot[(int64_t)cidx * H + h] = c;
+        // decay since the start of the step: the product over its tokens
+        const float f = fast_exp2(-gt * gh);
+        float F = f;
+        const int u = lane & (kG - 1);
+        float y = row_shr_zero<1>(F);
+        F = u >= 1 ? F * y : F;
+        y = row_shr_zero<2>(F);
+        F = u >= 2 ? F * y : F;
+        if constexpr (kG == 8) {
+          y = row_shr_zero<4>(F);
+          F = u >= 4 ? F * y : F;
         }
+        const float inv = fast_rcp(F);
+        *(f32x4*)&sDec[4 * lane] = f32x4{Ip * inv, inv, F, f};
+        const bool off = !__all(F >= kMinStepDecay && F <= 1.f);
+        if (lane == 0) *sPlain = off;
       }
       __syncthreads();
       // row j < kSub: weights of the tokens of the half for the state before step j; row kSub: for the state after token 31
@@ -488,51 +554,62 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         if (idx >= NT) { half_fetch(0, idx, y0); half_fetch(two, idx, y1); }
         half_put(0, idx, y0, sT0);
         if (two) half_put(1, idx, y1, sT1);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf(y0.x[t][u].get(e)), __builtin_fabsf(y1.x[t][u].get(e))));
       }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)kt[e]), __builtin_fabsf((float)kt1[e])));
       base_put(bs);
-      deposit(last);
+      float bigs = Ip;
+#pragma unroll
+      for (int x = 0; x < DT; ++x)
+#pragma unroll
+        for (int r = 0; r < DN; ++r) bigs = fmaxf(bigs, fmaxf(__builtin_fabsf(bs.m[x][r]), __builtin_fabsf(bs.y[x][r])));
+      if (!(big <= kMaxRow && bigs <= kMaxState)) *sPlain = 1;
       __syncthreads();
+      plain = __builtin_amdgcn_readfirstlane(*sPlain) != 0;
+      deposit(last);
       if (two) {
         state_at(kSub, sT0);
-        load_kt(1);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kt[e] = kt1[e];
 #pragma unroll
         for (int x = 0; x < DT; ++x) {
           *(f32x4*)(base + 256 * x) = f32x4{M[x][0], M[x][1], M[x][2], DN == 4 ? M[x][DN - 1] : 0.f};
           *(f32x4*)(base + 256 * (DT + x)) = f32x4{J[x][0], J[x][1], J[x][2], DN == 4 ? J[x][DN - 1] : 0.f};
         }
-        if constexpr (!BOTH) __syncthreads();
       }
+      __syncthreads();
     }
 
+    // dM, dJ at a step's end in time: the carry of the tokens after it, with the decay of the first of them
     float dM[DT][DN], dJ[DT][DN];
 #pragma unroll
     for (int x = 0; x < DT; ++x)
 #pragma unroll
       for (int r = 0; r < DN; ++r) { dM[x][r] = 0.f; dJ[x][r] = 0.f; }
-    // dq, dk: lanes with the two low bits clear store the columns oc (and, out2, oc + 1) of dq (lane bit 3 clear) or dk
+    // dq, dk: lane u of a quad stores the columns oc (and, out2, oc + 1) of token u (and, eight tokens a step, u + 4) of dq (lane
+    // bit 3 clear) or dk
     int lo = lane;
     asm volatile("" : "+v"(lo));
-    const int oc = nw + DN * (lo >> 4) + 2 * ((lo >> 2) & 1), ow = (lo >> 3) & 1;
+    const int oc = nw + DN * (lo >> 4) + 2 * ((lo >> 2) & 1), ow = (lo >> 3) & 1, ou = lo & 3;
     const bool out2 = DN == 4 || (lo & 4) == 0;
-    TIn* const po = (TIn*)(ow ? A.dk : A.dq) + tok0 * dk + oc;
+    TIn* const po = (TIn*)(ow ? A.dk : A.dq) + tok0 * dk + oc + ou * (int)dks;
     // bf16 rows: sums over the launches so far
-    float* const pacc = PARTS ? A.pQK + ((int64_t)blockIdx.y * A.tokens * H + tok0) * (2 * dk) + ow * dk + oc
-                              : A.wQK + tok0 * (2 * DNG) + ow * DNG + (oc - n0);
     const int accs = 2 * (PARTS ? dk : DNG) * H;   // per token
-    const bool out_on = (lane & 3) == 0;
-    // SLICE 2: what the launches over earlier value rows left for a token, requested two tokens ahead of its use
-    auto acc_load = [&](int t, float* was) {
-      t = t < clen ? t : 0;
-      const float* acc = F32 ? (const float*)po + t * (int)dks : pacc + t * accs;
-      was[0] = acc[0];
-      was[1] = acc[out2 ? 1 : 0];
-    };
-
+    float* const pacc = (PARTS ? A.pQK + ((int64_t)blockIdx.y * A.tokens * H + tok0) * (2 * dk) + ow * dk + oc
+                               : A.wQK + tok0 * (2 * DNG) + ow * DNG + (oc - n0)) + ou * accs;
+    auto steps = [&](auto form) {
+    constexpr bool SCALED = decltype(form)::value;
     for (int j = last; j >= 0; --j) {
       if (j == kSub / 2 - 1 && two) {   // on to the first half
         BaseIn bs;
         base_fetch(bs);
-        load_kt(0);
+        load_kt(0, kt);
         if constexpr (!BOTH) {
           int it0 = tid;
           asm volatile("" : "+v"(it0));
@@ -545,7 +622,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         base_put(bs);
         if constexpr (!BOTH) __syncthreads();
       }
-      if (j > 0) fetch(j - 1);
+      fetch(j - 1);   // (by every wave and also before the first step, when nothing is left: the registers are then set on one path)
       // what the step before left is summed over the waves here, beside the set-up of this step
       f32x4 fl = {0.f, 0.f, 0.f, 0.f};
       raw4 fw;
@@ -563,159 +640,173 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       }
       const float* krow = smem + L.oKQ + ((j & 1) * NBW + w) * kG * 32 + 4 * g;
       const float* vrow = smem + L.oVB + (j & 1) * kG * SV + i * DTP;
-      const float* fs = sF + kG * j;
+      const float* dec = sDec + 4 * kG * j;
       const int o_tok = kG * j * (int)dks;   // (64 tokens of a tile stay within 32 bits)
-      float sM[kG][DT][DN], sJ[kG][DT][DN];   // state after each token; in reverse mu and 1 / I in their place
-      // ---- forward over the step; a token's operands are requested during the arithmetic of the token before it
-      TokFwd<DT> xf[kG], xr[kG];
-      TokRev<DT, VAR> yr[kG];
-      xf[0].load(krow, vrow, fs, plane);
-#pragma unroll
-      for (int u = 0; u < kG; ++u) {
-        const TokFwd<DT>& x = xf[u];
-        __builtin_amdgcn_sched_barrier(0);
-        if (u + 1 < kG) xf[u + 1].load(krow + (u + 1) * 32, vrow + (u + 1) * SV, fs + u + 1, plane);
-        else yr[u].load(krow + u * 32, vrow + u * SV, fs + u, plane);
-#pragma unroll
-        for (int r = 0; r < DN; ++r) {
-          const float kk = x.k[r] * x.k[r];
-#pragma unroll
-          for (int d = 0; d < DT; ++d) {
-            sM[u][d][r] = fmaf(x.v[d], x.k[r], (u ? sM[u ? u - 1 : 0][d][r] : M[d][r]) * x.f);
-            sJ[u][d][r] = fmaf(x.b[d], kk, (u ? sJ[u ? u - 1 : 0][d][r] : J[d][r]) * x.f);
-          }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // the gate of the first token of the step after, which saw the state after this one
-      float next_gate = 0.f;
-#pragma unroll
-      for (int r = 0; r < DN; ++r)
-#pragma unroll
-        for (int d = 0; d < DT; ++d) next_gate = fmaf(dM[d][r], sM[kG - 1][d][r], fmaf(dJ[d][r], sJ[kG - 1][d][r], next_gate));
-      next_gate *= fs[kG];
-      asm volatile("" : "+v"(next_gate));
-      __builtin_amdgcn_sched_barrier(0);
-      // ---- and in reverse
       float* part = smem + L.oPart + ((j & 1) * NBW + w) * (kG * 32 * DT);
-      float xs[kG / 2], xo, oz[kG][2], was[kG][2], S = 0.f;
-      if constexpr (SLICE == 2) acc_load(kG * j + kG - 1, was[kG - 1]);
+      float was[kG / 4][2];
+      float xs[kG / 2], xo, oz[kG][2], inv_last = 1.f;
       TokSums<DT, DN> ts[2];
-      auto finish = [&](int u, TokSums<DT, DN>& z) {
+      auto finish = [&](int u, TokSums<DT, DN>& z, float inv) {
         z.stage_c();
-        oz[u][0] = SLICE == 2 ? z.z0 + was[u][0] : z.z0;
-        oz[u][1] = SLICE == 2 ? z.z1 + was[u][1] : z.z1;
+        oz[u][0] = z.z0;
+        oz[u][1] = z.z1;
         float* pu = part + u * (32 * DT);
         if constexpr (DT >= 3) {
           if (lane < 16 * DT) {
-            pu[lane] = z.p[0];
-            pu[16 * DT + lane] = z.q[0];
+            pu[lane] = z.p[0] * inv;
+            pu[16 * DT + lane] = z.q[0] * inv;
           }
         } else {
-          if (lane < 32 * DT) pu[lane] = z.p[0];
+          if (lane < 32 * DT) pu[lane] = z.p[0] * inv;
         }
         if (u & 1) xo = z.X;
         else xs[u >> 1] = pair_bit3(z.X, xo);
       };
+      {
+        float sM[kG][DT][DN], sJ[kG][DT][DN];   // state after each token; in reverse mu and 1 / I in their place
+        // ---- forward over the step; a token's operands are requested during the arithmetic of the token before it
+        TokFwd<DT, SCALED> xf[kG], xr[kG];
+        TokRev<DT, VAR, SCALED> yr[kG];
+        xf[0].load(krow, vrow, dec, plane);
 #pragma unroll
-      for (int u = kG - 1; u >= 0; --u) {
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (SLICE == 2) { if (u > 0) acc_load(kG * j + u - 1, was[u - 1]); }
-        const TokFwd<DT>& x = u + 1 < kG ? xr[u] : xf[u];
-        const TokRev<DT, VAR>& y = yr[u];
-        float dq[DN], dqv[DN], dkM[DN], dkJ[DN], dvp[DT], dbp[DT], gate = 0.f;
-        TokSums<DT, DN>& before = ts[(u + 1) & 1];   // of the token worked before this one
-        if (u + 1 < kG) before.stage_a();
+        for (int u = 0; u < kG; ++u) {
+          const TokFwd<DT, SCALED>& x = xf[u];
+          __builtin_amdgcn_sched_barrier(0);
+          if (u + 1 < kG) xf[u + 1].load(krow + (u + 1) * 32, vrow + (u + 1) * SV, dec + 4 * (u + 1), plane);
+          else yr[u].load(krow + u * 32, vrow + u * SV, dec + 4 * u, Ip, plane);
 #pragma unroll
-        for (int r = 0; r < DN; ++r) {
-          if (r > 0) __builtin_amdgcn_sched_barrier(0);
-          if (r == 1 && u + 1 < kG) before.stage_b();
-          if (r == 2 && u + 1 < kG) finish(u + 1, before);
-          if (r == DN - 2 && u > 0) {   // half of mu, r of this token are dead: room for the next token's operands
-            xr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, fs + u - 1, plane);
-            yr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, fs + u - 1, plane);
-          }
-          __builtin_amdgcn_s_setprio(3);
+          for (int r = 0; r < DN; ++r) {
+            const float kk = x.k[r] * x.k[r];
 #pragma unroll
-          for (int d = 0; d < DT; ++d) {
-            sJ[u][d][r] = fast_rcp(sJ[u][d][r] + Ip);
-            asm volatile("" : "+v"(sJ[u][d][r]));
-          }
-          __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-          for (int d = 0; d < DT; ++d) sM[u][d][r] *= sJ[u][d][r];
-          const float kk = x.k[r] * x.k[r], q2 = y.q[r] * y.q[r];
-#pragma unroll
-          for (int d = 0; d < DT; ++d) {
-            const float p = y.d_o[d] * y.q[r], ri = sJ[u][d][r], m = sM[u][d][r];
-            const float dl = p * ri;
-            float t;
-            if constexpr (VAR) {
-              const float go = y.d_ov[d] * q2;
-              t = fmaf(go, ri, p * m) * ri;
-              dqv[r] = d ? fmaf(y.d_ov[d], ri, dqv[r]) : y.d_ov[d] * ri;
-            } else {
-              t = dl * m;
+            for (int d = 0; d < DT; ++d) {
+              const float m = u ? sM[u ? u - 1 : 0][d][r] : M[d][r], y = u ? sJ[u ? u - 1 : 0][d][r] : J[d][r];
+              sM[u][d][r] = fmaf(x.v[d], x.k[r], SCALED ? m : m * x.f);
+              sJ[u][d][r] = fmaf(x.b[d], kk, SCALED ? y : y * x.f);
             }
-            dM[d][r] = fmaf(dM[d][r], y.fn, dl);
-            dJ[d][r] = fmaf(dJ[d][r], y.fn, -t);
-            S += t;
-            if (u > 0) gate = fmaf(dM[d][r], sM[u ? u - 1 : 0][d][r], fmaf(dJ[d][r], sJ[u ? u - 1 : 0][d][r], gate));
-            dq[r] = d ? fmaf(m, y.d_o[d], dq[r]) : m * y.d_o[d];
-            dkM[r] = d ? fmaf(dM[d][r], x.v[d], dkM[r]) : dM[d][r] * x.v[d];
-            dkJ[r] = d ? fmaf(dJ[d][r], x.b[d], dkJ[r]) : dJ[d][r] * x.b[d];
-            dvp[d] = r ? fmaf(dM[d][r], x.k[r], dvp[d]) : dM[d][r] * x.k[r];
-            dbp[d] = r ? fmaf(dJ[d][r], kk, dbp[d]) : dJ[d][r] * kk;
           }
         }
-        TokSums<DT, DN>& mine = ts[u & 1];
-        mine.X = u > 0 ? x.f * gate : next_gate;
-        asm volatile("" : "+v"(S), "+v"(mine.X));
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (SCALED) {
+          const float Fe = dec[4 * (kG - 1) + 2];
 #pragma unroll
-        for (int r = 0; r < DN; ++r) {
-          mine.o[r] = VAR ? fmaf(2.f * y.q[r], dqv[r], dq[r]) : dq[r];
-          mine.o[DN + r] = fmaf(2.f * x.k[r], dkJ[r], dkM[r]);
-        }
-        if constexpr (DT >= 3) {
+          for (int r = 0; r < DN; ++r)
 #pragma unroll
-          for (int d = 0; d < 4; ++d) { mine.p[d] = d < DT ? dvp[d < DT ? d : 0] : 0.f; mine.q[d] = d < DT ? dbp[d < DT ? d : 0] : 0.f; }
-        } else {
-          mine.p[0] = dvp[0];
-          mine.p[1] = DT == 2 ? dvp[DT - 1] : dbp[0];
-          mine.p[2] = DT == 2 ? dbp[0] : 0.f;
-          mine.p[3] = DT == 2 ? dbp[DT - 1] : 0.f;
+            for (int d = 0; d < DT; ++d) { dM[d][r] *= Fe; dJ[d][r] *= Fe; }
         }
+        // the gate of the first token of the step after, which saw the state after this one
+        float next_gate = 0.f;
+#pragma unroll
+        for (int r = 0; r < DN; ++r)
+#pragma unroll
+          for (int d = 0; d < DT; ++d) next_gate = fmaf(dM[d][r], sM[kG - 1][d][r], fmaf(dJ[d][r], sJ[kG - 1][d][r], next_gate));
+        asm volatile("" : "+v"(next_gate));
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- and in reverse
+        float S = 0.f, inv_before = 1.f;
+        // SLICE 2: what the launches over earlier value rows left for the lane's token
+        if constexpr (SLICE == 2) {
+#pragma unroll
+          for (int e = 0; e < kG / 4; ++e) {
+            const bool on = kG * j + 4 * e + ou < clen;
+            const int t = on ? kG * j + 4 * e : -ou;   // (or the first token)
+            const float* acc = F32 ? (const float*)po + t * (int)dks : pacc + t * accs;
+            was[e][0] = acc[0];
+            was[e][1] = acc[out2 ? 1 : 0];
+          }
+        }
+#pragma unroll
+        for (int u = kG - 1; u >= 0; --u) {
+          __builtin_amdgcn_sched_barrier(0);
+          const TokFwd<DT, SCALED>& x = u + 1 < kG ? xr[u] : xf[u];
+          const TokRev<DT, VAR, SCALED>& y = yr[u];
+          float dq[DN], dqv[DN], dk[DN], dvp[DT], dbp[DT], St = 0.f, gate = 0.f;
+          TokSums<DT, DN>& before = ts[(u + 1) & 1];   // of the token worked before this one
+          if (u + 1 < kG) before.stage_a();
+#pragma unroll
+          for (int r = 0; r < DN; ++r) {
+            if (r > 0) __builtin_amdgcn_sched_barrier(0);
+            if (r == 1 && u + 1 < kG) before.stage_b();
+            if (r == 2 && u + 1 < kG) finish(u + 1, before, inv_before);
+            if (r == DN - 2 && u > 0) {   // half of mu, r of this token are dead: room for the next token's operands
+              xr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, dec + 4 * (u - 1), plane);
+              yr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, dec + 4 * (u - 1), Ip, plane);
+            }
+            __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+              sJ[u][d][r] = fast_rcp(sJ[u][d][r] + y.ip);
+              asm volatile("" : "+v"(sJ[u][d][r]));
+            }
+            __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+            for (int d = 0; d < DT; ++d) sM[u][d][r] *= sJ[u][d][r];
+            const float kk = x.k[r] * x.k[r];
+            float dkM, dkJ, Sw;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+              const float ri = sJ[u][d][r], m = sM[u][d][r], p = y.d_o[d] * ri;
+              float t;   // G r mu over q
+              if constexpr (VAR) {
+                const float e = y.d_o[d] * m, n = y.d_ov[d] * ri;
+                dq[r] = d ? dq[r] + e : e;
+                dqv[r] = d ? dqv[r] + n : n;
+                t = fmaf(n, y.q[r], e) * ri;
+              } else {
+                dq[r] = d ? fmaf(m, y.d_o[d], dq[r]) : m * y.d_o[d];
+                t = p * m;
+              }
+              Sw = d ? Sw + t : t;
+              if constexpr (SCALED) {
+                dM[d][r] = fmaf(p, y.q[r], dM[d][r]);
+                dJ[d][r] = fmaf(-t, y.q[r], dJ[d][r]);
+              } else {
+                dM[d][r] = fmaf(dM[d][r], u + 1 < kG ? y.inv : 1.f, p * y.q[r]);
+                dJ[d][r] = fmaf(dJ[d][r], u + 1 < kG ? y.inv : 1.f, -t * y.q[r]);
+              }
+              if (u > 0) gate = fmaf(dM[d][r], sM[u ? u - 1 : 0][d][r], fmaf(dJ[d][r], sJ[u ? u - 1 : 0][d][r], gate));
+              dkM = d ? fmaf(dM[d][r], x.v[d], dkM) : dM[d][r] * x.v[d];
+              dkJ = d ? fmaf(dJ[d][r], x.b[d], dkJ) : dJ[d][r] * x.b[d];
+              dvp[d] = r ? fmaf(dM[d][r], x.k[r], dvp[d]) : dM[d][r] * x.k[r];
+              dbp[d] = r ? fmaf(dJ[d][r], kk, dbp[d]) : dJ[d][r] * kk;
+            }
+            St = fmaf(Sw, y.q[r], St);
+            dk[r] = fmaf(2.f * x.k[r], dkJ, dkM);
+          }
+          TokSums<DT, DN>& mine = ts[u & 1];
+          inv_before = SCALED ? y.inv : 1.f;
+          S = fmaf(St, inv_before, S);
+          mine.X = u == 0 ? next_gate : SCALED ? gate : x.f * gate;
+          asm volatile("" : "+v"(S), "+v"(mine.X));
+#pragma unroll
+          for (int r = 0; r < DN; ++r) {
+            mine.o[r] = VAR ? fmaf(2.f * y.q[r], dqv[r], dq[r]) : dq[r];
+            mine.o[DN + r] = dk[r];
+          }
+          if constexpr (DT >= 3) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) { mine.p[d] = d < DT ? dvp[d < DT ? d : 0] : 0.f; mine.q[d] = d < DT ? dbp[d < DT ? d : 0] : 0.f; }
+          } else {
+            mine.p[0] = dvp[0];
+            mine.p[1] = DT == 2 ? dvp[DT - 1] : dbp[0];
+            mine.p[2] = DT == 2 ? dbp[0] : 0.f;
+            mine.p[3] = DT == 2 ? dbp[DT - 1] : 0.f;
+          }
+          if constexpr (!SCALED) {
+            if (u == 0) {
+#pragma unroll
+              for (int r = 0; r < DN; ++r)
+#pragma unroll
+                for (int d = 0; d < DT; ++d) { dM[d][r] *= x.f; dJ[d][r] *= x.f; }
+            }
+          }
+        }
+        ssum += S;
+        inv_last = inv_before;
       }
       __builtin_amdgcn_sched_barrier(0);
       ts[0].stage_a();
       ts[0].stage_b();
-      finish(0, ts[0]);
-      if (out_on) {
-#pragma unroll
-        for (int u = 0; u < kG; ++u) {
-          if (kG * j + u < clen) {
-            TIn* o = po + (o_tok + u * (int)dks);
-            bool done = true;
-            if constexpr (PARTS || (SLICE != 0 && !F32)) {   // the value rows of the launches add up, in fp32
-              if (PARTS || (R.flags & kRectRowsAfter)) {
-                float* acc = pacc + (kG * j + u) * accs;
-                acc[0] = oz[u][0];
-                if (out2) acc[1] = oz[u][1];
-                done = false;
-              }
-            }
-            if (done) {
-              if constexpr (DN == 4) {
-                store_vec<2>(o, oz[u]);
-              } else {
-                o[0] = from_f32<TIn>(oz[u][0]);
-                if (out2) o[1] = from_f32<TIn>(oz[u][1]);
-              }
-            }
-          }
-        }
-      }
-      ssum += S;
+      finish(0, ts[0], inv_last);
       // gates: odd token of a pair by lane bit 3, pair of tokens by bit 2 (kG = 8: four of them by bit 5)
       {
         float x = quad_sum(pair_bit2(xs[0], xs[1]));
@@ -732,9 +823,44 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         if ((lane & (kG == 8 ? 19 : 51)) == 0)
           smem[L.oXS + ((j & 1) * NBW + w) * kG + (kG == 8 ? (lane >> 5) * 4 : 0) + ((lane >> 2) & 1) * 2 + ((lane >> 3) & 1)] = x;
       }
+      // (before the stores: what a wave waits for here, its fetched rows, would include stores that were just issued)
       if (j > 0) deposit(j - 1);
+#pragma unroll
+      for (int e = 0; e < kG / 4; ++e) {
+        float x[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          x[c] = quad_tokens(lane, oz[4 * e][c], oz[4 * e + 1][c], oz[4 * e + 2][c], oz[4 * e + 3][c]);
+          if constexpr (SLICE == 2) x[c] += was[e][c];
+        }
+        if (kG * j + 4 * e + ou < clen) {
+          bool done = true;
+          if constexpr (PARTS || (SLICE != 0 && !F32)) {   // the value rows of the launches add up, in fp32
+            if (PARTS || (R.flags & kRectRowsAfter)) {
+              float* acc = pacc + (kG * j + 4 * e) * accs;
+              acc[0] = x[0];
+              if (out2) acc[1] = x[1];
+              done = false;
+            }
+          }
+          if (done) {
+            TIn* o = po + (o_tok + 4 * e * (int)dks);
+            if constexpr (DN == 4) {
+              store_vec<2>(o, x);
+            } else {
+              o[0] = from_f32<TIn>(x[0]);
+              if (out2) o[1] = from_f32<TIn>(x[1]);
+            }
+          }
+        }
+      }
       __syncthreads();
     }
+    // (vmcnt(0): to the compiler one loop may follow the other, which would then wait for what this one has requested)
+    if constexpr (!SCALED) __builtin_amdgcn_s_waitcnt(0x0f70);
+    };
+    if (plain) steps(std::false_type{});
+    else steps(std::true_type{});
     {
       f32x4 x;
       raw4 fw;
@@ -760,7 +886,6 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       }
     }
     // carry handed to the previous tile
-    const float f_first = sF[0];
     int lx = lane;
     asm volatile("" : "+v"(lx));
     const int ci = lx & 15, cn = nw + DN * (lx >> 4);
@@ -769,7 +894,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       const int64_t co = tile_off + (r0 + 16 * x + ci) * dk + cn;
       float rm[DN], rj[DN];
 #pragma unroll
-      for (int r = 0; r < DN; ++r) { rm[r] = f_first * dM[x][r]; rj[r] = f_first * dJ[x][r]; }
+      for (int r = 0; r < DN; ++r) { rm[r] = dM[x][r]; rj[r] = dJ[x][r]; }
       if constexpr (DN == 4) {
         store_vec<4>((TIn*)A.wDM + co, rm);
         store_vec<4>((TIn*)A.wDJ + co, rj);
@@ -788,7 +913,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     float x = p[0], tot = -p[NBW];
 #pragma unroll
     for (int y = 1; y < NBW; ++y) { x += p[y]; tot -= p[NBW + y]; }
-    x = lane ? sX[lane] : sF[0] * x;
+    x = lane ? sX[lane] : x;
     const int rect = PARTS ? (R.group + blockIdx.z) * R.slices + blockIdx.y : 0;
     float* pe = (PARTS ? A.pE : A.wE) + ((int64_t)rect * H + h) * A.tokens + t0 + lane;
     float* ps = (PARTS ? A.pSig : A.wSig) + ((int64_t)rect * a.total_chunks + cidx) * H + h;
