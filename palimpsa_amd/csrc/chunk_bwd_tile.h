@@ -247,7 +247,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     auto fetch = [&](int j) {
       const int ntok = j < 0 ? 0 : min(kG, clen - kG * j);
       if constexpr (kByWave) {
-        const int bytes = j < 0 ? 0 : ntok == kG || f_full == 0 ? f_full : (int)(((ntok - 1) * (int)f_stride + f_width) * sizeof(TIn));
+        const int bytes = ntok <= 0 ? 0 : ntok == kG || f_full == 0 ? f_full : (int)(((ntok - 1) * (int)f_stride + f_width) * sizeof(TIn));
         auto take = [&](const TIn* p, int n) {
           const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, n, 0x00020000);
           if constexpr (F32) return __builtin_bit_cast(raw4, __builtin_amdgcn_raw_buffer_load_b128(rs, f_off, 0, 0));
@@ -328,33 +328,44 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
     // of both tensors per item), then put into LDS.
     bf16_t* const sT = (bf16_t*)(smem + L.oT);
     constexpr int PL = F32 ? 2 : 1, groups = DS >> 3, HI = 16 * groups;   // items of a half
-    struct HalfItem { Raw8<TIn> x[2][2]; };
+    // Rows come through descriptors that end with the tile's last token: what lies beyond reads as zero.
+    auto tile_rows = [&](const TIn* p, int64_t stride, int width) {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, clen > 0 ? (int)(unsigned)(((clen - 1) * stride + width) * sizeof(TIn)) : 0, 0x00020000);
+    };
+    struct HalfItem { TIn x[2][2][8]; };
     auto half_fetch = [&](int hf, int idx, HalfItem& y) {
       const int sp = idx / groups, c8 = idx - sp * groups;
-      const int s = kHalf * hf + 2 * sp;
+      const __amdgpu_buffer_rsrc_t vrs = tile_rows(vp + r0, vs, DS), brs = tile_rows(bp + r0, vs, DS);
+      const unsigned o = (unsigned)((kHalf * hf + 2 * sp) * (int)vs + 8 * c8) * (unsigned)sizeof(TIn);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const unsigned o = (unsigned)((s + u < clen ? s + u : 0) * (int)vs + r0 + 8 * c8);   // (or any row that exists)
-        y.x[0][u].load(vp + o);
-        y.x[1][u].load(bp + o);
-      }
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < (int)(sizeof(TIn) / 2); ++e) {
+          const unsigned at = o + (unsigned)(u * (int)vs * (int)sizeof(TIn) + 16 * e);
+          const auto xv = __builtin_amdgcn_raw_buffer_load_b128(vrs, at, 0, 0), xb = __builtin_amdgcn_raw_buffer_load_b128(brs, at, 0, 0);
+          __builtin_memcpy((char*)y.x[0][u] + 16 * e, &xv, 16);
+          __builtin_memcpy((char*)y.x[1][u] + 16 * e, &xb, 16);
+        }
     };
-    auto half_put = [&](int hf, int idx, const HalfItem& y, bf16_t* dst) {
+    auto half_put = [&](int idx, const HalfItem& y, bf16_t* dst) {
       const int sp = idx / groups, c8 = idx - sp * groups;
-      const int s = kHalf * hf + 2 * sp;
-      const bool on0 = s < clen, on1 = s + 1 < clen;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          float a0 = y.x[t][0].get(e), a1 = y.x[t][1].get(e);
-          a0 = on0 ? a0 : 0.f;
-          a1 = on1 ? a1 : 0.f;
+          const float a0 = (float)y.x[t][0][e], a1 = (float)y.x[t][1][e];
           bf16_t* p = dst + ((t * PL) * DS + 8 * c8 + e) * kHS + 2 * sp;
           const bf16x2 hi = pack2(a0, a1);
           *(bf16x2*)p = hi;
           if constexpr (F32) *(bf16x2*)(p + DS * kHS) = pack2(a0 - (float)hi[0], a1 - (float)hi[1]);
         }
+    };
+    auto largest = [&](const HalfItem& y, float big) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)y.x[t][0][e]), __builtin_fabsf((float)y.x[t][1][e])));
+      return big;
     };
     // the wave's k in operand layout (tokens 8g + j of the half; operand row i is column i & 3 of lane group i >> 2)
     TIn kt[8];
@@ -362,12 +373,15 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       int lx = lane;
       asm volatile("" : "+v"(lx));
       const int i = lx & 15, g = lx >> 4;
-      const int col = nw + DN * (i >> 2) + (i & 3);
+      const bool ok = DN == 4 || (i & 3) < DN;
+      const __amdgpu_buffer_rsrc_t krs = tile_rows(kp + nw, qks, WC);
+      const unsigned o = (unsigned)((kHalf * hf + 8 * g) * (int)qks + (ok ? DN * (i >> 2) + (i & 3) : 0)) * (unsigned)sizeof(TIn);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int s = kHalf * hf + 8 * g + j;
-        const bool ok = (DN == 4 || (i & 3) < DN) && s < clen;
-        const TIn x = kp[(int64_t)(ok ? s : 0) * qks + (ok ? col : 0)];
+        const unsigned at = o + (unsigned)(j * (int)qks * (int)sizeof(TIn));
+        TIn x;
+        if constexpr (F32) x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(krs, at, 0, 0));
+        else x = __builtin_bit_cast(bf16_t, __builtin_amdgcn_raw_buffer_load_b16(krs, at, 0, 0));
         kt[j] = ok ? x : (TIn)0.f;
       }
     };
@@ -509,17 +523,23 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       float big = 0.f;   // the largest of v, b and k
       bf16_t* const sT0 = BOTH || !two ? sT : (bf16_t*)(smem + L.oPart);
       bf16_t* const sT1 = BOTH ? sT + 2 * PL * DS * kHS : sT;
+      // (the gates first: the decays are what the rest waits for)
+      const int64_t gi = (int64_t)(t0 + (lane < clen ? lane : 0)) * H + h;
+      const unsigned gate_word = load_gate_word(a.gt, gi, a.gate_bf16);
+      const float gh = a.g[h] * kLog2e;
       fetch(last);
-      half_fetch(0, min(tp, HI - 1), y0);
-      half_fetch(two, min(tp, HI - 1), y1);
+      // items of both halves: one of either for a thread, or one of each
+      constexpr bool kOneEach = NT < 2 * HI;
+      const int hf1 = kOneEach ? 0 : tp >= HI, it1 = kOneEach ? tp : tp - HI * hf1;
+      half_fetch(hf1, min(it1, HI - 1), y0);
+      if constexpr (kOneEach) half_fetch(1, min(tp, HI - 1), y1);
       base_fetch(bs);
       TIn kt1[8];
       load_kt(0, kt);
-      load_kt(two, kt1);
+      load_kt(1, kt1);
       {
       if (w == 0) {
-        const float gh = a.g[h] * kLog2e;
-        const float gt = (lane < clen) ? load_gate(a.gt, (int64_t)(t0 + lane) * H + h, a.gate_bf16) : 0.f;
+        const float gt = lane < clen ? gate_value(gate_word, gi, a.gate_bf16) : 0.f;
         const float c = wave_inclusive_scan(-gt * gh, lane);
         sC[lane] = c;
         sX[lane] = 0.f;
@@ -543,23 +563,36 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       }
       __syncthreads();
       // row j < kSub: weights of the tokens of the half for the state before step j; row kSub: for the state after token 31
-      for (int idx = tp; idx < (kSub + 1) * kHalf; idx += NT) {
-        const int j = idx / kHalf, s = idx % kHalf;
-        const int hb = (j < kSub && j >= kSub / 2) ? kHalf : 0, at = j < kSub ? kG * j : kHalf;
-        sW[idx] = hb + s < at ? fast_exp2(sC[at - 1] - sC[hb + s]) : 0.f;
-        if (s == 0) sFB[j] = at == hb ? 1.f : fast_exp2(sC[at - 1] - (hb ? sC[hb - 1] : 0.f));
+      {
+        constexpr int kRows = NT / kHalf, kIts = (kSub + kRows) / kRows;
+        const int s = tp % kHalf;
+        const float c0 = sC[s], c1 = sC[kHalf + s], cm = sC[kHalf - 1];
+        float ce[kIts];
+#pragma unroll
+        for (int e = 0; e < kIts; ++e) {
+          const int j = min(tp / kHalf + e * kRows, kSub), at = j < kSub ? kG * j : kHalf;
+          ce[e] = sC[max(at - 1, 0)];
+        }
+#pragma unroll
+        for (int e = 0; e < kIts; ++e) {
+          const int j = min(tp / kHalf + e * kRows, kSub), at = j < kSub ? kG * j : kHalf;
+          const bool upper = j < kSub && j >= kSub / 2;
+          const int hb = upper ? kHalf : 0;
+          sW[j * kHalf + s] = hb + s < at ? fast_exp2(ce[e] - (upper ? c1 : c0)) : 0.f;
+          if (s == 0) sFB[j] = at == hb ? 1.f : fast_exp2(ce[e] - (upper ? cm : 0.f));
+        }
       }
       }
-      for (int idx = tp; idx < HI; idx += NT) {
-        if (idx >= NT) { half_fetch(0, idx, y0); half_fetch(two, idx, y1); }
-        half_put(0, idx, y0, sT0);
-        if (two) half_put(1, idx, y1, sT1);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf(y0.x[t][u].get(e)), __builtin_fabsf(y1.x[t][u].get(e))));
+      if constexpr (kOneEach) {
+        for (int idx = tp; idx < HI; idx += NT) {
+          if (idx >= NT) { half_fetch(0, idx, y0); half_fetch(1, idx, y1); }
+          half_put(idx, y0, sT0);
+          if (two) half_put(idx, y1, sT1);
+          big = largest(y1, largest(y0, big));
+        }
+      } else if (it1 < HI && (two || hf1 == 0)) {
+        half_put(it1, y0, hf1 ? sT1 : sT0);
+        big = largest(y0, big);
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)kt[e]), __builtin_fabsf((float)kt1[e])));
@@ -616,7 +649,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           for (int idx = it0; idx < HI; idx += NT) {
             HalfItem y;
             half_fetch(0, idx, y);
-            half_put(0, idx, y, sT);
+            half_put(idx, y, sT);
           }
         }
         base_put(bs);

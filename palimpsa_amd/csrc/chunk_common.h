@@ -38,7 +38,7 @@ struct ChunkArgs {
 
 // q and k rows of value head h: element offset of token t's row, and the token stride, in a [tokens, Hq, dk] tensor
 __device__ __forceinline__ int64_t qk_row(const ChunkArgs& a, int64_t t, int h) {
-  return (t * a.Hq + h / (a.H / a.Hq)) * a.dk;
+  return (t * a.Hq + (a.Hq == a.H ? h : h / (a.H / a.Hq))) * a.dk;   // (a division is forty instructions)
 }
 __device__ __forceinline__ int64_t qk_stride(const ChunkArgs& a) { return (int64_t)a.Hq * a.dk; }
 
