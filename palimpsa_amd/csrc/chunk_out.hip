@@ -12,18 +12,21 @@
 // the four, and rounds the operands.  What bounds the kernel is vector issue: per entry and token six fp32
 // instructions and one reciprocal, or (scaled form) six and half a reciprocal.
 //
-// Scaled form (bf16 rows without the uncertainty output): with F_t the decay since the start of a staging step of
-// eight tokens, M = F M', I - Ip = F J':
+// Scaled form (bf16 rows without the uncertainty output): with F_t the decay since the start of a group of tokens, M = F M',
+// I - Ip = F J':
 //   M' <- M' + (v_t / F_t) k_t^T,   J' <- J' + (b_t / F_t) (k_t*k_t)^T,   M / I = M' / (J' + Ip / F_t)
 // so that the decay costs an addition per entry and token instead of two products and one addition, v / F and b / F once a
-// row; two entries share a reciprocal, n1/x1 + n2/x2 = (n1 x2 + n2 x1) / (x1 x2).  Against a float64 recurrence the outputs
+// row; two entries share a reciprocal, n1/x1 + n2/x2 = (n1 x2 + n2 x1) / (x1 x2).  A group is 64, 32, 16 or 8 tokens, the longest
+// over which no group of the tile decays by more than 2^30 (a gate of 0.5 at a rate of 1: 2^-23 over 32): M', J' take the group's
+// decay, and the largest precision is looked for, only at its end.  Against a float64 recurrence the outputs
 // are as exact as in plain form to three digits (bf16 rounding is all of the error); in fp32 the error of the outputs would
 // be up to 0.5 % larger and that of the uncertainty 15 %, so fp32 rows and the uncertainty keep the plain form.  A walk
-// takes it where every step decays by less than 2^48, and is done again in plain form if a total is not finite
-// or a precision over F beyond 2^61 (then a product of two may have no reciprocal).  8 x 2048 tokens, 12 heads of 64x64 160 -> 148 us; 65536 of
-// 16 heads of 128x128 3060 -> 2870; 32768 of 16 of 96x96 945 -> 888.  (The issue rates below promise 22.6 -> 18.1 cycles; 26.1
-// of 27.9 are left: LDS reads of the operands 2.3, the totals over the lanes 2.  Four rows a lane halve both, but leave two
-// waves per SIMD: 193 us at 64x64.)
+// takes it where every eight tokens decay by less than 2^48, and is done again in plain form if a total is not finite
+// or a precision over F beyond 2^61 (then a product of two may have no reciprocal).  Plain form -> groups of
+// eight -> groups up to 64 and staging on all waves: 65536 tokens of 16 heads of 128x128 3060 -> 2805 -> 2750 us, 32768 of 16 of
+// 96x96 945 -> 871 -> 857, 8 x 2048 of 12 of 64x64 without a backward 168 -> 160 (the last step), of 16 of 48x48 144 -> 140.
+// (112 vector instructions a token for a lane's 16 entries at 64x64, 96 of them the entries' own; a step of eight tokens adds
+// 60 for staging.  Four rows a lane halve the reads of LDS and the totals over the lanes, but leave two waves per SIMD: 193 us at 64x64.)
 //
 // How a SIMD of gfx950 issues these (profiles/issue_rates.txt): a lone wave issues an fp32 add, mul or fma per 5 cycles; two waves
 // issue one each in the same cycles (2.4 to 2.6 per instruction), a reciprocal takes 8.2 with no other beside it, and the
@@ -48,9 +51,11 @@
 
 namespace pal {
 
-// Least decay over a staging step for the scaled form, and largest precision over F: the product of two of the latter still
+// Least decay over eight tokens for the scaled form, and largest precision over F: the product of two of the latter still
 // has a reciprocal in fp32.  Steps that decay more are rare (gates of 0.5 at a rate of 2: 2^-12) and gain least from it.
 constexpr float kMinDecay = 0x1p-48f, kMaxScaled = 0x1p61f;
+// Least decay over sixteen, 32 or 64 tokens for the decay to be applied to the state only after them.
+constexpr float kMinLong = 0x1p-30f;
 constexpr int kOT = 8;   // tokens per staging step: two buffers of them let four workgroups of four waves share a unit's LDS
 
 template <int DD>
@@ -121,7 +126,8 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   }
   float* sFC = smem;                        // [tokens][4] f_t (scaled form: F_t), c_t, factor of v and b, f_t
   int* sForm = (int*)(sFC + 4 * kC * a.every);   // whether the tiles are worked in scaled form
-  float* sRow = sFC + 4 * kC * a.every + 4;               // [2][kOT][STRIDE]
+  int* sLen = sForm + 1;                         // [every] scaled form: tokens after which the decay is applied
+  float* sRow = sFC + 4 * kC * a.every + 8;      // [2][kOT][STRIDE]
   const float Ip = a.Ip[h];
   // every fetch of the set-up is issued before the first is used
   const float gt = 64 * w + lane < clen ? load_gate(a.gt, (int64_t)(t0 + 64 * w + lane) * H + h, a.gate_bf16) : 0.f;
@@ -134,7 +140,9 @@ void chunk_out_kernel(ChunkArgs a, int W) {
   // staging items: (token, four columns) of k and q, (token, four rows) of v and b
   const int nk4 = dk >> 2, nv4 = min(VR, dv - r0) >> 2;
   raw4 rk, rq, rv, rb;
-  const int s_kq = tid / nk4, c_kq = tid - s_kq * nk4, s_vb = tid / nv4, c_vb = tid - s_vb * nv4;
+  // (v and b by the threads after those of k and q, where there are as many: the first waves of all workgroups share a SIMD)
+  const int o_vb = kOT * (nk4 + nv4) <= NT ? kOT * nk4 : 0, i_vb = tid >= o_vb ? tid - o_vb : NT;
+  const int s_kq = tid / nk4, c_kq = tid - s_kq * nk4, s_vb = i_vb / nv4, c_vb = i_vb - s_vb * nv4;
   auto fetch = [&](int s0) {
     if (s_kq < kOT && s0 + s_kq < clen) {
       rk = *(const raw4*)(kp + (int64_t)(s0 + s_kq) * qs + 4 * c_kq);
@@ -192,16 +200,30 @@ void chunk_out_kernel(ChunkArgs a, int W) {
     if (tid == 0) *sForm = 1;
     __syncthreads();
     tokens([&](int t, float f) {
-      float F = f;   // F_t: decay since the start of the staging step, the product over its tokens
-      const int s = lane & (kOT - 1);
+      // Decay since the start of a group of eight tokens (a staging step), of sixteen and so on: the product over its tokens
       // (each shift before its select: a lane that is switched off hands nothing on)
-      float y = dpp_shr<1>(F);
-      F = s >= 1 ? F * y : F;
-      y = dpp_shr<2>(F);
-      F = s >= 2 ? F * y : F;
-      y = dpp_shr<4>(F);
-      F = s >= 4 ? F * y : F;
+      float F = f, P = f;
+      auto shift = [&](auto by) {
+        constexpr int N = decltype(by)::value;
+        float y = dpp_shr<N>(F);
+        if constexpr (N < kOT) F = (lane & (kOT - 1)) >= N ? F * y : F;
+        y = dpp_shr<N>(P);
+        P = (lane & 15) >= N ? P * y : P;
+      };
+      shift(std::integral_constant<int, 1>{});
+      shift(std::integral_constant<int, 2>{});
+      shift(std::integral_constant<int, 4>{});
+      shift(std::integral_constant<int, 8>{});
       if (!__all(F >= kMinDecay && F <= 1.f && Ip <= kMinDecay * kMaxScaled)) *sForm = 0;
+      auto total = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, P), l)); };
+      const float t0 = total(15), t1 = total(31), t2 = total(47);
+      const int row = lane >> 4;
+      const float P32 = P * (row == 1 ? t0 : row == 3 ? t2 : 1.f), P64 = P32 * (row >= 2 ? t0 * t1 : 1.f);
+      int len = kOT;
+      if (__all(P >= kMinLong)) { F = P; len = 16; }
+      if (__all(P32 >= kMinLong)) { F = P32; len = 32; }
+      if (__all(P64 >= kMinLong)) { F = P64; len = 64; }
+      if (lane == 0) sLen[t / kC] = len;
       sFC[4 * t] = F;
       sFC[4 * t + 3] = f;
     });
@@ -265,6 +287,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       if (more) fetch(s0 + kOT);
       const int nt = min(kOT, clen - s0);
       const float* row = sRow + buf * kOT * STRIDE;
+      const int len = SCALED ? __builtin_amdgcn_readfirstlane(sLen[s0 / kC]) : 0;
       x.load(row, ng, d0);
 #pragma unroll 1
       for (int tt = 0; tt < nt; tt += TU, row += TU * STRIDE) {
@@ -330,18 +353,19 @@ void chunk_out_kernel(ChunkArgs a, int W) {
           if (wr) store_rt(a.o_var, oo, outv * a.scale, a.var_bf16);
         }
       }
-      if constexpr (SCALED) {   // (b and Ip are not negative: a step's precisions over F are largest at its end)
+      if constexpr (SCALED) {
+        if (!more || ((s0 + kOT) & (len - 1)) == 0) {
+          // (b and Ip are not negative: precisions over F are largest before the decay is applied)
 #pragma unroll
-        for (int i = 0; i < DN; ++i)
+          for (int i = 0; i < DN; ++i)
 #pragma unroll
-          for (int j = 0; j < DD; ++j) big = fmaxf(big, __builtin_fabsf(I[j][i]));
-      }
-      if (SCALED && more) {
-        const float Fe = sFC[4 * (s0 + kOT - 1)];
+            for (int j = 0; j < DD; ++j) big = fmaxf(big, __builtin_fabsf(I[j][i]));
+          const float Fe = sFC[4 * (s0 + kOT - 1)];   // (inside the last tile)
 #pragma unroll
-        for (int i = 0; i < DN; ++i)
+          for (int i = 0; i < DN; ++i)
 #pragma unroll
-          for (int j = 0; j < DD; ++j) { M[j][i] *= Fe; I[j][i] *= Fe; }
+            for (int j = 0; j < DD; ++j) { M[j][i] *= Fe; I[j][i] *= Fe; }
+        }
       }
       if (more) deposit(s0 + kOT, buf ^ 1);
       __syncthreads();
@@ -374,7 +398,7 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
   const int64_t walks = a.every > 1 ? (int64_t)a.n_seqs * (((a.T + kC - 1) / kC + a.every - 1) / a.every) : a.total_chunks;
   const int64_t blocks = tile_head_blocks(walks, a.H);
   if (blocks > 0x7fffffff) return PAL_E_DIM;
-  const size_t lds = sizeof(float) * (4 * kC * a.every + 4 + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
+  const size_t lds = sizeof(float) * (4 * kC * a.every + 8 + (2 * kOT + 1) * (4 + 3 * NG * DN + 2 * (size_t)W * ROWS));
   if (lds > kMaxLds) return PAL_E_HEADDIM;
   auto go = [&](auto kern) -> int {
     if (int rc = allow_lds((const void*)kern, lds)) return rc;

@@ -4,6 +4,8 @@ registers — must agree: same algorithm, same bf16 operands, fp32 sums taken in
 also checked against the oracle (Palimpsa) or the float64 closed form (scalar-gated path) on its own, so that
 neither is only ever compared with the other.
 """
+import math
+
 import pytest
 import torch
 
@@ -122,6 +124,27 @@ def test_scaled_and_plain_tiles(gpu_device, state_pass_mode, dk, dv, case):
     o_ref = hp.oracle_forward(inp, mu0=mu0, I0=I0, dtype=torch.float64)[0].float()
     assert torch.equal(torch.isnan(o), torch.isnan(o_ref))
     assert hp.max_abs(o.nan_to_num(), o_ref.nan_to_num()) <= hp.BF16_OUT_ABS_TOL
+
+
+@pytest.mark.parametrize("dk,dv", [(32, 32), (48, 48), (64, 64), (80, 96), (128, 64), (192, 48)])
+def test_decay_applied_after_8_to_64_tokens(gpu_device, state_pass_mode, dk, dv):
+    """The scaled form applies the decay to the state after 64, 32, 16 or 8 tokens, the longest whose decay stays above 2^-30:
+    heads on either side of each line and far from them, full and ragged tiles, against the oracle in float64.  bf16 rows:
+    half a unit of the result (2^-9) and as much for the rows' products."""
+    bits = torch.tensor([0.0, 0.3, 0.468, 0.47, 0.93, 0.945, 1.87, 1.88, 3.0, 6.0])   # of decay a token; 30 / 64 = 0.46875
+    H = bits.numel()
+    inp = _pal_inputs(1, 64 * 3 + 41, H, dk, dv, dk + dv, "cpu")
+    inp["g"] = bits * math.log(2.0)
+    inp["gt"] = torch.ones_like(inp["gt"])
+    inp["gt"][:, 64:128] = torch.rand(1, 64, H, generator=torch.Generator().manual_seed(3)) * 2.0   # one tile of uneven decays
+    gen = torch.Generator().manual_seed(dv)
+    mu0 = torch.randn(1, H, dv, dk, generator=gen) * 0.3
+    I0 = torch.rand(1, H, dv, dk, generator=gen) + inp["Ip"][None, :, None, None]
+    state_pass_mode(2)
+    o = _run_palimpsa(hp.to_device(inp, gpu_device), mu0.to(gpu_device), I0.to(gpu_device), None, False)[0].float().cpu()
+    o_ref = hp.oracle_forward(inp, mu0=mu0, I0=I0, dtype=torch.float64)[0].float()
+    for h in range(H):
+        assert hp.max_rel(o[:, :, h], o_ref[:, :, h]) <= 2.0 ** -8, h
 
 
 @pytest.mark.parametrize("tiles,dtype,case", [(257, torch.bfloat16, "usual"), (129, torch.bfloat16, "usual"),
