@@ -32,9 +32,23 @@ struct ChunkArgs {
   int32_t Hq;   // heads of q and k: H, or a divisor of it when a group of H / Hq value heads shares one q/k head
   int32_t gate_bf16, var_bf16;
   int32_t every;   // tiles per tile-start state that is kept: 1, or more where the output kernel walks that many from one
+  int32_t segs, seg_tiles;   // segments that a sequence's state pass is cut into, tiles of one (a multiple of `every`; 1, 0: none)
   uint32_t flags;
   float scale;
 };
+
+// Segments of the state pass (chunk_states.hip): the tile states that are kept are sums since the start of their segment, M and J as
+// they are, and the state before the segment is added where they are read.  Of the slots of a segment's tiles, of which only
+// every fourth is kept, the second holds the segment's total, in its place then the state before it; the third of chunk_mu the
+// decays since the start of the segment, [kept tile][head], and over the whole of it.
+__device__ __forceinline__ int64_t seg_slot(const ChunkArgs& a, int n, int seg, int h) {
+  const int tiles = (a.T + kC - 1) / kC;
+  return ((int64_t)(n * tiles + seg * a.seg_tiles + 1) * a.H + h) * a.dv * a.dk;
+}
+__device__ __forceinline__ float* seg_decays(const ChunkArgs& a, int n, int seg) {
+  const int tiles = (a.T + kC - 1) / kC;
+  return a.chunk_mu + (int64_t)(n * tiles + seg * a.seg_tiles + 2) * a.H * a.dv * a.dk;
+}
 
 // q and k rows of value head h: element offset of token t's row, and the token stride, in a [tokens, Hq, dk] tensor
 __device__ __forceinline__ int64_t qk_row(const ChunkArgs& a, int64_t t, int h) {

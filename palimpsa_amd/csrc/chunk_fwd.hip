@@ -340,6 +340,8 @@ void fill_chunk_args(ChunkArgs& a, const PalDims* d, const PalFwdTensors* t) {
   a.gate_bf16 = d->gate_dtype == PAL_DTYPE_BF16;
   a.var_bf16 = d->var_dtype == PAL_DTYPE_BF16;
   a.every = 1;
+  a.segs = 1;
+  a.seg_tiles = 0;
   a.flags = d->flags;
   a.scale = d->scale;
 }
@@ -350,7 +352,8 @@ namespace pal {
 // the outputs from the tile-start states, and how many tiles it walks from one where no one else reads them (chunk_out.hip)
 int out_tiles_per_state(const ChunkArgs& a);
 int launch_out(const ChunkArgs& a, int dtype, hipStream_t s);
-// the one-pass form of chunk_states.hip
+// the one-pass form of chunk_states.hip, and the segments that it cuts a sequence into where few states are kept
+int state_pass_segments(const ChunkArgs& a);
 bool state_pass_applies(const ChunkArgs& a, int dtype, bool has_j);
 int launch_state_pass(const ChunkArgs& a, bool has_j, void* tiles_a, float* tiles_b, const float* init_a,
                       const float* init_b, float* fin_a, float* fin_b, bool reverse, float fin_scale, int kern_id,
@@ -500,7 +503,12 @@ extern "C" int pal_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void* str
   }
   ChunkArgs a;
   fill_chunk_args(a, d, t);
-  if (d->flags & PAL_FLAG_SPARSE_STATES) a.every = out_tiles_per_state(a);
+  if (d->flags & PAL_FLAG_SPARSE_STATES) {
+    a.every = out_tiles_per_state(a);
+    if (state_pass_applies(a, d->dtype, true)) a.segs = state_pass_segments(a);
+    const int per = a.segs * a.every;
+    if (a.segs > 1) a.seg_tiles = ((a.T + kC - 1) / kC + per - 1) / per * a.every;
+  }
   hipStream_t s = (hipStream_t)stream;
   if (int rc2 = launch_tile_states(a, d->dtype, true, s)) return rc2;
   return launch_out(a, d->dtype, s);

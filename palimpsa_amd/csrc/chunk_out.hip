@@ -239,6 +239,9 @@ void chunk_out_kernel(ChunkArgs a, int W) {
     {
       const float* mu = a.chunk_mu + (((int64_t)cidx * H + h) * dv + r0) * dk;
       const float* Is = a.chunk_I + (((int64_t)cidx * H + h) * dv + r0) * dk;
+      const int seg = a.segs > 1 ? cis / a.seg_tiles : 0;
+      const int64_t before = a.segs > 1 ? seg_slot(a, seq, seg, h) + (int64_t)r0 * dk : 0;
+      const float Fseg = a.segs > 1 ? seg_decays(a, seq, seg)[(cis - seg * a.seg_tiles) / a.every * H + h] : 0.f;
 #pragma unroll
       for (int j = 0; j < DD; ++j) {
         const bool on = r0 + d0 + j < dv;
@@ -250,6 +253,20 @@ void chunk_out_kernel(ChunkArgs a, int W) {
           const bool in = DKP == 0 || c < dk;
           load_vec<VW>(mu + ro + (in ? c : 0), x);
           load_vec<VW>(Is + ro + (in ? c : 0), y);
+          if (a.segs > 1) {   // sums since the start of the segment: the state before it is added
+            float m[VW] = {}, J[VW] = {};
+            if (seg > 0) {
+              load_vec<VW>(a.chunk_mu + before + ro + (in ? c : 0), m);
+              load_vec<VW>(a.chunk_I + before + ro + (in ? c : 0), J);
+            }
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+              M[j][i + e] = on && in ? fmaf(Fseg, m[e], x[e]) : 0.f;
+              const float J1 = fmaf(Fseg, J[e], y[e]);
+              I[j][i + e] = on && in ? (SCALED ? J1 : J1 + Ip) : 1.f;
+            }
+            return;
+          }
 #pragma unroll
           for (int e = 0; e < VW; ++e) {
             M[j][i + e] = on && in ? x[e] * y[e] : 0.f;

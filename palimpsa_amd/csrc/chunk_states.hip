@@ -73,10 +73,19 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
   // A workgroup owns the state entries (value rows [d0, d0 + ds)) x (key columns [k0, k0 + dks)) of a (sequence, head).
   int n, h, sl;
   if (!walk_item(a, A.plan, lane, n, h, sl)) return;
+  const bool segs = HAS_J && a.segs > 1;
+  const int seg = segs ? n % a.segs : 0;
+  if (segs) n /= a.segs;
   const int d0 = (sl / A.ksplit) * ds, k0 = (sl % A.ksplit) * dks;
   const int nh = n * H + h;
   int bos, len, cbase;
   seq_lookup(a, n, bos, len, cbase);
+  if (segs) {
+    const int t = seg * a.seg_tiles * kC;
+    bos += t;
+    len = min(len - t, a.seg_tiles * kC);
+    cbase += seg * a.seg_tiles;
+  }
   const int nchunks = (len + kC - 1) / kC;
 
   float* sA = smem;                                   // [3][64] weight of token s in its tile (ring over tiles)
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     goff[jj] = (d0 + 16 * db + i) * dk + k0 + 16 * nb + 4 * g;
     accM[jj] = f32x4{0.f, 0.f, 0.f, 0.f};
     accJ[jj] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (sval[jj] && A.init_a) {
+    if (sval[jj] && A.init_a && seg == 0) {
       const int64_t off = (int64_t)nh * E + goff[jj];
       const f32x4 x = *(const f32x4*)(A.init_a + off);
       if (HAS_J) {
@@ -257,6 +266,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
   }
   __syncthreads();   // steps -2 and -1 of the feeding waves
   __syncthreads();
+  float Fseg = 1.f;   // decay since the start of the segment
   for (int p = 0; p < nchunks; ++p) {
     const int buf = p & 1;
     const int c = A.reverse ? nchunks - 1 - p : p;
@@ -266,6 +276,10 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     const bf16_t* vt = sV + buf * vbuf;
     const bf16_t* bt = sB + buf * vbuf;
     const bool kept = !HAS_J || (c & (a.every - 1)) == 0;
+    if (segs && w == 0) {
+      if (lane == 0 && sl == 0 && kept) seg_decays(a, n, seg)[c / a.every * H + h] = Fseg;
+      Fseg *= F;
+    }
     // operands, the tokens as contraction index (g, j) -> 32 ks + 16 (j / 4) + 4 g + j % 4; those of the next block are read
     // while a block is worked
     struct Ops { bf16x8 k[2], v[2], b[2]; } x[2];
@@ -292,7 +306,10 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
         if (HAS_J) {
           f32x4 mu, I;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) { I[r] = accJ[jj][r] + Ip; mu[r] = accM[jj][r] * fast_rcp(I[r]); }
+          for (int r = 0; r < 4; ++r) {
+            I[r] = segs ? accJ[jj][r] : accJ[jj][r] + Ip;
+            mu[r] = segs ? accM[jj][r] : accM[jj][r] * fast_rcp(I[r]);
+          }
           *(f32x4*)((float*)A.tiles_a + off) = mu;
           *(f32x4*)(A.tiles_b + off) = I;
         } else {
@@ -322,6 +339,17 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
   // the feeding waves take their steps in groups of four, starting at -2
   for (int p = nchunks; ((p + 2) & 3) != 0; ++p) __syncthreads();
 
+  if (segs) {
+    if (w == 0 && lane == 0 && sl == 0) seg_decays(a, n, seg)[a.seg_tiles / a.every * H + h] = Fseg;
+    const int64_t slot = seg_slot(a, n, seg, h);
+#pragma unroll
+    for (int jj = 0; jj < NSB; ++jj) {
+      if (!sval[jj]) continue;
+      *(f32x4*)((float*)A.tiles_a + slot + goff[jj]) = accM[jj];
+      *(f32x4*)(A.tiles_b + slot + goff[jj]) = accJ[jj];
+    }
+    return;
+  }
   if (A.fin_a) {
 #pragma unroll
     for (int jj = 0; jj < NSB; ++jj) {
@@ -337,6 +365,32 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
         *(f32x4*)(A.fin_a + off) = accM[jj] * A.fin_scale;
       }
     }
+  }
+}
+
+// The segments' totals become the states before them, and the last one the final state.  Four entries per thread.
+__global__ __launch_bounds__(256) void chunk_segments_kernel(ChunkArgs a) {
+  const int64_t E = (int64_t)a.dv * a.dk;
+  const int nblk = (int)((E + 1023) / 1024), nh = blockIdx.x / nblk, n = nh / a.H, h = nh - n * a.H;
+  const int64_t e = ((int64_t)(blockIdx.x % nblk) * 256 + threadIdx.x) * 4;
+  if (e >= E) return;
+  f32x4 M = {0.f, 0.f, 0.f, 0.f}, J = M;
+  for (int s = 0; s < a.segs; ++s) {
+    const int64_t slot = seg_slot(a, n, s, h) + e;
+    const float F = seg_decays(a, n, s)[a.seg_tiles / a.every * a.H + h];
+    const f32x4 m = *(const f32x4*)(a.chunk_mu + slot), j = *(const f32x4*)(a.chunk_I + slot);
+    *(f32x4*)(a.chunk_mu + slot) = M;
+    *(f32x4*)(a.chunk_I + slot) = J;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { M[r] = fmaf(F, M[r], m[r]); J[r] = fmaf(F, J[r], j[r]); }
+  }
+  if (a.final_mu) {
+    const float Ip = a.Ip[h];
+    f32x4 mu, I;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { I[r] = J[r] + Ip; mu[r] = M[r] * fast_rcp(I[r]); }
+    *(f32x4*)(a.final_mu + nh * E + e) = mu;
+    *(f32x4*)(a.final_I + nh * E + e) = I;
   }
 }
 
@@ -379,6 +433,26 @@ static int state_pass_key_slice(const ChunkArgs& a, int ds) {
   return a.dk;
 }
 
+// Segments for a pass that keeps every fourth tile's state (the windows of one long sequence, see out_tiles_per_state).  The walk
+// over the tiles is a chain of 0.7 us a tile, and 16 heads of 128x128 filled the compute units only in slices of 16 rows by 64
+// columns, each of which stages rows for little state.  As segments walked side by side, in slices as wide as the registers
+// hold, states that are kept since the start of the segment: the smallest number that gives three quarters of the units a workgroup.
+// 65536 tokens of 16 heads of 128x128, four windows: states 731 -> 415 us (1.34 GB at 3.2 TB/s), and 20 us of output kernel for the state
+// before the segment.  (Eight tiles to a kept state then: 360 us, and 100 more in the output kernel.)
+int state_pass_segments(const ChunkArgs& a) {
+  if (a.every < 4 || a.cu_seqlens) return 1;
+  const int64_t tiles = (a.T + kC - 1) / kC;
+  int ds = 16;
+  for (int c : {64, 48, 32})
+    if (a.dv % c == 0 && c * a.dk <= 256 * 4 * kStMaxBlocks) { ds = c; break; }
+  const int64_t per = (int64_t)a.n_seqs * a.H * (a.dv / ds);
+  int segs = 1;
+  while (segs < 16 && per * segs < 192) segs *= 2;
+  const int64_t seg_tiles = (tiles + (int64_t)segs * a.every - 1) / ((int64_t)segs * a.every) * a.every;
+  // (a segment needs the slots of three tiles for itself, and enough of them to be worth its own start)
+  return segs > 1 && seg_tiles >= 16 && tiles - (segs - 1) * seg_tiles >= a.every ? segs : 1;
+}
+
 // Whether the one-pass form serves this call: bf16 rows, and enough (sequence, head, slice) workgroups that
 // the serial walk over the tiles does not leave most of the GPU idle.
 bool state_pass_applies(const ChunkArgs& a, int dtype, bool has_j) {
@@ -409,24 +483,33 @@ int launch_state_pass(const ChunkArgs& a, bool has_j, void* tiles_a, float* tile
   const int cand[3] = {64, 48, 32};
   for (int c : cand) {
     if (a.dv % c || c * a.dk > 256 * 4 * kStMaxBlocks) continue;
-    if ((int64_t)a.n_seqs * a.H * (a.dv / c) >= 192) { ds = c; break; }
+    if ((int64_t)a.n_seqs * a.segs * a.H * (a.dv / c) >= 192) { ds = c; break; }
   }
   // key columns per workgroup: all of them, unless even slices of 16 value rows leave the GPU short of workgroups and
   // the key columns can be halved into slices of 64 (measured at one sequence of 16 heads, 128x128: 128 workgroups
   // 102 us per 64 tiles, 256 workgroups of 16 x 64 entries 72 us, the two-kernel form 96 us; slices of 32 columns or
   // 32 x 32 entries are slower again, and with enough workgroups splitting the columns gains nothing)
-  const int dks = state_pass_key_slice(a, ds);
+  const int dks = a.segs > 1 ? a.dk : state_pass_key_slice(a, ds);
   if (ds * dks > 256 * 4 * kStMaxBlocks) return PAL_E_HEADDIM;
   A.ds = ds;
   A.dks = dks;
   A.ksplit = a.dk / dks;
   if ((int64_t)a.n_seqs * a.H <= 0) return PAL_OK;
-  if (!walk_plan(a, a.dv / ds * A.ksplit, A.plan)) return PAL_E_DIM;
+  ChunkArgs walks = a;
+  walks.n_seqs *= a.segs;
+  if (!walk_plan(walks, a.dv / ds * A.ksplit, A.plan)) return PAL_E_DIM;
   const size_t lds = sizeof(float) * (3 * kC + 4) +
                      sizeof(bf16_t) * 2 * kC * (size_t)(staged_stride(dks) + staged_stride(ds) * (has_j ? 2 : 1));
   if (lds > kMaxLds) return PAL_E_HEADDIM;
   const unsigned grid = (unsigned)A.plan.per_xcd * 8;
-  return has_j ? launch_state_pass_j<true>(A, kern_id, grid, lds, s) : launch_state_pass_j<false>(A, kern_id, grid, lds, s);
+  if (int rc = has_j ? launch_state_pass_j<true>(A, kern_id, grid, lds, s) : launch_state_pass_j<false>(A, kern_id, grid, lds, s)) return rc;
+  if (a.segs > 1) {
+    const int64_t blocks = (int64_t)a.n_seqs * a.H * (((int64_t)a.dv * a.dk + 1023) / 1024);
+    if (blocks > 0x7fffffff) return PAL_E_DIM;
+    PAL_TIMED_LAUNCH(kern_id, s, chunk_segments_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+    PAL_HIP_LAUNCH_CHECK();
+  }
+  return PAL_OK;
 }
 
 }  // namespace pal

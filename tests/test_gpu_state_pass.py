@@ -179,6 +179,36 @@ def test_walks_over_several_tiles(gpu_device, monkeypatch, tiles, dtype, case):
             assert hp.max_abs(x.float(), y.float()) <= hp.BF16_OUT_ABS_TOL
 
 
+@pytest.mark.parametrize("H,dk,dv,tiles", [(16, 128, 128, 128), (16, 96, 192, 130), (24, 128, 64, 129), (16, 128, 112, 160)])
+@pytest.mark.parametrize("case", ["usual", "strong", "uncertainty", "no_init"])
+def test_state_pass_in_segments(gpu_device, monkeypatch, H, dk, dv, tiles, case):
+    """Windows that keep every fourth tile's state cut the walk that makes them into segments, whose states count from the
+    start of their segment (bf16 rows, few heads): final states and outputs against windows that keep all states.  A second
+    window of fewer tiles, the last of them ragged.  The states differ by the order of fp32 sums over 10^4 tokens."""
+    from palimpsa_amd import _lib
+    from palimpsa_amd.ops.palimpsa import chunk as chunk_mod, chunk_palimpsa
+    T = 64 * (2 * tiles - 27) - 20
+    monkeypatch.setattr(chunk_mod, "_WINDOW_STATE_BYTES", tiles * 2 * 4 * H * dk * dv)
+    inp = _pal_inputs(1, T, H, dk, dv, 77, gpu_device)
+    inp = {n: x.to(torch.bfloat16) if n in "qkvb" else x for n, x in inp.items()}
+    # slow decays: states of earlier segments reach far into the later ones; or none that survives a tile
+    inp["g"] = torch.linspace(0.5, 90.0, H, device=gpu_device) if case == "strong" else torch.logspace(-5, 0, H, device=gpu_device)
+    gen = torch.Generator().manual_seed(5)
+    kw = dict(output_final_state=True, output_uncertainty=case == "uncertainty")
+    if case != "no_init":
+        kw["initial_mu_state"] = (torch.randn(1, H, dv, dk, generator=gen) * 0.2).to(gpu_device)
+        kw["initial_I_state"] = (torch.rand(1, H, dv, dk, generator=gen) + 0.5).to(gpu_device)
+    with torch.no_grad():
+        o, mu, I = chunk_palimpsa(**inp, **kw)
+        monkeypatch.setattr(_lib, "PAL_FLAG_SPARSE_STATES", 0)
+        o_all, mu_all, I_all = chunk_palimpsa(**inp, **kw)
+    for h in range(H):
+        assert hp.max_rel(mu[:, h], mu_all[:, h]) <= 1e-5 and hp.max_rel(I[:, h], I_all[:, h]) <= 1e-5, h
+    o, o_all = ((z if isinstance(z, tuple) else (z,)) for z in (o, o_all))
+    for x, y in zip(o, o_all):
+        assert hp.max_abs(x.float(), y.float()) <= hp.BF16_OUT_ABS_TOL
+
+
 @pytest.mark.parametrize("T", [64, 64 * 9 + 5, 64 * 21])
 def test_scan_of_few_and_of_many_heads(gpu_device, state_pass_mode, T):
     """The scan over the tiles takes one or four state entries per thread, by the number of heads: the same sums in the same
