@@ -117,9 +117,10 @@ __global__ __launch_bounds__(256) void chunk_bwd_carry_scan_kernel(BwdArgs A) {
 // row is fetched once, serves as operand and as the factor of the results, and the sums go back to memory from the
 // registers.  Bound by HBM traffic (the rows, the gradients in and out, the carries, and the states for the boundary
 // term: 375 MB at 8 x 2048 tokens, 12 heads of 64x64) and by the latency that few workgroups hide: every fetch
-// is issued before the first is used, and there is one barrier between them and the results.  (With results parked in
-// LDS, phase by phase with a barrier and fetches in each, 112 us at that size, now 108; 16 heads of 48x48 120, 95; 32768 packed
-// tokens, 16 of 96x96 660, 527; 4 x 2048, 8 of 128x128 182, 96; fp32 rows 2 x 2048, 8 of 128x64 62, 39.)
+// is issued before the first is used, and there is one barrier between them and the results.  Carries and states are gone
+// through as they lie, whole kilobytes a wave instruction: in blocks of 16 rows by 32 or 64 bytes, as the products take them,
+// 107 us at that size, now 96.5 (3.9 TB/s); 16 heads of 48x48 89, 83; 32768 packed tokens, 16 of 96x96 529, 459; 8 x 2048, 8 of
+// 128x128 199, 175; 4 x 1531, 16 of 48x96 53.6, 50.5; fp32 rows 8 x 2048, 8 of 64x64 95.6, 93.2.
 // KSMAX = operand registers per product (32 contraction indices each: head dims up to 32 KSMAX).
 // PREC (fp32 rows): operands as two bf16 halves, three matrix instructions per product; the copy of the carries in LDS
 // then holds a second plane with the lo halves.
@@ -228,38 +229,42 @@ void chunk_bwd_carry_apply_kernel(BwdArgs A) {
     const float* sI = a.chunk_I + ((int64_t)cidx * H + h) * E;
     const float Ipb = a.Ip[h];
     float acc = 0.f;
-    // a wave instruction covers 16 value rows x 64 bytes, and a wave walks along the rows before it
-    // moves to other rows, so that both halves of a 128-byte line are used while it is still in L1;
-    // four blocks are fetched before the first is used
-    const int nc = dk >> 4, nblk = (dv >> 4) * nc, per = (nblk + 3) >> 2;
-    for (int j0 = 0; j0 < per; j0 += 4) {
-      raw4 rm[4], rj[4];
-      f32x4 mu[4], I[4];
+    // the workgroup goes through the states as they lie in memory, 16 bytes of the carries a lane; two pieces are fetched
+    // before the first is used
+    constexpr int VP = 16 / sizeof(TIn), kPass = 256 * VP;
+    typedef TIn piece __attribute__((ext_vector_type(VP)));
+    const int n_e = (int)E, step_row = kPass / dk, step_col = kPass - step_row * dk;
+    int row = VP * tid / dk, col = VP * tid - row * dk;
+    for (int e0 = 0; e0 < n_e; e0 += 2 * kPass) {
+      piece rm[2], rj[2];
+      f32x4 mu[2][VP / 4], I[2][VP / 4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int blk = w * per + j0 + u;
-        if (j0 + u < per && blk < nblk) {
-          const int64_t e = (int64_t)(16 * (blk / nc) + i) * dk + 4 * (4 * (blk % nc) + g);
-          rm[u] = *(const raw4*)(RM + e);
-          rj[u] = *(const raw4*)(RJ + e);
-          mu[u] = *(const f32x4*)(smu + e);
-          I[u] = *(const f32x4*)(sI + e);
+      for (int u = 0; u < 2; ++u) {
+        const int e = e0 + u * kPass + VP * tid;
+        if (e < n_e) {
+          rm[u] = *(const piece*)(RM + e);
+          rj[u] = *(const piece*)(RJ + e);
+#pragma unroll
+          for (int x = 0; x < VP / 4; ++x) {
+            mu[u][x] = *(const f32x4*)(smu + e + 4 * x);
+            I[u][x] = *(const f32x4*)(sI + e + 4 * x);
+          }
         }
       }
       if constexpr (AHEAD) {
-        if (j0 == 0) fetch_grads();
+        if (e0 == 0) fetch_grads();
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int blk = w * per + j0 + u;
-        if (j0 + u < per && blk < nblk) {
-          const int o = (16 * (blk / nc) + i) * RS + 4 * (4 * (blk % nc) + g);
-          bf16x4 mh, jh, ml, jl;
+      for (int u = 0; u < 2; ++u) {
+        if (e0 + u * kPass + VP * tid < n_e) {
+          const int o = row * RS + col;
+          typedef bf16_t half __attribute__((ext_vector_type(VP)));
+          half mh, jh, ml, jl;
 #pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const float m = (float)rm[u][x], y = (float)rj[u][x];
-            acc = fmaf(m, mu[u][x] * I[u][x], acc);
-            acc = fmaf(y, I[u][x] - Ipb, acc);
+          for (int x = 0; x < VP; ++x) {
+            const float m = (float)rm[u][x], y = (float)rj[u][x], In = I[u][x >> 2][x & 3];
+            acc = fmaf(m, mu[u][x >> 2][x & 3] * In, acc);
+            acc = fmaf(y, In - Ipb, acc);
             mh[x] = (bf16_t)m;
             jh[x] = (bf16_t)y;
             if constexpr (PREC) {
@@ -267,13 +272,16 @@ void chunk_bwd_carry_apply_kernel(BwdArgs A) {
               jl[x] = (bf16_t)(y - (float)jh[x]);
             }
           }
-          *(bf16x4*)&sR[o] = mh;
-          *(bf16x4*)&sR[dv * RS + o] = jh;
+          *(half*)&sR[o] = mh;
+          *(half*)&sR[dv * RS + o] = jh;
           if constexpr (PREC) {
-            *(bf16x4*)&sRl[o] = ml;
-            *(bf16x4*)&sRl[dv * RS + o] = jl;
+            *(half*)&sRl[o] = ml;
+            *(half*)&sRl[dv * RS + o] = jl;
           }
         }
+        row += step_row;
+        col += step_col;
+        if (col >= dk) { col -= dk; ++row; }
       }
     }
     acc = wave_sum(acc);
