@@ -61,23 +61,43 @@ inline int tile_rows(int cols, int n, bool f32) {
 // compute unit; at two for fp32 rows and for heads whose pieces come out small (80x80, 96x96), which are the dearest one after the other.
 // It bounds the parts too: 8 bytes per token, head, slice and key column, and per group and value column (190 MB at most at 96x192).
 constexpr int kPartsTiles = 384, kPartsTilesSmall = 512;   // tiles x heads
+// The slices are of 16 rows where their waves are one to a SIMD at most, of 32 else (16 / 32 rows, us, by tiles x heads:
+// 96x96 16 43.3 / 48.8, 32 53.4 / 51.9; 128x64 32 44.3 / 50.8, 64 53.5 / 53.7; 48x96 32 42.7 / 48.9, 64 51.8 / 51.2; 96x192 16
+// 55.1 / 51.8).  A head that is one piece is cut too, from 48 rows on, where the waves of its slices are two to a SIMD at most:
+// half to a quarter of the tile's serial work, and the sum kernel of 6 us (whole -> slices of 16 rows or, @, 32, us, bf16 rows):
+//            32            64            128            192            256
+//   64x64    68.7 -> 41.5  69.8 -> 44.2  71.4 -> 54.4   72.2 -> 64.9@  72.2 -> 65.9@
+//   64x48    60.0 -> 40.6  60.6 -> 42.7  62.1 -> 52.0   (63.0, 63.6)
+//   48x48    52.3 -> 40.8  53.1 -> 42.2  53.8 -> 51.9   (54.8, 61)
+//   32x64    69.7 -> 40.0  70.5 -> 42.0  71.7 -> 50.2   72.0 -> 52.2   72.3 -> 54.3
+// and 32x32, where it gains nothing (41.1 -> 39.4, 41.2 -> 40.3, 41.9 -> 42.2), stays whole.
+constexpr int kPartsWaves = 2048;
 struct TileParts {
   int on, rows, slices, groups;
 };
 inline int parts_cols(int dk, int n0) { return dk % 64 == 0 ? 64 : dk % 48 == 0 ? 48 : dk % 32 == 0 ? 32 : tile_piece(dk - n0); }
 inline TileParts tile_parts(int dk, int dv, bool f32, int64_t tile_heads) {
   TileParts P;
-  P.rows = dk > 16 && dv % 32 == 0 ? 32 : 16;
-  P.slices = dv / P.rows;
   P.groups = 0;
-  for (int n0 = 0; n0 < dk; n0 += parts_cols(dk, n0)) ++P.groups;
-  int pieces = 0;   // one after the other
+  int pieces = 0, waves = 0;   // one after the other; of the workgroups of a tile's slice
+  for (int n0 = 0, c; n0 < dk; n0 += c, ++P.groups) {
+    c = parts_cols(dk, n0);
+    waves += c >= 48 ? 4 : c / 16;
+  }
   for (int n0 = 0, c; n0 < dk; n0 += c) {
     c = tile_piece(dk - n0);
     for (int r0 = 0; r0 < dv; r0 += tile_rows(c, dv - r0, f32)) ++pieces;
   }
-  const bool small = f32 || dk * dv <= pieces * 48 * 48;
-  P.on = pieces > 1 && tile_heads <= (small ? kPartsTilesSmall : kPartsTiles);
+  auto fits = [&](int rows) { return tile_heads * (dv / rows) * waves <= (pieces > 1 ? kPartsWaves / 2 : kPartsWaves); };
+  const bool rows32 = dk > 16 && dv % 32 == 0;
+  if (pieces > 1) {
+    const bool small = f32 || dk * dv <= pieces * 48 * 48;
+    P.on = tile_heads <= (small ? kPartsTilesSmall : kPartsTiles);
+  } else {
+    P.on = dv >= 48 && (fits(16) || (rows32 && fits(32)));
+  }
+  P.rows = rows32 && !fits(16) ? 32 : 16;
+  P.slices = dv / P.rows;
   return P;
 }
 

@@ -156,3 +156,27 @@ def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
             for h in range(H):
                 err = hp.max_rel(x.select(dim, h), ref[n].select(dim, h))
                 assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (big, n, h, err)
+
+
+@pytest.mark.parametrize("few", [1, 5, 8, 10])
+@pytest.mark.parametrize("dk,dv", [(16, 48), (32, 64), (48, 48), (64, 48), (64, 64)])
+@pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_small_passes_of_heads_of_one_piece(gpu_device, dk, dv, rows, few):
+    """A head that is one piece is cut into slices of 16 or 32 value rows where a pass has few tiles: the same rows as such a
+    pass (24, 120, 192, 240 tiles of heads: either slice, on both sides of the lines) and as the first of 576, which are whole.
+    Bars as above."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    H, many, T = 4, 24, 64 * 6 - 11
+    inp = hp.to_device(hp.rounded(po.make_inputs(many, T, H, dk, dv, seed=dk * dv), rows), gpu_device)
+    gen = torch.Generator(device=gpu_device).manual_seed(few)
+    do, dov = (torch.randn(many, T, H, dv, generator=gen, device=gpu_device) for _ in range(2))
+    for var in (False, True):
+        got = []
+        for B in (few, many):
+            leaves = [(inp[n][:B] if inp[n].dim() > 1 else inp[n]).clone().requires_grad_(True) for n in NAMES]
+            out = chunk_palimpsa(*leaves, output_uncertainty=var)
+            out = list(out) if var else [out]
+            got.append(torch.autograd.grad(out, leaves[:5], [g[:B].to(rows) for g in (do, dov)][:len(out)]))
+        for n, x, y in zip(NAMES, *got):
+            bar = 4 * 2.0 ** -17 if rows == torch.float32 else (4 if n == "gt" else 6) * 2.0 ** -9
+            assert hp.max_rel(x, y[:few]) <= bar, (var, n, hp.max_rel(x, y[:few]))
