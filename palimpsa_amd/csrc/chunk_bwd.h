@@ -29,19 +29,24 @@ struct BwdArgs {
 // 32 or 16 value rows.  (96 columns as 64 + 32, 80 as 48 + 32: workgroups of four or two waves, two or four of them to a
 // compute unit.  One workgroup of eight waves has nothing to fill its barriers and its set-up with: 96x96, 32768 packed
 // tokens, 16 heads: 5.5 ms, as rectangles 4.2.  A rectangle costs, in ps per state entry and token at B=8 T=2048 H=16, bf16
-// rows, 0.68 (64x64: columns x rows), 0.77 (64x48, 64x32), 0.88 (48x64), 0.92 (48x48), 1.00 (48x32), 0.97 (32x64), 0.87 (32x48),
-// 0.89 (32x32), 1.6 (16x16), and fp32 rows 1.14 (64x64, whose LDS leaves one workgroup to a unit), 0.84 (64x48, 64x32), 1.45 (32x64),
-// 1.66 (32x48): hence 96 rows as 64 + 32 where the group has 64 columns and the rows are bf16 (96x96 B=8 T=2048 H=16: 2155 us
-// with 48 + 48 everywhere, 2055 so; 64x96 1299, 1202), as 48 + 48 otherwise (fp32 rows 96x96 2970 us, 3230 with 64 + 32).)
+// rows, 0.63 (64x64: columns x rows), 0.71 (64x48), 0.70 (64x32), 0.81 (48x64), 0.82 (48x48), 0.90 (48x32), 0.89 (32x64), 0.82
+// (32x48), 0.80 (32x32), 1.4 (16x16): hence 96 rows of bf16 as 64 + 32 where the group has 64 columns, as 48 + 48 otherwise (96x96
+// B=8 T=2048 H=16, kernels of that time: 2155 us with 48 + 48 everywhere, 2055 so; 64x96 1299, 1202).)
 struct TileRect {
   int n0, cols, r0, flags;
   int group, groups, slices;   // small pass: first column group, their number (grid z), slices of value rows (grid y)
 };
 constexpr int kRectColsBefore = 1, kRectRowsBefore = 2, kRectRowsAfter = 4, kRectParts = 8;   // launches that came before, come after; a small pass
 inline int tile_piece(int n) { return n == 80 ? 48 : n >= 64 ? 64 : n; }
-inline int tile_rows(int cols, int n, bool f32) {
+// fp32 rows: 64 columns by 64 rows and 48 or 32 columns by 48 or 64 take 87 KB of LDS or more than half of a unit's registers'
+// worth of waves, and one or two workgroups of them run on a compute unit; slices of 32 rows, twice as many (ps per entry 1.07
+// against 0.77 for 64 columns, 1.38 and 1.34 against 0.97 for 48, 1.53 and 1.35 against 1.07 for 32; us at 256 tiles of 8 heads,
+// 64x64 578 -> 463, 48x48 416 -> 340, 48x96 878 -> 628, 128x64 1169 -> 882, 64x64 with the uncertainty 819 -> 497).  48 rows would
+// leave a slice of 16 and stay together where a pass has `few` tiles (512 tiles x heads, 48x48: 108 us, 116).
+inline int tile_rows(int cols, int n, bool f32, bool few) {
   if (cols == 16) return n >= 48 ? 48 : 16;   // (one wave's staging)
-  return n == 96 && (f32 || cols < 64) ? 48 : tile_piece(n);
+  if (f32) return (cols == 64 && n % 48 == 0) || (few && n == 48) ? 48 : n < 32 ? 16 : 32;
+  return n == 96 && cols < 64 ? 48 : tile_piece(n);
 }
 
 // A pass with too few tiles to fill the chip: all rectangles of a group width in one launch, side by side, each with
@@ -61,7 +66,7 @@ inline int tile_rows(int cols, int n, bool f32) {
 // compute unit; at two for fp32 rows and for heads whose pieces come out small (80x80, 96x96), which are the dearest one after the other.
 // It bounds the parts too: 8 bytes per token, head, slice and key column, and per group and value column (190 MB at most at 96x192).
 constexpr int kPartsTiles = 384, kPartsTilesSmall = 512;   // tiles x heads
-// The slices are of 16 rows where their waves are one to a SIMD at most, of 32 else (16 / 32 rows, us, by tiles x heads:
+// The slices are of 16 rows where their waves are one to a SIMD at most (two, where there is one column group), of 32 else (16 / 32 rows, us, by tiles x heads:
 // 96x96 16 43.3 / 48.8, 32 53.4 / 51.9; 128x64 32 44.3 / 50.8, 64 53.5 / 53.7; 48x96 32 42.7 / 48.9, 64 51.8 / 51.2; 96x192 16
 // 55.1 / 51.8).  A head that is one piece is cut too, from 48 rows on, where the waves of its slices are two to a SIMD at most:
 // half to a quarter of the tile's serial work, and the sum kernel of 6 us (whole -> slices of 16 rows or, @, 32, us, bf16 rows):
@@ -74,11 +79,13 @@ constexpr int kPartsTiles = 384, kPartsTilesSmall = 512;   // tiles x heads
 constexpr int kPartsWaves = 2048;
 struct TileParts {
   int on, rows, slices, groups;
+  bool few;   // tiles x heads at most kPartsTilesSmall
 };
 inline int parts_cols(int dk, int n0) { return dk % 64 == 0 ? 64 : dk % 48 == 0 ? 48 : dk % 32 == 0 ? 32 : tile_piece(dk - n0); }
 inline TileParts tile_parts(int dk, int dv, bool f32, int64_t tile_heads) {
   TileParts P;
   P.groups = 0;
+  P.few = tile_heads <= kPartsTilesSmall;
   int pieces = 0, waves = 0;   // one after the other; of the workgroups of a tile's slice
   for (int n0 = 0, c; n0 < dk; n0 += c, ++P.groups) {
     c = parts_cols(dk, n0);
@@ -86,9 +93,9 @@ inline TileParts tile_parts(int dk, int dv, bool f32, int64_t tile_heads) {
   }
   for (int n0 = 0, c; n0 < dk; n0 += c) {
     c = tile_piece(dk - n0);
-    for (int r0 = 0; r0 < dv; r0 += tile_rows(c, dv - r0, f32)) ++pieces;
+    for (int r0 = 0; r0 < dv; r0 += tile_rows(c, dv - r0, f32, P.few)) ++pieces;
   }
-  auto fits = [&](int rows) { return tile_heads * (dv / rows) * waves <= (pieces > 1 ? kPartsWaves / 2 : kPartsWaves); };
+  auto fits = [&](int rows) { return tile_heads * (dv / rows) * waves <= (P.groups > 1 ? kPartsWaves / 2 : kPartsWaves); };
   const bool rows32 = dk > 16 && dv % 32 == 0;
   if (pieces > 1) {
     const bool small = f32 || dk * dv <= pieces * 48 * 48;

@@ -554,7 +554,7 @@ static BwdLayout bwd_layout(const PalDims* d) {
     L.oPVB = o; o = align256(o + P.groups * rows * 2 * d->dv * 4);
     L.oPE = o; o = align256(o + rects * rows * 4);
     L.oPSig = o; o = align256(o + rects * tiles * 4);
-  } else if (row == 2 && tile_rows(cols, d->dv, false) < d->dv) o = align256(o + tokens * d->n_heads * cols * 2 * 4);
+  } else if (row == 2 && tile_rows(cols, d->dv, false, P.few) < d->dv) o = align256(o + tokens * d->n_heads * cols * 2 * 4);
   L.total = o;
   return L;
 }

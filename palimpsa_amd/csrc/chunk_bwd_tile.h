@@ -1005,14 +1005,16 @@ int launch_tile_t(const BwdArgs& A, const TileParts& P, hipStream_t s) {
     R.slices = P.on ? P.slices : 1;
     int rows;
     for (R.r0 = 0; R.r0 < dv; R.r0 += rows * R.slices) {
-      rows = P.on ? P.rows : tile_rows(R.cols, dv - R.r0, sizeof(TIn) == 4);
+      rows = P.on ? P.rows : tile_rows(R.cols, dv - R.r0, sizeof(TIn) == 4, P.few);
       R.flags = P.on ? kRectParts : (R.n0 ? kRectColsBefore : 0) | (R.r0 ? kRectRowsBefore : 0) | (R.r0 + rows < dv ? kRectRowsAfter : 0);
       int rc;
       switch (rows) {
         case 16: rc = launch_tile_d<TIn, 1, VAR>(A, R, s); break;
         case 32: rc = launch_tile_d<TIn, 2, VAR>(A, R, s); break;
         case 48: rc = launch_tile_d<TIn, 3, VAR>(A, R, s); break;
-        case 64: rc = launch_tile_d<TIn, 4, VAR>(A, R, s); break;
+        case 64:
+          if constexpr (sizeof(TIn) == 2) { rc = launch_tile_d<TIn, 4, VAR>(A, R, s); break; }   // (fp32 rows: slices of at most 48)
+          [[fallthrough]];
         default: rc = PAL_E_HEADDIM;
       }
       if (rc) return rc;
