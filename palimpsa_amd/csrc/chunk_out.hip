@@ -95,7 +95,9 @@ __device__ __forceinline__ float dpp_shr(float x) {   // lane i of a row of 16 t
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x110 + N, 0xf, 0xf, true));
 }
 
-template <typename TIn, int NG, int DN, int DD, bool HAS_VAR>
+// SEGS: the states are kept since the start of a segment (state_pass_segments; an instance of its own: the branch and its
+// values took 1 to 2 % from calls that have none)
+template <typename TIn, int NG, int DN, int DD, bool HAS_VAR, bool SEGS>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(HAS_VAR ? 2 : 4)))
 void chunk_out_kernel(ChunkArgs a, int W) {
   extern __shared__ float smem[];
@@ -239,9 +241,9 @@ void chunk_out_kernel(ChunkArgs a, int W) {
     {
       const float* mu = a.chunk_mu + (((int64_t)cidx * H + h) * dv + r0) * dk;
       const float* Is = a.chunk_I + (((int64_t)cidx * H + h) * dv + r0) * dk;
-      const int seg = a.segs > 1 ? cis / a.seg_tiles : 0;
-      const int64_t before = a.segs > 1 ? seg_slot(a, seq, seg, h) + (int64_t)r0 * dk : 0;
-      const float Fseg = a.segs > 1 ? seg_decays(a, seq, seg)[(cis - seg * a.seg_tiles) / a.every * H + h] : 0.f;
+      const int seg = SEGS ? cis / a.seg_tiles : 0;
+      const int64_t before = SEGS ? seg_slot(a, seq, seg, h) + (int64_t)r0 * dk : 0;
+      const float Fseg = SEGS ? seg_decays(a, seq, seg)[(cis - seg * a.seg_tiles) / a.every * H + h] : 0.f;
 #pragma unroll
       for (int j = 0; j < DD; ++j) {
         const bool on = r0 + d0 + j < dv;
@@ -253,24 +255,22 @@ void chunk_out_kernel(ChunkArgs a, int W) {
           const bool in = DKP == 0 || c < dk;
           load_vec<VW>(mu + ro + (in ? c : 0), x);
           load_vec<VW>(Is + ro + (in ? c : 0), y);
-          if (a.segs > 1) {   // sums since the start of the segment: the state before it is added
-            float m[VW] = {}, J[VW] = {};
-            if (seg > 0) {
-              load_vec<VW>(a.chunk_mu + before + ro + (in ? c : 0), m);
-              load_vec<VW>(a.chunk_I + before + ro + (in ? c : 0), J);
-            }
+          if constexpr (SEGS) {   // sums since the start of the segment: the state before it is added
+            float m[VW], J[VW];
+            load_vec<VW>(a.chunk_mu + before + ro + (in ? c : 0), m);
+            load_vec<VW>(a.chunk_I + before + ro + (in ? c : 0), J);
 #pragma unroll
             for (int e = 0; e < VW; ++e) {
               M[j][i + e] = on && in ? fmaf(Fseg, m[e], x[e]) : 0.f;
               const float J1 = fmaf(Fseg, J[e], y[e]);
               I[j][i + e] = on && in ? (SCALED ? J1 : J1 + Ip) : 1.f;
             }
-            return;
-          }
+          } else {
 #pragma unroll
-          for (int e = 0; e < VW; ++e) {
-            M[j][i + e] = on && in ? x[e] * y[e] : 0.f;
-            I[j][i + e] = on && in ? (SCALED ? y[e] - Ip : y[e]) : 1.f;
+            for (int e = 0; e < VW; ++e) {
+              M[j][i + e] = on && in ? x[e] * y[e] : 0.f;
+              I[j][i + e] = on && in ? (SCALED ? y[e] - Ip : y[e]) : 1.f;
+            }
           }
         };
 #pragma unroll
@@ -422,7 +422,17 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
     PAL_TIMED_LAUNCH(kKernChunkOut, s, kern, dim3((unsigned)blocks, (unsigned)slices), dim3(64 * W), lds, s, a, W);
     return 0;
   };
-  const int rc = (a.flags & PAL_FLAG_HAS_VAR) ? go(&chunk_out_kernel<TIn, NG, DN, DD, true>) : go(&chunk_out_kernel<TIn, NG, DN, DD, false>);
+  const bool var = a.flags & PAL_FLAG_HAS_VAR;
+  int rc;
+  if (a.segs <= 1) {
+    rc = var ? go(&chunk_out_kernel<TIn, NG, DN, DD, true, false>) : go(&chunk_out_kernel<TIn, NG, DN, DD, false, false>);
+  } else {
+    if constexpr (DD == 2 && sizeof(TIn) == 2) {
+      rc = var ? go(&chunk_out_kernel<TIn, NG, DN, DD, true, true>) : go(&chunk_out_kernel<TIn, NG, DN, DD, false, true>);
+    } else {
+      rc = PAL_E_DIM;   // (segments are of bf16 rows, and only where two rows to a lane fill the SIMDs: out_tiles_per_state)
+    }
+  }
   if (rc) return rc;
   PAL_HIP_LAUNCH_CHECK();
   return PAL_OK;
