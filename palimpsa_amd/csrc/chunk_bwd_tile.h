@@ -26,9 +26,9 @@
 // What bounds it: vector issue, of waves that are two to a SIMD (the registers).  By the counters 24 instructions per entry and
 // token at 64x64, 16 of them fp32 arithmetic of the entry and one a reciprocal, 7 for the sums over lanes, the recomputed states,
 // staging and the sums over waves; a wave alone issues one per 5 cycles, and waits (reads of LDS, barriers, what the other
-// wave has in the way) for two fifths of its time.  B=8 T=2048 H=12 64x64 564 -> 528 us, 48x48 H=16 549 -> 513, 48x96 4 x 1531 456 -> 406,
-// packed 32768 tokens 96x96 4060 -> 3780, fp32 rows 64x64 H=8 604 -> 586 (plain form throughout -> this, with the fetches and stores
-// below).  As products on the matrix cores (12 prefix and 12 suffix instructions of 16 cycles per 16 entries of a lane, operands
+// wave has in the way) for two fifths of its time.  B=8 T=2048 H=12 64x64 564 -> 528 us, 48x48 H=16 549 -> 491, 48x96 4 x 1531 456 -> 393,
+// packed 32768 tokens 96x96 4050 -> 3650, fp32 rows 64x64 H=8 604 -> 460 (plain form throughout -> this, with the fetches and stores
+// below; fp32 rows also as slices of 32 value rows).  As products on the matrix cores (12 prefix and 12 suffix instructions of 16 cycles per 16 entries of a lane, operands
 // exchanged through LDS between waves of different roles) the same pass took 822 us at 64x64.
 // Waits that the compiler places (counted in order, for loads and stores alike) cost more than instructions here: rows are
 // fetched by every wave on one path, nothing is stored between a fetch and its use, and a token's dq, dk leave from the four

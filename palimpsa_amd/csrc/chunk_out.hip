@@ -35,7 +35,8 @@
 // (s_setprio; B=8 T=2048 H=12 64x64: 185 -> 161 us); (2) fp32 instructions with a scalar-register operand do not pair
 // (every operand comes from LDS into vector registers, wave-uniform ones too); (3) an odd number of waves on a
 // SIMD leaves one without a partner (two or four waves, not three: at most 128 registers).
-// Ideal by these rates in plain form: 6 x 2.4 + 8.2 = 22.6 cycles per entry and wave; measured 27.9 (profiles/bench_c1.sq_counters_pmc.txt).
+// Ideal by these rates: 6 x 2.4 + 8.2 = 22.6 cycles per entry and wave in plain form, 18.5 in scaled form; measured 27.9 and 25.3
+// (profiles/bench_c1.sq_counters_pmc.txt).
 // Against the earlier kernels on the matrix cores: 64x64 B=8 T=2048 H=12 250 -> 155 us, 128x128 B=2 T=4096 H=16
 // 568 -> 388, 96x96 B=8 T=2048 H=16 0.287 -> 0.202 ps per entry, fp32 rows at 64x64 570 -> 160 us (they ran split operands).
 //
