@@ -373,6 +373,11 @@ int pal_epilogue_bwd(const PalGlueDims *dims, const PalEpilogueTensors *t, const
  * pal_gla_chunk_fwd never touches its fp32 scratch (chunk_mu), which may then be NULL-sized by the caller. */
 int pal_state_pass_applies(const PalDims *dims, int has_precision_state);
 
+/* Segments of a sequence that pal_chunk_fwd would walk side by side for its tile-start states (1: none, the sequence is walked as
+ * a whole; more only with PAL_FLAG_SPARSE_STATES), tiles per state that is kept and, for two segments or more, tiles per segment;
+ * negative: an argument error. */
+int pal_chunk_fwd_segments(const PalDims *dims, int32_t *tiles_per_state, int32_t *tiles_per_segment);
+
 /* PAL_OK if pal_chunk_bwd serves this head-dim pair for rows of `dtype` under `flags` (PAL_FLAG_FP32_FAST is
  * the bit that matters), PAL_E_HEADDIM otherwise (see pal_chunk_bwd); lets a caller refuse in its forward what
  * its backward could not do. */

@@ -133,6 +133,8 @@ def load() -> C.CDLL:
         fn.argtypes = [P(PalGlueDims)]
     lib.pal_state_pass_applies.restype = C.c_int
     lib.pal_state_pass_applies.argtypes = [P(PalDims), C.c_int]
+    lib.pal_chunk_fwd_segments.restype = C.c_int
+    lib.pal_chunk_fwd_segments.argtypes = [P(PalDims), P(C.c_int32), P(C.c_int32)]
     lib.pal_gla_walk_applies.restype = C.c_int
     lib.pal_gla_walk_applies.argtypes = [P(PalDims), C.c_int64]
     lib.pal_chunk_bwd_supported.restype = C.c_int

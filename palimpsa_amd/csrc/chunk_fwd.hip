@@ -352,8 +352,8 @@ namespace pal {
 // the outputs from the tile-start states, and how many tiles it walks from one where no one else reads them (chunk_out.hip)
 int out_tiles_per_state(const ChunkArgs& a);
 int launch_out(const ChunkArgs& a, int dtype, hipStream_t s);
-// the one-pass form of chunk_states.hip, and the segments that it cuts a sequence into where few states are kept
-int state_pass_segments(const ChunkArgs& a);
+// the one-pass form of chunk_states.hip, and the segments (a.segs, a.seg_tiles) that it cuts a sequence into where few states are kept
+void state_pass_segments(ChunkArgs& a);
 bool state_pass_applies(const ChunkArgs& a, int dtype, bool has_j);
 int launch_state_pass(const ChunkArgs& a, bool has_j, void* tiles_a, float* tiles_b, const float* init_a,
                       const float* init_b, float* fin_a, float* fin_b, bool reverse, float fin_scale, int kern_id,
@@ -478,6 +478,24 @@ extern "C" int pal_chunk_fwd_static(const PalDims* d, const PalFwdTensors* t, vo
   return launch_out(a, d->dtype, s);
 }
 
+// tiles per kept state, and the segments of the pass that makes them, where the caller needs no state afterwards
+static void sparse_states(pal::ChunkArgs& a, int dtype) {
+  a.every = pal::out_tiles_per_state(a);
+  if (pal::state_pass_applies(a, dtype, true)) pal::state_pass_segments(a);
+}
+
+extern "C" int pal_chunk_fwd_segments(const PalDims* d, int32_t* tiles_per_state, int32_t* tiles_per_segment) {
+  if (!tiles_per_state || !tiles_per_segment) return PAL_E_NULL;
+  if (int rc = pal_validate_dims(d)) return rc;
+  const PalFwdTensors none = {};
+  pal::ChunkArgs a;
+  pal::fill_chunk_args(a, d, &none);
+  if (d->flags & PAL_FLAG_SPARSE_STATES) sparse_states(a, d->dtype);
+  *tiles_per_state = a.every;
+  *tiles_per_segment = a.seg_tiles;
+  return a.segs;
+}
+
 extern "C" int pal_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void* stream) {
   using namespace pal;
   if (d && t && (d->flags & PAL_FLAG_STATES_ONLY)) {
@@ -503,12 +521,7 @@ extern "C" int pal_chunk_fwd(const PalDims* d, const PalFwdTensors* t, void* str
   }
   ChunkArgs a;
   fill_chunk_args(a, d, t);
-  if (d->flags & PAL_FLAG_SPARSE_STATES) {
-    a.every = out_tiles_per_state(a);
-    if (state_pass_applies(a, d->dtype, true)) a.segs = state_pass_segments(a);
-    const int per = a.segs * a.every;
-    if (a.segs > 1) a.seg_tiles = ((a.T + kC - 1) / kC + per - 1) / per * a.every;
-  }
+  if (d->flags & PAL_FLAG_SPARSE_STATES) sparse_states(a, d->dtype);
   hipStream_t s = (hipStream_t)stream;
   if (int rc2 = launch_tile_states(a, d->dtype, true, s)) return rc2;
   return launch_out(a, d->dtype, s);

@@ -439,8 +439,8 @@ static int state_pass_key_slice(const ChunkArgs& a, int ds) {
 // hold, states that are kept since the start of the segment: the smallest number that gives three quarters of the units a workgroup.
 // 65536 tokens of 16 heads of 128x128, four windows: states 731 -> 415 us (1.34 GB at 3.2 TB/s), and 20 us of output kernel for the state
 // before the segment.  (Eight tiles to a kept state then: 360 us, and 100 more in the output kernel.)
-int state_pass_segments(const ChunkArgs& a) {
-  if (a.every < 4 || a.cu_seqlens) return 1;
+void state_pass_segments(ChunkArgs& a) {
+  if (a.every < 4 || a.cu_seqlens || (a.flags & PAL_FLAG_VARLEN)) return;
   const int64_t tiles = (a.T + kC - 1) / kC;
   int ds = 16;
   for (int c : {64, 48, 32})
@@ -449,8 +449,12 @@ int state_pass_segments(const ChunkArgs& a) {
   int segs = 1;
   while (segs < 16 && per * segs < 192) segs *= 2;
   const int64_t seg_tiles = (tiles + (int64_t)segs * a.every - 1) / ((int64_t)segs * a.every) * a.every;
-  // (a segment needs the slots of three tiles for itself, and enough of them to be worth its own start)
-  return segs > 1 && seg_tiles >= 16 && tiles - (segs - 1) * seg_tiles >= a.every ? segs : 1;
+  // (a segment needs the slots of three tiles for itself, and enough of them to be worth its own start; its decays, one per kept
+  // tile and head and one more, have the third of these: sequences so long for the size of their states are walked whole)
+  if (segs < 2 || seg_tiles < 16 || tiles - (segs - 1) * seg_tiles < a.every) return;
+  if (seg_tiles / a.every + 1 > (int64_t)a.dv * a.dk) return;
+  a.segs = segs;
+  a.seg_tiles = (int32_t)seg_tiles;
 }
 
 // Whether the one-pass form serves this call: bf16 rows, and enough (sequence, head, slice) workgroups that

@@ -360,3 +360,48 @@ def test_chunk_bwd_workspace_of_bf16_rows(L):
         carries, sums, rest = 2 * tiles * H * dk * dv * 2, T * H * 2 * cols * 4, T * H * 4 + 4 * tiles * H * 4 + 16 * 1024
         need = lib.pal_chunk_bwd_workspace_bytes(d)
         assert carries + sums <= need <= carries + sums + rest, (dk, dv, need)
+
+
+def test_segments_of_the_state_pass_leave_room_for_their_decays(L):
+    """Segments exist only where few states are kept, in the slots of the tiles whose states are not.  A segment begins with a
+    kept tile; its decays, one per kept tile and head and one more, fill the slot of its third tile (H dv dk floats) at most,
+    the next kept state being the fifth's; the last segment has tiles of its own for the same slots."""
+    def split(one_pass=False, **kw):
+        flags = L.PAL_FLAG_SPARSE_STATES | (L.PAL_FLAG_STATES_ONE_PASS if one_pass else 0)
+        n, T = kw["n_seqs"], kw["seq_len"]
+        d = _dims(L, batch=n, total_chunks=n * ((T + 63) // 64), flags=flags, **kw)
+        every, per = C.c_int32(-1), C.c_int32(-1)
+        segs = L.load().pal_chunk_fwd_segments(d, C.byref(every), C.byref(per))
+        assert segs >= 1
+        return segs, every.value, per.value
+
+    def holds(segs, every, per, T, dk, dv):
+        tiles = (T + 63) // 64
+        assert every == 4 and per % every == 0 and per >= 16, (segs, every, per)
+        assert segs * per >= tiles and tiles - (segs - 1) * per >= every, (segs, per, tiles)
+        assert per // every + 1 <= dk * dv, (segs, per, dk, dv)
+
+    # the windows of a long sequence at the default window size
+    segs, every, per = split(n_seqs=1, seq_len=16384, n_heads=16, dk=128, dv=128)
+    assert segs == 4 and every == 4 and per == 64
+    # decays that would not fit: walked whole
+    for n, T, H, dk, dv, one_pass in ((1, 64 * 98304, 1, 16, 16, True), (2, 1300000, 48, 16, 16, False)):
+        assert split(one_pass, n_seqs=n, seq_len=T, n_heads=H, dk=dk, dv=dv)[0] == 1
+    seen = 0
+    for H in (1, 2, 3, 8, 16, 24, 48):
+        for dk, dv in ((16, 16), (16, 32), (32, 32), (48, 96), (64, 64), (128, 128)):
+            for n in (1, 2, 4):
+                for T in (640, 16384, 16385, 65536 * 3 - 77, 640000, 1100000, 4000000, 10000000):
+                    if n * T * H * max(dk, dv) > 1 << 40:
+                        continue
+                    for one_pass in (False, True):
+                        segs, every, per = split(one_pass, n_seqs=n, seq_len=T, n_heads=H, dk=dk, dv=dv)
+                        if segs > 1:
+                            seen += 1
+                            holds(segs, every, per, T, dk, dv)
+    assert seen > 100
+    none = C.c_int32()
+    assert L.load().pal_chunk_fwd_segments(_dims(L), None, C.byref(none)) == L.PAL_E_NULL
+    assert L.load().pal_chunk_fwd_segments(_dims(L, dk=31), C.byref(none), C.byref(none)) == L.PAL_E_HEADDIM
+    assert L.load().pal_chunk_fwd_segments(_dims(L, batch=1, n_seqs=1, seq_len=16384, total_chunks=256, n_heads=16, dk=128, dv=128),
+                                           C.byref(none), C.byref(none)) == 1      # every state is kept
