@@ -39,15 +39,27 @@ struct ChunkArgs {
 
 // Segments of the state pass (chunk_states.hip): the tile states that are kept are sums since the start of their segment, M and J as
 // they are, and the state before the segment is added where they are read.  Of the slots of a segment's tiles, of which only
-// every fourth is kept, the second holds the segment's total, in its place then the state before it; the third of chunk_mu the
-// decays since the start of the segment, [kept tile][head], and over the whole of it.
+// every fourth is kept, the second holds the segment's total, in its place then the state before it; the third and fourth of
+// chunk_mu the decays since the start of the segment, [kept tile][head], and over the whole of it.
+// A decay over thousands of tokens is kept as a number in [1/2, 1) and a power of two: as one fp32 number it leaves the range where
+// tokens grow (f > 1) or a state is large, when the state itself, which the walk multiplies tile by tile, does not.
+struct SegDecay {
+  float m, e;
+  __device__ __forceinline__ void times(float F) {   // (infinities, NaN and zero stay in m)
+    m *= F;
+    e += (float)__builtin_amdgcn_frexp_expf(m);
+    m = __builtin_amdgcn_frexp_mantf(m);
+  }
+  // the state x after the decay, plus y: one rounding, as of a product with the number itself
+  __device__ __forceinline__ float apply(float x, float y) const { return fmaf(m, __builtin_amdgcn_ldexpf(x, (int)e), y); }
+};
 __device__ __forceinline__ int64_t seg_slot(const ChunkArgs& a, int n, int seg, int h) {
   const int tiles = (a.T + kC - 1) / kC;
   return ((int64_t)(n * tiles + seg * a.seg_tiles + 1) * a.H + h) * a.dv * a.dk;
 }
-__device__ __forceinline__ float* seg_decays(const ChunkArgs& a, int n, int seg) {
+__device__ __forceinline__ SegDecay* seg_decays(const ChunkArgs& a, int n, int seg) {
   const int tiles = (a.T + kC - 1) / kC;
-  return a.chunk_mu + (int64_t)(n * tiles + seg * a.seg_tiles + 2) * a.H * a.dv * a.dk;
+  return (SegDecay*)(a.chunk_mu + (int64_t)(n * tiles + seg * a.seg_tiles + 2) * a.H * a.dv * a.dk);
 }
 
 // q and k rows of value head h: element offset of token t's row, and the token stride, in a [tokens, Hq, dk] tensor

@@ -244,7 +244,7 @@ void chunk_out_kernel(ChunkArgs a, int W) {
       const float* Is = a.chunk_I + (((int64_t)cidx * H + h) * dv + r0) * dk;
       const int seg = SEGS ? cis / a.seg_tiles : 0;
       const int64_t before = SEGS ? seg_slot(a, seq, seg, h) + (int64_t)r0 * dk : 0;
-      const float Fseg = SEGS ? seg_decays(a, seq, seg)[(cis - seg * a.seg_tiles) / a.every * H + h] : 0.f;
+      const SegDecay Fseg = SEGS ? seg_decays(a, seq, seg)[(cis - seg * a.seg_tiles) / a.every * H + h] : SegDecay{};
 #pragma unroll
       for (int j = 0; j < DD; ++j) {
         const bool on = r0 + d0 + j < dv;
@@ -262,8 +262,8 @@ void chunk_out_kernel(ChunkArgs a, int W) {
             load_vec<VW>(a.chunk_I + before + ro + (in ? c : 0), J);
 #pragma unroll
             for (int e = 0; e < VW; ++e) {
-              M[j][i + e] = on && in ? fmaf(Fseg, m[e], x[e]) : 0.f;
-              const float J1 = fmaf(Fseg, J[e], y[e]);
+              M[j][i + e] = on && in ? Fseg.apply(m[e], x[e]) : 0.f;
+              const float J1 = Fseg.apply(J[e], y[e]);
               I[j][i + e] = on && in ? (SCALED ? J1 : J1 + Ip) : 1.f;
             }
           } else {

@@ -266,7 +266,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
   }
   __syncthreads();   // steps -2 and -1 of the feeding waves
   __syncthreads();
-  float Fseg = 1.f;   // decay since the start of the segment
+  SegDecay Fseg = {1.f, 0.f};   // decay since the start of the segment
   for (int p = 0; p < nchunks; ++p) {
     const int buf = p & 1;
     const int c = A.reverse ? nchunks - 1 - p : p;
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(768) void chunk_states_kernel(StatePassArgs A) {
     const bool kept = !HAS_J || (c & (a.every - 1)) == 0;
     if (segs && w == 0) {
       if (lane == 0 && sl == 0 && kept) seg_decays(a, n, seg)[c / a.every * H + h] = Fseg;
-      Fseg *= F;
+      Fseg.times(F);
     }
     // operands, the tokens as contraction index (g, j) -> 32 ks + 16 (j / 4) + 4 g + j % 4; those of the next block are read
     // while a block is worked
@@ -377,12 +377,12 @@ __global__ __launch_bounds__(256) void chunk_segments_kernel(ChunkArgs a) {
   f32x4 M = {0.f, 0.f, 0.f, 0.f}, J = M;
   for (int s = 0; s < a.segs; ++s) {
     const int64_t slot = seg_slot(a, n, s, h) + e;
-    const float F = seg_decays(a, n, s)[a.seg_tiles / a.every * a.H + h];
+    const SegDecay F = seg_decays(a, n, s)[a.seg_tiles / a.every * a.H + h];
     const f32x4 m = *(const f32x4*)(a.chunk_mu + slot), j = *(const f32x4*)(a.chunk_I + slot);
     *(f32x4*)(a.chunk_mu + slot) = M;
     *(f32x4*)(a.chunk_I + slot) = J;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) { M[r] = fmaf(F, M[r], m[r]); J[r] = fmaf(F, J[r], j[r]); }
+    for (int r = 0; r < 4; ++r) { M[r] = F.apply(M[r], m[r]); J[r] = F.apply(J[r], j[r]); }
   }
   if (a.final_mu) {
     const float Ip = a.Ip[h];
@@ -449,10 +449,10 @@ void state_pass_segments(ChunkArgs& a) {
   int segs = 1;
   while (segs < 16 && per * segs < 192) segs *= 2;
   const int64_t seg_tiles = (tiles + (int64_t)segs * a.every - 1) / ((int64_t)segs * a.every) * a.every;
-  // (a segment needs the slots of three tiles for itself, and enough of them to be worth its own start; its decays, one per kept
-  // tile and head and one more, have the third of these: sequences so long for the size of their states are walked whole)
+  // (a segment needs the slots of four tiles for itself, and enough of them to be worth its own start; its decays, two numbers per
+  // kept tile and head and two more, have the last two of these: sequences so long for the size of their states are walked whole)
   if (segs < 2 || seg_tiles < 16 || tiles - (segs - 1) * seg_tiles < a.every) return;
-  if (seg_tiles / a.every + 1 > (int64_t)a.dv * a.dk) return;
+  if (2 * (seg_tiles / a.every + 1) > 2 * (int64_t)a.dv * a.dk) return;
   a.segs = segs;
   a.seg_tiles = (int32_t)seg_tiles;
 }

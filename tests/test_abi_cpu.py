@@ -364,8 +364,8 @@ def test_chunk_bwd_workspace_of_bf16_rows(L):
 
 def test_segments_of_the_state_pass_leave_room_for_their_decays(L):
     """Segments exist only where few states are kept, in the slots of the tiles whose states are not.  A segment begins with a
-    kept tile; its decays, one per kept tile and head and one more, fill the slot of its third tile (H dv dk floats) at most,
-    the next kept state being the fifth's; the last segment has tiles of its own for the same slots."""
+    kept tile; its decays, two numbers per kept tile and head and two more, fill the slots of its third and fourth tile (H dv
+    dk floats each) at most, the next kept state being the fifth's; the last segment has tiles of its own for the same slots."""
     def split(one_pass=False, **kw):
         flags = L.PAL_FLAG_SPARSE_STATES | (L.PAL_FLAG_STATES_ONE_PASS if one_pass else 0)
         n, T = kw["n_seqs"], kw["seq_len"]
@@ -379,7 +379,7 @@ def test_segments_of_the_state_pass_leave_room_for_their_decays(L):
         tiles = (T + 63) // 64
         assert every == 4 and per % every == 0 and per >= 16, (segs, every, per)
         assert segs * per >= tiles and tiles - (segs - 1) * per >= every, (segs, per, tiles)
-        assert per // every + 1 <= dk * dv, (segs, per, dk, dv)
+        assert 2 * (per // every + 1) <= 2 * dk * dv, (segs, per, dk, dv)
 
     # the windows of a long sequence at the default window size
     segs, every, per = split(n_seqs=1, seq_len=16384, n_heads=16, dk=128, dv=128)

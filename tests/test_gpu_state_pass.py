@@ -209,6 +209,46 @@ def test_state_pass_in_segments(gpu_device, monkeypatch, H, dk, dv, tiles, case)
         assert hp.max_abs(x.float(), y.float()) <= hp.BF16_OUT_ABS_TOL
 
 
+@pytest.mark.parametrize("H,dk,dv", [(16, 128, 128), (16, 128, 112)])
+def test_segments_whose_decay_leaves_the_range_of_fp32(gpu_device, monkeypatch, H, dk, dv):
+    """Gates above 1, or states far above 1, over more tokens than fp32 has powers of two: what the tile by tile walk over the
+    same window keeps finite stays finite in segments, to the rounding of fp32 sums.  Heads: nothing before a growth of 2^368;
+    a state of 2^-100 that grows by 2^184; one of 2^100 that decays by 2^-184; and ordinary ones."""
+    from palimpsa_amd import _lib
+    from palimpsa_amd.ops.palimpsa import chunk as chunk_mod, chunk_palimpsa
+    tiles, grown = 128, 80
+    T = 64 * tiles + 64 * 8
+    monkeypatch.setattr(chunk_mod, "_WINDOW_STATE_BYTES", tiles * 2 * 4 * H * dk * dv)
+    inp = _pal_inputs(1, T, H, dk, dv, 78, gpu_device)
+    inp = {n: x.to(torch.bfloat16) if n in "qkvb" else x for n, x in inp.items()}
+    inp["g"] = torch.full((H,), 0.6931472, device=gpu_device)        # f = 2^-gt
+    inp["gt"] = 0.02 * torch.rand(1, T, H, generator=torch.Generator().manual_seed(3)).to(gpu_device)
+    quiet = slice(0, 64 * grown)
+    inp["gt"][:, quiet, :12] = 0
+    inp["gt"][:, :64 * grown, 0:4] = inp["gt"][:, :32 * grown, 4:8] = -0.071875     # 2^147 over a segment of 32 tiles
+    inp["gt"][:, :32 * grown, 8:12] = 0.071875
+    for n in ("v", "b"):
+        inp[n][:, quiet, :12] = 0
+    gen = torch.Generator().manual_seed(5)
+    mu0, I0 = torch.randn(1, H, dv, dk, generator=gen) * 0.2, inp["Ip"].cpu().view(1, H, 1, 1).expand(1, H, dv, dk).clone()
+    mu0[:, 0:4], mu0[:, 4:8], mu0[:, 8:12] = 0, mu0[:, 4:8] * 2.0 ** -100, mu0[:, 8:12] * 2.0 ** 100
+    kw = dict(output_final_state=True, initial_mu_state=mu0.to(gpu_device), initial_I_state=I0.to(gpu_device))
+    with torch.no_grad():
+        o, mu, I = chunk_palimpsa(**inp, **kw)
+        monkeypatch.setattr(_lib, "PAL_FLAG_SPARSE_STATES", 0)
+        o_all, mu_all, I_all = chunk_palimpsa(**inp, **kw)
+    for x in (o_all, mu_all, I_all, o, mu, I):
+        assert bool(torch.isfinite(x).all())
+    for h in range(H):
+        assert hp.max_rel(mu[:, h], mu_all[:, h]) <= 1e-5 and hp.max_rel(I[:, h], I_all[:, h]) <= 1e-5, h
+        for w in (slice(0, 64 * grown), slice(64 * grown, None)):
+            x, y = o[:, w, h].float(), o_all[:, w, h].float()
+            if float(y.abs().max()) < hp.BF16_OUT_ABS_TOL or float(y.abs().max()) > 100:   # one bf16 rounding on either side
+                assert hp.max_rel(x, y) <= 2.0 ** -7, (h, w)
+            else:
+                assert hp.max_abs(x, y) <= hp.BF16_OUT_ABS_TOL, (h, w)
+
+
 @pytest.mark.parametrize("T", [64, 64 * 9 + 5, 64 * 21])
 def test_scan_of_few_and_of_many_heads(gpu_device, state_pass_mode, T):
     """The scan over the tiles takes one or four state entries per thread, by the number of heads: the same sums in the same
