@@ -14,21 +14,27 @@
 // most 32 tokens (k weighted by the decay against v, and k^2 against b; bf16 operands, two halves of each for fp32
 // rows), the step's tokens are advanced forward leaving their states in registers, then worked in reverse.
 //
-// Scaled form: with F_t the decay since the start of the step, M = F M', J = F J' and dM' = F dM, dJ' = F dJ
+// Scaled form (bf16 rows without the uncertainty output): with F_t the decay since the start of the step, M = F M', J = F J' and
+// dM' = F dM, dJ' = F dJ
 //   M' <- M' + (v_t / F_t) k_t    J' <- J' + (b_t / F_t) k_t^2    r' = 1 / (J' + Ip / F_t) = F_t r    mu = M' r'
 //   dM' <- dM' + (do_t r') q_t    dJ' <- dJ' - (do_t r' mu) q_t    dv = (1 / F_t) sum_n dM' k,  dk = sum_d dM' (v / F) + ...
 // so that a decay costs nothing per entry (17 instructions instead of 20; dM, dJ take the step's whole decay once), v / F and
 // b / F are formed where the rows are staged, and F dM of the step's first token is the carry that the step before it takes.
-// Rounding is that of the plain form but for one more of 2^-24 in v / F, b / F and 1 / F.  A tile is worked in plain form
-// where a step decays below 2^-56, a token grows (f > 1), or a row's entry is above 2^20 or a state or Ip above 2^66: then nothing
-// over F leaves fp32's range.  (Two copies of the loop: both forms of a step in one loop keep too many registers.)
+// A tile is worked in plain form where a step decays below 2^-56, the decay since the start of a step exceeds 1, or a row's
+// entry is above 2^20 or a state or Ip above 2^66: then nothing over F leaves fp32's range.  (Two copies of the loop: both forms of
+// a step in one loop keep too many registers.)
+// 1 / F (a product and a hardware reciprocal, one ulp) and the products with it round once more: under the rounding of bf16 rows that is
+// nothing (gradients against a float64 recurrence: the same three digits), but fp32 rows' gradients were up to 12 % further off where
+// tokens decay by e^-2 or more (dk, 96x96 and 64x64), for 4 % of the time (64x64 B=8 T=2048 H=8 444 us, plain 458).  With the
+// uncertainty the scaled form was no faster (bf16 64x64 H=8 490 us, plain 459), and dovar / F needs a bound of its own.
 //
 // What bounds it: vector issue, of waves that are two to a SIMD (the registers).  By the counters 24 instructions per entry and
 // token at 64x64, 16 of them fp32 arithmetic of the entry and one a reciprocal, 7 for the sums over lanes, the recomputed states,
 // staging and the sums over waves; a wave alone issues one per 5 cycles, and waits (reads of LDS, barriers, what the other
 // wave has in the way) for two fifths of its time.  B=8 T=2048 H=12 64x64 564 -> 528 us, 48x48 H=16 549 -> 491, 48x96 4 x 1531 456 -> 393,
-// packed 32768 tokens 96x96 4050 -> 3650, fp32 rows 64x64 H=8 604 -> 460 (plain form throughout -> this, with the fetches and stores
-// below; fp32 rows also as slices of 32 value rows).  As products on the matrix cores (12 prefix and 12 suffix instructions of 16 cycles per 16 entries of a lane, operands
+// packed 32768 tokens 96x96 4050 -> 3600 (plain form throughout -> this, with the fetches and stores below), with every tile in plain
+// form 554, 537, 433 and 3840; fp32 rows 64x64 H=8 604 -> 460 (slices of 32 value rows, fetches and stores), with the uncertainty bf16 64x64
+// H=8 512 -> 459.  As products on the matrix cores (12 prefix and 12 suffix instructions of 16 cycles per 16 entries of a lane, operands
 // exchanged through LDS between waves of different roles) the same pass took 822 us at 64x64.
 // Waits that the compiler places (counted in order, for loads and stores alike) cost more than instructions here: rows are
 // fetched by every wave on one path, nothing is stored between a fetch and its use, and a token's dq, dk leave from the four
@@ -188,9 +194,10 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   constexpr int NT = NBW * 64, DNG = WC * NBW;
   constexpr TileLds L = tile_lds(DT, DN, NBW, VAR, F32);
   constexpr int kG = tile_g(DT, DN), kSub = kC / kG;   // tokens per step, steps per tile
+  constexpr bool kScaled = !F32 && !VAR;    // whether there is a scaled form
   constexpr bool BOTH = L.both != 0;
   float* sC = smem;
-  float* sDec = smem + L.oDec;   // [64] Ip / F_t, 1 / F_t, F_t, f_t
+  float* sDec = smem + L.oDec;   // [64] (scaled form: Ip / F_t, 1 / F_t, F_t,) f_t
   int* sPlain = (int*)(smem + L.oDec + 4 * kC);   // whether the tile is worked in plain form
   float* sW = smem + L.oW;
   float* sFB = smem + L.oFB;
@@ -282,8 +289,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         }
       }
     };
-    // value rows are staged with the DT rows of a lane next to each other; v, b and dovar over F
-    bool plain = false;
+    // value rows are staged with the DT rows of a lane next to each other; v and b over F
+    bool plain = true;
     auto deposit = [&](int j) {
       int tx = tid;
       asm volatile("" : "+v"(tx));
@@ -314,13 +321,13 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         }
       } else if (c < DS) {
         float* p = smem + L.oVB + ((j & 1) * kG + t) * SV + (c & 15) * DTP + (c >> 4);
-        const float inv = plain ? 1.f : sDec[4 * (kG * j + t) + 1];
+        const float inv = !kScaled || plain ? 1.f : sDec[4 * (kG * j + t) + 1];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           p[e * DTP] = ok ? inv * (float)r1[e] : 0.f;
           p[e * DTP + plane] = ok ? inv * (float)r2[e] : 0.f;
           p[e * DTP + 2 * plane] = ok ? scale * (float)r3[e] : 0.f;
-          if constexpr (VAR) p[e * DTP + 3 * plane] = kG * j + t < clen ? (inv * scale) * rdv[e] : 0.f;
+          if constexpr (VAR) p[e * DTP + 3 * plane] = kG * j + t < clen ? scale * rdv[e] : 0.f;
         }
       }
     };
@@ -544,22 +551,26 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
         sC[lane] = c;
         sX[lane] = 0.f;
         if (lane == 63 && (!PARTS || (n0 | r0) == 0)) A.wFtot[(int64_t)cidx * H + h] = c;
-        // decay since the start of the step: the product over its tokens
         const float f = fast_exp2(-gt * gh);
-        float F = f;
-        const int u = lane & (kG - 1);
-        float y = row_shr_zero<1>(F);
-        F = u >= 1 ? F * y : F;
-        y = row_shr_zero<2>(F);
-        F = u >= 2 ? F * y : F;
-        if constexpr (kG == 8) {
-          y = row_shr_zero<4>(F);
-          F = u >= 4 ? F * y : F;
+        if constexpr (kScaled) {
+          // decay since the start of the step: the product over its tokens
+          float F = f;
+          const int u = lane & (kG - 1);
+          float y = row_shr_zero<1>(F);
+          F = u >= 1 ? F * y : F;
+          y = row_shr_zero<2>(F);
+          F = u >= 2 ? F * y : F;
+          if constexpr (kG == 8) {
+            y = row_shr_zero<4>(F);
+            F = u >= 4 ? F * y : F;
+          }
+          const float inv = fast_rcp(F);
+          *(f32x4*)&sDec[4 * lane] = f32x4{Ip * inv, inv, F, f};
+          const bool off = !__all(F >= kMinStepDecay && F <= 1.f);
+          if (lane == 0) *sPlain = off;
+        } else {
+          sDec[4 * lane + 3] = f;
         }
-        const float inv = fast_rcp(F);
-        *(f32x4*)&sDec[4 * lane] = f32x4{Ip * inv, inv, F, f};
-        const bool off = !__all(F >= kMinStepDecay && F <= 1.f);
-        if (lane == 0) *sPlain = off;
       }
       __syncthreads();
       // row j < kSub: weights of the tokens of the half for the state before step j; row kSub: for the state after token 31
@@ -588,23 +599,25 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           if (idx >= NT) { half_fetch(0, idx, y0); half_fetch(1, idx, y1); }
           half_put(idx, y0, sT0);
           if (two) half_put(idx, y1, sT1);
-          big = largest(y1, largest(y0, big));
+          if constexpr (kScaled) big = largest(y1, largest(y0, big));
         }
       } else if (it1 < HI && (two || hf1 == 0)) {
         half_put(it1, y0, hf1 ? sT1 : sT0);
-        big = largest(y0, big);
+        if constexpr (kScaled) big = largest(y0, big);
       }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)kt[e]), __builtin_fabsf((float)kt1[e])));
       base_put(bs);
-      float bigs = Ip;
+      if constexpr (kScaled) {
 #pragma unroll
-      for (int x = 0; x < DT; ++x)
+        for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)kt[e]), __builtin_fabsf((float)kt1[e])));
+        float bigs = Ip;
 #pragma unroll
-        for (int r = 0; r < DN; ++r) bigs = fmaxf(bigs, fmaxf(__builtin_fabsf(bs.m[x][r]), __builtin_fabsf(bs.y[x][r])));
-      if (!(big <= kMaxRow && bigs <= kMaxState)) *sPlain = 1;
+        for (int x = 0; x < DT; ++x)
+#pragma unroll
+          for (int r = 0; r < DN; ++r) bigs = fmaxf(bigs, fmaxf(__builtin_fabsf(bs.m[x][r]), __builtin_fabsf(bs.y[x][r])));
+        if (!(big <= kMaxRow && bigs <= kMaxState)) *sPlain = 1;
+      }
       __syncthreads();
-      plain = __builtin_amdgcn_readfirstlane(*sPlain) != 0;
+      if constexpr (kScaled) plain = __builtin_amdgcn_readfirstlane(*sPlain) != 0;
       deposit(last);
       if (two) {
         state_at(kSub, sT0);
@@ -890,10 +903,10 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       __syncthreads();
     }
     // (vmcnt(0): to the compiler one loop may follow the other, which would then wait for what this one has requested)
-    if constexpr (!SCALED) __builtin_amdgcn_s_waitcnt(0x0f70);
+    if constexpr (kScaled && !SCALED) __builtin_amdgcn_s_waitcnt(0x0f70);
     };
     if (plain) steps(std::false_type{});
-    else steps(std::true_type{});
+    else if constexpr (kScaled) steps(std::true_type{});
     {
       f32x4 x;
       raw4 fw;

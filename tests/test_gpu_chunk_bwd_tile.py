@@ -158,6 +158,47 @@ def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
                 assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (big, n, h, err)
 
 
+@pytest.mark.parametrize("dk,dv", [(16, 16), (32, 64), (48, 48), (64, 64), (96, 80)])
+@pytest.mark.parametrize("case", ["fp32", "fp32-var", "bf16-var"])
+@pytest.mark.parametrize("end", ["large", "small"])
+def test_gradients_at_the_ends_of_the_range(gpu_device, dk, dv, case, end):
+    """Strong decays inside a step (f = 2^-54.5), where what is divided by a decay is largest and what is multiplied by one
+    least: gradients of the outputs of 2^90 stay finite, and with a precision of 2^60 gradients of 2^-32 keep their bits.  Head
+    by head against the float64 recurrence; as a small pass, and repeated in the batch until its pieces run one after the other."""
+    from palimpsa_amd.ops.palimpsa import chunk_palimpsa
+    rows, var = torch.float32 if case.startswith("fp32") else torch.bfloat16, case.endswith("var")
+    H, T, many = 4, 64 * 3 + 21, 33                   # 4 tiles of 4 heads, or 528 of them
+    inp = hp.rounded(po.make_inputs(1, T, H, dk, dv, seed=dk + dv), rows)
+    inp["g"] = torch.full((H,), 0.6931472)            # f = 2^-gt
+    inp["gt"] = 0.3 * torch.rand(1, T, H, generator=torch.Generator().manual_seed(1))
+    inp["gt"][:, 97::8] = 54.5
+    gen = torch.Generator().manual_seed(T)
+    mu0 = 0.1 * torch.randn(1, H, dv, dk, generator=gen)
+    if end == "small":
+        inp["Ip"] = inp["Ip"] * 2.0 ** 60
+    I0 = inp["Ip"].view(1, H, 1, 1) * (1 + torch.rand(1, H, dv, dk, generator=gen))
+    size = 2.0 ** 90 if end == "large" else 2.0 ** -32
+    do = (size * torch.randn(1, T, H, dv, generator=gen)).to(rows).float()
+    dov = (size * torch.rand(1, T, H, dv, generator=gen)).to(rows).float() if var else None
+    ref = hp.oracle_grads(inp, do, dov, mu0=mu0, I0=I0)
+    for n_copies in (1, many):
+        per_row = {n: x.to(gpu_device).repeat(n_copies, *[1] * (x.dim() - 1)) for n, x in inp.items() if x.dim() > 1}
+        leaves = {n: per_row.get(n, inp[n].to(gpu_device)).clone().requires_grad_(True) for n in NAMES}
+        states = [x.to(gpu_device).repeat(n_copies, 1, 1, 1) for x in (mu0, I0)]
+        out = chunk_palimpsa(*[leaves[n] for n in NAMES], *states, output_uncertainty=var)
+        grads = [x.to(rows).to(gpu_device).repeat(n_copies, 1, 1, 1) for x in ((do, dov) if var else (do,))]
+        got = torch.autograd.grad(list(out) if var else [out], [leaves[n] for n in "qkvb"], grads)
+        for n, x in zip("qkvb", got):
+            assert bool(torch.isfinite(x).all()), (n_copies, n)
+            for h in range(H):
+                err = hp.max_rel(x[-1:, :, h], ref[n][:, :, h])
+                assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (n_copies, n, h, err)
+                if n == "b" and end == "small":
+                    continue   # (in the strong steps do r mu k^2 itself is below fp32's range)
+                err = hp.max_rel(x[-1:, 97:104, h], ref[n][:, 97:104, h])   # tokens of the strong steps by themselves
+                assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (n_copies, n, h, err)
+
+
 @pytest.mark.parametrize("few", [1, 5, 8, 10])
 @pytest.mark.parametrize("dk,dv", [(16, 48), (32, 64), (48, 48), (64, 48), (64, 64)])
 @pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
