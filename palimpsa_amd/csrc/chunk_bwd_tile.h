@@ -20,9 +20,9 @@
 //   dM' <- dM' + (do_t r') q_t    dJ' <- dJ' - (do_t r' mu) q_t    dv = (1 / F_t) sum_n dM' k,  dk = sum_d dM' (v / F) + ...
 // so that a decay costs nothing per entry (17 instructions instead of 20; dM, dJ take the step's whole decay once), v / F and
 // b / F are formed where the rows are staged, and F dM of the step's first token is the carry that the step before it takes.
-// A tile is worked in plain form where a step decays below 2^-56, the decay since the start of a step exceeds 1, or a row's
-// entry is above 2^20 or a state or Ip above 2^66: then nothing over F leaves fp32's range.  (Two copies of the loop: both forms of
-// a step in one loop keep too many registers.)
+// A tile is worked in plain form where a step decays below 2^-40, the decay since the start of a step exceeds 1, or rows, the state
+// at its start or Ip are large (kMaxV and so on): then nothing over F leaves fp32's range, and nothing times F that counts.  (Two
+// copies of the loop: both forms of a step in one loop keep too many registers.)
 // 1 / F (a product and a hardware reciprocal, one ulp) and the products with it round once more: under the rounding of bf16 rows that is
 // nothing (gradients against a float64 recurrence: the same three digits), but fp32 rows' gradients were up to 12 % further off where
 // tokens decay by e^-2 or more (dk, 96x96 and 64x64), for 4 % of the time (64x64 B=8 T=2048 H=8 444 us, plain 458).  With the
@@ -175,8 +175,11 @@ struct TokRev {
   }
 };
 
-// Least decay over a step, and largest row entries and states, for the scaled form: then nothing over F leaves fp32's range.
-constexpr float kMinStepDecay = 0x1p-56f, kMaxRow = 0x1p20f, kMaxState = 0x1p66f;
+// Least decay over a step, and largest entries of v, b, k and of the state at the tile's start (and Ip), for the scaled form.  At
+// the upper end nothing over F then leaves fp32's range (M' < 2^71, J' + Ip / F < 2^63).  At the lower end a tile's precisions stay below
+// 2^20 + 64 x 2^7 x 2^8 < 2^22, so that r' = F r is at least 2^-62, and what is left of a gradient's term do r mu q after F has
+// 12 bits above fp32's last one (2^-149) for terms down to 2^-97: r, mu of 2^-22, 2^-25 and q of 2^-4 leave do down to 2^-46.
+constexpr float kMinStepDecay = 0x1p-40f, kMaxV = 0x1p20f, kMaxB = 0x1p7f, kMaxK = 0x1p4f, kMaxState = 0x1p20f;
 
 // waves per SIMD that a lane's E state entries leave registers for
 constexpr int tile_waves(int E) { return E > 4 ? 2 : 3; }
@@ -367,12 +370,13 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           if constexpr (F32) *(bf16x2*)(p + DS * kHS) = pack2(a0 - (float)hi[0], a1 - (float)hi[1]);
         }
     };
-    auto largest = [&](const HalfItem& y, float big) {
+    float largest[3] = {0.f, 0.f, 0.f};   // |v|, |b|, |k| of the thread's items
+    auto look = [&](const HalfItem& y) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)y.x[t][0][e]), __builtin_fabsf((float)y.x[t][1][e])));
-      return big;
+        for (int e = 0; e < 8; ++e)
+          largest[t] = fmaxf(largest[t], fmaxf(__builtin_fabsf((float)y.x[t][0][e]), __builtin_fabsf((float)y.x[t][1][e])));
     };
     // the wave's k in operand layout (tokens 8g + j of the half; operand row i is column i & 3 of lane group i >> 2)
     TIn kt[8];
@@ -527,7 +531,6 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       asm volatile("" : "+v"(tp));
       BaseIn bs;
       HalfItem y0, y1;
-      float big = 0.f;   // the largest of v, b and k
       bf16_t* const sT0 = BOTH || !two ? sT : (bf16_t*)(smem + L.oPart);
       bf16_t* const sT1 = BOTH ? sT + 2 * PL * DS * kHS : sT;
       // (the gates first: the decays are what the rest waits for)
@@ -599,22 +602,22 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           if (idx >= NT) { half_fetch(0, idx, y0); half_fetch(1, idx, y1); }
           half_put(idx, y0, sT0);
           if (two) half_put(idx, y1, sT1);
-          if constexpr (kScaled) big = largest(y1, largest(y0, big));
+          if constexpr (kScaled) { look(y0); look(y1); }
         }
       } else if (it1 < HI && (two || hf1 == 0)) {
         half_put(it1, y0, hf1 ? sT1 : sT0);
-        if constexpr (kScaled) big = largest(y0, big);
+        if constexpr (kScaled) look(y0);
       }
       base_put(bs);
       if constexpr (kScaled) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) big = fmaxf(big, fmaxf(__builtin_fabsf((float)kt[e]), __builtin_fabsf((float)kt1[e])));
-        float bigs = Ip;
+        for (int e = 0; e < 8; ++e) largest[2] = fmaxf(largest[2], fmaxf(__builtin_fabsf((float)kt[e]), __builtin_fabsf((float)kt1[e])));
+        float state = __builtin_fabsf(Ip);
 #pragma unroll
         for (int x = 0; x < DT; ++x)
 #pragma unroll
-          for (int r = 0; r < DN; ++r) bigs = fmaxf(bigs, fmaxf(__builtin_fabsf(bs.m[x][r]), __builtin_fabsf(bs.y[x][r])));
-        if (!(big <= kMaxRow && bigs <= kMaxState)) *sPlain = 1;
+          for (int r = 0; r < DN; ++r) state = fmaxf(state, fmaxf(__builtin_fabsf(bs.m[x][r]), __builtin_fabsf(bs.y[x][r])));
+        if (!(largest[0] <= kMaxV && largest[1] <= kMaxB && largest[2] <= kMaxK && state <= kMaxState)) *sPlain = 1;
       }
       __syncthreads();
       if constexpr (kScaled) plain = __builtin_amdgcn_readfirstlane(*sPlain) != 0;

@@ -159,7 +159,7 @@ def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
 
 
 @pytest.mark.parametrize("dk,dv", [(16, 16), (32, 64), (48, 48), (64, 64), (96, 80)])
-@pytest.mark.parametrize("case", ["fp32", "fp32-var", "bf16-var"])
+@pytest.mark.parametrize("case", ["fp32", "fp32-var", "bf16", "bf16-var"])
 @pytest.mark.parametrize("end", ["large", "small"])
 def test_gradients_at_the_ends_of_the_range(gpu_device, dk, dv, case, end):
     """Strong decays inside a step (f = 2^-54.5), where what is divided by a decay is largest and what is multiplied by one
