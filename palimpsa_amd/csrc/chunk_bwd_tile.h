@@ -280,8 +280,10 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           const bool on = t < ntok && c < (kq ? DNG : DS);
           if (ntok > 0) {
             const int64_t o = kq ? (int64_t)n0 + (on ? s * qks + t * qks + c : 0) : (int64_t)r0 + (on ? s * vs + t * vs + c : 0);
-            r1 = *(const raw4*)((kq ? kp : vp) + o);
-            r2 = *(const raw4*)((kq ? qp : bp) + o);
+            const TIn *p1 = kp, *p2 = qp;   // (opaque: of a choice between two pointers the compiler makes one between places in scratch memory)
+            asm volatile("" : "+s"(p1), "+s"(p2));
+            r1 = *(const raw4*)((kq ? p1 : vp) + o);
+            r2 = *(const raw4*)((kq ? p2 : bp) + o);
             r3 = *(const raw4*)(dop + (kq ? (int64_t)r0 : o));
           }
         }
