@@ -116,7 +116,12 @@ __host__ __device__ constexpr int tile_g(int DT, int DN) { return DT * DN <= 9 ?
 __host__ __device__ constexpr int rows_pad(int DT) { return DT == 3 ? 4 : DT; }
 __host__ __device__ constexpr int vb_stride(int DT, bool var) { return (var ? 4 : 3) * 16 * rows_pad(DT) + 4; }
 
-// LDS (floats): running decay, decays of every token (and which tokens rule scaled form out), decay weights of every step's state, their factors of the base state,
+// whether the tile kernel has a scaled form (chunk_bwd_tile.h), and the numbers that it keeps per token: Ip / F, 1 / F and F with it, f
+__host__ __device__ constexpr bool tile_scales(bool var, bool f32) { return !var && !f32; }
+__host__ __device__ constexpr int tile_decs(bool var, bool f32) { return tile_scales(var, f32) ? 4 : 1; }
+
+// LDS (floats): running decay, decays of every token (and whether the tile is worked in plain form), decay weights of every step's
+// state, their factors of the base state,
 // gamma_t, its partial sums; base states; transposed v, b of both halves (of one, and the first half's in the
 // partial sums' memory at the start, where that lets two workgroups share a compute unit); two buffers of staged rows
 // and of partial dv, db
@@ -128,7 +133,7 @@ __host__ __device__ constexpr TileLds tile_lds(int DT, int DN, int nbw, bool var
   const int G = tile_g(DT, DN), half = (f32 ? 2 : 1) * 16 * DT * kHS;   // (two tensors of bf16)
   for (int both = 1; both >= 0; --both) {
     int o = kC;
-    L.oDec = o; o += 4 * kC + 8;
+    L.oDec = o; o += tile_decs(var, f32) * kC + (tile_scales(var, f32) ? 8 : 4);
     L.oW = o; o += (kC / G + 1) * kHalf;
     L.oFB = o; o += kC / G + 4;
     L.oX = o; o += kC + 4;

@@ -150,19 +150,19 @@ __device__ __forceinline__ void lds_vals(const float* p, float* out) {
 }
 
 // what both sweeps read of a token: its k, v and b (over F in scaled form), and in plain form f
-template <int DT, bool SCALED>
+template <int DT, bool SCALED, int DS>
 struct TokFwd {
   f32x4 k;
   float v[DT], b[DT], f;
   __device__ __forceinline__ void load(const float* kq, const float* vb, const float* dec, int plane) {
-    if constexpr (!SCALED) f = dec[3];
+    if constexpr (!SCALED) f = dec[DS - 1];
     k = *(const f32x4*)kq;
     lds_vals<DT>(vb, v);
     lds_vals<DT>(vb + plane, b);
   }
 };
 // and the reverse sweep: q, do, (dovar), Ip and 1 / F or, in plain form, the next token's f
-template <int DT, bool VAR, bool SCALED>
+template <int DT, bool VAR, bool SCALED, int DS>
 struct TokRev {
   f32x4 q;
   float d_o[DT], d_ov[VAR ? DT : 1], ip, inv;
@@ -171,7 +171,7 @@ struct TokRev {
     lds_vals<DT>(vb + 2 * plane, d_o);
     if constexpr (VAR) lds_vals<DT>(vb + 3 * plane, d_ov);
     ip = SCALED ? dec[0] : Ip;
-    inv = dec[SCALED ? 1 : 7];
+    inv = dec[SCALED ? 1 : 2 * DS - 1];
   }
 };
 
@@ -197,11 +197,12 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   constexpr int NT = NBW * 64, DNG = WC * NBW;
   constexpr TileLds L = tile_lds(DT, DN, NBW, VAR, F32);
   constexpr int kG = tile_g(DT, DN), kSub = kC / kG;   // tokens per step, steps per tile
-  constexpr bool kScaled = !F32 && !VAR;    // whether there is a scaled form
+  constexpr bool kScaled = tile_scales(VAR, F32);
+  constexpr int kDS = tile_decs(VAR, F32);   // numbers kept per token, f the last of them
   constexpr bool BOTH = L.both != 0;
   float* sC = smem;
   float* sDec = smem + L.oDec;   // [64] (scaled form: Ip / F_t, 1 / F_t, F_t,) f_t
-  int* sPlain = (int*)(smem + L.oDec + 4 * kC);   // whether the tile is worked in plain form
+  int* sPlain = (int*)(smem + L.oDec + kDS * kC);   // (scaled form) whether the tile is worked in plain form
   float* sW = smem + L.oW;
   float* sFB = smem + L.oFB;
   float* sX = smem + L.oX;
@@ -574,7 +575,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
           const bool off = !__all(F >= kMinStepDecay && F <= 1.f);
           if (lane == 0) *sPlain = off;
         } else {
-          sDec[4 * lane + 3] = f;
+          sDec[lane] = f;
         }
       }
       __syncthreads();
@@ -691,7 +692,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       }
       const float* krow = smem + L.oKQ + ((j & 1) * NBW + w) * kG * 32 + 4 * g;
       const float* vrow = smem + L.oVB + (j & 1) * kG * SV + i * DTP;
-      const float* dec = sDec + 4 * kG * j;
+      const float* dec = sDec + kDS * kG * j;
       const int o_tok = kG * j * (int)dks;   // (64 tokens of a tile stay within 32 bits)
       float* part = smem + L.oPart + ((j & 1) * NBW + w) * (kG * 32 * DT);
       float was[kG / 4][2];
@@ -716,15 +717,15 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
       {
         float sM[kG][DT][DN], sJ[kG][DT][DN];   // state after each token; in reverse mu and 1 / I in their place
         // ---- forward over the step; a token's operands are requested during the arithmetic of the token before it
-        TokFwd<DT, SCALED> xf[kG], xr[kG];
-        TokRev<DT, VAR, SCALED> yr[kG];
+        TokFwd<DT, SCALED, kDS> xf[kG], xr[kG];
+        TokRev<DT, VAR, SCALED, kDS> yr[kG];
         xf[0].load(krow, vrow, dec, plane);
 #pragma unroll
         for (int u = 0; u < kG; ++u) {
-          const TokFwd<DT, SCALED>& x = xf[u];
+          const TokFwd<DT, SCALED, kDS>& x = xf[u];
           __builtin_amdgcn_sched_barrier(0);
-          if (u + 1 < kG) xf[u + 1].load(krow + (u + 1) * 32, vrow + (u + 1) * SV, dec + 4 * (u + 1), plane);
-          else yr[u].load(krow + u * 32, vrow + u * SV, dec + 4 * u, Ip, plane);
+          if (u + 1 < kG) xf[u + 1].load(krow + (u + 1) * 32, vrow + (u + 1) * SV, dec + kDS * (u + 1), plane);
+          else yr[u].load(krow + u * 32, vrow + u * SV, dec + kDS * u, Ip, plane);
 #pragma unroll
           for (int r = 0; r < DN; ++r) {
             const float kk = x.k[r] * x.k[r];
@@ -768,8 +769,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
 #pragma unroll
         for (int u = kG - 1; u >= 0; --u) {
           __builtin_amdgcn_sched_barrier(0);
-          const TokFwd<DT, SCALED>& x = u + 1 < kG ? xr[u] : xf[u];
-          const TokRev<DT, VAR, SCALED>& y = yr[u];
+          const TokFwd<DT, SCALED, kDS>& x = u + 1 < kG ? xr[u] : xf[u];
+          const TokRev<DT, VAR, SCALED, kDS>& y = yr[u];
           float dq[DN], dqv[DN], dk[DN], dvp[DT], dbp[DT], St = 0.f, gate = 0.f;
           TokSums<DT, DN>& before = ts[(u + 1) & 1];   // of the token worked before this one
           if (u + 1 < kG) before.stage_a();
@@ -779,8 +780,8 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
             if (r == 1 && u + 1 < kG) before.stage_b();
             if (r == 2 && u + 1 < kG) finish(u + 1, before, inv_before);
             if (r == DN - 2 && u > 0) {   // half of mu, r of this token are dead: room for the next token's operands
-              xr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, dec + 4 * (u - 1), plane);
-              yr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, dec + 4 * (u - 1), Ip, plane);
+              xr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, dec + kDS * (u - 1), plane);
+              yr[u - 1].load(krow + (u - 1) * 32, vrow + (u - 1) * SV, dec + kDS * (u - 1), Ip, plane);
             }
             __builtin_amdgcn_s_setprio(3);
 #pragma unroll
