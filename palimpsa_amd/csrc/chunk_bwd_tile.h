@@ -796,24 +796,28 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
             float dkM, dkJ, Sw;
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
-              const float ri = sJ[u][d][r], m = sM[u][d][r], p = y.d_o[d] * ri;
-              float t;   // G r mu over q
+              const float ri = sJ[u][d][r], m = sM[u][d][r];
+              const float fn = !SCALED && u + 1 < kG ? y.inv : 1.f;   // (plain form)
               if constexpr (VAR) {
-                const float e = y.d_o[d] * m, n = y.d_ov[d] * ri;
+                const float e = y.d_o[d] * m, n = y.d_ov[d] * ri, t = fmaf(n, y.q[r], e) * ri;   // G r mu over q
                 dq[r] = d ? dq[r] + e : e;
                 dqv[r] = d ? dqv[r] + n : n;
-                t = fmaf(n, y.q[r], e) * ri;
+                Sw = d ? Sw + t : t;
+                dM[d][r] = fmaf(dM[d][r], fn, y.d_o[d] * ri * y.q[r]);
+                dJ[d][r] = fmaf(dJ[d][r], fn, -t * y.q[r]);
               } else {
                 dq[r] = d ? fmaf(m, y.d_o[d], dq[r]) : m * y.d_o[d];
-                t = p * m;
-              }
-              Sw = d ? Sw + t : t;
-              if constexpr (SCALED) {
-                dM[d][r] = fmaf(p, y.q[r], dM[d][r]);
-                dJ[d][r] = fmaf(-t, y.q[r], dJ[d][r]);
-              } else {
-                dM[d][r] = fmaf(dM[d][r], u + 1 < kG ? y.inv : 1.f, p * y.q[r]);
-                dJ[d][r] = fmaf(dJ[d][r], u + 1 < kG ? y.inv : 1.f, -t * y.q[r]);
+                if constexpr (SCALED) {
+                  const float p = y.d_o[d] * ri, t = p * m;   // G r mu over q
+                  Sw = d ? Sw + t : t;
+                  dM[d][r] = fmaf(p, y.q[r], dM[d][r]);
+                  dJ[d][r] = fmaf(-t, y.q[r], dJ[d][r]);
+                } else {
+                  const float p = y.d_o[d] * y.q[r] * ri, t = p * m;   // G r mu
+                  Sw = d ? Sw + t : t;
+                  dM[d][r] = fmaf(dM[d][r], fn, p);
+                  dJ[d][r] = fmaf(dJ[d][r], fn, -t);
+                }
               }
               if (u > 0) gate = fmaf(dM[d][r], sM[u ? u - 1 : 0][d][r], fmaf(dJ[d][r], sJ[u ? u - 1 : 0][d][r], gate));
               dkM = d ? fmaf(dM[d][r], x.v[d], dkM) : dM[d][r] * x.v[d];
@@ -821,7 +825,7 @@ void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
               dvp[d] = r ? fmaf(dM[d][r], x.k[r], dvp[d]) : dM[d][r] * x.k[r];
               dbp[d] = r ? fmaf(dJ[d][r], kk, dbp[d]) : dJ[d][r] * kk;
             }
-            St = fmaf(Sw, y.q[r], St);
+            St = VAR || SCALED ? fmaf(Sw, y.q[r], St) : St + Sw;
             dk[r] = fmaf(2.f * x.k[r], dkJ, dkM);
           }
           TokSums<DT, DN>& mine = ts[u & 1];
