@@ -181,11 +181,13 @@ struct TokRev {
 // 12 bits above fp32's last one (2^-149) for terms down to 2^-97: r, mu of 2^-22, 2^-25 and q of 2^-4 leave do down to 2^-46.
 constexpr float kMinStepDecay = 0x1p-40f, kMaxV = 0x1p20f, kMaxB = 0x1p7f, kMaxK = 0x1p4f, kMaxState = 0x1p20f;
 
-// waves per SIMD that a lane's E state entries leave registers for
-constexpr int tile_waves(int E) { return E > 4 ? 2 : 3; }
+// Waves per SIMD that a lane's E state entries leave registers for.  Three entries (48 columns by 16 rows) take 131 to 136 and are held to
+// 128, for up to four spilled: 80x80 at 192 tiles x heads 138 -> 123 us, with the uncertainty 172 -> 154, at 384 242 -> 232; not where
+// that spills more (`four`: earlier launches' sums added, or fp32 rows with the uncertainty).
+constexpr int tile_waves(int E, bool four) { return E > 4 ? 2 : E == 3 && four ? 4 : 3; }
 
 template <typename TIn, int DT, int DN, int NBW, bool VAR, int SLICE>
-__global__ __attribute__((amdgpu_flat_work_group_size(NBW * 64, NBW * 64), amdgpu_waves_per_eu(tile_waves(DT * DN))))
+__global__ __attribute__((amdgpu_flat_work_group_size(NBW * 64, NBW * 64), amdgpu_waves_per_eu(tile_waves(DT * DN, SLICE != 2 && !(VAR && sizeof(TIn) == 4)))))
 void chunk_bwd_tile_kernel(BwdArgs A, TileRect R) {
   const ChunkArgs& a = A.c;
   extern __shared__ float smem[];
