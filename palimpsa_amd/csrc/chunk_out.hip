@@ -99,7 +99,7 @@ __device__ __forceinline__ float dpp_shr(float x) {   // lane i of a row of 16 t
 // SEGS: the states are kept since the start of a segment (state_pass_segments; an instance of its own: the branch and its
 // values took 1 to 2 % from calls that have none)
 template <typename TIn, int NG, int DN, int DD, bool HAS_VAR, bool SEGS>
-__global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(HAS_VAR ? 2 : 4)))
+__global__ __attribute__((amdgpu_flat_work_group_size(64, 512), amdgpu_waves_per_eu(HAS_VAR ? 2 : 4, !HAS_VAR && DD == 2 ? 4 : 8)))
 void chunk_out_kernel(ChunkArgs a, int W) {
   extern __shared__ float smem[];
   typedef typename Raw4<TIn>::type raw4;
