@@ -108,17 +108,19 @@ def test_small_passes_agree_with_large_ones(gpu_device, dk, dv, rows):
 @pytest.mark.parametrize("dk,dv", [(16, 16), (32, 64), (48, 48), (64, 64), (96, 80)])
 @pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
-    """A tile is worked with the decay of a step taken out of the state, or in plain form where a step decays below 2^-56, a
-    token grows, or rows, states or Ip are large.  Heads on either side of each line (every one with tiles of both kinds),
+    """A tile of bf16 rows without the uncertainty is worked with the decay of a step taken out of the state, or in plain form
+    where a step decays below 2^-40, the decay since its start exceeds 1, or v, b, k, the state or Ip are large; fp32 rows and the
+    uncertainty always in plain form.  Heads on either side of each line (every one with tiles of both kinds), as a small pass, in
+    slices of 16 rows and mostly eight tokens a step, and repeated in the batch until the pieces run whole, one after the other;
     gradients head by head against the float64 recurrence."""
     from palimpsa_amd.ops.palimpsa import chunk_palimpsa
-    H, T = 6, 64 * 4 + 21
+    H, T, many = 6, 64 * 4 + 21, 18                  # 5 tiles of 6 heads, or 540 of them
     base = po.make_inputs(1, T, H, dk, dv, seed=dk + dv)
     base["g"] = torch.full((H,), 0.6931472)          # f = 2^-gt
     gt = 0.3 * torch.rand(1, T, H, generator=torch.Generator().manual_seed(1))
-    gt[:, 70:, 1] = 13.9                             # four tokens: 2^-55.6, eight 2^-111
-    gt[:, 70:90, 2] = 6.99                           # eight: 2^-55.92
-    gt[:, 70:90, 3] = 7.01                           # eight: 2^-56.08
+    gt[:, 70:, 1] = 9.9                              # four tokens: 2^-39.6, eight 2^-79
+    gt[:, 70:90, 2] = 4.99                           # eight: 2^-39.92
+    gt[:, 70:90, 3] = 5.01                           # eight: 2^-40.08
     gt[:, 100::64, 4] = 80.0                         # single tokens
     gt[:, 100:120, 5] = -0.05                        # f > 1
     base["gt"] = gt
@@ -126,36 +128,46 @@ def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
     mu0 = 0.1 * torch.randn(1, H, dv, dk, generator=gen)
     I0 = base["Ip"].view(1, H, 1, 1) + torch.rand(1, H, dv, dk, generator=gen)
     noise = torch.randn(1, T, H, dv, generator=gen)
-    for big in ("none", "v", "b", "k", "state", "Ip"):
+    unc = 0.3 * torch.rand(1, T, H, dv, generator=gen)
+    # rows and states beyond their lines, and just inside
+    cases = [("none", 1.0)] + [(n, 2.0 ** 24) for n in "vbk"] + [("state", 2.0 ** 70), ("Ip", 2.0 ** 70)]
+    cases += [("v", 2.0 ** 17), ("b", 2.0 ** 6), ("k", 2.0 ** 3), ("Ip", 2.0 ** 17)]
+    for what, size in cases:
         raw, m0, i0 = dict(base), mu0, I0
-        if big in ("v", "b"):
-            raw[big] = base[big].clone()
-            raw[big][:, 130:140] *= 2.0 ** 24
-        if big == "k":
-            raw["k"] = base["k"].clone()
-            raw["k"][:, 130:140] *= 2.0 ** 24
-        if big == "state":
+        if what in "vbk":
+            raw[what] = base[what].clone()
+            raw[what][:, 130:140] *= size
+        if what == "state":
             m0, i0 = mu0.clone(), I0.clone()
-            i0[:, ::2] *= 2.0 ** 70
-        if big == "Ip":
-            raw["Ip"] = base["Ip"] * torch.tensor([2.0 ** 70, 1, 2.0 ** 70, 1, 2.0 ** 70, 1])
+            i0[:, ::2] *= size
+        if what == "Ip":
+            raw["Ip"] = base["Ip"] * torch.tensor([size, 1, size, 1, size, 1])
             i0 = raw["Ip"].view(1, H, 1, 1) * (I0 / base["Ip"].view(1, H, 1, 1))
         inp = hp.rounded(raw, rows)
         o_ref, _, _, _ = hp.oracle_forward(inp, mu0=m0, I0=i0, dtype=torch.float64)
         do = (o_ref - 0.3 * noise * o_ref.abs().mean(dim=(0, 1, 3), keepdim=True)).float()   # as large as the head's outputs
-        ref = hp.oracle_grads(inp, do, None, mu0=m0, I0=i0)
-        leaves = {n: inp[n].to(gpu_device).clone().requires_grad_(True) for n in NAMES}
-        leaves["mu0"], leaves["I0"] = (x.to(gpu_device).requires_grad_(True) for x in (m0, i0))
-        out = chunk_palimpsa(*[leaves[n] for n in NAMES], initial_mu_state=leaves["mu0"], initial_I_state=leaves["I0"])
-        got = torch.autograd.grad((out.float() * do.to(gpu_device)).sum(), list(leaves.values()))
-        for n, x in zip(leaves, got):
-            assert bool(torch.isfinite(x).all()), (big, n)
-            if big in ("state", "Ip") and n in ("gt", "g", "I0", "Ip"):
-                continue   # <dM, M> + <dJ, J> with M = mu I: two terms whose difference is smaller by the 2^70
-            dim = {"g": 0, "Ip": 0, "mu0": 1, "I0": 1}.get(n, 2)
-            for h in range(H):
-                err = hp.max_rel(x.select(dim, h), ref[n].select(dim, h))
-                assert err <= (hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL), (big, n, h, err)
+        do = do.to(rows).float()
+        for var in (False, True) if what in ("none", "b") else (False,):
+            dov = unc.to(rows).float() if var else None
+            ref = hp.oracle_grads(inp, do, dov, mu0=m0, I0=i0)
+            for copies in (1, many):
+                rep = lambda x: x.to(gpu_device).repeat(copies, *[1] * (x.dim() - 1)) if x.dim() > 1 else x.to(gpu_device)
+                leaves = {n: rep(inp[n]).clone().requires_grad_(True) for n in NAMES}
+                leaves["mu0"], leaves["I0"] = (rep(x).clone().requires_grad_(True) for x in (m0, i0))
+                out = chunk_palimpsa(*[leaves[n] for n in NAMES], initial_mu_state=leaves["mu0"], initial_I_state=leaves["I0"],
+                                     output_uncertainty=var)
+                grads = [rep(x).to(rows) for x in ((do, dov) if var else (do,))]
+                got = torch.autograd.grad(list(out) if var else [out], list(leaves.values()), grads)
+                for n, x in zip(leaves, got):
+                    assert bool(torch.isfinite(x).all()), (what, size, var, copies, n)
+                    if what in ("state", "Ip") and size > 1 and n in ("gt", "g", "I0", "Ip"):
+                        continue   # <dM, M> + <dJ, J> with M = mu I: two terms whose difference is smaller by the size of I
+                    x = x[-1:] if x.dim() > 1 else x / copies
+                    dim = {"g": 0, "Ip": 0, "mu0": 1, "I0": 1}.get(n, 2)
+                    for h in range(H):
+                        err = hp.max_rel(x.select(dim, h), ref[n].select(dim, h))
+                        bar = hp.CHUNK_FP32_GRAD_TOL if rows == torch.float32 else hp.BF16_GRAD_NORM_TOL
+                        assert err <= bar, (what, size, var, copies, n, h, err)
 
 
 @pytest.mark.parametrize("dk,dv", [(16, 16), (32, 64), (48, 48), (64, 64), (96, 80)])
