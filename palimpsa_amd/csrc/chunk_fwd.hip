@@ -351,6 +351,7 @@ void fill_chunk_args(ChunkArgs& a, const PalDims* d, const PalFwdTensors* t) {
 namespace pal {
 // the outputs from the tile-start states, and how many tiles it walks from one where no one else reads them (chunk_out.hip)
 int out_tiles_per_state(const ChunkArgs& a);
+bool out_takes_segments(const ChunkArgs& a, int dtype);
 int launch_out(const ChunkArgs& a, int dtype, hipStream_t s);
 // the one-pass form of chunk_states.hip, and the segments (a.segs, a.seg_tiles) that it cuts a sequence into where few states are kept
 void state_pass_segments(ChunkArgs& a);
@@ -481,7 +482,7 @@ extern "C" int pal_chunk_fwd_static(const PalDims* d, const PalFwdTensors* t, vo
 // tiles per kept state, and the segments of the pass that makes them, where the caller needs no state afterwards
 static void sparse_states(pal::ChunkArgs& a, int dtype) {
   a.every = pal::out_tiles_per_state(a);
-  if (pal::state_pass_applies(a, dtype, true)) pal::state_pass_segments(a);
+  if (pal::state_pass_applies(a, dtype, true) && pal::out_takes_segments(a, dtype)) pal::state_pass_segments(a);
 }
 
 extern "C" int pal_chunk_fwd_segments(const PalDims* d, int32_t* tiles_per_state, int32_t* tiles_per_segment) {

@@ -431,7 +431,7 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
     if constexpr (DD == 2 && sizeof(TIn) == 2) {
       rc = var ? go(&chunk_out_kernel<TIn, NG, DN, DD, true, true>) : go(&chunk_out_kernel<TIn, NG, DN, DD, false, true>);
     } else {
-      rc = PAL_E_DIM;   // (segments are of bf16 rows, and only where two rows to a lane fill the SIMDs: out_tiles_per_state)
+      rc = PAL_E_DIM;   // (out_takes_segments)
     }
   }
   if (rc) return rc;
@@ -439,14 +439,23 @@ static int launch_out_dd(const ChunkArgs& a, hipStream_t s) {
   return PAL_OK;
 }
 
+// Two value rows per lane where that still gives every SIMD two waves; below, one row: half the work per wave and
+// twice the waves (one sequence of 777 tokens, 16 heads of 64x64: 28 us with two rows, 23 with one; B=2 T=2048 H=12 64x64,
+// three waves per SIMD: 49.6 against 51.0).
+static int out_lane_rows(const ChunkArgs& a, int NG) {
+  return (int64_t)a.total_chunks / a.every * a.H * ((a.dv * NG + 127) / 128) <= 2048 ? 1 : 2;
+}
+
 template <typename TIn, int NG, int DN>
 static int launch_out_dn(const ChunkArgs& a, hipStream_t s) {
-  // Two value rows per lane where that still gives every SIMD two waves; below, one row: half the work per wave and
-  // twice the waves (one sequence of 777 tokens, 16 heads of 64x64: 28 us with two rows, 23 with one; B=2 T=2048 H=12 64x64,
-  // three waves per SIMD: 49.6 against 51.0).
-  const int64_t waves = (int64_t)a.total_chunks / a.every * a.H * ((a.dv * NG + 127) / 128);
-  if (waves <= 2048) return launch_out_dd<TIn, NG, DN, 1>(a, s);
-  return launch_out_dd<TIn, NG, DN, 2>(a, s);
+  return out_lane_rows(a, NG) == 1 ? launch_out_dd<TIn, NG, DN, 1>(a, s) : launch_out_dd<TIn, NG, DN, 2>(a, s);
+}
+
+// Whether launch_out takes states of segments: there are instances for them with two rows to a lane only (as many tiles as
+// make segments fill the SIMDs; see out_tiles_per_state).
+bool out_takes_segments(const ChunkArgs& a, int dtype) {
+  const int NG = a.dk <= 32 ? 4 : a.dk <= 64 ? 8 : a.dk <= 128 ? 16 : 32;   // (as launch_out_t)
+  return dtype == PAL_DTYPE_BF16 && out_lane_rows(a, NG) == 2;
 }
 
 template <typename TIn>
