@@ -42,7 +42,9 @@ inline int tile_piece(int n) { return n == 80 ? 48 : n >= 64 ? 64 : n; }
 // worth of waves, and one or two workgroups of them run on a compute unit; slices of 32 rows, twice as many (ps per entry 1.07
 // against 0.77 for 64 columns, 1.38 and 1.34 against 0.97 for 48, 1.53 and 1.35 against 1.07 for 32; us at 256 tiles of 8 heads,
 // 64x64 578 -> 463, 48x48 416 -> 340, 48x96 878 -> 628, 128x64 1169 -> 882, 64x64 with the uncertainty 819 -> 497).  48 rows would
-// leave a slice of 16 and stay together where a pass has `few` tiles (512 tiles x heads, 48x48: 108 us, 116).
+// leave a slice of 16 and stay together where a pass has `few` tiles, one workgroup to a compute unit (whole / in slices, us, by
+// tiles x heads: 48x48 192 60 / 68, 256 59 / 68, 384 110 / 97, 512 113 / 110, 1024 217 / 185, with the uncertainty 256 73 / 73, 384 138 /
+// 108; 32x48 256 67 / 66, 384 89 / 72, 512 90 / 94, 1024 168 / 161).
 inline int tile_rows(int cols, int n, bool f32, bool few) {
   if (cols == 16) return n >= 48 ? 48 : 16;   // (one wave's staging)
   if (f32) return (cols == 64 && n % 48 == 0) || (few && n == 48) ? 48 : n < 32 ? 16 : 32;
@@ -65,7 +67,7 @@ inline int tile_rows(int cols, int n, bool f32, bool few) {
 // fp32 rows 96x96 288 -> 70, 301 -> 184, 382 -> 266, 387 -> 355, 631 -> 528.  The line lies at one and a half workgroups per
 // compute unit; at two for fp32 rows and for heads whose pieces come out small (80x80, 96x96), which are the dearest one after the other.
 // It bounds the parts too: 8 bytes per token, head, slice and key column, and per group and value column (190 MB at most at 96x192).
-constexpr int kPartsTiles = 384, kPartsTilesSmall = 512;   // tiles x heads
+constexpr int kPartsTiles = 384, kPartsTilesSmall = 512, kFewTiles = 256;   // tiles x heads
 // The slices are of 16 rows where their waves are one to a SIMD at most (two, where there is one column group), of 32 else (16 / 32 rows, us, by tiles x heads:
 // 96x96 16 43.3 / 48.8, 32 53.4 / 51.9; 128x64 32 44.3 / 50.8, 64 53.5 / 53.7; 48x96 32 42.7 / 48.9, 64 51.8 / 51.2; 96x192 16
 // 55.1 / 51.8).  A head that is one piece is cut too, from 48 rows on, where the waves of its slices are two to a SIMD at most:
@@ -79,13 +81,13 @@ constexpr int kPartsTiles = 384, kPartsTilesSmall = 512;   // tiles x heads
 constexpr int kPartsWaves = 2048;
 struct TileParts {
   int on, rows, slices, groups;
-  bool few;   // tiles x heads at most kPartsTilesSmall
+  bool few;   // tiles x heads at most kFewTiles
 };
 inline int parts_cols(int dk, int n0) { return dk % 64 == 0 ? 64 : dk % 48 == 0 ? 48 : dk % 32 == 0 ? 32 : tile_piece(dk - n0); }
 inline TileParts tile_parts(int dk, int dv, bool f32, int64_t tile_heads) {
   TileParts P;
   P.groups = 0;
-  P.few = tile_heads <= kPartsTilesSmall;
+  P.few = tile_heads <= kFewTiles;
   int pieces = 0, waves = 0;   // one after the other; of the workgroups of a tile's slice
   for (int n0 = 0, c; n0 < dk; n0 += c, ++P.groups) {
     c = parts_cols(dk, n0);
