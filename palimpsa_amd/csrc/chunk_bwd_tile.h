@@ -20,7 +20,7 @@
 //   dM' <- dM' + (do_t r') q_t    dJ' <- dJ' - (do_t r' mu) q_t    dv = (1 / F_t) sum_n dM' k,  dk = sum_d dM' (v / F) + ...
 // so that a decay costs nothing per entry (17 instructions instead of 20; dM, dJ take the step's whole decay once), v / F and
 // b / F are formed where the rows are staged, and F dM of the step's first token is the carry that the step before it takes.
-// A tile is worked in plain form where a step decays below 2^-40, the decay since the start of a step exceeds 1, or rows, the state
+// A tile is worked in plain form where a step decays below 2^-48, the decay since the start of a step exceeds 1, or rows, the state
 // at its start or Ip are large (kMaxV and so on): then nothing over F leaves fp32's range, and nothing times F that counts.  (Two
 // copies of the loop: both forms of a step in one loop keep too many registers.)
 // 1 / F (a product and a hardware reciprocal, one ulp) and the products with it round once more: under the rounding of bf16 rows that is
@@ -176,10 +176,11 @@ struct TokRev {
 };
 
 // Least decay over a step, and largest entries of v, b, k and of the state at the tile's start (and Ip), for the scaled form.  At
-// the upper end nothing over F then leaves fp32's range (M' < 2^71, J' + Ip / F < 2^63).  At the lower end a tile's precisions stay below
-// 2^20 + 64 x 2^7 x 2^8 < 2^22, so that r' = F r is at least 2^-62, and what is left of a gradient's term do r mu q after F has
-// 12 bits above fp32's last one (2^-149) for terms down to 2^-97: r, mu of 2^-22, 2^-25 and q of 2^-4 leave do down to 2^-46.
-constexpr float kMinStepDecay = 0x1p-40f, kMaxV = 0x1p20f, kMaxB = 0x1p7f, kMaxK = 0x1p4f, kMaxState = 0x1p20f;
+// the upper end nothing over F then leaves fp32's range (M' < 2^80, J' + Ip / F < 2^68).  At the lower end a tile's precisions stay below
+// 2^16 + 64 x 2^4 x 2^8 < 2^19, so that r' = F r is at least 2^-67, and what is left of a gradient's term do r mu q after F has
+// 12 bits above fp32's last one (2^-149) for terms down to 2^-89: r, mu of 2^-19, 2^-22 and q of 2^-4 leave do down to 2^-44.
+// (A step of eight tokens at gates of 0.5 and a rate of 4.5, strong for a layer, decays by 2^26 on average.)
+constexpr float kMinStepDecay = 0x1p-48f, kMaxV = 0x1p20f, kMaxB = 0x1p4f, kMaxK = 0x1p4f, kMaxState = 0x1p16f;
 
 // Waves per SIMD that a lane's E state entries leave registers for.  Three entries (48 columns by 16 rows) take 131 to 136 and are held to
 // 128, for up to four spilled: 80x80 at 192 tiles x heads 138 -> 123 us, with the uncertainty 172 -> 154, at 384 242 -> 232; not where

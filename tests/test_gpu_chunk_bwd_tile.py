@@ -109,7 +109,7 @@ def test_small_passes_agree_with_large_ones(gpu_device, dk, dv, rows):
 @pytest.mark.parametrize("rows", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
     """A tile of bf16 rows without the uncertainty is worked with the decay of a step taken out of the state, or in plain form
-    where a step decays below 2^-40, the decay since its start exceeds 1, or v, b, k, the state or Ip are large; fp32 rows and the
+    where a step decays below 2^-48, the decay since its start exceeds 1, or v, b, k, the state or Ip are large; fp32 rows and the
     uncertainty always in plain form.  Heads on either side of each line (every one with tiles of both kinds), as a small pass, in
     slices of 16 rows and mostly eight tokens a step, and repeated in the batch until the pieces run whole, one after the other;
     gradients head by head against the float64 recurrence."""
@@ -118,9 +118,9 @@ def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
     base = po.make_inputs(1, T, H, dk, dv, seed=dk + dv)
     base["g"] = torch.full((H,), 0.6931472)          # f = 2^-gt
     gt = 0.3 * torch.rand(1, T, H, generator=torch.Generator().manual_seed(1))
-    gt[:, 70:, 1] = 9.9                              # four tokens: 2^-39.6, eight 2^-79
-    gt[:, 70:90, 2] = 4.99                           # eight: 2^-39.92
-    gt[:, 70:90, 3] = 5.01                           # eight: 2^-40.08
+    gt[:, 70:, 1] = 11.9                             # four tokens: 2^-47.6, eight 2^-95
+    gt[:, 70:90, 2] = 5.99                           # eight: 2^-47.92
+    gt[:, 70:90, 3] = 6.01                           # eight: 2^-48.08
     gt[:, 100::64, 4] = 80.0                         # single tokens
     gt[:, 100:120, 5] = -0.05                        # f > 1
     base["gt"] = gt
@@ -131,7 +131,7 @@ def test_scaled_and_plain_tiles(gpu_device, dk, dv, rows):
     unc = 0.3 * torch.rand(1, T, H, dv, generator=gen)
     # rows and states beyond their lines, and just inside
     cases = [("none", 1.0)] + [(n, 2.0 ** 24) for n in "vbk"] + [("state", 2.0 ** 70), ("Ip", 2.0 ** 70)]
-    cases += [("v", 2.0 ** 17), ("b", 2.0 ** 6), ("k", 2.0 ** 3), ("Ip", 2.0 ** 17)]
+    cases += [("v", 2.0 ** 17), ("b", 2.0 ** 3), ("k", 2.0 ** 3), ("Ip", 2.0 ** 13)]
     for what, size in cases:
         raw, m0, i0 = dict(base), mu0, I0
         if what in "vbk":
