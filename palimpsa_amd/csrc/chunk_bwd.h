@@ -29,7 +29,7 @@ struct BwdArgs {
 // 32 or 16 value rows.  (96 columns as 64 + 32, 80 as 48 + 32: workgroups of four or two waves, two or four of them to a
 // compute unit.  One workgroup of eight waves has nothing to fill its barriers and its set-up with: 96x96, 32768 packed
 // tokens, 16 heads: 5.5 ms, as rectangles 4.2.  A rectangle costs, in ps per state entry and token at B=8 T=2048 H=16, bf16
-// rows, 0.63 (64x64: columns x rows), 0.71 (64x48), 0.70 (64x32), 0.81 (48x64), 0.82 (48x48), 0.90 (48x32), 0.89 (32x64), 0.82
+// rows, 0.63 (64x64: columns x rows), 0.71 (64x48), 0.70 (64x32), 0.80 (48x64), 0.82 (48x48), 0.89 (48x32), 0.90 (32x64), 0.78
 // (32x48), 0.80 (32x32), 1.4 (16x16): hence 96 rows of bf16 as 64 + 32 where the group has 64 columns, as 48 + 48 otherwise (96x96
 // B=8 T=2048 H=16, kernels of that time: 2155 us with 48 + 48 everywhere, 2055 so; 64x96 1299, 1202).)
 struct TileRect {
@@ -39,9 +39,9 @@ struct TileRect {
 constexpr int kRectColsBefore = 1, kRectRowsBefore = 2, kRectRowsAfter = 4, kRectParts = 8;   // launches that came before, come after; a small pass
 inline int tile_piece(int n) { return n == 80 ? 48 : n >= 64 ? 64 : n; }
 // fp32 rows: 64 columns by 64 rows and 48 or 32 columns by 48 or 64 take 87 KB of LDS or more than half of a unit's registers'
-// worth of waves, and one or two workgroups of them run on a compute unit; slices of 32 rows, twice as many (ps per entry 1.07
-// against 0.77 for 64 columns, 1.38 and 1.34 against 0.97 for 48, 1.53 and 1.35 against 1.07 for 32; us at 256 tiles of 8 heads,
-// 64x64 578 -> 463, 48x48 416 -> 340, 48x96 878 -> 628, 128x64 1169 -> 882, 64x64 with the uncertainty 819 -> 497).  48 rows would
+// worth of waves, and one or two workgroups of them run on a compute unit; slices of 32 rows, twice as many (ps per entry, when both
+// were launched, 1.07 against 0.77 for 64 columns, 1.38 and 1.34 against 0.97 for 48, 1.53 and 1.35 against 1.07 for 32; us at 256 tiles
+// of 8 heads, 64x64 578 -> 463, 48x48 416 -> 340, 48x96 878 -> 628, 128x64 1169 -> 882, 64x64 with the uncertainty 819 -> 497).  48 rows would
 // leave a slice of 16 and stay together where a pass has `few` tiles, one workgroup to a compute unit (whole / in slices, us, by
 // tiles x heads: 48x48 192 60 / 68, 256 59 / 68, 384 110 / 97, 512 113 / 110, 1024 217 / 185, with the uncertainty 256 73 / 73, 384 138 /
 // 108; 32x48 256 67 / 66, 384 89 / 72, 512 90 / 94, 1024 168 / 161).

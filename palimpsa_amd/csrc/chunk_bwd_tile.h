@@ -31,9 +31,9 @@
 // What bounds it: vector issue, of waves that are two to a SIMD (the registers).  By the counters 24 instructions per entry and
 // token at 64x64, 16 of them fp32 arithmetic of the entry and one a reciprocal, 7 for the sums over lanes, the recomputed states,
 // staging and the sums over waves; a wave alone issues one per 5 cycles, and waits (reads of LDS, barriers, what the other
-// wave has in the way) for two fifths of its time.  B=8 T=2048 H=12 64x64 564 -> 528 us, 48x48 H=16 549 -> 491, 48x96 4 x 1531 456 -> 393,
+// wave has in the way) for two fifths of its time.  B=8 T=2048 H=12 64x64 554 -> 515 us, 48x48 H=16 549 -> 491, 48x96 4 x 1531 456 -> 392,
 // packed 32768 tokens 96x96 4050 -> 3600 (plain form throughout -> this, with the fetches and stores below), with every tile in plain
-// form 554, 537, 433 and 3840; fp32 rows 64x64 H=8 604 -> 460 (slices of 32 value rows, fetches and stores), with the uncertainty bf16 64x64
+// form 552, 532, 428 and 3840; fp32 rows 64x64 H=8 604 -> 458 (slices of 32 value rows, fetches and stores), with the uncertainty bf16 64x64
 // H=8 512 -> 459.  As products on the matrix cores (12 prefix and 12 suffix instructions of 16 cycles per 16 entries of a lane, operands
 // exchanged through LDS between waves of different roles) the same pass took 822 us at 64x64.
 // Waits that the compiler places (counted in order, for loads and stores alike) cost more than instructions here: rows are
@@ -183,8 +183,8 @@ struct TokRev {
 constexpr float kMinStepDecay = 0x1p-48f, kMaxV = 0x1p20f, kMaxB = 0x1p4f, kMaxK = 0x1p4f, kMaxState = 0x1p16f;
 
 // Waves per SIMD that a lane's E state entries leave registers for.  Three entries (48 columns by 16 rows) take 131 to 136 and are held to
-// 128, for up to four spilled: 80x80 at 192 tiles x heads 138 -> 123 us, with the uncertainty 172 -> 154, at 384 242 -> 232; not where
-// that spills more (`four`: earlier launches' sums added, or fp32 rows with the uncertainty).
+// 128 (`four`), for up to four spilled: 80x80 at 192 tiles x heads 138 -> 123 us, with the uncertainty 172 -> 154, at 384 242 -> 232; but
+// not where that spills 14 to 27: earlier launches' sums added, fp32 rows with the uncertainty.
 constexpr int tile_waves(int E, bool four) { return E > 4 ? 2 : E == 3 && four ? 4 : 3; }
 
 template <typename TIn, int DT, int DN, int NBW, bool VAR, int SLICE>

@@ -23,8 +23,11 @@
 // be up to 0.5 % larger and that of the uncertainty 15 %, so fp32 rows and the uncertainty keep the plain form.  A walk
 // takes it where every eight tokens decay by less than 2^48, and is done again in plain form if a total is not finite
 // or a precision over F beyond 2^61 (then a product of two may have no reciprocal).  Plain form -> groups of
-// eight -> groups up to 64 and staging on all waves: 65536 tokens of 16 heads of 128x128 3060 -> 2805 -> 2750 us, 32768 of 16 of
-// 96x96 945 -> 871 -> 857, 8 x 2048 of 12 of 64x64 without a backward 168 -> 160 (the last step), of 16 of 48x48 144 -> 140.
+// eight -> groups up to 64 and staging on all waves: 65536 tokens of 16 heads of 128x128 3060 -> 2805 -> 2750 us (2820 with
+// states of segments to add up), 32768 of 16 of
+// 96x96 945 -> 871 -> 857, 8 x 2048 of 12 of 64x64 without a backward 168 -> 160 (the last step), of 16 of 48x48 144 -> 140.  (Two rows a lane are held
+// to four waves a SIMD: five, which 16 key columns would allow, leave some compute units 18 workgroups where an even share is 16 and the
+// fifth wave without a partner: 8 x 2048, 16 heads of 16x16 40.5 -> 45.4 us.)
 // (112 vector instructions a token for a lane's 16 entries at 64x64, 96 of them the entries' own; a step of eight tokens adds
 // 60 for staging.  Four rows a lane halve the reads of LDS and the totals over the lanes, but leave two waves per SIMD: 193 us at 64x64.)
 //
